@@ -14,9 +14,8 @@
 //   3. Gram matrix per sector on the grouped MFMA GEMM: A*A^T for
 //      MoveFromLeft (the left factor U is what must be orthonormal),
 //      A^T*A for MoveFromRight;
-//   4. one workgroup per sector: parallel cyclic Jacobi eigensolver
-//      (round-robin pairs, packed upper triangle in LDS when it fits) with
-//      the eigenvectors accumulated in HBM;  s = sqrt(max(lambda, 0));
+//   4. Jacobi eigensolver per sector: one workgroup for up to 64 rows, block
+//      Jacobi over workgroups above;  s = sqrt(max(lambda, 0));
 //   5. truncation on the device: per-sector rank-K cap, sum of s^2 and the
 //      sequential cumsum rule in one thread, in the reference's order;
 //   6. the absorbed factor as a second grouped GEMM (U^T A or A V), then the
@@ -28,6 +27,7 @@
 
 #include "ttg_device.h"
 #include "ttg_internal.h"
+#include "ttg_jacobi.h"
 #include "ttg_plan.h"
 
 namespace ttg {
@@ -196,12 +196,9 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
   }
 }
 
-// 4. parallel cyclic Jacobi, one workgroup per sector.  n even (padded with
-// a zero row/column when odd; the pad never rotates).  Packed upper triangle
-// (i <= j at j(j+1)/2 + i).  Dynamic LDS holds, when they fit: the triangle,
-// the eigenvector matrix V and the table of 2x2 block pairs of a round;
-// otherwise V, then also the triangle, live in HBM (scratch / output).
-// A sweep converges when no rotation is significant: |a_pq| above 1e-12 of
+// 4. sectors of up to 64 rows: one workgroup per sector sweeps (ttg_jacobi.h)
+// the matrix, padded with zeros to 16, 32 or 64 (the padding never rotates), in
+// LDS until a sweep holds no significant rotation: |a_pq| above 1e-12 of
 // sqrt(a_pp a_qq) (an off-diagonal d moves eigenvalues by ~d^2 / gap, so
 // the eigenvalues are exact to ~1e-24 relative) and above 1e-14 of the
 // largest diagonal.  Below that floor
@@ -209,170 +206,69 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // values below 1e-7 of the largest, under the Gram matrix's own resolution of
 // ~sqrt(eps)), and the rounding noise in the null space of a rank-deficient
 // sector's Gram matrix never passes the relative test alone.
-constexpr int kJacThreads = 1024;
 constexpr double kJacFloor = 1e-14;   // convergence floor relative to the largest diagonal
-constexpr int kLdsDoubles = 20000;   // dynamic LDS (160 000 B of the CU's 160 KiB)
 
-__device__ inline int pk(int i, int j) { return i <= j ? j * (j + 1) / 2 + i : i * (i + 1) / 2 + j; }
-
-// LDS placement of one sector of size n (doubles): rotation arrays always;
-// then the packed triangle, V and the pair table in that priority.  Bit 0 of
-// *where: triangle in LDS, bit 1: V in LDS, bit 2: pair table in LDS.
-struct JacLayout {
-  int64_t rot, tri, v, tab, total;
-  int where;
-};
-__host__ __device__ inline JacLayout jac_layout(int n) {
-  const int64_t np = n + (n & 1), npair = np / 2;
-  JacLayout L;
-  L.rot = 3 * npair;   // c, s (doubles) and the (p, q) pairs (two ints)
-  L.tri = np * (np + 1) / 2;
-  L.v = (int64_t)n * n;
-  L.tab = (npair * (npair + 1) / 2 + 1) / 2;
-  L.where = 0;
-  int64_t used = L.rot;
-  if (used + L.tri <= kLdsDoubles) { used += L.tri; L.where |= 1; }
-  if (used + L.v <= kLdsDoubles) { used += L.v; L.where |= 2; }
-  if (used + L.tab <= kLdsDoubles) { used += L.tab; L.where |= 4; }
-  L.total = used;
-  return L;
-}
-
-__device__ inline void tri_index(int64_t w, int& i, int& j) {   // w -> (i <= j)
-  j = (int)((sqrt(8.0 * (double)w + 1.0) - 1.0) / 2.0);
-  while ((int64_t)j * (j + 1) / 2 > w) j--;
-  while ((int64_t)(j + 1) * (j + 2) / 2 <= w) j++;
-  i = (int)(w - (int64_t)j * (j + 1) / 2);
-}
-
-__global__ void __launch_bounds__(kJacThreads)
-k_jacobi(const int* __restrict__ nq, const int64_t* __restrict__ goff,
-         const double* __restrict__ Gin, double* __restrict__ gscratch,
-         const int64_t* __restrict__ poff, double* __restrict__ Vout,
-         double* __restrict__ evals, const int64_t* __restrict__ eoff, int max_sweeps,
-         int nmax_here, double floor_rel) {
-  extern __shared__ double lds_g[];
-  __shared__ int any_rot;
-  __shared__ double red[kJacThreads / 64];
-  const int q = blockIdx.x;
-  const int n = nq[q];                 // true size
-  if (n == 0 || n > nmax_here) return;   // larger sectors: block Jacobi
-  const int np = n + (n & 1);          // padded even size
-  const int npair = np / 2;
-  const int64_t psize = (int64_t)np * (np + 1) / 2;
-  const int nblk = npair * (npair + 1) / 2;
-  const JacLayout lay = jac_layout(n);
-  double* cs_c = lds_g;
-  double* cs_s = lds_g + npair;
-  int* pp = (int*)(lds_g + 2 * npair);
-  int* qq = pp + npair;
-  double* next = lds_g + lay.rot;
-  double* g = (lay.where & 1) ? next : gscratch + poff[q];
-  if (lay.where & 1) next += psize;
-  double* Vg = Vout + goff[q];         // n x n column-major eigenvectors (output)
-  double* V = (lay.where & 2) ? next : Vg;
-  if (lay.where & 2) next += (int64_t)n * n;
-  int* tab = (lay.where & 4) ? (int*)next : nullptr;
-  const double* G0 = Gin + goff[q];    // full n x n column-major
-  // load packed triangle (pad row/col zero), V = I, block-pair table
+template <int NPR>
+__device__ __forceinline__ void jacobi_sector(double* S, double* Qts, int* sig, double* red, int n, const double* G0,
+                                              double* Vg, double* ev, int max_sweeps, double floor_rel) {
+  constexpr int W = 16 * NPR;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 #pragma unroll 8
-  for (int64_t e = threadIdx.x; e < psize; e += blockDim.x) {
-    int i, j;
-    tri_index(e, i, j);
-    g[e] = (i < n && j < n) ? 0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]) : 0.0;
+  for (int e = tid; e < W * W; e += kJThreads) {
+    const int i = e % W, j = e / W;
+    S[j * kJP + i] = (i < n && j < n) ? 0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]) : 0.0;
   }
-  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += blockDim.x)
-    V[e] = (e % n == e / n) ? 1.0 : 0.0;
-  if (tab)
-    for (int w = threadIdx.x; w < nblk; w += blockDim.x) {
-      int k1, k2;
-      tri_index(w, k1, k2);
-      tab[w] = k1 | (k2 << 16);
-    }
-  // largest diagonal element: the scale of the convergence floor
-  double dmax = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x)
-    dmax = fmax(dmax, fabs(G0[i + (int64_t)n * i]));
-  for (int o = 32; o > 0; o >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dmax;
+  double vt[2 * NPR][2];
+  jac_identity<NPR>(vt, wave, lane);
   __syncthreads();
-  dmax = 0.0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); i++) dmax = fmax(dmax, red[i]);
-  const double floor_abs = floor_rel * dmax;
-  const int m1 = np - 1;
+  if (wave == 0) {   // largest diagonal element: the scale of the convergence floor
+    double m = lane < W ? fabs(S[lane * kJP + lane]) : 0.0;
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    if (lane == 0) *red = m;
+  }
+  int par = 0;
   for (int sweep = 0; sweep < max_sweeps; sweep++) {
-    if (threadIdx.x == 0) any_rot = 0;
+    if (tid == 0) *sig = 0;
     __syncthreads();
-    for (int round = 0; round < m1; round++) {
-      // circle method: player m1 fixed, pairs (round, m1) and (round+k, round-k)
-      for (int k = threadIdx.x; k < npair; k += blockDim.x) {
-        int a, b;
-        if (k == 0) { a = round; b = m1; }
-        else { a = (round + k) % m1; b = (round - k + m1) % m1; }
-        if (a > b) { int t = a; a = b; b = t; }
-        pp[k] = a;
-        qq[k] = b;
-        const double app = g[pk(a, a)], aqq = g[pk(b, b)], apq = g[pk(a, b)];
-        double c = 1.0, s = 0.0;
-        if (apq != 0.0) {
-          if (fabs(apq) > 1e-12 * sqrt(fabs(app * aqq)) && fabs(apq) > floor_abs) any_rot = 1;
-          const double theta = (aqq - app) / (2.0 * apq);
-          const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-          c = 1.0 / sqrt(t * t + 1.0);
-          s = t * c;
-        }
-        cs_c[k] = c;
-        cs_s[k] = s;
-      }
-      __syncthreads();
-      // G <- J^T G J over 2x2 blocks (k1 <= k2) of the packed triangle
-      for (int w = threadIdx.x; w < nblk; w += blockDim.x) {
-        int k1, k2;
-        if (tab) { k1 = tab[w] & 0xffff; k2 = tab[w] >> 16; }
-        else tri_index(w, k1, k2);
-        const int a = pp[k1], b = qq[k1], c2i = pp[k2], d = qq[k2];
-        const double c1 = cs_c[k1], s1 = cs_s[k1], c2 = cs_c[k2], s2 = cs_s[k2];
-        if (k1 == k2) {
-          const double gaa = g[pk(a, a)], gab = g[pk(a, b)], gbb = g[pk(b, b)];
-          // rows then columns of the symmetric 2x2 block
-          const double ra0 = c1 * gaa - s1 * gab, ra1 = c1 * gab - s1 * gbb;
-          const double rb0 = s1 * gaa + c1 * gab, rb1 = s1 * gab + c1 * gbb;
-          g[pk(a, a)] = c1 * ra0 - s1 * ra1;
-          g[pk(a, b)] = s1 * ra0 + c1 * ra1;
-          g[pk(b, b)] = s1 * rb0 + c1 * rb1;
-        } else {
-          const int iac = pk(a, c2i), iad = pk(a, d), ibc = pk(b, c2i), ibd = pk(b, d);
-          const double gac = g[iac], gad = g[iad], gbc = g[ibc], gbd = g[ibd];
-          const double ra_c = c1 * gac - s1 * gbc, ra_d = c1 * gad - s1 * gbd;
-          const double rb_c = s1 * gac + c1 * gbc, rb_d = s1 * gad + c1 * gbd;
-          g[iac] = c2 * ra_c - s2 * ra_d;
-          g[iad] = s2 * ra_c + c2 * ra_d;
-          g[ibc] = c2 * rb_c - s2 * rb_d;
-          g[ibd] = s2 * rb_c + c2 * rb_d;
-        }
-      }
-      // V <- V J (columns of real indices only)
-      for (int w = threadIdx.x; w < npair * n; w += blockDim.x) {
-        const int k = w / n, i = w % n;
-        const int a = pp[k], b = qq[k];
-        if (b >= n) continue;   // pad never rotates (apq == 0)
-        const double c = cs_c[k], s = cs_s[k];
-        const double va = V[i + (int64_t)n * a], vb = V[i + (int64_t)n * b];
-        V[i + (int64_t)n * a] = c * va - s * vb;
-        V[i + (int64_t)n * b] = s * va + c * vb;
-      }
-      __syncthreads();
-    }
+    jac_sweep<NPR>(S, Qts, vt, wave, lane, par, floor_rel * *red, sig);
+    __syncthreads();
     // every thread reads the flag before thread 0 may clear it for the next
     // sweep: the barrier between the read and the reset keeps the decision
     // uniform over the workgroup
-    const int rotated = any_rot;
+    const int rotated = *sig;
     __syncthreads();
     if (!rotated) break;
   }
-  for (int i = threadIdx.x; i < n; i += blockDim.x) evals[eoff[q] + i] = g[pk(i, i)];
-  if (lay.where & 2)
-    for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += blockDim.x) Vg[e] = V[e];
+  for (int i = tid; i < n; i += kJThreads) ev[i] = S[i * kJP + i];
+  if (wave >= 4) {   // V(i, c) = V^T(c, i): consecutive lanes down a column of V
+    const int i = 16 * (wave - 4) + (lane & 15);
+#pragma unroll
+    for (int b = 0; b < 2 * NPR; b++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int c = 8 * b + (lane >> 4) + 4 * h;
+        if (i < n && c < n) Vg[i + (int64_t)n * c] = vt[b][h];
+      }
+  }
+}
+
+__global__ void __launch_bounds__(kJThreads)
+k_jacobi(const int* __restrict__ nq, const int64_t* __restrict__ goff, const double* __restrict__ Gin,
+         double* __restrict__ Vout, double* __restrict__ evals, const int64_t* __restrict__ eoff, int max_sweeps,
+         int nmax_here, double floor_rel) {
+  __shared__ __attribute__((aligned(16))) double lds[kJLds];
+  __shared__ double red;
+  __shared__ int sig;
+  const int q = blockIdx.x;
+  const int n = nq[q];
+  if (n == 0 || n > nmax_here) return;   // larger sectors: block Jacobi
+  const double* G0 = Gin + goff[q];      // full n x n column-major
+  double* Vg = Vout + goff[q];           // eigenvectors, the same layout
+  double* ev = evals + eoff[q];
+  double* Qts = lds + kJS;
+  if (n <= 16) jacobi_sector<1>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
+  else if (n <= 32) jacobi_sector<2>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
+  else jacobi_sector<4>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
 }
 
 // 4b. Sectors larger than kJacBlockMin: two-sided block Jacobi.  The padded
@@ -390,8 +286,7 @@ k_jacobi(const int* __restrict__ nq, const int64_t* __restrict__ goff,
 // above the sector's floor, 1e-14 of the largest diagonal.  A subproblem
 // with nothing to rotate leaves Q_IJ = I and marks its pair unrotated; the
 // tile products of a round skip the tiles whose pairs were both unrotated.
-constexpr int kJacBlockMin = 64;
-constexpr double kBJRel = 1e-12;
+constexpr int kJacBlockMin = kJW;
 constexpr int kBJ = 32;                // block width; subproblems are 2 kBJ
 constexpr int kSub = 2 * kBJ;
 
@@ -450,80 +345,22 @@ __global__ void k_bjac_init(const BJSector* sec, int nsec, const int64_t* goff, 
   }
 }
 
-// Jacobi rotation zeroing a_pq of [[app, apq], [apq, aqq]]: rows/columns
-// (p, q) <- (c x_p - s x_q, s x_p + c x_q), t = s/c the smaller root of
-// t^2 + 2 theta t - 1 = 0, theta = (aqq - app) / (2 apq).  Reciprocal and
-// reciprocal square root from the hardware estimates with two Newton steps
-// each (full double precision; c^2 + s^2 = 1 to rounding).
-__device__ inline double rcp_nr(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  double e = fma(-b, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-b, r, 1.0);
-  return fma(r, e, r);
-}
-__device__ inline double rsq_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  double e = fma(-x * y, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  e = fma(-x * y, y, 1.0);
-  return fma(0.5 * y, e, y);
-}
-__device__ inline void jac_rotation(double app, double aqq, double apq, double& c, double& s) {
-  c = 1.0;
-  s = 0.0;
-  if (!(fabs(apq) > 1e-290)) return;   // nothing to rotate (and no overflow below)
-  const double theta = (aqq - app) * (0.5 * rcp_nr(apq));
-  const double at = fabs(theta);
-  double t;
-  if (at < 1e150) {
-    const double h = fma(theta, theta, 1.0);
-    t = rcp_nr(at + h * rsq_nr(h));
-  } else {
-    t = 0.5 * rcp_nr(at);
-  }
-  if (theta < 0) t = -t;
-  c = rsq_nr(fma(t, t, 1.0));
-  s = t * c;
-}
-
-// one workgroup per (sector, pair): the 64 x 64 subproblem, one cyclic
-// sweep of 63 rounds of 32 disjoint rotations (circle method), in slot
-// order: slot k holds the pair of round r at positions (2k, 2k+1), so every
-// rotation acts on adjacent rows and columns.  Between rounds the indices
-// move by the fixed permutation slot_next (period 63); a round reads S and
-// Q^T from one buffer and writes the rotated values to their next-round
-// positions in the other.  A round, one barrier:
-//   1. every wave: lane k < 32 computes the rotation of slot k from its 2x2
-//      diagonal block (the four waves compute the same values from the same
-//      LDS words), and each thread takes the rotations it needs from those
-//      lanes by cross-lane shuffles, so no rotation table passes through LDS;
-//   2. all threads: S <- M S M^T (thread t: rows 2k, 2k+1, k = t/8, and the
-//      column pairs k' = t%8 + 8u) and Q^T <- M Q^T (the same rows).
-constexpr int kSP = 72;                    // LDS row pitch (doubles) of S and Q^T
-constexpr int kSlotMat = kSub * kSP;
-constexpr size_t kSolveLds = 4 * kSlotMat * sizeof(double) + (2 * kSub + 1) * sizeof(int);
-__device__ inline int slot_of(int x) { return x < kBJ ? 2 * x : 2 * (kSub - 1 - x) + 1; }
-__device__ inline int slot_next(int p) {
-  const int k = p >> 1;
-  if (!(p & 1)) return k ? 2 * (k - 1) : 3;
-  if (k == 0) return 1;
-  return k < kBJ - 1 ? 2 * k + 3 : 2 * kBJ - 2;
-}
-
-constexpr int kSolveThreads = 256;
-__global__ void __launch_bounds__(kSolveThreads)
+// one workgroup per (sector, pair): the 64 x 64 subproblem, one cyclic sweep
+// (ttg_jacobi.h)
+static_assert(kSub == kJW, "a subproblem is one Jacobi matrix");
+__global__ void __launch_bounds__(kJThreads)
 k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const int* active, int* flag,
              int* rotated, const double* Gp, double* Qp) {
-  extern __shared__ __attribute__((aligned(16))) double bj_lds[];
-  int* perm = (int*)(bj_lds + 4 * kSlotMat);
-  int* cnt = perm + kSub;
-  int* sig = cnt + kSub;
+  __shared__ __attribute__((aligned(16))) double lds[kJLds];
+  __shared__ int perm[kSub], cnt[kSub];
+  __shared__ int sig;
   const int2 it = items[blockIdx.x];
   const int li = it.x, k = it.y;
   const BJSector S = sec[li];
   if (!active[li] || r >= S.nbk - 1) return;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double* M = lds;
+  double* Qts = lds + kJS;
   // the pair's two blocks (uniform): subproblem entry t is global index
   // (t < 32 ? ba : bb) * 32 + t % 32; the sector's own indices (global index
   // < n) are entries [0, na) and [32, 32 + nbb)
@@ -532,47 +369,43 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
   const int na = min(max(S.n - kBJ * ba, 0), kBJ), nbb = min(max(S.n - kBJ * bb, 0), kBJ);
   auto gidx = [&](int t) { return (t >= kBJ ? bb : ba) * kBJ + (t & (kBJ - 1)); };
   auto own = [&](int t) { return t < kBJ ? t < na : t - kBJ < nbb; };
-  if (tid == 0) *sig = 0;
+  if (tid == 0) sig = 0;
   if (tid < kSub) cnt[tid] = 0;
   {
     // all of a thread's loads are issued before the first LDS store (a loop
     // with one load per iteration would wait one memory latency per entry)
-    constexpr int kPer = kSub * kSub / kSolveThreads;
-    double* S0 = bj_lds;
-    double* Q0 = bj_lds + 2 * kSlotMat;
+    constexpr int kPer = kSub * kSub / kJThreads;
     double gv[kPer];
 #pragma unroll
     for (int u = 0; u < kPer; u++) {
-      const int e = tid + kSolveThreads * u, i = e % kSub, j = e / kSub;   // G is exactly symmetric
+      const int e = tid + kJThreads * u, i = e % kSub, j = e / kSub;   // G is exactly symmetric
       gv[u] = Gp[S.gp + gidx(i) + (int64_t)S.N * gidx(j)];
     }
 #pragma unroll
     for (int u = 0; u < kPer; u++) {
-      const int e = tid + kSolveThreads * u, i = e % kSub, j = e / kSub;
-      S0[slot_of(i) * kSP + slot_of(j)] = gv[u];
-      Q0[slot_of(j) * kSP + i] = i == j ? 1.0 : 0.0;
+      const int e = tid + kJThreads * u, i = e % kSub, j = e / kSub;
+      M[j * kJP + i] = gv[u];
     }
   }
   __syncthreads();
   {
     // significance test of this subproblem (before rotating):
-    // |v| > 1e-12 sqrt(g_pp g_qq), compared squared; thread t's rows p are
-    // all t % 64 (so one diagonal load), its columns q = t / 64 + 4 i
-    const double* S0 = bj_lds;
+    // |v| > 1e-12 sqrt(g_pp g_qq), compared squared; thread t's columns p are
+    // all t % 64 (so one diagonal load), its rows q = t / 64 + 8 i
     const int p = tid % kSub;
-    const double gpp = S0[p * kSP + p];
+    const double gpp = M[p * kJP + p];
     bool any = false;
-    for (int q = tid / kSub; q < kSub; q += kSolveThreads / kSub) {
+    for (int q = tid / kSub; q < kSub; q += kJThreads / kSub) {
       if (p == q) continue;
-      const double v = S0[p * kSP + q];
-      any |= v * v > (kBJRel * kBJRel) * fabs(gpp * S0[q * kSP + q]) && fabs(v) > S.floor;
+      const double v = M[q * kJP + p];
+      any |= v * v > (kJacRel * kJacRel) * fabs(gpp * M[q * kJP + q]) && fabs(v) > S.floor;
     }
-    if (any) *sig = 1;
+    if (any) sig = 1;
   }
   __syncthreads();
   double* Qg = Qp + S.qp + (int64_t)k * kSub * kSub;   // column-major 64 x 64
-  if (!*sig) {   // already diagonal: Q = I
-    for (int e = tid; e < kSub * kSub; e += kSolveThreads) Qg[e] = (e % kSub == e / kSub) ? 1.0 : 0.0;
+  if (!sig) {   // already diagonal: Q = I
+    for (int e = tid; e < kSub * kSub; e += kJThreads) Qg[e] = (e % kSub == e / kSub) ? 1.0 : 0.0;
     if (tid == 0) rotated[blockIdx.x] = 0;
     return;
   }
@@ -580,83 +413,28 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
     atomicOr(&flag[li], 1);
     rotated[blockIdx.x] = 1;
   }
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  const int kk = tid >> 3, c8 = tid & 7, lane = tid & 63;
-  const int r0 = 2 * kk, r1 = 2 * kk + 1;
-  const int nr0 = slot_next(r0) * kSP, nr1 = slot_next(r1) * kSP;
-  int ncol[4][2];
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    ncol[u][0] = slot_next(2 * c8 + 16 * u);
-    ncol[u][1] = slot_next(2 * c8 + 16 * u + 1);
-  }
-  for (int round = 0; round < kSub - 1; round++) {
-    const double* Sc = bj_lds + (round & 1) * kSlotMat;
-    double* Sn = bj_lds + ((round & 1) ^ 1) * kSlotMat;
-    const double* Qc = bj_lds + (2 + (round & 1)) * kSlotMat;
-    double* Qn = bj_lds + (2 + ((round & 1) ^ 1)) * kSlotMat;
-    // lane k (k < 32) of every wave: the rotation of slot k from its 2x2
-    // diagonal block; lanes 32..63 compute slot k - 32 again (same words, no
-    // divergence).  The block's three words are read before the round's S and
-    // Q^T rows (the scheduling barriers keep that order), so the rotation's
-    // arithmetic runs while those 16 reads stream in.
-    d2 x0[4], x1[4], q0[4], q1[4], cp[4];
-    const int pd = 2 * (lane & (kBJ - 1));
-    const double app = Sc[pd * kSP + pd], aqq = Sc[(pd + 1) * kSP + pd + 1], apq = Sc[pd * kSP + pd + 1];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      x0[u] = *(const d2*)&Sc[r0 * kSP + 2 * c8 + 16 * u];
-      x1[u] = *(const d2*)&Sc[r1 * kSP + 2 * c8 + 16 * u];
-      q0[u] = *(const d2*)&Qc[r0 * kSP + 2 * c8 + 16 * u];
-      q1[u] = *(const d2*)&Qc[r1 * kSP + 2 * c8 + 16 * u];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    double cl, sl;
-    jac_rotation(app, aqq, apq, cl, sl);
-#pragma unroll
-    for (int u = 0; u < 4; u++) cp[u] = d2{__shfl(cl, c8 + 8 * u), __shfl(sl, c8 + 8 * u)};
-    const double c1 = __shfl(cl, kk), s1 = __shfl(sl, kk);
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      // rows 2k, 2k+1 of the 2x2 block (k, k' = c8 + 8u), then its columns
-      const double y00 = c1 * x0[u].x - s1 * x1[u].x, y01 = c1 * x0[u].y - s1 * x1[u].y;
-      const double y10 = s1 * x0[u].x + c1 * x1[u].x, y11 = s1 * x0[u].y + c1 * x1[u].y;
-      const double c2 = cp[u].x, s2 = cp[u].y;
-      double z00 = c2 * y00 - s2 * y01, z01 = s2 * y00 + c2 * y01;
-      double z10 = c2 * y10 - s2 * y11, z11 = s2 * y10 + c2 * y11;
-      if (c8 + 8 * u == kk) { z01 = 0.0; z10 = 0.0; }   // the pair's own element is rotated away
-      Sn[nr0 + ncol[u][0]] = z00;
-      Sn[nr0 + ncol[u][1]] = z01;
-      Sn[nr1 + ncol[u][0]] = z10;
-      Sn[nr1 + ncol[u][1]] = z11;
-      *(d2*)&Qn[nr0 + 2 * c8 + 16 * u] = c1 * q0[u] - s1 * q1[u];
-      *(d2*)&Qn[nr1 + 2 * c8 + 16 * u] = s1 * q0[u] + c1 * q1[u];
-    }
-    __syncthreads();
-  }
-  // 63 rounds return every index to its first slot; the result is in buffer 1.
+  double vt[8][2];
+  jac_identity<4>(vt, wave, lane);
+  int par = 0;
+  jac_sweep<4>(M, Qts, vt, wave, lane, par, S.floor, &sig);
   // Eigenpairs in descending order (the larger values to the pair's lower
   // block): a fixed order keeps values from swapping between blocks from
   // round to round, which otherwise holds the outer iteration at a linear rate.
   // Only the sector's own indices are ordered, over their own positions; a
   // padding index (global index >= n, never rotated) keeps its column, so no
   // eigenvector moves into the padding that k_bjac_finish drops.
-  const double* Sf = bj_lds + kSlotMat;
-  const double* Qf = bj_lds + 3 * kSlotMat;
   {
     // rank of own entry x among the own entries (descending eigenvalue,
-    // ties to the lower entry), counted by the four waves over a quarter of
+    // ties to the lower entry), counted by the eight waves over an eighth of
     // the entries each
     const int x = tid % kSub, part = tid / kSub;
     if (own(x)) {
-      const double d = Sf[slot_of(x) * kSP + slot_of(x)];
+      const double d = M[x * kJP + x];
       int c = 0;
-      for (int u = 16 * part; u < 16 * part + 16; u++) {
-        if (!own(u)) continue;
-        const int pu = slot_of(u);
-        const double du = Sf[pu * kSP + pu];
-        c += (du > d) || (du == d && u < x);
+#pragma unroll
+      for (int u = 8 * part; u < 8 * part + 8; u++) {
+        const double du = M[u * kJP + u];
+        c += own(u) && ((du > d) || (du == d && u < x));
       }
       if (c) atomicAdd(&cnt[x], c);
     }
@@ -671,12 +449,15 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
       const int rk = cnt[x];
       dst = rk < na ? rk : kBJ + (rk - na);
     }
-    perm[slot_of(x)] = dst;   // column of Q for the eigenvector in slot slot_of(x)
+    perm[x] = dst;   // column of Q for the eigenvector of entry x
   }
   __syncthreads();
-  for (int e = tid; e < kSub * kSub; e += kSolveThreads) {
-    const int i = e % kSub, p = e / kSub;
-    Qg[i + kSub * perm[p]] = Qf[p * kSP + i];
+  if (wave >= 4) {   // Q(i, perm(c)) = V^T(c, i)
+    const int i = 16 * (wave - 4) + (lane & 15);
+#pragma unroll
+    for (int b = 0; b < 8; b++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) Qg[i + kSub * perm[8 * b + (lane >> 4) + 4 * h]] = vt[b][h];
   }
 }
 
@@ -876,8 +657,6 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
   TTG_TRY(h2d_vec(d_pit, pitems));
   TTG_TRY(h2d_vec(d_tit, titems));
   TTG_TRY(h2d_vec(act, hact));
-  TTG_HIP(hipFuncSetAttribute((const void*)k_bjac_solve, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kSolveLds));
   // largest diagonal per sector and the convergence floor, on the device
   if (floor_rel > 0)
     hipLaunchKernelGGL(k_bjac_floor, dim3(ns), dim3(256), 0, s, d_sec, ns, d_goff, G, floor_rel);
@@ -894,7 +673,7 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
   int sweep = 0;
   for (; sweep < max_sweeps; sweep++) {
     for (int r = 0; r < maxr; r++) {
-      hipLaunchKernelGGL(k_bjac_solve, dim3((unsigned)pitems.size()), dim3(kSolveThreads), kSolveLds, s, d_sec, d_pit,
+      hipLaunchKernelGGL(k_bjac_solve, dim3((unsigned)pitems.size()), dim3(kJThreads), 0, s, d_sec, d_pit,
                          (int)pitems.size(), r, act, flag, rot, Gp, Qp);
       hipLaunchKernelGGL(k_bjac_apply, dim3((unsigned)titems.size()), dim3(256), 0, s, d_sec, d_tit,
                          (int)titems.size(), r, act, rot, Gp, Vp, Qp);
@@ -1610,31 +1389,26 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
     prev_panels = std::min(need, all_panels);
   }
   std::vector<int> r2(ns);
-  std::vector<int64_t> goff2(ns + 1, 0), poff2(ns + 1, 0), eoff2(ns + 1, 0);
-  int64_t lds_need = 1;
+  std::vector<int64_t> goff2(ns + 1, 0), eoff2(ns + 1, 0);
   bool any_small = false;
   std::vector<int> big2;
   for (int li = 0; li < ns; li++) {
     const int r = rk[li] < 0 ? ps[li].n : rk[li];
     r2[li] = r;
     goff2[li + 1] = goff2[li] + (int64_t)r * r;
-    const int64_t np = r + (r & 1);
-    poff2[li + 1] = poff2[li] + np * (np + 1) / 2;
     eoff2[li + 1] = eoff2[li] + r;
     if (r > kJacBlockMin) big2.push_back(li);
-    else if (r > 0) { any_small = true; lds_need = std::max(lds_need, jac_layout(r).total); }
+    else if (r > 0) any_small = true;
   }
   double* G2 = sc.get<double>(std::max<int64_t>(1, goff2[ns]));
   double* W2 = sc.get<double>(std::max<int64_t>(1, goff2[ns]));
-  double* gs2 = sc.get<double>(std::max<int64_t>(1, poff2[ns]));
   double* ev2 = sc.get<double>(std::max<int64_t>(1, eoff2[ns]));
   TTG_TRY(sc.ok("svd: LR step"));
   Pack pk;
-  const size_t o_r2 = pk.add(r2), o_goff2 = pk.add(goff2), o_poff2 = pk.add(poff2), o_eoff2 = pk.add(eoff2);
+  const size_t o_r2 = pk.add(r2), o_goff2 = pk.add(goff2), o_eoff2 = pk.add(eoff2);
   TTG_TRY(pk.upload(sc, "svd: LR step"));
   int* d_r2 = pk.at<int>(o_r2);
   int64_t* d_goff2 = pk.at<int64_t>(o_goff2);
-  int64_t* d_poff2 = pk.at<int64_t>(o_poff2);
   int64_t* d_eoff2 = pk.at<int64_t>(o_eoff2);
   // G' = R R^T: A(k, j) = R[k n + j], B(j, k') = R[k' n + j]
   {
@@ -1650,11 +1424,8 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
   }
   // eigenpairs of G' (relative convergence test only)
   if (any_small) {
-    const size_t lb = sizeof(double) * (size_t)std::min<int64_t>(lds_need, kLdsDoubles);
-    TTG_HIP(hipFuncSetAttribute((const void*)k_jacobi, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * kLdsDoubles)));
-    hipLaunchKernelGGL(k_jacobi, dim3(ns), dim3(256), lb, s, d_r2, d_goff2, G2, gs2, d_poff2, W2, ev2,
-                       d_eoff2, 40, kJacBlockMin, 0.0);
+    hipLaunchKernelGGL(k_jacobi, dim3(ns), dim3(kJThreads), 0, s, d_r2, d_goff2, G2, W2, ev2, d_eoff2, 40,
+                       kJacBlockMin, 0.0);
     TTG_HIP(hipGetLastError());
   }
   if (!big2.empty()) TTG_TRY(block_jacobi(big2, r2, d_goff2, d_eoff2, G2, W2, ev2, s, 40, 0.0));
@@ -1746,7 +1517,7 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   tab(t.qR1, qR1.data(), sizeof(int));
   // ---- host layout of the per-sector work arrays
   const bool fromLeft = direction == TTG_MOVE_FROM_LEFT;
-  std::vector<int64_t> moff(nQ + 1, 0), goff(nQ + 1, 0), poff(nQ + 1, 0), eoff(nQ + 1, 0);
+  std::vector<int64_t> moff(nQ + 1, 0), goff(nQ + 1, 0), eoff(nQ + 1, 0);
   std::vector<int> nq(nQ), kq(nQ);
   for (int q = 0; q < nQ; q++) {
     const int64_t n = fromLeft ? rows[q] : cols[q];
@@ -1756,8 +1527,6 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
     kq[q] = K > 0 ? (int)std::min<int64_t>(K, kd) : kd;   // rank-K SVD per sector
     moff[q + 1] = moff[q] + rows[q] * cols[q];
     goff[q + 1] = goff[q] + n * n;
-    const int64_t np = n + (n & 1);
-    poff[q + 1] = poff[q] + np * (np + 1) / 2;
     eoff[q + 1] = eoff[q] + n;
   }
   std::vector<int64_t> soff(nQ + 1, 0), selo(nQ + 1, 0);
@@ -1768,7 +1537,6 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   double* mat = sc.get<double>(moff[nQ]);
   double* G = sc.get<double>(goff[nQ]);
   double* Vev = sc.get<double>(goff[nQ]);
-  double* gs = sc.get<double>(poff[nQ]);
   double* ev = sc.get<double>(eoff[nQ]);
   double* Esel = sc.get<double>(selo[nQ]);
   int* selidx = sc.get<int>(soff[nQ]);
@@ -1780,12 +1548,11 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   double* tout = sc.get<double>(2);
   TTG_TRY(sc.ok("svd"));
   Pack pk;
-  const size_t o_moff = pk.add(moff), o_goff = pk.add(goff), o_poff = pk.add(poff), o_eoff = pk.add(eoff),
+  const size_t o_moff = pk.add(moff), o_goff = pk.add(goff), o_eoff = pk.add(eoff),
                o_soff = pk.add(soff), o_selo = pk.add(selo), o_nq = pk.add(nq), o_kq = pk.add(kq);
   TTG_TRY(pk.upload(sc, "svd"));
   int64_t* d_moff = pk.at<int64_t>(o_moff);
   int64_t* d_goff = pk.at<int64_t>(o_goff);
-  int64_t* d_poff = pk.at<int64_t>(o_poff);
   int64_t* d_eoff = pk.at<int64_t>(o_eoff);
   int64_t* d_soff = pk.at<int64_t>(o_soff);
   int64_t* d_selo = pk.at<int64_t>(o_selo);
@@ -1823,30 +1590,23 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   }
   // ---- 4. eigensolver
   std::vector<int> big;
-  int64_t lds_need = 1;
   int nsmall = 0;
   for (int q = 0; q < nQ; q++) {
     if (nq[q] > kJacBlockMin) { big.push_back(q); continue; }
-    lds_need = std::max(lds_need, jac_layout(nq[q]).total);
     nsmall = std::max(nsmall, nq[q]);
   }
   // The small sectors' one-workgroup Jacobi runs on the side stream, beside
   // the large sectors' solver on the main stream: the two read and write
-  // disjoint sector ranges of G, the packed triangles, Vev and ev.
+  // disjoint sector ranges of G, Vev and ev.
   bool forked = false;
   if (nsmall > 0) {
-    const size_t lds_bytes = sizeof(double) * (size_t)std::min<int64_t>(lds_need, kLdsDoubles);
-    TTG_HIP(hipFuncSetAttribute((const void*)k_jacobi, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(sizeof(double) * kLdsDoubles)));
-    // small sectors: fewer waves per workgroup (cheaper barriers per round)
-    const int jac_threads = nsmall <= 96 ? 256 : kJacThreads;
     hipStream_t js = s;
     if (!big.empty()) {
       TTG_TRY(side_fork(&js));
       forked = true;
     }
-    hipLaunchKernelGGL(k_jacobi, dim3(nQ), dim3(jac_threads), lds_bytes, js, d_nq, d_goff, G, gs,
-                       d_poff, Vev, ev, d_eoff, 40, kJacBlockMin, kJacFloor);
+    hipLaunchKernelGGL(k_jacobi, dim3(nQ), dim3(kJThreads), 0, js, d_nq, d_goff, G, Vev, ev, d_eoff, 40,
+                       kJacBlockMin, kJacFloor);
     TTG_HIP(hipGetLastError());
   }
   // large sectors: the LR step when the truncation drops zero singular
