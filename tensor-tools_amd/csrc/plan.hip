@@ -25,75 +25,261 @@ __device__ inline uint32_t qcode(int q0, int q1) {
   return ((uint32_t)(q0 + 32768) << 16) | (uint32_t)(q1 + 32768);
 }
 
-struct KeyArrays {
-  uint64_t *kUL, *kSA, *kUR, *kUM, *kSB;     // raw keys
-  int *vSA, *vSB;                            // block ids
-  uint64_t *sUL, *sSA, *sUR, *sUM, *sSB;     // sorted
-  int *svSA, *svSB;
+// Sorted keys and groups of one plan (device scratch, nmax entries each).
+// q is a function of the left tuple, so the blocks of A with one left tuple are
+// a run of sSA, in ascending mid order: the candidates of every result block
+// with that left tuple, in the reference's mid order.
+struct PlanSets {
+  uint64_t *kUL, *kSA, *kUR, *kSB;   // keys by block (the path of many blocks)
+  uint64_t *sUL, *sSA, *sUR, *sSB;   // sorted: (q, left), (left, mid), (q, right), (mid, right)
+  int *svSA, *svUR, *svSB;           // block ids in those orders
+  uint64_t *uL, *uR;                 // unique (q, left), (q, right)
+  int *lsa0, *lcnt, *lpre;           // per left tuple: first entry of sSA, blocks, blocks of all earlier ones (nuL + 1)
+  int *rrep;                         // per right tuple: one block of B that has it
+  int *qL0, *qL1, *qR0, *qR1;        // per q: ranges of uL and uR
+  int64_t *qbase, *qcand;            // per q: first result block, first candidate (nQ + 1)
 };
 
-// ---- K1: per-block keys ------------------------------------------------
-// Block 0 also clears the plan header that the later planning kernels fill
-// (in place of a separate memset launch before this one).
-static_assert(sizeof(PlanHdr) % sizeof(int64_t) == 0, "plan header is whole 8-byte words");
-__global__ void k_plan_keys(MetaView A, MetaView B, PairSpec ps, KeyArrays k, PlanHdr* hdr) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0)
-    for (int w = threadIdx.x; w < (int)(sizeof(PlanHdr) / sizeof(int64_t)); w += blockDim.x)
-      ((int64_t*)hdr)[w] = 0;
-  if (i < A.nblocks) {
-    const int* qi = A.qi + (size_t)i * A.rank;
-    int q0 = 0, q1 = 0;
-    uint64_t left = 0, mid = 0;
-    for (int j = 0; j < ps.nfa; j++) {
-      int p = ps.fa[j], s = qi[p];
-      const int* e = A.idx + 3 * (A.idx_off[p] + s);
-      int sg = A.arrow[p] == 0 ? 1 : -1;          // Inward +, Outward - (:617-621)
-      q0 += sg * e[0];
-      q1 += sg * e[1];
-      left = left * A.nsec[p] + s;
-    }
-    for (int t = 0; t < ps.np; t++) {
-      int p = ps.pa[t];
-      mid = mid * A.nsec[p] + qi[p];
-    }
-    k.kUL[i] = ((uint64_t)qcode(q0, q1) << 32) | left;
-    k.kSA[i] = (left << 32) | mid;
-    k.vSA[i] = i;
+__device__ inline void plan_key_a(const MetaView& A, const PairSpec& ps, int i, uint64_t& ul, uint64_t& sa) {
+  const int* qi = A.qi + (size_t)i * A.rank;
+  int q0 = 0, q1 = 0;
+  uint64_t left = 0, mid = 0;
+  for (int j = 0; j < ps.nfa; j++) {
+    int p = ps.fa[j], s = qi[p];
+    const int* e = A.idx + 3 * (A.idx_off[p] + s);
+    int sg = A.arrow[p] == 0 ? 1 : -1;          // Inward +, Outward - (:617-621)
+    q0 += sg * e[0];
+    q1 += sg * e[1];
+    left = left * A.nsec[p] + s;
   }
-  if (i < B.nblocks) {
-    const int* qi = B.qi + (size_t)i * B.rank;
-    int q0 = 0, q1 = 0;
-    uint64_t right = 0, mid = 0;
-    for (int j = 0; j < ps.nfb; j++) {
-      int p = ps.fb[j], s = qi[p];
-      const int* e = B.idx + 3 * (B.idx_off[p] + s);
-      int sg = B.arrow[p] == 0 ? -1 : 1;          // Inward -, Outward + (:629-633)
-      q0 += sg * e[0];
-      q1 += sg * e[1];
-      right = right * B.nsec[p] + s;
+  for (int t = 0; t < ps.np; t++) {
+    int p = ps.pa[t];
+    mid = mid * A.nsec[p] + qi[p];
+  }
+  ul = ((uint64_t)qcode(q0, q1) << 32) | left;
+  sa = (left << 32) | mid;
+}
+__device__ inline void plan_key_b(const MetaView& B, const PairSpec& ps, int i, uint64_t& ur, uint64_t& sb) {
+  const int* qi = B.qi + (size_t)i * B.rank;
+  int q0 = 0, q1 = 0;
+  uint64_t right = 0, mid = 0;
+  for (int j = 0; j < ps.nfb; j++) {
+    int p = ps.fb[j], s = qi[p];
+    const int* e = B.idx + 3 * (B.idx_off[p] + s);
+    int sg = B.arrow[p] == 0 ? -1 : 1;          // Inward -, Outward + (:629-633)
+    q0 += sg * e[0];
+    q1 += sg * e[1];
+    right = right * B.nsec[p] + s;
+  }
+  for (int t = 0; t < ps.np; t++) {
+    int p = ps.pb[t];
+    mid = mid * B.nsec[p] + qi[p];
+  }
+  ur = ((uint64_t)qcode(q0, q1) << 32) | right;
+  sb = (mid << 32) | right;
+}
+
+// ---- groups of the sorted keys (one workgroup) ---------------------------
+constexpr int kPlanThreads = 1024;   // most threads of the one-workgroup planning kernels
+
+// rank of the calling thread's set flag among the workgroup's, and the count
+__device__ inline int block_rank(bool f, int* lds, int* total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const uint64_t m = __ballot(f);
+  if (lane == 0) lds[w] = __popcll(m);
+  __syncthreads();
+  int base = 0, tot = 0;
+  for (int k = 0; k < nw; k++) {
+    const int c = lds[k];
+    base += k < w ? c : 0;
+    tot += c;
+  }
+  __syncthreads();
+  *total = tot;
+  return base + __popcll(m & ((1ull << lane) - 1ull));
+}
+// exclusive prefix sum over the workgroup
+__device__ inline int64_t block_prefix(int64_t v, int64_t* lds, int64_t* total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int64_t x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int64_t y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) lds[w] = x;
+  __syncthreads();
+  int64_t base = 0, tot = 0;
+  for (int k = 0; k < nw; k++) {
+    const int64_t c = lds[k];
+    base += k < w ? c : 0;
+    tot += c;
+  }
+  __syncthreads();
+  *total = tot;
+  return base + x - v;
+}
+
+// Unique left and right tuples, q groups, and the first result block and first
+// candidate of every group.  The sorted keys are read from, and the unique
+// ones written to, LDS or global memory (cuL may be sUL, cuR may be sUR); the
+// other results go to w's global arrays and the header to both headers.
+__device__ __forceinline__ void plan_groups(const uint64_t* sUL, const uint64_t* sSA, const uint64_t* sUR, const int* svUR,
+                                            uint64_t* cuL, uint64_t* cuR, int nA, int nB, const PlanSets& w,
+                                            int* lds_i, int64_t* lds_l, PlanHdr* hdr, PlanHdr* host) {
+  const int nt = blockDim.x, tid = threadIdx.x;
+  int nuL = 0, nuR = 0, nQ = 0;
+  int64_t blocks_before = 0;   // blocks of A before the chunk
+  for (int base = 0; base < nA; base += nt) {
+    const int i = base + tid;
+    const uint64_t key = i < nA ? sUL[i] : 0;
+    const bool f = i < nA && (i == 0 || key != sUL[i - 1]);
+    int tot;
+    const int pos = nuL + block_rank(f, lds_i, &tot);
+    int cnt = 0, a0 = 0;
+    if (f) {
+      const uint64_t left = key & 0xffffffffull;
+      a0 = lower_bound_u64(sSA, nA, left << 32);
+      cnt = lower_bound_u64(sSA, nA, (left + 1) << 32) - a0;
     }
-    for (int t = 0; t < ps.np; t++) {
-      int p = ps.pb[t];
-      mid = mid * B.nsec[p] + qi[p];
+    int64_t all;
+    const int64_t pre = block_prefix(cnt, lds_l, &all);
+    if (f) {
+      cuL[pos] = key;
+      w.lsa0[pos] = a0;
+      w.lcnt[pos] = cnt;
+      w.lpre[pos] = (int)(blocks_before + pre);
     }
-    uint64_t qc = (uint64_t)qcode(q0, q1) << 32;
-    k.kUR[i] = qc | right;
-    k.kUM[i] = qc | mid;
-    k.kSB[i] = (mid << 32) | right;
-    k.vSB[i] = i;
+    nuL += tot;
+    blocks_before += all;
+  }
+  for (int base = 0; base < nB; base += nt) {
+    const int i = base + tid;
+    const uint64_t key = i < nB ? sUR[i] : 0;
+    const bool f = i < nB && (i == 0 || key != sUR[i - 1]);
+    int tot;
+    const int pos = nuR + block_rank(f, lds_i, &tot);   // (its barriers: every read of the chunk comes before a write)
+    if (f) {
+      cuR[pos] = key;
+      w.uR[pos] = key;
+      w.rrep[pos] = svUR[i];
+    }
+    nuR += tot;
+  }
+  if (tid == 0) w.lpre[nuL] = (int)blocks_before;
+  __syncthreads();
+  // q groups of the left tuples (ascending q; A's mid-QN set, :622-623)
+  for (int base = 0; base < nuL; base += nt) {
+    const int i = base + tid;
+    const bool f = i < nuL && (i == 0 || (cuL[i] >> 32) != (cuL[i - 1] >> 32));
+    int tot;
+    const int pos = nQ + block_rank(f, lds_i, &tot);
+    if (f) w.qL0[pos] = i;
+    nQ += tot;
+  }
+  __syncthreads();
+  int64_t nblk = 0, ncand = 0;
+  for (int base = 0; base < nQ; base += nt) {
+    const int t = base + tid;
+    int64_t cnt = 0, cand = 0;
+    if (t < nQ) {
+      const int l0 = w.qL0[t], l1 = t + 1 < nQ ? w.qL0[t + 1] : nuL;
+      const uint64_t qc = cuL[l0] >> 32;
+      const int r0 = lower_bound_u64(cuR, nuR, qc << 32), r1 = lower_bound_u64(cuR, nuR, (qc + 1) << 32);
+      w.qL1[t] = l1;
+      w.qR0[t] = r0;
+      w.qR1[t] = r1;
+      cnt = (int64_t)(l1 - l0) * (r1 - r0);
+      cand = (int64_t)(w.lpre[l1] - w.lpre[l0]) * (r1 - r0);
+    }
+    int64_t tot, tot2;
+    const int64_t pb = block_prefix(cnt, lds_l, &tot), pc = block_prefix(cand, lds_l, &tot2);
+    if (t < nQ) {
+      w.qbase[t] = nblk + pb;
+      w.qcand[t] = ncand + pc;
+    }
+    nblk += tot;
+    ncand += tot2;
+  }
+  if (tid == 0) {
+    w.qbase[nQ] = nblk;
+    w.qcand[nQ] = ncand;
+    hdr->nQ = host->nQ = nQ;
+    hdr->nblocksC = host->nblocksC = nblk;
+    hdr->ncand = host->ncand = ncand;
   }
 }
 
-// ---- K2: stable rank sort (five arrays, grid.y selects) -----------------
+// ---- up to kPlanSmall blocks per operand: keys, sorts and groups in one
+// workgroup's LDS (one launch and 12 us where the three kernels below take
+// 23 us and two launch gaps at a few hundred blocks).  The four key arrays
+// are sorted together by bitonic networks of P entries, P the power of two
+// above both block counts.
+constexpr int kPlanSmall = 1024;
+__global__ void __launch_bounds__(kPlanThreads) k_plan_small(MetaView A, MetaView B, PairSpec ps, int P, PlanSets w,
+                                                             PlanHdr* hdr, PlanHdr* host) {
+  __shared__ uint64_t K[4][kPlanSmall];   // (q, left), (left, mid), (q, right), (mid, right)
+  __shared__ int V[3][kPlanSmall];        // block ids of the last three
+  __shared__ int lds_i[kPlanThreads / 64];
+  __shared__ int64_t lds_l[kPlanThreads / 64];
+  const int tid = threadIdx.x, nA = A.nblocks, nB = B.nblocks;
+  for (int i = tid; i < P; i += blockDim.x) {
+    uint64_t ul = ~0ull, sa = ~0ull, ur = ~0ull, sb = ~0ull;   // above every key: a tuple's half is below 2^32 - 1
+    if (i < nA) plan_key_a(A, ps, i, ul, sa);
+    if (i < nB) plan_key_b(B, ps, i, ur, sb);
+    K[0][i] = ul;
+    K[1][i] = sa;
+    K[2][i] = ur;
+    K[3][i] = sb;
+    V[0][i] = V[1][i] = V[2][i] = i;
+  }
+  const int half = P >> 1, hs = 31 - __builtin_clz(half | 1);   // half = 1 << hs (P >= 2)
+  for (int k = 2; k <= P; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      __syncthreads();
+      for (int c = tid; c < 4 * half; c += blockDim.x) {
+        const int a = c >> hs, e = c & (half - 1);
+        const int i = 2 * e - (e & (j - 1)), l = i + j;
+        const uint64_t x = K[a][i], y = K[a][l];
+        // equal keys keep block order (a repeated block is found at its first id)
+        const bool after = x > y || (x == y && a > 0 && V[a - 1][i] > V[a - 1][l]);
+        if (after == ((i & k) == 0)) {
+          K[a][i] = y;
+          K[a][l] = x;
+          if (a > 0) {
+            const int t = V[a - 1][i];
+            V[a - 1][i] = V[a - 1][l];
+            V[a - 1][l] = t;
+          }
+        }
+      }
+    }
+  __syncthreads();
+  for (int i = tid; i < nA; i += blockDim.x) {
+    w.sSA[i] = K[1][i];
+    w.svSA[i] = V[0][i];
+  }
+  for (int i = tid; i < nB; i += blockDim.x) {
+    w.sSB[i] = K[3][i];
+    w.svSB[i] = V[2][i];
+  }
+  plan_groups(K[0], K[1], K[2], V[1], K[0], K[2], nA, nB, w, lds_i, lds_l, hdr, host);
+}
+
+// ---- more blocks: keys, stable rank sort (grid.y selects the array), groups
+__global__ void k_plan_keys(MetaView A, MetaView B, PairSpec ps, PlanSets w) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < A.nblocks) plan_key_a(A, ps, i, w.kUL[i], w.kSA[i]);
+  if (i < B.nblocks) plan_key_b(B, ps, i, w.kUR[i], w.kSB[i]);
+}
+
 struct SortJob {
   const uint64_t* in;
-  const int* vin;
   uint64_t* out;
-  int* vout;
+  int* vout;   // ids of the sorted entries, or null
   int n;
 };
-struct SortJobs { SortJob j[5]; };
+struct SortJobs { SortJob j[4]; };
 
 __global__ void __launch_bounds__(256) k_rank_sort(SortJobs jobs) {
   const SortJob& J = jobs.j[blockIdx.y];
@@ -114,177 +300,92 @@ __global__ void __launch_bounds__(256) k_rank_sort(SortJobs jobs) {
   }
   if (i < J.n) {
     J.out[rank] = key;
-    if (J.vout) J.vout[rank] = J.vin ? J.vin[i] : i;
+    if (J.vout) J.vout[rank] = i;
   }
 }
 
-// ---- K3: unique sets, per-q ranges, result-block bases -------------------
-struct QTab {
-  int *qL0, *qL1, *qR0, *qR1, *qM0, *qM1;
-  int64_t* qbase;   // nQ + 1
+__global__ void __launch_bounds__(kPlanThreads) k_plan_groups(int nA, int nB, PlanSets w, PlanHdr* hdr, PlanHdr* host) {
+  __shared__ int lds_i[kPlanThreads / 64];
+  __shared__ int64_t lds_l[kPlanThreads / 64];
+  plan_groups(w.sUL, w.sSA, w.sUR, w.svUR, w.uL, w.uR, nA, nB, w, lds_i, lds_l, hdr, host);
+}
+
+// ---- per result block: tuple, dims, task enumeration ---------------------
+// what the scan kernel and the host need of a result block
+struct BlkStat {
+  int64_t t0;          // first task slot
+  int64_t opmax;       // largest operand block (elements) of its tasks
+  double flops;
+  int M, N, nt, nkt;   // nt tasks, nkt k-tiles
+  int ktmax, bad;      // largest K; a task with more than two strides per dimension
+  int votes[4];        // tasks with unit stride: A m, A k, B k, B n
 };
 
-__device__ int compact_unique(const uint64_t* s, int n, uint64_t* u, int64_t* lds) {
-  int64_t carry = 0;
-  for (int base = 0; base < n; base += 1024) {
-    int i = base + threadIdx.x;
-    int f = 0;
-    if (i < n) f = (i == 0) || (s[i] != s[i - 1]);
-    int64_t tot;
-    int64_t pos = block_excl_scan<1024>((int64_t)f, lds, &tot);
-    if (f) u[carry + pos] = s[i];
-    carry += tot;
+// fold (extent, stride) components in order: extent-1 ones are dropped,
+// contiguous runs merged; n counts the components, the first two are kept.
+// 32 bits: an operand block of 2^28 elements or more is refused (opmax).
+struct Fold {
+  int n = 0;
+  unsigned e0 = 1, ce = 0, cs = 0, s0 = 0, s1 = 0;   // ce: extent of the open component (0: none)
+  __device__ __forceinline__ void close() {
+    const bool open = ce != 0;
+    e0 = open && n == 0 ? ce : e0;
+    s0 = open && n == 0 ? cs : s0;
+    s1 = open && n == 1 ? cs : s1;
+    n += open;
+    ce = 0;
   }
-  __syncthreads();
-  return (int)carry;
-}
-
-__global__ void __launch_bounds__(1024) k_plan_unique(KeyArrays k, int nA, int nB, uint64_t* uL,
-                                                      uint64_t* uR, uint64_t* uM, QTab q,
-                                                      PlanHdr* hdr) {
-  __shared__ int64_t lds[32];
-  const int nuL = compact_unique(k.sUL, nA, uL, lds);
-  const int nuR = compact_unique(k.sUR, nB, uR, lds);
-  const int nuM = compact_unique(k.sUM, nB, uM, lds);
-  // q groups of uL (ascending q; A's mid-QN set, :622-623)
-  int64_t carry = 0;
-  for (int base = 0; base < nuL; base += 1024) {
-    int i = base + threadIdx.x;
-    int f = 0;
-    if (i < nuL) f = (i == 0) || ((uL[i] >> 32) != (uL[i - 1] >> 32));
-    int64_t tot;
-    int64_t pos = block_excl_scan<1024>((int64_t)f, lds, &tot);
-    if (f) q.qL0[carry + pos] = i;
-    carry += tot;
+  __device__ __forceinline__ void add(unsigned ext, unsigned st) {
+    if (ext == 1) return;
+    if (ce != 0 && st == ce * cs) { ce *= ext; return; }
+    close();
+    ce = ext;
+    cs = st;
   }
-  __syncthreads();
-  const int nQ = (int)carry;
-  for (int t = threadIdx.x; t < nQ; t += 1024) {
-    int l0 = q.qL0[t];
-    int l1 = (t + 1 < nQ) ? q.qL0[t + 1] : nuL;
-    q.qL1[t] = l1;
-    uint64_t qc = uL[l0] >> 32;
-    q.qR0[t] = lower_bound_u64(uR, nuR, qc << 32);
-    q.qR1[t] = lower_bound_u64(uR, nuR, (qc + 1) << 32);
-    q.qM0[t] = lower_bound_u64(uM, nuM, qc << 32);
-    q.qM1[t] = lower_bound_u64(uM, nuM, (qc + 1) << 32);
-  }
-  __syncthreads();
-  carry = 0;
-  int64_t ncand = 0;   // every result block of group t tries each of its nM mids
-  for (int base = 0; base < nQ; base += 1024) {
-    int t = base + threadIdx.x;
-    int64_t cnt = 0, cand = 0;
-    if (t < nQ) {
-      cnt = (int64_t)(q.qL1[t] - q.qL0[t]) * (q.qR1[t] - q.qR0[t]);
-      cand = cnt * (q.qM1[t] - q.qM0[t]);
-    }
-    int64_t tot, tot2;
-    int64_t pos = block_excl_scan<1024>(cnt, lds, &tot);
-    (void)block_excl_scan<1024>(cand, lds, &tot2);
-    if (t < nQ) q.qbase[t] = carry + pos;
-    carry += tot;
-    ncand += tot2;
-  }
-  if (threadIdx.x == 0) {
-    q.qbase[nQ] = carry;
-    hdr->nuL = nuL;
-    hdr->nuR = nuR;
-    hdr->nuM = nuM;
-    hdr->nQ = nQ;
-    hdr->nblocksC = carry;
-    hdr->ncand = ncand;
-  }
-}
-
-// ---- K4: per result block: tuple, dims, task enumeration ----------------
-struct BlkArrays {
-  int64_t* size;      // nblocksC
-  int64_t* ntask;     // nblocksC
-  double* flops;      // nblocksC
-  const int64_t* task_off;   // nblocksC + 1 (phase 1)
-  int* c_qi;          // nblocksC * rankC
-  const int64_t* c_off;      // nblocksC + 1 (phase 1)
 };
-struct EmitArrays {
-  GemmTask* tasks;
-  CBlock* cblk;
-  int* tuples;
+// the same for K, whose components have a stride in each operand
+struct FoldK {
+  int n = 0;
+  unsigned e0 = 1, ce = 0, ca = 0, cb = 0, a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+  __device__ __forceinline__ void close() {
+    const bool open = ce != 0, first = open && n == 0, second = open && n == 1;
+    e0 = first ? ce : e0;
+    a0 = first ? ca : a0;
+    b0 = first ? cb : b0;
+    a1 = second ? ca : a1;
+    b1 = second ? cb : b1;
+    n += open;
+    ce = 0;
+  }
+  __device__ __forceinline__ void add(unsigned ext, unsigned sa, unsigned sb) {
+    if (ext == 1) return;
+    if (ce != 0 && sa == ce * ca && sb == ce * cb) { ce *= ext; return; }
+    close();
+    ce = ext;
+    ca = sa;
+    cb = sb;
+  }
 };
-
-__device__ inline int find_sorted(const uint64_t* a, int n, uint64_t key) {
-  int p = lower_bound_u64(a, n, key);
-  return (p < n && a[p] == key) ? p : -1;
+// extent and stride of index p (uniform, runtime) of a block of extents d:
+// products of selects, so the array stays in registers
+__device__ __forceinline__ unsigned ext_of(const unsigned (&d)[MAXR], int p) {
+  unsigned r = 1;
+#pragma unroll
+  for (int j = 0; j < MAXR; j++) r *= j == p ? d[j] : 1u;
+  return r;
+}
+__device__ __forceinline__ unsigned stride_of(const unsigned (&d)[MAXR], int p) {
+  unsigned r = 1;
+#pragma unroll
+  for (int j = 0; j < MAXR - 1; j++) r *= j < p ? d[j] : 1u;
+  return r;
 }
 
-// fold (extent, stride) components: drop extent-1, merge contiguous runs;
-// returns the component count (components beyond 2 are reported, not kept)
-__device__ inline int fold2(int n, const int* ext, const int64_t* st, int& e0, int64_t& s0,
-                            int64_t& s1) {
-  int cnt = 0;
-  int64_t ce = 1, cs = 0;
-  e0 = 1; s0 = 0; s1 = 0;
-  int ncomp = 0;
-  int64_t ce0 = 0;
-  for (int j = 0; j < n; j++) {
-    if (ext[j] == 1) continue;
-    if (cnt > 0 && st[j] == ce * cs) {
-      ce *= ext[j];
-      continue;
-    }
-    if (cnt > 0) {  // close previous
-      if (ncomp == 0) { ce0 = ce; s0 = cs; }
-      else if (ncomp == 1) { s1 = cs; }
-      ncomp++;
-    }
-    cnt = 1;
-    ce = ext[j];
-    cs = st[j];
-  }
-  if (cnt > 0) {
-    if (ncomp == 0) { ce0 = ce; s0 = cs; }
-    else if (ncomp == 1) { s1 = cs; }
-    ncomp++;
-  }
-  e0 = ncomp >= 1 ? (int)ce0 : 1;
-  return ncomp;
-}
-
-// K fold with two operands sharing the contraction index order
-__device__ inline int foldk(int n, const int* ext, const int64_t* sa, const int64_t* sb, int& e0,
-                            int64_t& a0, int64_t& a1, int64_t& b0, int64_t& b1) {
-  int ncomp = 0, open = 0;
-  int64_t ce = 1, ca = 0, cb = 0, ce0 = 1;
-  a0 = a1 = b0 = b1 = 0;
-  for (int j = 0; j < n; j++) {
-    if (ext[j] == 1) continue;
-    if (open && sa[j] == ce * ca && sb[j] == ce * cb) {
-      ce *= ext[j];
-      continue;
-    }
-    if (open) {
-      if (ncomp == 0) { ce0 = ce; a0 = ca; b0 = cb; }
-      else if (ncomp == 1) { a1 = ca; b1 = cb; }
-      ncomp++;
-    }
-    open = 1;
-    ce = ext[j]; ca = sa[j]; cb = sb[j];
-  }
-  if (open) {
-    if (ncomp == 0) { ce0 = ce; a0 = ca; b0 = cb; }
-    else if (ncomp == 1) { a1 = ca; b1 = cb; }
-    ncomp++;
-  }
-  e0 = ncomp >= 1 ? (int)ce0 : 1;
-  return ncomp;
-}
-
-// One wave per result block.  The block's tasks are its mid tuples in
-// ascending order (qtensor.cpp:696-722); the lanes take 64 mids at a time,
-// and each task's position in the list and the k-tile offset of its walk
-// are exclusive prefix sums over the lanes in mid order, so the task list is
-// the one a walk over the mids in order gives.
 __device__ inline int64_t wave_sum_i64(int64_t v) {
+  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+  return v;
+}
+__device__ inline int wave_sum_i32(int v) {
   for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
   return v;
 }
@@ -300,221 +401,270 @@ __device__ inline int64_t wave_max_i64(int64_t v) {
   return v;
 }
 
-__global__ void __launch_bounds__(256) k_plan_blocks(MetaView A, MetaView B, PairSpec ps,
-                                                     KeyArrays k, const uint64_t* uL,
-                                                     const uint64_t* uR, const uint64_t* uM,
-                                                     QTab q, int nQ, int nblocksC, int phase,
-                                                     BlkArrays ba, EmitArrays ea, PlanHdr* hdr,
-                                                     int nA, int nB, int TK) {
+// One wave per result block (q -> right -> left).  Its candidates are A's
+// blocks with its left tuple, in ascending mid order (qtensor.cpp:696-722); the
+// lanes take 64 at a time and look up the B block (mid, right).  The tasks of
+// the block are written one after another from its first candidate slot, each
+// at the prefix sum of the matches before it, so the tasks, their k-tile
+// offsets and the counts come out of one pass.  The B keys are staged in LDS
+// when they fit (stage_b): the lookups are a chain of dependent loads.
+constexpr int kPlanStageB = 4096;
+__global__ void __launch_bounds__(256) k_plan_blocks(MetaView A, MetaView B, PairSpec ps, PlanSets w, int stage_b,
+                                                     const PlanHdr* hdr, BlkStat* stat, int* c_qi, GemmTask* tasks,
+                                                     int* tuples, int TK) {
+  extern __shared__ uint64_t lds_sb[];
+  const int nB = B.nblocks;
+  if (stage_b) {
+    for (int i = threadIdx.x; i < nB; i += 256) lds_sb[i] = w.sSB[i];
+    __syncthreads();
+  }
   const int lane = threadIdx.x & 63;
   const int b = (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
-  if (b >= nblocksC) return;   // the whole wave
-  // q group containing b: last t with qbase[t] <= b
-  int lo = 0, hi = nQ;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (q.qbase[mid] <= b) lo = mid + 1;
-    else hi = mid;
-  }
-  const int t = lo - 1;
-  const int64_t local = b - q.qbase[t];
-  const int nL = q.qL1[t] - q.qL0[t];
-  const int ri = (int)(local / nL), li = (int)(local % nL);
-  const uint64_t left = uL[q.qL0[t] + li] & 0xffffffffull;
-  const uint64_t right = uR[q.qR0[t] + ri] & 0xffffffffull;
-  // decode tuples (first position most significant)
-  int lq[MAXR], rq[MAXR];
-  {
-    uint64_t x = left;
-    for (int j = ps.nfa - 1; j >= 0; j--) { int p = ps.fa[j]; lq[j] = (int)(x % A.nsec[p]); x /= A.nsec[p]; }
-    x = right;
-    for (int j = ps.nfb - 1; j >= 0; j--) { int p = ps.fb[j]; rq[j] = (int)(x % B.nsec[p]); x /= B.nsec[p]; }
-  }
+  const int nQ = (int)hdr->nQ;
+  if (b >= hdr->nblocksC) return;   // the whole wave
+  // q group containing b: the last t with qbase[t] <= b
+  int t = -1;
+  for (int i = 0; i < nQ; i += 64)
+    t += __popcll(__ballot(i + lane < nQ && w.qbase[i + lane] <= b));
+  const int local = (int)(b - w.qbase[t]);
+  const int l0 = w.qL0[t], nL = w.qL1[t] - l0;
+  const int ri = local / nL, l = l0 + local % nL, r = w.qR0[t] + ri;
+  const int sa0 = w.lsa0[l], cnt = w.lcnt[l];
+  const int64_t t0 = w.qcand[t] + (int64_t)ri * (w.lpre[l0 + nL] - w.lpre[l0]) + (w.lpre[l] - w.lpre[l0]);
+  const uint32_t right = (uint32_t)w.uR[r];
+  const int rep = w.rrep[r];
+  unsigned freeA = 0, freeB = 0;   // uniform
+  for (int j = 0; j < ps.nfa; j++) freeA |= 1u << ps.fa[j];
+  for (int j = 0; j < ps.nfb; j++) freeB |= 1u << ps.fb[j];
   const int rankC = ps.nfa + ps.nfb;
-  int64_t M = 1, N = 1;
-  for (int j = 0; j < ps.nfa; j++) M *= A.idx[3 * (A.idx_off[ps.fa[j]] + lq[j]) + 2];
-  for (int j = 0; j < ps.nfb; j++) N *= B.idx[3 * (B.idx_off[ps.fb[j]] + rq[j]) + 2];
-  if (phase == 0 && lane == 0) {
-    for (int j = 0; j < ps.nfa; j++) ba.c_qi[(size_t)b * rankC + j] = lq[j];
-    for (int j = 0; j < ps.nfb; j++) ba.c_qi[(size_t)b * rankC + ps.nfa + j] = rq[j];
-    ba.size[b] = M * N;
+  int64_t N = 1;
+  {
+    int k = ps.nfa;
+#pragma unroll
+    for (int j = 0; j < MAXR; j++)
+      if ((freeB >> j) & 1) {
+        const int s = B.qi[(size_t)rep * B.rank + j];
+        N *= B.idx[3 * (B.idx_off[j] + s) + 2];
+        if (lane == 0) c_qi[(size_t)b * rankC + k] = s;
+        k++;
+      }
   }
-  const int64_t tw = phase == 1 ? ba.task_off[b] : 0;
-  int64_t nt = 0;   // tasks of the block so far (uniform)
-  int64_t kt = 0;   // k-tiles of the block's walk so far (uniform)
-  // per-lane partial sums and maxima, reduced over the wave at the end
+  int64_t M = 1;
+  int nt = 0, kt = 0;   // tasks and k-tiles of the block so far (uniform)
   double fl = 0.0;
-  int64_t sumK = 0;
-  int64_t votes[4] = {0, 0, 0, 0};
-  int64_t ktmax = 0, opmax = 0;
-  int64_t bad = 0;
-  for (int m0 = q.qM0[t]; m0 < q.qM1[t]; m0 += 64) {
-    const int m = m0 + lane;
+  int votes[4] = {0, 0, 0, 0}, ktmax = 0, bad = 0;
+  int64_t opmax = 0;
+  for (int c0 = 0; c0 < cnt; c0 += 64) {
+    const int ca = c0 + lane;
     bool valid = false;
     GemmTask g{};
-    int64_t K = 1, ktl = 0;
-    int ablk = 0, bblk = 0;
-    if (m < q.qM1[t]) {
-      const uint64_t mid = uM[m] & 0xffffffffull;
-      const int ia = find_sorted(k.sSA, nA, (left << 32) | mid);
-      const int ib = ia < 0 ? -1 : find_sorted(k.sSB, nB, (mid << 32) | right);
-      if (ib >= 0) {
+    int64_t K = 1;
+    int ktl = 0, ablk = 0, bblk = 0;
+    if (ca < cnt) {
+      ablk = w.svSA[sa0 + ca];
+      const uint64_t akey = w.sSA[sa0 + ca];
+      const bool again = ca > 0 && w.sSA[sa0 + ca - 1] == akey;   // a repeated block counts once
+      const uint64_t key = (akey << 32) | right;                  // (mid, right)
+      unsigned dA[MAXR];
+      int qA[MAXR];
+#pragma unroll
+      for (int j = 0; j < MAXR; j++) qA[j] = j < A.rank ? A.qi[(size_t)ablk * A.rank + j] : 0;
+#pragma unroll
+      for (int j = 0; j < MAXR; j++) dA[j] = j < A.rank ? A.idx[3 * (A.idx_off[j] + qA[j]) + 2] : 1;
+      M = 1;
+#pragma unroll
+      for (int j = 0; j < MAXR; j++) M *= (freeA >> j) & 1 ? dA[j] : 1;
+      if (ca == 0) {
+        int k = 0;
+#pragma unroll
+        for (int j = 0; j < MAXR; j++)
+          if ((freeA >> j) & 1) c_qi[(size_t)b * rankC + k++] = qA[j];
+      }
+      const uint64_t* sb = stage_b ? lds_sb : w.sSB;
+      const int ib = lower_bound_u64(sb, nB, key);
+      if (!again && ib < nB && sb[ib] == key) {
         valid = true;
-        ablk = k.svSA[ia];
-        bblk = k.svSB[ib];
-        // strides of the stored (unpermuted) blocks
-        int dA[MAXR], dB[MAXR];
-        int64_t sA[MAXR], sB[MAXR];
-        int64_t acc = 1;
-        for (int j = 0; j < A.rank; j++) {
-          dA[j] = A.idx[3 * (A.idx_off[j] + A.qi[(size_t)ablk * A.rank + j]) + 2];
-          sA[j] = acc;
-          acc *= dA[j];
-        }
-        acc = 1;
-        for (int j = 0; j < B.rank; j++) {
-          dB[j] = B.idx[3 * (B.idx_off[j] + B.qi[(size_t)bblk * B.rank + j]) + 2];
-          sB[j] = acc;
-          acc *= dB[j];
-        }
-        int em[MAXR], ek[MAXR], en[MAXR];
-        int64_t smA[MAXR], skA[MAXR], skB[MAXR], snB[MAXR];
-        for (int j = 0; j < ps.nfa; j++) { em[j] = dA[ps.fa[j]]; smA[j] = sA[ps.fa[j]]; }
-        for (int p = 0; p < ps.np; p++) {
-          ek[p] = dB[ps.pb[p]];
-          skA[p] = sA[ps.pa[p]];
-          skB[p] = sB[ps.pb[p]];
-          K *= ek[p];
-        }
-        for (int j = 0; j < ps.nfb; j++) { en[j] = dB[ps.fb[j]]; snB[j] = sB[ps.fb[j]]; }
+        bblk = w.svSB[ib];
+        unsigned dB[MAXR];
+#pragma unroll
+        for (int j = 0; j < MAXR; j++)
+          dB[j] = j < B.rank ? B.idx[3 * (B.idx_off[j] + B.qi[(size_t)bblk * B.rank + j]) + 2] : 1;
         g.a_off = A.off[ablk];
         g.b_off = B.off[bblk];
+        Fold fm, fn;
+        unsigned sA = 1, sB = 1;   // strides of the stored (unpermuted) blocks
+#pragma unroll
+        for (int j = 0; j < MAXR; j++) {
+          if ((freeA >> j) & 1) fm.add(dA[j], sA);
+          if ((freeB >> j) & 1) fn.add(dB[j], sB);
+          sA *= dA[j];
+          sB *= dB[j];
+        }
+        fm.close();
+        fn.close();
+        g.em0 = fm.e0; g.sam0 = fm.s0; g.sam1 = fm.s1;
+        g.en0 = fn.e0; g.sbn0 = fn.s0; g.sbn1 = fn.s1;
+        // the contraction order forwards, and reversed: taken when it folds
+        // better, or when it puts the longer component first (the GEMM walks k
+        // in chunks of the first component, so a short first component wastes
+        // chunk slots)
+        FoldK fk, fr;
+        for (int p = 0; p < ps.np; p++) {
+          const int z = ps.np - 1 - p;
+          const unsigned ext = ext_of(dB, ps.pb[p]);
+          K *= ext;
+          fk.add(ext, stride_of(dA, ps.pa[p]), stride_of(dB, ps.pb[p]));
+          fr.add(ext_of(dB, ps.pb[z]), stride_of(dA, ps.pa[z]), stride_of(dB, ps.pb[z]));
+        }
+        fk.close();
+        fr.close();
+        const bool rev = (fk.n > 2 && fr.n <= 2) || (fk.n == 2 && fr.n == 2 && fr.e0 > fk.e0);
+        g.ek0 = rev ? fr.e0 : fk.e0;
+        g.sak0 = rev ? fr.a0 : fk.a0;
+        g.sak1 = rev ? fr.a1 : fk.a1;
+        g.sbk0 = rev ? fr.b0 : fk.b0;
+        g.sbk1 = rev ? fr.b1 : fk.b1;
         g.K = (int)K;
-        int cm = fold2(ps.nfa, em, smA, g.em0, g.sam0, g.sam1);
-        int cn = fold2(ps.nfb, en, snB, g.en0, g.sbn0, g.sbn1);
-        int ck = foldk(ps.np, ek, skA, skB, g.ek0, g.sak0, g.sak1, g.sbk0, g.sbk1);
-        {  // reversed contraction order: taken when it folds better, or when it
-           // puts the longer component first (the GEMM walks k in chunks of the
-           // first component, so a short first component wastes chunk slots)
-          int ekr[MAXR];
-          int64_t skAr[MAXR], skBr[MAXR];
-          for (int p = 0; p < ps.np; p++) {
-            ekr[p] = ek[ps.np - 1 - p];
-            skAr[p] = skA[ps.np - 1 - p];
-            skBr[p] = skB[ps.np - 1 - p];
-          }
-          int e0r;
-          int64_t a0r, a1r, b0r, b1r;
-          const int ckr = foldk(ps.np, ekr, skAr, skBr, e0r, a0r, a1r, b0r, b1r);
-          if ((ck > 2 && ckr <= 2) || (ck == 2 && ckr == 2 && e0r > g.ek0)) {
-            ck = ckr;
-            g.ek0 = e0r; g.sak0 = a0r; g.sak1 = a1r; g.sbk0 = b0r; g.sbk1 = b1r;
-          }
-        }
-        if (cm > 2 || cn > 2 || ck > 2) bad = 1;
-        ktl = (int64_t)(K / g.ek0) * (int64_t)((g.ek0 + TK - 1) / TK);
-        if (phase == 0) {
-          votes[0] += (g.sam0 == 1) || M == 1;
-          votes[1] += (g.sak0 == 1) || K == 1;
-          votes[2] += (g.sbk0 == 1) || K == 1;
-          votes[3] += (g.sbn0 == 1) || N == 1;
-        }
-        ktmax = K > ktmax ? K : ktmax;
-        opmax = M * K > opmax ? M * K : opmax;
-        opmax = K * N > opmax ? K * N : opmax;
-        // K walk in TK-wide chunks of the first k component (gemm.hip)
-        sumK += (int64_t)(K / g.ek0) * (int64_t)((g.ek0 + TK - 1) / TK * TK);
+        g.nk1 = (int)(K / g.ek0);
+        if (fm.n > 2 || fn.n > 2 || (rev ? fr.n : fk.n) > 2) bad = 1;
+        ktl = g.nk1 * ((g.ek0 + TK - 1) / TK);   // K walk in TK-wide chunks of the first k component (gemm.hip)
+        votes[0] += g.sam0 == 1 || M == 1;
+        votes[1] += g.sak0 == 1 || K == 1;
+        votes[2] += g.sbk0 == 1 || K == 1;
+        votes[3] += g.sbn0 == 1 || N == 1;
+        ktmax = max(ktmax, (int)K);
+        const int64_t oa = M * K, ob = K * N;
+        opmax = oa > opmax ? oa : opmax;
+        opmax = ob > opmax ? ob : opmax;
         fl += 2.0 * (double)M * (double)N * (double)K;
       }
     }
     // position and k-tile offset: exclusive prefix sums over the lanes
     const uint64_t vm = __ballot(valid);
     const int pos = __popcll(vm & ((1ull << lane) - 1ull));
-    int64_t incl = valid ? ktl : 0;
+    int incl = ktl;
     for (int d = 1; d < 64; d <<= 1) {
-      const int64_t y = __shfl_up(incl, d);
+      const int y = __shfl_up(incl, d);
       if (lane >= d) incl += y;
     }
-    if (valid && phase == 1) {
-      g.kt0 = (int)(kt + incl - ktl);
-      g.nk1 = (int)(K / g.ek0);
-      ea.tasks[tw + nt + pos] = g;
-      if (ea.tuples) {
-        int* tu = ea.tuples + 6 * (tw + nt + pos);
-        tu[0] = b; tu[1] = ablk; tu[2] = bblk; tu[3] = (int)M; tu[4] = (int)N; tu[5] = (int)K;
-      }
+    if (valid) {
+      g.kt0 = kt + incl - ktl;
+      tasks[t0 + nt + pos] = g;
+      int* tu = tuples + 6 * (t0 + nt + pos);
+      tu[0] = b; tu[1] = ablk; tu[2] = bblk; tu[3] = (int)M; tu[4] = (int)N; tu[5] = (int)K;
     }
     nt += __popcll(vm);
     kt += __shfl(incl, 63);
   }
-  if (phase == 0) {
-    fl = wave_sum_f64(fl);
-    sumK = wave_sum_i64(sumK);
-    for (int v = 0; v < 4; v++) votes[v] = wave_sum_i64(votes[v]);
-    ktmax = wave_max_i64(ktmax);
-    opmax = wave_max_i64(opmax);
-    bad = wave_max_i64(bad);
-    if (lane != 0) return;
-    ba.ntask[b] = nt;
-    ba.flops[b] = fl;
-    for (int c = 0; c < TILE_NCFG; c++) {
-      const int TMc = cfg_tm(c), TNc = cfg_tn(c);
-      int64_t tm = (M + TMc - 1) / TMc, tn = (N + TNc - 1) / TNc;
-      atomicAdd((unsigned long long*)&hdr->tiles[c], (unsigned long long)(tm * tn));
-      atomicAdd(&hdr->padded[c], (double)(tm * TMc) * (double)(tn * TNc) * (double)sumK);
-    }
-    atomicMax((unsigned long long*)&hdr->kmax, (unsigned long long)sumK);
-    if (nt) {
-      atomicMax((unsigned long long*)&hdr->nmax, (unsigned long long)N);
-      atomicMax((unsigned long long*)&hdr->ktmax, (unsigned long long)ktmax);
-      atomicMax((unsigned long long*)&hdr->opmax, (unsigned long long)opmax);
-    }
-    for (int v = 0; v < 4; v++)
-      if (votes[v]) atomicAdd((unsigned long long*)&hdr->votes[v], (unsigned long long)votes[v]);
-    if (bad) atomicAdd((unsigned long long*)&hdr->err, 1ull);
-  } else if (lane == 0) {
-    CBlock cb;
-    cb.c_off = ba.c_off[b];
-    cb.M = (int)M;
-    cb.N = (int)N;
-    cb.t0 = (int)tw;
-    cb.t1 = (int)(tw + nt);
-    cb.nkt = (int)kt;
-    cb.pad = 0;
-    ea.cblk[b] = cb;
+  fl = wave_sum_f64(fl);
+  for (int v = 0; v < 4; v++) votes[v] = wave_sum_i32(votes[v]);
+  for (int d = 32; d >= 1; d >>= 1) {
+    ktmax = max(ktmax, __shfl_xor(ktmax, d));
+    bad = max(bad, __shfl_xor(bad, d));
   }
+  opmax = wave_max_i64(opmax);
+  if (lane == 0)   // lane 0 holds the block's first candidate, so its M
+    stat[b] = BlkStat{t0, opmax, fl, (int)M, (int)N, nt, kt, ktmax, bad, {votes[0], votes[1], votes[2], votes[3]}};
 }
 
-// ---- K5: scans over result blocks ---------------------------------------
-__global__ void __launch_bounds__(1024) k_plan_scan(int n, const int64_t* size, const int64_t* ntask,
-                                                    const double* flops, int64_t* c_off,
-                                                    int64_t* task_off, PlanHdr* hdr) {
-  __shared__ int64_t lds[32];
-  __shared__ double red[16];
-  int64_t cs = 0, ct = 0;
-  double fsum = 0.0;
-  for (int base = 0; base < n; base += 1024) {
-    int i = base + threadIdx.x;
-    int64_t s = i < n ? size[i] : 0, t = i < n ? ntask[i] : 0;
-    double f = i < n ? flops[i] : 0.0;
-    int64_t ts, tt;
-    int64_t ps = block_excl_scan<1024>(s, lds, &ts);
-    int64_t pt = block_excl_scan<1024>(t, lds, &tt);
+// ---- scan over the result blocks (one workgroup) --------------------------
+// Packed offsets and the block table, on the device and in pinned host memory
+// (hcb, when the table is read back that way), the result's index table, and
+// the totals.  The per-shape totals of the tile choice are a wave's each.
+__global__ void __launch_bounds__(kPlanThreads) k_plan_scan(MetaView A, MetaView B, PairSpec ps, const BlkStat* stat,
+                                                            int TK, int64_t* c_off, int* c_idx, CBlock* cblk,
+                                                            CBlock* hcb, PlanHdr* hdr, PlanHdr* host) {
+  __shared__ int64_t lds[kPlanThreads / 64];
+  __shared__ PlanHdr H;
+  const int n = (int)hdr->nblocksC, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
+  for (int k = tid; k < (int)(sizeof(PlanHdr) / 8); k += blockDim.x) ((int64_t*)&H)[k] = 0;
+  __syncthreads();
+  if (tid == 0) {
+    H.nQ = hdr->nQ;
+    H.nblocksC = n;
+    H.ncand = hdr->ncand;
+  }
+  int64_t total = 0, nt = 0, opmax = 0;
+  int vote[4] = {0, 0, 0, 0}, nkt = 0, nmax = 0, ktmax = 0, bad = 0;
+  double fl = 0.0;
+  for (int base = 0; base < n; base += blockDim.x) {
+    const int i = base + tid;
+    BlkStat s{};
+    if (i < n) s = stat[i];
+    int64_t tot;
+    const int64_t off = total + block_prefix((int64_t)s.M * s.N, lds, &tot);
     if (i < n) {
-      c_off[i] = cs + ps;
-      task_off[i] = ct + pt;
+      const CBlock cb{off, s.M, s.N, (int)s.t0, (int)(s.t0 + s.nt), s.nkt, 0};
+      c_off[i] = off;
+      cblk[i] = cb;
+      if (hcb) hcb[i] = cb;
+      nt += s.nt;
+      fl += s.flops;
+      nkt = max(nkt, s.nkt);
+      if (s.nt) nmax = max(nmax, s.N);
+      ktmax = max(ktmax, s.ktmax);
+      opmax = s.opmax > opmax ? s.opmax : opmax;
+      bad |= s.bad;
+      for (int v = 0; v < 4; v++) vote[v] += s.votes[v];
     }
-    fsum += block_sum<1024>(f, red);
-    cs += ts;
-    ct += tt;
+    total += tot;
   }
-  if (threadIdx.x == 0) {
-    c_off[n] = cs;
-    task_off[n] = ct;
-    hdr->totalC = cs;
-    hdr->ntasks = ct;
-    hdr->flops = fsum;
+  // the workgroup's totals: a wave's by shuffles, the waves' by LDS atomics
+  // (integers and maxima; the FLOP count is a sum of whole numbers)
+  nt = wave_sum_i64(nt);
+  fl = wave_sum_f64(fl);
+  opmax = wave_max_i64(opmax);
+  for (int v = 0; v < 4; v++) vote[v] = wave_sum_i32(vote[v]);
+  for (int d = 32; d >= 1; d >>= 1) {
+    nkt = max(nkt, __shfl_xor(nkt, d));
+    nmax = max(nmax, __shfl_xor(nmax, d));
+    ktmax = max(ktmax, __shfl_xor(ktmax, d));
+    bad |= __shfl_xor(bad, d);
   }
+  typedef unsigned long long u64;
+  if (lane == 0) {
+    atomicAdd((u64*)&H.ntasks, (u64)nt);
+    atomicAdd(&H.flops, fl);
+    atomicMax((u64*)&H.kmax, (u64)((int64_t)nkt * TK));
+    atomicMax((u64*)&H.nmax, (u64)nmax);
+    atomicMax((u64*)&H.ktmax, (u64)ktmax);
+    atomicMax((u64*)&H.opmax, (u64)opmax);
+    for (int v = 0; v < 4; v++) atomicAdd((u64*)&H.votes[v], (u64)vote[v]);
+    if (bad) atomicAdd((u64*)&H.err, 1ull);
+  }
+  // tile-choice totals: wave w takes shapes w, w + nw, ...
+  for (int c = wave; c < TILE_NCFG; c += nw) {
+    const int TM = cfg_tm(c), TN = cfg_tn(c);
+    int64_t tiles = 0;
+    double padded = 0.0;
+    for (int i = lane; i < n; i += 64) {
+      const int tm = (stat[i].M + TM - 1) / TM, tn = (stat[i].N + TN - 1) / TN;
+      tiles += (int64_t)tm * tn;
+      padded += (double)(tm * TM) * (double)(tn * TN) * ((double)stat[i].nkt * TK);
+    }
+    tiles = wave_sum_i64(tiles);
+    padded = wave_sum_f64(padded);
+    if (lane == 0) {
+      H.tiles[c] = tiles;
+      H.padded[c] = padded;
+    }
+  }
+  // the result's sectors: A's free indices, then B's
+  {
+    int o = 0;
+    for (int j = 0; j < ps.nfa + ps.nfb; j++) {
+      const MetaView& S = j < ps.nfa ? A : B;
+      const int p = j < ps.nfa ? ps.fa[j] : ps.fb[j - ps.nfa], len = 3 * S.nsec[p];
+      for (int e = tid; e < len; e += blockDim.x) c_idx[o + e] = S.idx[3 * S.idx_off[p] + e];
+      o += len;
+    }
+  }
+  if (tid == 0) {
+    c_off[n] = total;
+    H.totalC = total;
+  }
+  __syncthreads();
+  for (int k = tid; k < (int)(sizeof(PlanHdr) / 8); k += blockDim.x) ((int64_t*)host)[k] = ((const int64_t*)&H)[k];
 }
 
 }  // namespace ttg
@@ -687,11 +837,12 @@ int plan_clone(const ttg_plan_s& src, int prec, ttg_plan* out) {
   p->prec = prec;
   p->nblocksC = src.nblocksC;
   p->ntasks = src.ntasks;
+  p->ncand = src.ncand;
   p->flops = src.flops;
   p->cfg = src.cfg;   // packed_in / split_out start false: the new operator sets them
   p->a_mcontig = src.a_mcontig;
   p->b_kcontig = src.b_kcontig;
-  const int64_t nt = std::max<int64_t>(1, p->ntasks);
+  const int64_t nt = p->ncand;
   const int64_t nb = std::max<int64_t>(1, p->nblocksC);
   p->d_tasks = dalloc<GemmTask>(nt);
   p->d_cblk = dalloc<CBlock>(nb);
@@ -716,11 +867,18 @@ int plan_clone(const ttg_plan_s& src, int prec, ttg_plan* out) {
   return 0;
 }
 
-// pinned host copy of a plan header, allocated once for the process: plans
-// are built one at a time, and every read of it follows a stream sync
-static PlanHdr* pinned_hdr() {
-  static PlanHdr* h = nullptr;
-  if (!h && hipHostMalloc((void**)&h, sizeof(PlanHdr)) != hipSuccess) {
+// pinned host memory that the planning kernels write: two headers (group
+// pass, scan pass) and the block table of plans of up to kPlanHostBlocks
+// blocks.  Allocated once for the process: plans are built one at a time, and
+// every read of it follows a stream sync.
+constexpr int kPlanHostBlocks = 8192;
+struct PlanHost {
+  PlanHdr groups, scan;
+  CBlock cb[kPlanHostBlocks];
+};
+static PlanHost* plan_host() {
+  static PlanHost* h = nullptr;
+  if (!h && hipHostMalloc((void**)&h, sizeof(PlanHost)) != hipSuccess) {
     (void)hipGetLastError();
     h = nullptr;
   }
@@ -764,90 +922,89 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
   hipStream_t s = stream();
   // scratch (returned to the pool on every exit path)
   Scratch sc;
-  KeyArrays k{};
+  PlanSets w{};
   const int nmax = std::max(1, std::max(nA, nB));
-  k.kUL = sc.get<uint64_t>(nmax); k.kSA = sc.get<uint64_t>(nmax); k.kUR = sc.get<uint64_t>(nmax);
-  k.kUM = sc.get<uint64_t>(nmax); k.kSB = sc.get<uint64_t>(nmax);
-  k.sUL = sc.get<uint64_t>(nmax); k.sSA = sc.get<uint64_t>(nmax); k.sUR = sc.get<uint64_t>(nmax);
-  k.sUM = sc.get<uint64_t>(nmax); k.sSB = sc.get<uint64_t>(nmax);
-  k.vSA = sc.get<int>(nmax); k.vSB = sc.get<int>(nmax); k.svSA = sc.get<int>(nmax); k.svSB = sc.get<int>(nmax);
-  uint64_t* uL = sc.get<uint64_t>(nmax);
-  uint64_t* uR = sc.get<uint64_t>(nmax);
-  uint64_t* uM = sc.get<uint64_t>(nmax);
-  QTab q{};
-  q.qL0 = sc.get<int>(nmax); q.qL1 = sc.get<int>(nmax); q.qR0 = sc.get<int>(nmax);
-  q.qR1 = sc.get<int>(nmax); q.qM0 = sc.get<int>(nmax); q.qM1 = sc.get<int>(nmax);
-  q.qbase = sc.get<int64_t>(nmax + 1);
+  const bool small = nmax <= kPlanSmall;
+  for (uint64_t** k : {&w.sUL, &w.sSA, &w.sUR, &w.sSB, &w.uL, &w.uR}) *k = sc.get<uint64_t>(nmax);
+  for (int** v : {&w.svSA, &w.svUR, &w.svSB, &w.lsa0, &w.lcnt, &w.rrep, &w.qL0, &w.qL1, &w.qR0, &w.qR1})
+    *v = sc.get<int>(nmax);
+  w.lpre = sc.get<int>(nmax + 1);
+  w.qbase = sc.get<int64_t>(nmax + 1);
+  w.qcand = sc.get<int64_t>(nmax + 1);
+  if (!small)
+    for (uint64_t** k : {&w.kUL, &w.kSA, &w.kUR, &w.kSB}) *k = sc.get<uint64_t>(nmax);
   PlanHdr* d_hdr = sc.get<PlanHdr>(1);
   TTG_TRY(sc.ok("plan"));
-  PlanHdr* h_hdr = pinned_hdr();
-  TTG_REQUIRE(h_hdr, "plan: pinned host header allocation failed");
+  PlanHost* host = plan_host();
+  TTG_REQUIRE(host, "plan: pinned host memory allocation failed");
+  // One host wait when every (A, B) block pair could be a result block or a
+  // task without much memory: the arrays take that size.  Otherwise the counts
+  // are read back first.
+  constexpr int64_t kPlanPairs = 4096;
+  const bool one_wait = (int64_t)nA * nB <= kPlanPairs;
+  int64_t nbcap = std::max<int64_t>(1, (int64_t)nA * nB), ncap = nbcap;
 
-  hipLaunchKernelGGL(k_plan_keys, dim3((nmax + 255) / 256), dim3(256), 0, s, A->view(), B->view(),
-                     ps, k, d_hdr);
-  SortJobs jobs;
-  jobs.j[0] = {k.kUL, nullptr, k.sUL, nullptr, nA};
-  jobs.j[1] = {k.kSA, k.vSA, k.sSA, k.svSA, nA};
-  jobs.j[2] = {k.kUR, nullptr, k.sUR, nullptr, nB};
-  jobs.j[3] = {k.kUM, nullptr, k.sUM, nullptr, nB};
-  jobs.j[4] = {k.kSB, k.vSB, k.sSB, k.svSB, nB};
-  hipLaunchKernelGGL(k_rank_sort, dim3((nmax + 255) / 256, 5), dim3(256), 0, s, jobs);
-  hipLaunchKernelGGL(k_plan_unique, dim3(1), dim3(1024), 0, s, k, nA, nB, uL, uR, uM, q, d_hdr);
-  TTG_HIP(hipMemcpyAsync(h_hdr, d_hdr, sizeof(PlanHdr), hipMemcpyDeviceToHost, s));
-  TTG_HIP(hipStreamSynchronize(s));
-  const int64_t nblocksC = h_hdr->nblocksC;
-  const int nQ = (int)h_hdr->nQ;
-  const int64_t ncand = h_hdr->ncand;
-  TTG_REQUIRE(nblocksC < (1 << 30), "plan: too many result blocks");
-  TTG_REQUIRE(ncand < (1 << 30), "plan: too many block pairs");
+  if (small) {
+    int P = 2;
+    while (P < nmax) P *= 2;
+    hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(std::min(kPlanThreads, std::max(256, P))), 0, s, A->view(), B->view(),
+                       ps, P, w, d_hdr, &host->groups);
+  } else {
+    hipLaunchKernelGGL(k_plan_keys, dim3((nmax + 255) / 256), dim3(256), 0, s, A->view(), B->view(), ps, w);
+    SortJobs jobs;
+    jobs.j[0] = {w.kUL, w.sUL, nullptr, nA};
+    jobs.j[1] = {w.kSA, w.sSA, w.svSA, nA};
+    jobs.j[2] = {w.kUR, w.sUR, w.svUR, nB};
+    jobs.j[3] = {w.kSB, w.sSB, w.svSB, nB};
+    hipLaunchKernelGGL(k_rank_sort, dim3((nmax + 255) / 256, 4), dim3(256), 0, s, jobs);
+    hipLaunchKernelGGL(k_plan_groups, dim3(1), dim3(kPlanThreads), 0, s, nA, nB, w, d_hdr, &host->groups);
+  }
+  if (!one_wait) {
+    TTG_HIP(hipStreamSynchronize(s));
+    TTG_REQUIRE(host->groups.nblocksC < (1 << 30), "plan: too many result blocks");
+    TTG_REQUIRE(host->groups.ncand < (1 << 30), "plan: too many block pairs");
+    nbcap = std::max<int64_t>(1, host->groups.nblocksC);
+    ncap = std::max<int64_t>(1, host->groups.ncand);
+  }
 
-  // result structure
+  // result structure (its index table is written by the scan kernel)
   std::vector<std::pair<const TMeta*, int>> cidx;
   for (int j = 0; j < ps.nfa; j++) cidx.push_back({A.get(), ps.fa[j]});
   for (int j = 0; j < ps.nfb; j++) cidx.push_back({B.get(), ps.fb[j]});
-  MetaPtr C = meta_from_indices(cidx);
+  MetaPtr C = meta_from_indices(cidx, false);
   if (!C) return 1;
-  TTG_TRY(meta_alloc_blocks(*C, (int)nblocksC, 0));
-  BlkArrays ba{};
-  ba.size = sc.get<int64_t>(nblocksC + 1);
-  ba.ntask = sc.get<int64_t>(nblocksC + 1);
-  ba.flops = sc.get<double>(nblocksC + 1);
-  int64_t* task_off = sc.get<int64_t>(nblocksC + 1);
+  TTG_TRY(meta_alloc_blocks(*C, (int)nbcap, 0));
+  BlkStat* stat = sc.get<BlkStat>(nbcap);
   TTG_TRY(sc.ok("plan"));
-  ba.c_qi = C->d_qi;
-  EmitArrays ea{};
-  const unsigned gb = (unsigned)std::max<int64_t>(1, (nblocksC + 3) / 4);   // one wave per result block
-  // the task list is emitted right after the count pass, into arrays sized
-  // by the candidate count (an upper bound of the task count), so one
-  // read-back (header and block table) serves both passes
+  // the task list is emitted with the counts, into slots by candidate
   std::unique_ptr<ttg_plan_s> p(new ttg_plan_s());
-  const int64_t ncap = std::max<int64_t>(1, ncand);
   p->d_tasks = dalloc<GemmTask>(ncap);
-  p->d_cblk = dalloc<CBlock>(std::max<int64_t>(1, nblocksC));
+  p->d_cblk = dalloc<CBlock>(nbcap);
   p->d_tuples = dalloc<int>(6 * ncap);
   if (!p->d_tasks || !p->d_cblk || !p->d_tuples) {
     set_error(std::string("plan: ") + ttg_last_error());
     return 1;
   }
-  hipLaunchKernelGGL(k_plan_blocks, dim3(gb), dim3(256), 0, s, A->view(), B->view(), ps, k, uL, uR,
-                     uM, q, nQ, (int)nblocksC, 0, ba, ea, d_hdr, nA, nB, tk_of(prec));
-  hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(1024), 0, s, (int)nblocksC, ba.size, ba.ntask,
-                     ba.flops, C->d_off, task_off, d_hdr);
-  ba.task_off = task_off;
-  ba.c_off = C->d_off;
-  ea.tasks = p->d_tasks;
-  ea.cblk = p->d_cblk;
-  ea.tuples = p->d_tuples;
-  hipLaunchKernelGGL(k_plan_blocks, dim3(gb), dim3(256), 0, s, A->view(), B->view(), ps, k, uL, uR,
-                     uM, q, nQ, (int)nblocksC, 1, ba, ea, d_hdr, nA, nB, tk_of(prec));
+  const int stage_b = nB <= kPlanStageB;
+  hipLaunchKernelGGL(k_plan_blocks, dim3((unsigned)((nbcap + 3) / 4)), dim3(256), stage_b ? sizeof(uint64_t) * nB : 0, s,
+                     A->view(), B->view(), ps, w, stage_b, d_hdr, stat, C->d_qi, p->d_tasks, p->d_tuples, tk_of(prec));
+  const bool hcb_pinned = nbcap <= kPlanHostBlocks;
+  hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(nbcap <= 256 ? 256 : kPlanThreads), 0, s, A->view(), B->view(), ps, stat,
+                     tk_of(prec), C->d_off, C->d_idx, p->d_cblk, hcb_pinned ? host->cb : nullptr, d_hdr, &host->scan);
+  TTG_HIP(hipGetLastError());
+  TTG_HIP(hipStreamSynchronize(s));
+  const PlanHdr* h_hdr = &host->scan;
+  const int64_t nblocksC = h_hdr->nblocksC;
+  C->nblocks = (int)nblocksC;
+  p->ncand = std::max<int64_t>(1, h_hdr->ncand);
   p->hcb.resize(nblocksC);
-  {
-    const D2HPiece pc[2] = {{h_hdr, d_hdr, sizeof(PlanHdr)},
-                            {p->hcb.data(), p->d_cblk, sizeof(CBlock) * (size_t)nblocksC}};
-    TTG_TRY(d2h_wait(pc, 2));
+  if (hcb_pinned) {
+    std::copy(host->cb, host->cb + nblocksC, p->hcb.begin());
+  } else {
+    const D2HPiece pc{p->hcb.data(), p->d_cblk, sizeof(CBlock) * (size_t)nblocksC};
+    TTG_TRY(d2h_wait(&pc, 1));
   }
   TTG_REQUIRE(!h_hdr->err, "plan: operand layout needs more than two strides per GEMM dimension");
-  TTG_REQUIRE(h_hdr->ntasks <= ncand, "plan: task count above its bound");
   C->total = (size_t)h_hdr->totalC;
   // the GEMM's 32-bit byte offsets per block
   TTG_REQUIRE(h_hdr->opmax < (int64_t(1) << 28), "plan: an operand block exceeds 2^28 elements");
@@ -900,10 +1057,14 @@ int ttg_plan_info(ttg_plan p, int* nblocks, int64_t* ntasks, double* flops) {
 
 int ttg_plan_tasks_download(ttg_plan p, int* tasks6) {
   TTG_REQUIRE(p, "null plan");
+  // a block's tasks start at its first candidate's slot: packed here
+  std::vector<int> all(6 * (size_t)p->ncand);
   if (p->ntasks)
-    TTG_HIP(hipMemcpyAsync(tasks6, p->d_tuples, sizeof(int) * 6 * (size_t)p->ntasks,
-                           hipMemcpyDeviceToHost, stream()));
+    TTG_HIP(hipMemcpyAsync(all.data(), p->d_tuples, sizeof(int) * all.size(), hipMemcpyDeviceToHost, stream()));
   TTG_HIP(hipStreamSynchronize(stream()));
+  if (p->ntasks)
+    for (const CBlock& b : p->hcb)
+      tasks6 = std::copy(all.begin() + 6 * (size_t)b.t0, all.begin() + 6 * (size_t)b.t1, tasks6);
   return 0;
 }
 

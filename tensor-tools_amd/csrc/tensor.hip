@@ -77,7 +77,7 @@ int meta_shell(int rank, const int* arrows, const int* nsec, const int* qn, cons
   return 0;
 }
 
-MetaPtr meta_from_indices(const std::vector<std::pair<const TMeta*, int>>& src) {
+MetaPtr meta_from_indices(const std::vector<std::pair<const TMeta*, int>>& src, bool upload) {
   auto m = std::make_shared<TMeta>();
   m->rank = (int)src.size();
   int off = 0;
@@ -95,7 +95,15 @@ MetaPtr meta_from_indices(const std::vector<std::pair<const TMeta*, int>>& src) 
     off += s->nsec[k];
   }
   m->idx_off[m->rank] = off;
-  if (upload_idx(*m) != 0) return nullptr;
+  if (upload) {
+    if (upload_idx(*m) != 0) return nullptr;
+  } else {
+    m->d_idx = dalloc<int>(m->h_idx.size());
+    if (!m->d_idx) {
+      set_error(std::string("meta: ") + ttg_last_error());
+      return nullptr;
+    }
+  }
   return m;
 }
 

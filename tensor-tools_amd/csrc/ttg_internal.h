@@ -199,8 +199,9 @@ using MetaPtr = std::shared_ptr<TMeta>;
 // index tables only (no blocks yet)
 int meta_shell(int rank, const int* arrows, const int* nsec, const int* qn, const int* qdim,
                MetaPtr* out);
-// index tables copied from selected indices of other metas
-MetaPtr meta_from_indices(const std::vector<std::pair<const TMeta*, int>>& src);
+// index tables copied from selected indices of other metas; upload = false
+// leaves the device table for a kernel to write
+MetaPtr meta_from_indices(const std::vector<std::pair<const TMeta*, int>>& src, bool upload = true);
 int meta_alloc_blocks(TMeta& m, int nblocks, size_t total);
 
 }  // namespace ttg

@@ -70,7 +70,7 @@ __host__ __device__ inline int cfg_tn(int c) {
 
 // device header filled by the planning kernels
 struct PlanHdr {
-  int64_t nuL, nuR, nuM, nQ, nblocksC;
+  int64_t nQ, nblocksC;
   int64_t totalC, ntasks;
   double flops;
   int64_t tiles[TILE_NCFG];
@@ -80,7 +80,7 @@ struct PlanHdr {
   int64_t nmax, ktmax;           // widest output block with tasks; largest task K
   int64_t opmax;                 // largest operand block (elements) of any task
   int64_t err;
-  int64_t ncand;                 // (result block, mid) candidates: an upper bound of ntasks
+  int64_t ncand;                 // (result block, A block) candidates: an upper bound of ntasks
 };
 
 }  // namespace ttg
@@ -91,6 +91,7 @@ struct ttg_plan_s {
   int prec = TTG_FP64;
   int nblocksC = 0;
   int64_t ntasks = 0;
+  int64_t ncand = 1;             // task slots: a block's tasks are [t0, t1) of its candidates' slots
   double flops = 0;
   int cfg = ttg::TILE_64x64;
   int ntiles = 0;
