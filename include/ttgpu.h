@@ -140,7 +140,8 @@ int ttg_heff_time(ttg_heff h, ttg_tensor x, ttg_tensor y, int n, double* ms_per_
 int ttg_heff_stage_time(ttg_heff h, ttg_tensor x, int n, double* ms3);
 /* work shape the planner chose for each stage (0..10: MFMA tiles 64x64,
  * 32x32, 64x32, 32x64, 128x64, 256x16, 128x16, 64x16, 96x96, 96x32, 32x96;
- * 11: the vector-ALU kernel for K <= 32, N <= 16) and its work-item count */
+ * 11: the vector-ALU kernel for K <= 32, N <= 16; 12, 13: MFMA tiles 96x64 and
+ * 64x96, timed for operators only) and its work-item count */
 int ttg_heff_tiles(ttg_heff h, int* tile_cfg3, int* ntiles3);
 /* the plan of stage 0, 1 or 2 (L*x, *W12, *R), borrowed: valid while h
  * lives and never passed to ttg_plan_free.  For the bit-exact checks of each

@@ -1,21 +1,22 @@
-// gemm.hip -- persistent grouped block GEMM over a plan's tile list.
+// gemm.hip -- grouped block GEMM over a plan's work list.
 //
 // Every uneven block pair of a contraction runs in ONE launch.  A work item
 // is a TM x TN piece of one output block and a range of its k walk (all of
-// the block's tasks, the K contributions in the reference's mid order).  An
-// item owning the whole walk writes the tile once, so no atomics and no
-// zero-fill pass are needed (blocks without tasks are written as zeros);
-// long walks are split into pieces that write partial tiles, added in fixed
-// order by k_split_reduce (deterministic split-K).  Operand tiles are staged
-// through LDS; the next k-slice is prefetched into registers while the MFMA
-// pipe works on the current one.
+// the block's tasks, the K contributions in the reference's mid order), run by
+// one workgroup.  An item owning the whole walk writes the tile once, so no
+// atomics and no zero-fill pass are needed (blocks without tasks are written as
+// zeros); long walks are split into pieces that write partial tiles, added in
+// fixed order by k_split_reduce (deterministic split-K).  Operand tiles are
+// staged through LDS; the next k-slice is prefetched into registers while the
+// MFMA pipe works on the current one.
 //
 // K walk: a task's contraction index is k = k0 + e0*k1 (two stride
 // components).  k-tiles never straddle a k1 boundary: for each k1 the
 // k0 range is cut into chunks of TK (the last one partial, zero-filled), so
 // an operand element's address is base + row_offset + (c + kl)*s0 + k1*s1
 // with no division inside the loop; row offsets (the M or N mixed-radix
-// decomposition) are computed once per task.
+// decomposition) are computed once per task, and what is uniform in a k-tile's
+// address is a scalar register.
 //
 // MFMA building block: 16x16 output fragment per wave-instruction.
 //   FP64:   v_mfma_f64_16x16x4_f64      (A,B one double per lane)
@@ -27,288 +28,274 @@
 // The kernels pass the B fragment as the first operand and the A fragment as
 // the second, so D is the transposed tile (B^T A^T): lane l holds output
 // row l%16, and a column of C is stored by 16 consecutive lanes.
+//
+// What bounds the FP64 kernel (m=8192 and m=2048 H_eff operators): the FP64
+// matrix cores, busy for 55-70% of a launch, plus padding to 16 x 16 fragments
+// (6% and 25% more products).  Against the kernel this one replaced (8-byte
+// loads and [row][k] LDS tiles for every operand, a persistent grid with one
+// run of items per workgroup, padding to the whole tile), stage times, FP64:
+// m=8192 2.56 -> 1.9 and 2.51 -> 1.8 ms (98 and 81 GFLOP), m=2048 70 -> 57 and
+// 81 -> 77 us (1.77 GFLOP each), m=2048 on few large sectors 466 -> 383 and
+// 539 -> 410 us (15.5 GFLOP each).
 #include <algorithm>
 #include <unordered_map>
 
-#include "ttg_internal.h"
-#include "ttg_plan.h"
+#include "ttg_gemm.h"
 
 namespace ttg {
 
-typedef double v4d __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-template <typename T>
-struct MfmaOp;
-template <>
-struct MfmaOp<double> {
-  typedef v4d acc_t;
-  static __device__ __forceinline__ acc_t mac(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <>
-struct MfmaOp<float> {
-  typedef v4f acc_t;
-  static __device__ __forceinline__ acc_t mac(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
-__device__ __forceinline__ int64_t off2(int x, int e0, int64_t s0, int64_t s1) {
-  return (int64_t)(x % e0) * s0 + (int64_t)(x / e0) * s1;
+// One workgroup per work item.  Workgroups are dispatched round-robin over the
+// 8 XCDs, so workgroup b runs on XCD b % 8; the mapping gives an XCD runs of
+// kXcdRun consecutive items (neighbouring tiles of one output block share their
+// A rows / B columns through that XCD's L2).  Short runs keep the XCDs evenly
+// loaded: item costs vary along the list (sector by sector), and with one run
+// per XCD, an eighth of the list each, the CUs were idle for 23-30% of a launch.
+constexpr int kXcdRun = 16;
+__device__ __forceinline__ int xcd_item() {
+  constexpr int R = 8 * kXcdRun;
+  const int b = blockIdx.x;
+  return b / R * R + (b & 7) * kXcdRun + (b % R >> 3);
 }
-// the same in 32 bits: operand blocks are below 2^28 elements (checked by the
-// planner), so element offsets and their byte offsets fit an unsigned
-__device__ __forceinline__ unsigned off2u(int x, int e0, unsigned s0, unsigned s1) {
-  return (unsigned)(x % e0) * s0 + (unsigned)(x / e0) * s1;
+static dim3 item_grid(int nitems) {
+  constexpr int R = 8 * kXcdRun;
+  return dim3((unsigned)((nitems + R - 1) / R * R));
 }
 
-constexpr int kThreads = 256;
+// ------------------------------------------------------------------ staging
+// One operand of a workgroup's tile: TR rows (A's rows, B's columns) by TK = 16
+// k, copied from the operand's block to LDS.  A staging slot is 16 bytes: V
+// consecutive rows at one k (RC: rows contiguous in memory) or V consecutive k
+// of one row, and the LDS tile keeps that direction ([k][row] or [row][k]), so a
+// slot is stored as it was loaded and neither the stores nor the fragment reads
+// meet bank conflicts (with [row][k] for both, two thirds of the LDS cycles of a
+// row-contiguous operand were conflicts, and the LDS was 77% busy).
+// 8-byte loads take the vector memory path as long as 16-byte ones (15 cycles
+// per wave instruction and CU, whatever the alignment and the segments: 33
+// against 67 bytes per cycle).  A 16-byte load needs dword alignment only; at
+// a block's last row it reads past the row's end, by less than 16 bytes
+// (kAllocTail), and what it reads there only reaches rows of the tile that are
+// not stored.
+template <typename T, int TR, bool RC>
+struct Operand {
+  static constexpr int TK = 16, ESZ = (int)sizeof(T), V = 16 / ESZ;
+  // LDS pitches: rows of 16 k spread over the banks; rows of TR values of which
+  // the four lane groups read k and k + 4, + 8, + 12
+  static constexpr int P = RC ? TR + 4 : ESZ == 8 ? TK + 2 : TK + 4;
+  static constexpr int LDS = (RC ? TK : TR) * P;
+  static constexpr int S = TR * TK / V, N = (S + kThreads - 1) / kThreads;
+  typedef T vec __attribute__((ext_vector_type(V)));
 
-// k-walk state of one tile: task t, second k component k1, chunk start c
-struct KWalk {
-  int t, k1, c;
-};
-__device__ __forceinline__ void kwalk_next(KWalk& w, const GemmTask& g, int TK) {
-  w.c += TK;
-  if (w.c >= g.ek0) {
-    w.c = 0;
-    if (++w.k1 >= g.nk1) {
-      w.k1 = 0;
-      w.t++;
+  int row[N], k[N];        // the slots' places in the tile
+  unsigned off[N];         // their byte offsets in the block (kOOB: nothing to load)
+  vec v[N];
+  __amdgpu_buffer_rsrc_t rs;
+  unsigned sk0, sk1;       // byte strides of the two k components
+  unsigned sr0, sr1;       // and of the two row components, the first of e0 rows
+  int e0, r0, rows;        // the tile's first row, the block's rows
+  bool wide;               // slots are 16 consecutive bytes (uniform)
+
+  __device__ __forceinline__ void init(int tid) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int e = tid + kThreads * i;
+      row[i] = RC ? e % (TR / V) * V : e / (TK / V);
+      k[i] = RC ? e / (TR / V) : e % (TK / V) * V;
     }
   }
-}
-// position of k-tile kt of block cb's walk: the last task whose first k-tile
-// is <= kt (tasks[t0..t1) hold ascending kt0), then (k1, chunk) inside it
-__device__ __forceinline__ KWalk kwalk_start(const GemmTask* __restrict__ tasks, const CBlock& cb,
-                                             int kt, int TK) {
-  if (kt == 0) return KWalk{cb.t0, 0, 0};   // the walk's start (every item without split-K)
-  int lo = cb.t0, hi = cb.t1;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tasks[mid].kt0 <= kt) lo = mid;
-    else hi = mid;
+  __device__ __forceinline__ unsigned row_off(int r) const {
+    return r0 + TR <= e0 || rows <= e0 ? (unsigned)r * sr0 : off2u(r, e0, sr0, sr1);
   }
-  const int ek0 = tasks[lo].ek0, local = kt - tasks[lo].kt0;
-  const int nch = (ek0 + TK - 1) / TK;
-  return KWalk{lo, local / nch, (local % nch) * TK};
-}
-
-// Work items are taken with stride gridDim.x starting from a permuted block
-// id: workgroups are dispatched round-robin over the 8 XCDs, so block b runs
-// on XCD b % 8; the permutation gives each XCD a run of consecutive items
-// (neighbouring tiles of one output block share their A rows / B columns).
-__device__ __forceinline__ int xcd_first_item() {
-  const int G = gridDim.x, b = blockIdx.x;
-  return (G & 7) ? b : (b & 7) * (G >> 3) + (b >> 3);
-}
-
-// ------------------------------------------------------------------ operand loads
-// Raw buffer loads over one operand block: the resource's base is the block
-// start, offsets are bytes, and an offset at or above 2^31 reads as zero.
-// Row padding and the ragged end of a k chunk become such offsets, so the
-// staging loop has no branches.  Blocks are below 2^31 bytes (checked by the
-// planner), so a padding offset plus a k offset cannot wrap into range.
-constexpr unsigned kOOB = 0x80000000u;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_rsrc(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, 0x7FFFFFFF,
-                                           0x00020000);
-}
-template <typename T>
-__device__ __forceinline__ T buf_load(__amdgpu_buffer_rsrc_t r, unsigned off);
-template <>
-__device__ __forceinline__ double buf_load<double>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-}
-template <>
-__device__ __forceinline__ float buf_load<float>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-template <>
-__device__ __forceinline__ unsigned buf_load<unsigned>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
-}
+  __device__ __forceinline__ void prepare(const T* block, int64_t k0, int64_t k1, int64_t s0, int64_t s1, int em,
+                                          int first, int n) {
+    rs = block_rsrc(block);
+    sk0 = (unsigned)k0 * ESZ;
+    sk1 = (unsigned)k1 * ESZ;
+    sr0 = (unsigned)s0 * ESZ;
+    sr1 = (unsigned)s1 * ESZ;
+    e0 = em;
+    r0 = first;
+    rows = n;
+    wide = RC ? sr0 == ESZ && (rows <= e0 || e0 % V == 0) : sk0 == ESZ;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int r = r0 + row[i];
+      const bool in = (S % kThreads == 0 || (int)threadIdx.x + kThreads * i < S) && r < rows;
+      off[i] = in ? row_off(r) + (unsigned)k[i] * sk0 : kOOB;
+    }
+  }
+  // the k-tile at chunk start c of second component k1, klim k of it in the chunk
+  __device__ __forceinline__ void load(int c, int k1, int klim) {
+    const unsigned u0 = (unsigned)c * sk0 + (unsigned)k1 * sk1;
+    if (wide && klim >= TK) {
+#pragma unroll
+      for (int i = 0; i < N; i++)
+        v[i] = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(rs, off[i], u0, 0));
+    } else if (RC && wide) {
+#pragma unroll
+      for (int i = 0; i < N; i++)
+        v[i] = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(rs, k[i] < klim ? off[i] : kOOB, u0, 0));
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; i++)
+#pragma unroll
+        for (int u = 0; u < V; u++) {
+          unsigned o = off[i];
+          if (RC) {
+            const int r = r0 + row[i] + u;
+            o = o != kOOB && k[i] < klim && r < rows ? row_off(r) + (unsigned)k[i] * sk0 : kOOB;
+          } else {
+            o = o != kOOB && k[i] + u < klim ? o + u * sk0 : kOOB;
+          }
+          v[i][u] = buf_load<T>(rs, o, u0);
+        }
+    }
+  }
+  __device__ __forceinline__ void store(T* lds) const {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (S % kThreads != 0 && (int)threadIdx.x + kThreads * i >= S) continue;
+      *(vec*)&lds[RC ? k[i] * P + row[i] : row[i] * P + k[i]] = v[i];
+    }
+  }
+  // the four k (q4 .. q4 + 3) of tile row r
+  static __device__ __forceinline__ void frag(const T* lds, int r, int q4, T (&f)[4]) {
+    if constexpr (RC) {
+#pragma unroll
+      for (int u = 0; u < 4; u++) f[u] = lds[(q4 + u) * P + r];
+    } else {
+      typedef T v2t __attribute__((ext_vector_type(2)));
+      const v2t x = *(const v2t*)&lds[r * P + q4], y = *(const v2t*)&lds[r * P + q4 + 2];
+      f[0] = x[0];
+      f[1] = x[1];
+      f[2] = y[0];
+      f[3] = y[1];
+    }
+  }
+};
 
 // ------------------------------------------------------------------ FP64/FP32
-// WM x (4/WM) waves; each wave owns (TM/WM) x (TN/WN) of the tile.
+// One work item per workgroup: WM x (4/WM) waves, each (TM/WM) x (TN/WN) of the
+// tile.  The LDS tiles are double-buffered: one barrier per k-tile, the next
+// k-tile's loads in flight during the MFMAs.  MFMA j of a 16-deep k-tile takes
+// tile k = 4q + j from lane group q = lane / 16.  A wave skips the 16 x 16
+// fragments that lie outside the block, so ragged blocks pay for padding to
+// 16, not to the tile.
 //
-// Staging: element e = tid + 256 i of the TM x TK A tile (TN x TK B tile)
-// is slot i of thread tid, laid along the operand's contiguous HBM
-// direction (AM: rows, else k; BK: k, else columns) so that a wave's loads
-// coalesce.  Per task each slot keeps one 32-bit byte offset into the
-// operand block; per k-tile only the uniform (chunk, k1) offset is added.
-// LDS holds [row][k] tiles (row pitch LDK), double-buffered: one barrier per
-// k-tile.  MFMA j of a 16-deep k-tile takes tile k = 4q + j from lane group
-// q = lane / 16, so each lane reads its four k values of a row with 16-byte
-// LDS loads.
+// least waves per SIMD the register allocator has to allow
+template <typename T>
+constexpr int gemm_waves(int tm, int tn) {
+  const int f = tm * tn / 1024;   // fragments per wave
+  return tn == 16 ? 2 : sizeof(T) == 8 ? (f <= 4 ? 4 : f <= 6 ? 3 : 2) : (f <= 4 ? 4 : 3);
+}
+
 template <typename T, int TM, int TN, int WM, bool AM, bool BK, typename OutT>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(gemm_waves<T>(TM, TN))))
 k_gemm(const Tile* __restrict__ tiles, int ntiles, const CBlock* __restrict__ cblk,
        const GemmTask* __restrict__ tasks, const T* __restrict__ A, const T* __restrict__ B,
        OutT* __restrict__ C, T* __restrict__ part) {
-  constexpr int TK = 16;
-  constexpr int LDK = sizeof(T) == 8 ? TK + 2 : TK + 4;   // 16-row bank spread
-  constexpr int ESZ = (int)sizeof(T);
-  constexpr int WN = 4 / WM;
-  constexpr int FM = TM / (16 * WM), FN = TN / (16 * WN);
-  constexpr int NA = TM * TK / kThreads, NB = TN * TK / kThreads;
-  static_assert(FM >= 1 && FN >= 1 && NA >= 1 && NB >= 1, "tile shape");
-  static_assert(TM * TK % kThreads == 0 && TN * TK % kThreads == 0, "staging slots");
+  typedef Operand<T, TM, AM> OpA;
+  typedef Operand<T, TN, !BK> OpB;
+  constexpr int TK = OpA::TK;
+  constexpr int WN = 4 / WM, FM = TM / (16 * WM), FN = TN / (16 * WN);
+  static_assert(FM >= 1 && FN >= 1, "tile shape");
   typedef typename MfmaOp<T>::acc_t acc_t;
-  typedef T v2t __attribute__((ext_vector_type(2)));
-  __shared__ __attribute__((aligned(16))) T As[2][TM * LDK];
-  __shared__ __attribute__((aligned(16))) T Bs[2][TN * LDK];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
-  const int q4 = 4 * (lane >> 4), r16 = lane & 15;
-  int ar[NA], ak[NA], br[NB], bk[NB];
+  __shared__ __attribute__((aligned(16))) T As[2][OpA::LDS];
+  __shared__ __attribute__((aligned(16))) T Bs[2][OpB::LDS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM;
+  const int r16 = lane & 15, q4 = 4 * (lane >> 4);
+  const int ti = xcd_item();
+  if (ti >= ntiles) return;
+  const Tile tl = tiles[ti];
+  const CBlock cb = cblk[tl.c];
+  // fragments of this wave that lie in the block
+  const int fa = min(FM, max(0, (cb.M - tl.m0 - wm * 16 * FM + 15) >> 4));
+  const int fb = min(FN, max(0, (cb.N - tl.n0 - wn * 16 * FN + 15) >> 4));
+  acc_t acc[FM][FN];
 #pragma unroll
-  for (int i = 0; i < NA; i++) {
-    const int e = tid + kThreads * i;
-    ar[i] = AM ? e % TM : e / TK;
-    ak[i] = AM ? e / TM : e % TK;
-  }
+  for (int i = 0; i < FM; i++)
 #pragma unroll
-  for (int i = 0; i < NB; i++) {
-    const int e = tid + kThreads * i;
-    br[i] = BK ? e / TK : e % TN;
-    bk[i] = BK ? e % TK : e / TN;
-  }
-
-  for (int ti = xcd_first_item(); ti < ntiles; ti += gridDim.x) {
-    const Tile tl = tiles[ti];
-    const CBlock cb = cblk[tl.c];
-    acc_t acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++) acc[i][j] = acc_t{0, 0, 0, 0};
-
-    T ra[NA], rb[NB];
-    unsigned aoff[NA], boff[NB];
-    __amdgpu_buffer_rsrc_t rsA, rsB;
-    int cur_task = -1;
-    GemmTask g;
-    auto prepare = [&](int tt) {
-      g = tasks[tt];
-      cur_task = tt;
-      rsA = block_rsrc(A + g.a_off);
-      rsB = block_rsrc(B + g.b_off);
-      // a tile whose rows (columns) all lie in the first folded component
-      // (uniform test) needs no division to place them
-      const unsigned sam0 = (unsigned)g.sam0, sam1 = (unsigned)g.sam1, sak0 = (unsigned)g.sak0;
-      const unsigned sbn0 = (unsigned)g.sbn0, sbn1 = (unsigned)g.sbn1, sbk0 = (unsigned)g.sbk0;
-      if (tl.m0 + TM <= g.em0) {
-#pragma unroll
-        for (int i = 0; i < NA; i++) {
-          const int mg = tl.m0 + ar[i];
-          aoff[i] = mg < cb.M ? ((unsigned)mg * sam0 + (unsigned)ak[i] * sak0) * ESZ : kOOB;
+    for (int j = 0; j < FN; j++) acc[i][j] = acc_t{0, 0, 0, 0};
+  OpA oa;
+  OpB ob;
+  oa.init(tid);
+  ob.init(tid);
+  int ek0, nk1;
+  auto prepare = [&](int t) {
+    const GemmTask& g = tasks[t];
+    ek0 = g.ek0;
+    nk1 = g.nk1;
+    oa.prepare(A + g.a_off, g.sak0, g.sak1, g.sam0, g.sam1, g.em0, tl.m0, cb.M);
+    ob.prepare(B + g.b_off, g.sbk0, g.sbk1, g.sbn0, g.sbn1, g.en0, tl.n0, cb.N);
+  };
+  int left = tl.kt1 - tl.kt0;   // k-tiles still to compute
+  if (left > 0) {
+    KWalk w = kwalk_start(tasks, cb, tl.kt0, TK);
+    prepare(w.t);
+    oa.load(w.c, w.k1, ek0 - w.c);
+    ob.load(w.c, w.k1, ek0 - w.c);
+    oa.store(As[0]);
+    ob.store(Bs[0]);
+    __syncthreads();
+    int buf = 0;
+    while (left > 0) {
+      if (--left > 0) {   // next k-tile in flight during the MFMAs
+        w.c += TK;
+        if (w.c >= ek0) {
+          w.c = 0;
+          if (++w.k1 >= nk1) {
+            w.k1 = 0;
+            w.t++;
+            prepare(w.t);
+          }
         }
-      } else {
+        oa.load(w.c, w.k1, ek0 - w.c);
+        ob.load(w.c, w.k1, ek0 - w.c);
+      }
+      T bf[FN][4];
 #pragma unroll
-        for (int i = 0; i < NA; i++) {
-          const int mg = tl.m0 + ar[i];
-          aoff[i] = mg < cb.M ? (off2u(mg, g.em0, sam0, sam1) + (unsigned)ak[i] * sak0) * ESZ : kOOB;
+      for (int j = 0; j < FN; j++) OpB::frag(Bs[buf], wn * 16 * FN + j * 16 + r16, q4, bf[j]);
+#pragma unroll
+      for (int i = 0; i < FM; i++) {
+        if (i < fa) {
+          T af[4];
+          OpA::frag(As[buf], wm * 16 * FM + i * 16 + r16, q4, af);
+#pragma unroll
+          for (int j = 0; j < FN; j++)
+            if (j < fb) {
+#pragma unroll
+              for (int u = 0; u < 4; u++) acc[i][j] = MfmaOp<T>::mac(bf[j][u], af[u], acc[i][j]);
+            }
         }
       }
-      if (tl.n0 + TN <= g.en0) {
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-          const int ng = tl.n0 + br[i];
-          boff[i] = ng < cb.N ? ((unsigned)ng * sbn0 + (unsigned)bk[i] * sbk0) * ESZ : kOOB;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-          const int ng = tl.n0 + br[i];
-          boff[i] = ng < cb.N ? (off2u(ng, g.en0, sbn0, sbn1) + (unsigned)bk[i] * sbk0) * ESZ : kOOB;
-        }
+      if (left > 0) {
+        oa.store(As[buf ^ 1]);
+        ob.store(Bs[buf ^ 1]);
       }
-    };
-    auto load = [&](const KWalk& w) {
-      if (w.t != cur_task) prepare(w.t);
-      const unsigned ua = (unsigned)(((int64_t)w.c * g.sak0 + (int64_t)w.k1 * g.sak1) * ESZ);
-      const unsigned ub = (unsigned)(((int64_t)w.c * g.sbk0 + (int64_t)w.k1 * g.sbk1) * ESZ);
-      const int klim = g.ek0 - w.c;
-      if (klim >= TK) {   // the whole k-tile lies inside the chunk (uniform): no per-element test
-#pragma unroll
-        for (int i = 0; i < NA; i++) ra[i] = buf_load<T>(rsA, aoff[i] + ua);
-#pragma unroll
-        for (int i = 0; i < NB; i++) rb[i] = buf_load<T>(rsB, boff[i] + ub);
-      } else {
-#pragma unroll
-        for (int i = 0; i < NA; i++) ra[i] = buf_load<T>(rsA, ak[i] < klim ? aoff[i] + ua : kOOB);
-#pragma unroll
-        for (int i = 0; i < NB; i++) rb[i] = buf_load<T>(rsB, bk[i] < klim ? boff[i] + ub : kOOB);
-      }
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-      for (int i = 0; i < NA; i++) As[buf][ar[i] * LDK + ak[i]] = ra[i];
-#pragma unroll
-      for (int i = 0; i < NB; i++) Bs[buf][br[i] * LDK + bk[i]] = rb[i];
-    };
-    int left = tl.kt1 - tl.kt0;   // k-tiles still to compute
-    if (left > 0) {
-      KWalk w = kwalk_start(tasks, cb, tl.kt0, TK);
-      load(w);
-      store(0);
       __syncthreads();
-      int buf = 0;
-      while (left > 0) {
-        kwalk_next(w, g, TK);
-        if (--left > 0) load(w);   // next k-tile in flight during the MFMAs
-        v2t af[FM][2], bf[FN][2];
+      buf ^= 1;
+    }
+  }
+  // epilogue: the fragments hold the transposed tile (B^T A^T: the B
+  // fragment goes in as the MFMA's first operand), so lane l has rows
+  // m = l % 16 of output columns n = row(l, r) and the 16 lanes of a column
+  // store 128 contiguous bytes of the column-major M x N C block; a split
+  // piece writes its part of a TM x TN partial (column-major) to its slot
+  T* pt = tl.slot >= 0 ? part + (int64_t)tl.slot * (TM * TN) : nullptr;
 #pragma unroll
-        for (int i = 0; i < FM; i++) {
-          const T* p = &As[buf][(wm * (TM / WM) + i * 16 + r16) * LDK + q4];
-          af[i][0] = *(const v2t*)p;
-          af[i][1] = *(const v2t*)(p + 2);
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+      const int ml = wm * 16 * FM + i * 16 + r16, m = tl.m0 + ml;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int nl = wn * 16 * FN + j * 16 + MfmaOp<T>::row(lane, r), n = tl.n0 + nl;
+        if (m < cb.M && n < cb.N) {
+          if (pt) pt[ml + TM * nl] = acc[i][j][r];
+          else C[cb.c_off + m + (int64_t)cb.M * n] = (OutT)acc[i][j][r];
         }
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-          const T* p = &Bs[buf][(wn * (TN / WN) + j * 16 + r16) * LDK + q4];
-          bf[j][0] = *(const v2t*)p;
-          bf[j][1] = *(const v2t*)(p + 2);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-#pragma unroll
-          for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++)
-              acc[i][j] = MfmaOp<T>::mac(bf[j][kk >> 1][kk & 1], af[i][kk >> 1][kk & 1], acc[i][j]);
-        if (left > 0) store(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
       }
     }
-    // epilogue: the fragments hold the transposed tile (B^T A^T: the B
-    // fragment goes in as the MFMA's first operand), so lane l has rows
-    // m = l % 16 of output columns n = row(l, r) and the 16 lanes of a column
-    // store 128 contiguous bytes of the column-major M x N C block; a split
-    // piece writes its whole TM x TN partial (column-major) to its slot
-    T* pt = tl.slot >= 0 ? part + (int64_t)tl.slot * (TM * TN) : nullptr;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++) {
-        const int ml = wm * (TM / WM) + i * 16 + r16, m = tl.m0 + ml;
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const int nl = wn * (TN / WN) + j * 16 + MfmaOp<T>::row(lane, r), n = tl.n0 + nl;
-          if (pt) pt[ml + TM * nl] = acc[i][j][r];
-          else if (m < cb.M && n < cb.N) C[cb.c_off + m + (int64_t)cb.M * n] = (OutT)acc[i][j][r];
-        }
-      }
-  }
 }
 
 // ------------------------------------------------------------------ BF16X3
@@ -406,7 +393,7 @@ k_gemm_bf16x3(const Tile* __restrict__ tiles, int ntiles, const CBlock* __restri
     bkg[i] = BK ? e % 4 : e / TN;
   }
 
-  for (int ti = xcd_first_item(); ti < ntiles; ti += gridDim.x) {
+  if (const int ti = xcd_item(); ti < ntiles) {
     const Tile tl = tiles[ti];
     const CBlock cb = cblk[tl.c];
     v4f acc[FM][FN];
@@ -684,7 +671,7 @@ static void launch_reduce(const ttg_plan_s& p, void* C, hipStream_t s) {
   X(TILE_64x64, 64, 64, 2) X(TILE_32x32, 32, 32, 2) X(TILE_64x32, 64, 32, 2)                     \
   X(TILE_32x64, 32, 64, 2) X(TILE_128x64, 128, 64, 2) X(TILE_256x16, 256, 16, 4)                 \
   X(TILE_128x16, 128, 16, 4) X(TILE_64x16, 64, 16, 4) X(TILE_96x96, 96, 96, 2)                   \
-  X(TILE_96x32, 96, 32, 2) X(TILE_32x96, 32, 96, 2)
+  X(TILE_96x32, 96, 32, 2) X(TILE_32x96, 32, 96, 2) X(TILE_96x64, 96, 64, 2) X(TILE_64x96, 64, 96, 2)
 
 // the kernel instantiation that serves (precision, shape, operand layout)
 template <typename T, int TM, int TN, int WM, typename OutT>
@@ -735,16 +722,9 @@ int gemm_occupancy(int prec, int cfg, bool a_mcontig, bool b_kcontig) {
   return k ? occupancy_of(k) : 1;
 }
 
-// persistent grid: every workgroup the CUs can hold at once for this kernel,
-// at most one per work item
-static dim3 persistent_grid(const ttg_plan_s& p, const void* kernel) {
-  const int64_t g = (int64_t)occupancy_of(kernel) * rt().num_cu;
-  return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(g, p.ntiles)));
-}
-
 template <typename T, int TM, int TN, int WM, typename OutT>
 static void launch_mode(const ttg_plan_s& p, const void* A, const void* B, void* C, hipStream_t s) {
-  const dim3 grid = persistent_grid(p, fp_kernel<T, TM, TN, WM, OutT>(p.a_mcontig, p.b_kcontig));
+  const dim3 grid = item_grid(p.ntiles);
 #define TTG_L(AMv, BKv)                                                                           \
   hipLaunchKernelGGL((k_gemm<T, TM, TN, WM, AMv, BKv, OutT>), grid, dim3(kThreads), 0, s,        \
                      p.d_tiles, p.ntiles, p.d_cblk, p.d_tasks, (const T*)A, (const T*)B,        \
@@ -758,7 +738,7 @@ static void launch_mode(const ttg_plan_s& p, const void* A, const void* B, void*
 
 template <int TM, int TN, int WM, typename OutT, typename In>
 static void launch_bf16(const ttg_plan_s& p, const void* A, const void* B, void* C, hipStream_t s) {
-  const dim3 grid = persistent_grid(p, bf_kernel<TM, TN, WM, OutT, In>(p.a_mcontig, p.b_kcontig));
+  const dim3 grid = item_grid(p.ntiles);
 #define TTG_L(AMv, BKv)                                                                             \
   hipLaunchKernelGGL((k_gemm_bf16x3<TM, TN, WM, AMv, BKv, OutT, In>), grid, dim3(kThreads), 0, s, \
                      p.d_tiles, p.ntiles, p.d_cblk, p.d_tasks, (const In*)A, (const In*)B,       \

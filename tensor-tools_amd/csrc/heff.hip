@@ -147,11 +147,11 @@ int tune_stage(ttg_plan p, int stage, const void* A, const void* B, void* C, boo
   if (it != g_tuned.end()) return it->second == p->cfg ? keep() : rebuild_tiles(*p, it->second);
   int best = p->cfg;
   float best_ms = 1e30f;
-  // candidates: the analytic choice and the shapes that win on the DMRG
-  // stages (32x32, 64x32, 32x64, 96x32, 32x96: narrow tiles, many work
-  // items; 96x96 for the split-BF16 L x stage)
+  // candidates: the analytic choice and the shapes that were fastest, in some
+  // precision, on a stage of the m=512 to m=8192 operators with many small or
+  // few large sectors
   std::vector<int> cand{p->cfg};
-  for (int c : {TILE_32x32, TILE_64x32, TILE_32x64, TILE_96x32, TILE_32x96, TILE_96x96})
+  for (int c : {TILE_32x32, TILE_64x32, TILE_32x64, TILE_96x32, TILE_64x64, TILE_96x64, TILE_64x96, TILE_128x64})
     if (c != p->cfg) cand.push_back(c);
   // One timed launch per candidate, all queued before one wait.  A kernel
   // instantiation's first launch in the process (code object load) is run
@@ -173,8 +173,8 @@ int tune_stage(ttg_plan p, int stage, const void* A, const void* B, void* C, boo
   }
   for (size_t i = 0; i < cand.size(); i++) {
     const int c = cand[i];
-    const int kid = c | (p->prec << 4) | (p->a_mcontig ? 64 : 0) | (p->b_kcontig ? 128 : 0) |
-                    (out_f64 ? 256 : 0) | (p->packed_in ? 512 : 0);
+    const int kid = c | (p->prec << 5) | (p->a_mcontig ? 128 : 0) | (p->b_kcontig ? 256 : 0) |
+                    (out_f64 ? 512 : 0) | (p->packed_in ? 1024 : 0);
     // (the first candidate's extra launch: it is not timed on an idle GPU's
     // lower clock)
     const int warm = i == 0 ? 2 : (warmed.count(kid) ? 0 : 1);

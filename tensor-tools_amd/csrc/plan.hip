@@ -739,10 +739,8 @@ static int choose_cfg(const PlanHdr& h, int prec, int ncu, bool am, bool bk) {
 // slot order by the reduction pass (deterministic).  `piece` is the whole
 // walk over 6 x the CU count, so the longest item is short against the
 // launch while the partial tiles (written, then read by the reduction) stay
-// few: at 8 x the CU count the m=2048 operator's FP64 stage 3 spent ~30 us of
-// 116 us on them, at 6 x it runs in 88 us (whole matvec 0.253 ms against
-// 0.257-0.261 ms at 4 x and 5 x and 0.281 ms at 8 x; the m=8192 operator is
-// unchanged within 2%).  Items keep output-block order.
+// few: the m=2048 operator's FP64 stage 3 takes 77 us, 80-85 us at 4 x and
+// 78-79 us at 8 x and 12 x; the m=8192 operator is unchanged within 3%.
 int build_tiles(ttg_plan_s& p, const std::vector<CBlock>& cb) {
   const int TM = cfg_tm(p.cfg), TN = cfg_tn(p.cfg);
   const int64_t G = 3 * (int64_t)rt().num_cu;
@@ -774,11 +772,21 @@ int build_tiles(ttg_plan_s& p, const std::vector<CBlock>& cb) {
       }
   }
   TTG_REQUIRE(tiles.size() < (size_t)INT32_MAX && nslots < INT32_MAX, "plan: work list too long");
-  // Items stay in output-block creation order (q -> right -> left): the
-  // tiles of one block share A rows, and consecutive blocks share B blocks,
-  // so consecutive items (one XCD's run, see xcd_first_item) reuse its L2.
-  // A longest-walk-first order balanced the tail no better and ran the
-  // m=2048 and m=8192 operators 1-4% slower.
+  // Longest walks first (a counting sort, stable): workgroups are dispatched in
+  // list order as others end, so the last ones to start are the short ones.
+  // Items of equal walks stay in output-block creation order (q -> right ->
+  // left): the tiles of one block share A rows, and consecutive blocks share B
+  // blocks, through an XCD's L2.
+  if (p.cfg != TILE_SKINNY) {
+    int most = 0;
+    for (const Tile& t : tiles) most = std::max(most, t.kt1 - t.kt0);
+    std::vector<int> at(most + 2, 0);
+    for (const Tile& t : tiles) at[most - (t.kt1 - t.kt0) + 1]++;
+    for (int k = 1; k <= most + 1; k++) at[k] += at[k - 1];
+    std::vector<Tile> order(tiles.size());
+    for (const Tile& t : tiles) order[at[most - (t.kt1 - t.kt0)]++] = t;
+    tiles.swap(order);
+  }
   p.ntiles = (int)tiles.size();
   p.ngroups = (int)groups.size();
   p.nslots = nslots;
@@ -797,7 +805,7 @@ int build_tiles(ttg_plan_s& p, const std::vector<CBlock>& cb) {
 
 // replace a plan's work list by one for tile shape cfg (an MFMA shape)
 int rebuild_tiles(ttg_plan_s& p, int cfg) {
-  TTG_REQUIRE(cfg >= 0 && (cfg < TILE_NCFG || cfg == TILE_SKINNY), "plan: bad tile shape");
+  TTG_REQUIRE(cfg >= 0 && cfg < TILE_ALL, "plan: bad tile shape");
   if ((int)p.hcb.size() != p.nblocksC) {
     p.hcb.resize(p.nblocksC);
     const D2HPiece pc{p.hcb.data(), p.d_cblk, sizeof(CBlock) * p.nblocksC};
@@ -1026,6 +1034,7 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
   const bool skinny_ok = h_hdr->nmax <= kSkinnyN && h_hdr->ktmax <= kSkinnyK;
   if (force_cfg == TILE_SKINNY && skinny_ok) p->cfg = TILE_SKINNY;
   else if (force_cfg >= 0 && force_cfg < TILE_NCFG) p->cfg = force_cfg;
+  else if (force_cfg > TILE_SKINNY && force_cfg < TILE_ALL) p->cfg = force_cfg;
   else p->cfg = skinny_ok ? TILE_SKINNY
                           : choose_cfg(*h_hdr, prec, rt().num_cu, p->a_mcontig, p->b_kcontig);
   if (defer_tiles) p->tiles_pending = true;

@@ -61,7 +61,7 @@ void* dmalloc(size_t bytes) {
     set_error("device allocation of " + std::to_string(bytes) + " bytes refused (injected failure)");
     return nullptr;
   }
-  size_t sz = size_class(bytes);
+  size_t sz = size_class(bytes + kAllocTail);
   auto it = g_pool.free_list.lower_bound(sz);
   void* p = nullptr;
   if (it != g_pool.free_list.end() && it->first <= sz + sz / 4) {

@@ -100,6 +100,9 @@ int d2h_wait(const D2HPiece* pieces, int n);
 
 // caching device pool (size classes; buffers go back to the pool, reuse is
 // ordered by the library's single stream)
+// every buffer is followed by kAllocTail readable bytes, for 16-byte loads that
+// start inside it
+constexpr size_t kAllocTail = 16;
 void* dmalloc(size_t bytes);
 void dfree(void* p);
 template <class T>

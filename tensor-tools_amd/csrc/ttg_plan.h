@@ -57,14 +57,14 @@ struct PairSpec {
 enum TileCfg { TILE_64x64 = 0, TILE_32x32 = 1, TILE_64x32 = 2, TILE_32x64 = 3, TILE_128x64 = 4,
                TILE_256x16 = 5, TILE_128x16 = 6, TILE_64x16 = 7, TILE_96x96 = 8, TILE_96x32 = 9,
                TILE_32x96 = 10, TILE_NCFG = 11,
-               TILE_SKINNY = 11 };
+               TILE_SKINNY = 11, TILE_96x64 = 12, TILE_64x96 = 13, TILE_ALL };
 constexpr int kSkinnyN = 16, kSkinnyK = 32, kSkinnyRows = 256;
 __host__ __device__ inline int cfg_tm(int c) {
-  const int t[] = {64, 32, 64, 32, 128, 256, 128, 64, 96, 96, 32, kSkinnyRows};
+  const int t[] = {64, 32, 64, 32, 128, 256, 128, 64, 96, 96, 32, kSkinnyRows, 96, 64};
   return t[c];
 }
 __host__ __device__ inline int cfg_tn(int c) {
-  const int t[] = {64, 32, 32, 64, 64, 16, 16, 16, 96, 32, 96, kSkinnyN};
+  const int t[] = {64, 32, 32, 64, 64, 16, 16, 16, 96, 32, 96, kSkinnyN, 64, 96};
   return t[c];
 }
 
