@@ -7,7 +7,7 @@ dimension at the middle bond reported as w), two-site effective Hamiltonian
 L * (W35 W36) * R around the middle bond; MPS bond dimension m=2048 over
 Sz sectors -30..30 with Gaussian (sigma=9) sector dims; L, R, x N(0,1) from a
 fixed seed.  One step = one H_eff matvec y = ((L*x)*W12)*R (three grouped
-MFMA GEMM launches replayed from a HIP graph) with all operands resident in
+MFMA GEMM stages launched back to back) with all operands resident in
 HBM.  FP64 is the reported `value`; FP32 and split-BF16 (3 bf16 MFMA
 products, FP32 accumulation) are measured on the same inputs with their error
 against the FP64 result.

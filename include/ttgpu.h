@@ -116,13 +116,12 @@ int ttg_contract(ttg_tensor A, ttg_tensor B, int npairs, const int* pa, const in
  * y = ((L*x)*W12)*R with the three stages planned once for x's block list.
  * pairs3: for stage s = 0,1,2: [np, pa0, pb0, pa1, pb1, ...] concatenated.
  * prec: TTG_FP64, TTG_FP32 or TTG_BF16X3 (split-BF16, three MFMA products,
- * FP32 accumulation); the output y is always FP64.  Applies are launched
- * as one captured HIP graph per operator. */
+ * FP32 accumulation); the output y is always FP64.  An apply launches its
+ * stages on the library stream. */
 int ttg_heff_create(ttg_tensor L, ttg_tensor W12, ttg_tensor R, ttg_tensor x_like,
                     const int* pairs3, int prec, ttg_heff* out);
 /* the same operator at another precision, on src's plans (output blocks and
- * task lists copied on the device, no QN bookkeeping) and src's tile shapes,
- * applied by direct stage launches (no graph: it serves a few products);
+ * task lists copied on the device, no QN bookkeeping) and src's tile shapes;
  * src's L, W12 and R are read by both.  The FP64 twin serves the residual
  * correction of the reduced forms (tensor_davidson.cpp:255-276 computes its
  * products with the one FP64 operator) */
@@ -132,7 +131,7 @@ int ttg_heff_apply(ttg_heff h, ttg_tensor x, ttg_tensor y);
 /* algorithmic FLOPs of one apply (sum of 2*M*N*K over the 3 stages) and the
  * per-stage task counts */
 int ttg_heff_info(ttg_heff h, double* flops, int64_t* ntasks3, double* stage_flops3);
-/* device time of n whole applies (x copied in, graph launch, y copied out)
+/* device time of n whole applies
  * measured with HIP events on the library stream (ms per apply) */
 int ttg_heff_time(ttg_heff h, ttg_tensor x, ttg_tensor y, int n, double* ms_per_apply);
 /* per-stage device time (ms, mean over n runs) of the three grouped-GEMM

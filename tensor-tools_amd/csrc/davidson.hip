@@ -9,61 +9,71 @@
 
 namespace ttg {
 
-// Cyclic Jacobi (Golub & Van Loan 8.5) on an n x n symmetric matrix, one
-// thread (n <= 16).  Values ascending, vectors in columns (column-major).
-__global__ void k_small_eigh(int n, const double* __restrict__ Min, double* __restrict__ evals,
-                             double* __restrict__ evecs) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double a[16 * 16], v[16 * 16];
-  for (int i = 0; i < n * n; i++) a[i] = Min[i];
-  for (int i = 0; i < n * n; i++) v[i] = 0.0;
-  for (int i = 0; i < n; i++) v[i + n * i] = 1.0;
+// Cyclic Jacobi (Golub & Van Loan 8.5) on an n x n symmetric matrix, one wave
+// (n <= 16): every lane computes a rotation, lane k applies it to row and
+// column entries k.  The matrix comes in the kernel arguments; values
+// (ascending) and vectors (columns, column-major) go to pinned host memory.
+// (One thread with its arrays in scratch memory took 16-21 us at n = 2 and 3,
+// and three copies.)
+struct SmallMat {
+  double m[16 * 16];
+};
+__global__ void __launch_bounds__(64) k_small_eigh(int n, SmallMat Min, double* __restrict__ evals,
+                                                   double* __restrict__ evecs) {
+  __shared__ double a[16 * 16], v[16 * 16];
+  const int k = threadIdx.x;
+  for (int i = k; i < n * n; i += 64) {
+    a[i] = Min.m[i];
+    v[i] = i % n == i / n ? 1.0 : 0.0;
+  }
+  __syncthreads();
   for (int sweep = 0; sweep < 100; sweep++) {
     double off = 0.0, tot = 0.0;
     for (int i = 0; i < n * n; i++) tot += a[i] * a[i];
     for (int i = 0; i < n; i++)
       for (int j = 0; j < n; j++)
         if (i != j) off += a[i + n * j] * a[i + n * j];
-    if (off == 0.0 || off <= 1e-32 * tot) break;
+    if (off == 0.0 || off <= 1e-32 * tot) break;   // the same in every lane
     for (int p = 0; p < n - 1; p++)
       for (int q = p + 1; q < n; q++) {
-        double apq = a[p + n * q];
+        const double apq = a[p + n * q];
         if (apq == 0.0) continue;
-        double theta = (a[q + n * q] - a[p + n * p]) / (2.0 * apq);
-        double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-        double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        for (int k = 0; k < n; k++) {
-          double x = a[k + n * p], y = a[k + n * q];
+        const double theta = (a[q + n * q] - a[p + n * p]) / (2.0 * apq);
+        const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
+        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
+        __syncthreads();
+        if (k < n) {
+          const double x = a[k + n * p], y = a[k + n * q];
           a[k + n * p] = c * x - s * y;
           a[k + n * q] = s * x + c * y;
         }
-        for (int k = 0; k < n; k++) {
-          double x = a[p + n * k], y = a[q + n * k];
+        __syncthreads();
+        if (k < n) {
+          const double x = a[p + n * k], y = a[q + n * k];
           a[p + n * k] = c * x - s * y;
           a[q + n * k] = s * x + c * y;
+          const double z = v[k + n * p], w = v[k + n * q];
+          v[k + n * p] = c * z - s * w;
+          v[k + n * q] = s * z + c * w;
         }
-        for (int k = 0; k < n; k++) {
-          double x = v[k + n * p], y = v[k + n * q];
-          v[k + n * p] = c * x - s * y;
-          v[k + n * q] = s * x + c * y;
-        }
+        __syncthreads();
       }
   }
-  // stable selection sort by eigenvalue
-  int ord[16];
-  for (int i = 0; i < n; i++) ord[i] = i;
-  for (int i = 1; i < n; i++) {
-    int o = ord[i];
-    int j = i - 1;
-    while (j >= 0 && a[ord[j] + n * ord[j]] > a[o + n * o]) {
-      ord[j + 1] = ord[j];
-      j--;
+  // stable insertion sort by eigenvalue (every place gets a column, also when
+  // some of the values are not numbers)
+  __shared__ int ord[16];
+  if (k == 0)
+    for (int i = 0; i < n; i++) {
+      const double e = a[i + n * i];
+      int j = i - 1;
+      for (; j >= 0 && a[ord[j] + n * ord[j]] > e; j--) ord[j + 1] = ord[j];
+      ord[j + 1] = i;
     }
-    ord[j + 1] = o;
-  }
-  for (int j = 0; j < n; j++) {
-    evals[j] = a[ord[j] + n * ord[j]];
-    for (int i = 0; i < n; i++) evecs[i + n * j] = v[i + n * ord[j]];
+  __syncthreads();
+  if (k < n) {
+    const int o = ord[k];
+    evals[k] = a[o + n * o];
+    for (int i = 0; i < n; i++) evecs[i + n * k] = v[i + n * o];
   }
 }
 
@@ -203,13 +213,16 @@ int ttg_small_eigh(int n, const double* M, double* evals, double* evecs) {
   PhaseTimer _phase("ttg_small_eigh");
   TTG_TRY(ensure_init());
   TTG_REQUIRE(n >= 1 && n <= 16, "small_eigh: 1 <= n <= 16");
-  Scratch sc;
-  double* d = sc.get<double>(n * n * 2 + n);
-  TTG_TRY(sc.ok("small_eigh"));
-  TTG_TRY(h2d(d, M, sizeof(double) * n * n));
-  hipLaunchKernelGGL(k_small_eigh, dim3(1), dim3(64), 0, stream(), n, d, d + 2 * n * n, d + n * n);
-  const D2HPiece pc[2] = {{evecs, d + n * n, sizeof(double) * n * n}, {evals, d + 2 * n * n, sizeof(double) * n}};
-  return d2h_wait(pc, 2);
+  static double* host = nullptr;   // pinned: values, vectors
+  if (!host) TTG_HIP(hipHostMalloc((void**)&host, sizeof(double) * (16 + 16 * 16)));
+  SmallMat m;
+  std::copy(M, M + n * n, m.m);
+  hipLaunchKernelGGL(k_small_eigh, dim3(1), dim3(64), 0, stream(), n, m, host, host + 16);
+  TTG_HIP(hipGetLastError());
+  TTG_HIP(hipStreamSynchronize(stream()));
+  std::copy(host, host + n, evals);
+  std::copy(host + 16, host + 16 + n * n, evecs);
+  return 0;
 }
 
 int ttg_embed(ttg_tensor src, ttg_tensor dst) {

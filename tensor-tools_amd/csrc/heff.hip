@@ -1,6 +1,6 @@
 // heff.hip -- lazy effective Hamiltonian y = prime(-1)[((L*x)*W12)*R]
 // (big_qtensor::product, big_qtensor.cpp:23-40) as three planned grouped
-// GEMM stages replayed from one HIP graph.
+// GEMM stages on the library stream.
 //
 // The three stage plans are built once per operator (the block structure of
 // L, W12, R and x does not change inside a Davidson call).  Stage outputs
@@ -9,12 +9,17 @@
 // made once per operator).  The split-BF16 form keeps the operands of its
 // two MFMA stages (L, x, T2, R) as pre-split words (bf16 hi << 16 | bf16
 // lo, the same 4 bytes per element): L and R are split once per operator,
-// x by the graph's first kernel and T2 by the vector-ALU stage that writes
+// x by the apply's first kernel and T2 by the vector-ALU stage that writes
 // it, so the MFMA stages only regroup halves where they would split.  The
-// last stage writes y in FP64 directly into x's block layout: every output
-// block's offset is remapped to the offset of the same sector tuple in x, so
-// y and x share one block list and the Davidson vector ops stay plain
-// packed-array BLAS-1.
+// first stage reads x and the last one writes y in FP64 in x's block layout:
+// every output block's offset is remapped to the offset of the same sector
+// tuple in x, so y and x share one block list and the Davidson vector ops stay
+// plain packed-array BLAS-1.
+//
+// An apply launches its stages directly (three to six kernels).  As a captured
+// graph it needed x and y copied in and out of fixed buffers: two copies and
+// a graph launch cost 12-25 us per apply, and capturing and instantiating the
+// graph cost an operator more than the launches of the few products it serves.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -37,18 +42,12 @@ struct ttg_heff_s {
   void *Lr = nullptr, *Rr = nullptr, *xr = nullptr;
   float* W32 = nullptr;
   bool packed = false;
-  double* xbuf = nullptr;        // graph-bound input / output buffers
-  double* ybuf = nullptr;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
+  bool covers = false;           // the last stage writes every block of y
   double flops = 0;
   ~ttg_heff_s() {
     for (auto* q : p) delete q;
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     ttg::dfree(T1); ttg::dfree(T2);
     ttg::dfree(Lr); ttg::dfree(W32); ttg::dfree(Rr); ttg::dfree(xr);
-    ttg::dfree(xbuf); ttg::dfree(ybuf);
   }
 };
 
@@ -206,22 +205,22 @@ int tune_stage(ttg_plan p, int stage, const void* A, const void* B, void* C, boo
   return rebuild_tiles(*p, best);
 }
 
-// operands, output and output type (FP64 or not) of stage st
+// operands, output and output type (FP64 or not) of stage st of y = H x
 struct StageIO {
   const void* a;
   const void* b;
   void* c;
   bool f64;
 };
-static StageIO stage_io(ttg_heff h, int st) {
+static StageIO stage_io(ttg_heff h, int st, const double* x, double* y) {
   if (h->prec == TTG_FP64) {
-    if (st == 0) return {h->L->d_data, h->xbuf, h->T1, true};
+    if (st == 0) return {h->L->d_data, x, h->T1, true};
     if (st == 1) return {h->T1, h->W->d_data, h->T2, true};
-    return {h->T2, h->R->d_data, h->ybuf, true};
+    return {h->T2, h->R->d_data, y, true};
   }
   if (st == 0) return {h->Lr, h->xr, h->T1, false};
   if (st == 1) return {h->T1, h->W32, h->T2, false};
-  return {h->T2, h->Rr, h->ybuf, true};
+  return {h->T2, h->Rr, y, true};
 }
 
 // n FP64 values into a reduced form's operand format (FP32 or split words)
@@ -230,32 +229,44 @@ static void reduce_copy(const ttg_heff h, const double* src, void* dst, size_t n
   else hipLaunchKernelGGL(k_cvt_f32, dim3(grid_n(n)), dim3(256), 0, s, src, (float*)dst, n);
 }
 
-static int record(ttg_heff h, hipStream_t s) {
-  if (h->prec != TTG_FP64) reduce_copy(h, h->xbuf, h->xr, h->xm->total, s);
+// y = H x.  x is read by the first stage (or its conversion) only and y written
+// by the last one only, so they may be the same array.
+static int run(ttg_heff h, const double* x, double* y, hipStream_t s) {
+  if (h->prec != TTG_FP64) reduce_copy(h, x, h->xr, h->xm->total, s);
   for (int st = 0; st < 3; st++) {
-    const StageIO io = stage_io(h, st);
+    if (st == 2 && !h->covers) fill_f64(y, h->xm->total, 0.0);   // blocks of y no stage writes are zero
+    const StageIO io = stage_io(h, st, x, y);
     TTG_TRY(gemm_launch(*h->p[st], io.a, io.b, io.c, io.f64, s));
   }
   return 0;
 }
 
-// intermediates, reduced-form operand copies (FP32 or split words), the measured tile
-// shapes when `tune`, and (when `capture`) the captured apply graph of an
-// operator whose three plans exist; 1 with the error set on failure (the
-// caller deletes h).  An operator without a graph launches its stages
-// directly on each apply.
-static int heff_finish(ttg_heff h, bool tune, bool capture) {
+// the same for tensors: a y that is one of the operator's own operands is
+// written after the last stage has read them
+static int apply(ttg_heff h, ttg_tensor x, ttg_tensor y, hipStream_t s) {
+  if (y != h->L && y != h->W && y != h->R) return run(h, x->d_data, y->d_data, s);
+  Scratch sc;
+  double* t = sc.get<double>(h->xm->total);
+  TTG_TRY(sc.ok("heff_apply"));
+  TTG_TRY(run(h, x->d_data, t, s));
+  TTG_HIP(hipMemcpyAsync(y->d_data, t, h->xm->total * sizeof(double), hipMemcpyDeviceToDevice, s));
+  return 0;
+}
+
+// intermediates, reduced-form operand copies (FP32 or split words) and, with
+// `tune`, the measured tile shapes (on the values of x_like) of an operator
+// whose three plans exist; 1 with the error set on failure (the caller
+// deletes h)
+static int heff_finish(ttg_heff h, const double* x_like, bool tune) {
   const bool red = h->prec != TTG_FP64;
   const size_t es = red ? sizeof(float) : sizeof(double);
+  h->covers = h->p[2]->C->nblocks == h->xm->nblocks;   // distinct tuples, each remapped to a block of x
   h->T1 = dmalloc(std::max<size_t>(1, h->p[0]->C->total) * es);
   h->T2 = dmalloc(std::max<size_t>(1, h->p[1]->C->total) * es);
-  h->xbuf = dalloc<double>(h->xm->total);
-  h->ybuf = dalloc<double>(h->xm->total);
-  if (!h->T1 || !h->T2 || !h->xbuf || !h->ybuf) {
+  if (!h->T1 || !h->T2) {
     set_error("heff: allocation failed");
     return 1;
   }
-  fill_f64(h->ybuf, h->xm->total, 0.0);   // blocks of x never produced stay zero
   hipStream_t s = stream();
   if (red) {
     // split words need the vector-ALU kernel to write T2 (it does for the
@@ -278,28 +289,14 @@ static int heff_finish(ttg_heff h, bool tune, bool capture) {
     hipLaunchKernelGGL(k_cvt_f32, dim3(grid_n(h->W->m->total)), dim3(256), 0, s, h->W->d_data, h->W32,
                        h->W->m->total);
   }
-  if (tune) {   // measured tile shapes of the MFMA stages (before the graph is captured)
+  if (tune) {   // measured tile shapes of the MFMA stages
+    Scratch sc;
+    double* y = sc.get<double>(h->xm->total);
+    TTG_TRY(sc.ok("heff"));
     for (int st = 0; st < 3; st++) {
-      const StageIO io = stage_io(h, st);
+      const StageIO io = stage_io(h, st, x_like, y);
       if (tune_stage(h->p[st], st, io.a, io.b, io.c, io.f64, s)) return 1;
     }
-  }
-  if (!capture) return 0;
-  // capture the apply sequence once
-  TTG_HIP(hipStreamSynchronize(s));
-  TTG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  int rr = record(h, s);
-  hipGraph_t g = nullptr;
-  hipError_t e = hipStreamEndCapture(s, &g);
-  if (rr || e != hipSuccess) {
-    if (g) (void)hipGraphDestroy(g);
-    set_error("heff: graph capture failed");
-    return 1;
-  }
-  h->graph = g;
-  {
-    PhaseTimer _inst("heff_create: graph instantiate");
-    TTG_HIP(hipGraphInstantiate(&h->exec, g, nullptr, nullptr, 0));
   }
   return 0;
 }
@@ -338,7 +335,7 @@ int ttg_heff_create(ttg_tensor L, ttg_tensor W12, ttg_tensor R, ttg_tensor x_lik
     set_error("heff: L*x*W12*R does not reproduce x's index sectors");
     return 1;
   }
-  if (remap_to_x(h->p[2], h->xm) || heff_finish(h, true, true)) {
+  if (remap_to_x(h->p[2], h->xm) || heff_finish(h, x_like->d_data, true)) {
     delete h;
     return 1;
   }
@@ -361,10 +358,9 @@ int ttg_heff_create_twin(ttg_heff src, int prec, ttg_heff* out) {
       return 1;
     }
   }
-  // the source's tile shapes and no graph (a twin serves a few products:
-  // timing candidate shapes or capturing and instantiating a graph for it
-  // would cost more than they save)
-  if (heff_finish(h, false, false)) {
+  // the source's tile shapes (a twin serves a few products: timing candidate
+  // shapes for it would cost more than it saves)
+  if (heff_finish(h, nullptr, false)) {
     delete h;
     return 1;
   }
@@ -382,12 +378,7 @@ int ttg_heff_apply(ttg_heff h, ttg_tensor x, ttg_tensor y) {
   TTG_REQUIRE(h && x && y, "heff_apply: null argument");
   TTG_REQUIRE(same_meta(x->m, h->xm) && same_meta(y->m, h->xm),
               "heff_apply: x/y do not have the operator's block list");
-  hipStream_t s = stream();
-  const size_t bytes = h->xm->total * sizeof(double);
-  TTG_HIP(hipMemcpyAsync(h->xbuf, x->d_data, bytes, hipMemcpyDeviceToDevice, s));
-  if (h->exec) TTG_HIP(hipGraphLaunch(h->exec, s));
-  else TTG_TRY(record(h, s));
-  TTG_HIP(hipMemcpyAsync(y->d_data, h->ybuf, bytes, hipMemcpyDeviceToDevice, s));
+  TTG_TRY(apply(h, x, y, stream()));
   mark_written(y);
   return 0;
 }
@@ -407,17 +398,11 @@ int ttg_heff_time(ttg_heff h, ttg_tensor x, ttg_tensor y, int n, double* ms) {
   TTG_REQUIRE(same_meta(x->m, h->xm) && same_meta(y->m, h->xm),
               "heff_time: x/y do not have the operator's block list");
   hipStream_t s = stream();
-  const size_t bytes = h->xm->total * sizeof(double);
   hipEvent_t e0, e1;
   TTG_HIP(hipEventCreate(&e0));
   TTG_HIP(hipEventCreate(&e1));
   TTG_HIP(hipEventRecord(e0, s));
-  for (int i = 0; i < n; i++) {   // whole applies: x in, graph, y out
-    TTG_HIP(hipMemcpyAsync(h->xbuf, x->d_data, bytes, hipMemcpyDeviceToDevice, s));
-    if (h->exec) TTG_HIP(hipGraphLaunch(h->exec, s));
-    else TTG_TRY(record(h, s));
-    TTG_HIP(hipMemcpyAsync(y->d_data, h->ybuf, bytes, hipMemcpyDeviceToDevice, s));
-  }
+  for (int i = 0; i < n; i++) TTG_TRY(apply(h, x, y, s));
   TTG_HIP(hipEventRecord(e1, s));
   TTG_HIP(hipEventSynchronize(e1));
   float t = 0;
@@ -433,16 +418,17 @@ int ttg_heff_stage_time(ttg_heff h, ttg_tensor x, int n, double* ms3) {
   TTG_REQUIRE(h && x && n > 0 && ms3, "heff_stage_time: bad argument");
   TTG_REQUIRE(same_meta(x->m, h->xm), "heff_stage_time: x does not have the operator's block list");
   hipStream_t s = stream();
-  const size_t bytes = h->xm->total * sizeof(double);
-  TTG_HIP(hipMemcpyAsync(h->xbuf, x->d_data, bytes, hipMemcpyDeviceToDevice, s));
-  if (h->prec != TTG_FP64) reduce_copy(h, h->xbuf, h->xr, h->xm->total, s);
+  Scratch sc;
+  double* y = sc.get<double>(h->xm->total);
+  TTG_TRY(sc.ok("heff_stage_time"));
+  if (h->prec != TTG_FP64) reduce_copy(h, x->d_data, h->xr, h->xm->total, s);
   hipEvent_t ev[4];
   for (auto& e : ev) TTG_HIP(hipEventCreate(&e));
   float acc[3] = {0, 0, 0};
   for (int it = 0; it < n; it++) {
     TTG_HIP(hipEventRecord(ev[0], s));
     for (int st = 0; st < 3; st++) {
-      const StageIO io = stage_io(h, st);
+      const StageIO io = stage_io(h, st, x->d_data, y);
       TTG_TRY(gemm_launch(*h->p[st], io.a, io.b, io.c, io.f64, s));
       TTG_HIP(hipEventRecord(ev[st + 1], s));
     }
@@ -474,8 +460,7 @@ int ttg_heff_stage_plan(ttg_heff h, int stage, ttg_plan* out) {
 }
 
 int ttg_heff_free(ttg_heff h) {
-  if (h) TTG_HIP(hipStreamSynchronize(stream()));
-  delete h;
+  delete h;   // its buffers go back to the pool, whose reuse is ordered by the stream
   return 0;
 }
 

@@ -210,35 +210,83 @@ __global__ void k_lincomb(LinArgs a, double* __restrict__ y, size_t n) {
   }
 }
 
-// Deterministic two-pass dot: fixed 512 partial sums, then one workgroup.
-constexpr int kDotGrid = 512;
-__global__ void __launch_bounds__(256) k_dot_partial(const double* __restrict__ x,
-                                                     const double* __restrict__ y, size_t n,
-                                                     double* __restrict__ part) {
+// Deterministic dot: 512 partial sums (number c takes elements 256 c .. 256 c +
+// 255 of every stretch of 512 * 256), added in a fixed tree by the workgroup that
+// finishes last, which writes the result to pinned host memory.  A workgroup
+// forms four partial sums: what is paid besides the reading is one agent-scope
+// fence and counter update a workgroup, and 512 workgroups of 256 threads took
+// 13.3 us for 2 x 8 MB where these take 7.3.  Workgroups without elements are not
+// launched; their partial sums are zero.  (As two kernels and a copy of the
+// result a dot took 16 us of the stream, most of it between the three.)
+constexpr int kDotGrid = 128, kDotParts = 512;
+__global__ void __launch_bounds__(1024) k_dot(const double* __restrict__ x, const double* __restrict__ y, size_t n,
+                                              double* part, unsigned* done, double* out) {
+  __shared__ double red[16];
+  __shared__ bool last;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  auto wave_sum = [](double v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
+  };
   double s = 0.0;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    s += x[i] * y[i];
-  __shared__ double red[256];
-  s = block_sum<256>(s, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-__global__ void __launch_bounds__(512) k_dot_final(const double* __restrict__ part, int n,
-                                                   double* __restrict__ out) {
-  __shared__ double red[512];
-  double s = threadIdx.x < n ? part[threadIdx.x] : 0.0;
-  s = block_sum<512>(s, red);
-  if (threadIdx.x == 0) *out = s;
+  constexpr size_t S = (size_t)kDotParts * 256;
+  size_t i = blockIdx.x * (size_t)1024 + tid;
+  for (; i + 7 * S < n; i += 8 * S) {   // eight pairs of loads under way at once
+    double a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      a[j] = x[i + j * S];
+      b[j] = y[i + j * S];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) s += a[j] * b[j];
+  }
+  for (; i < n; i += S) s += x[i] * y[i];
+  s = wave_sum(s);
+  if (lane == 0) red[w] = s;
+  __syncthreads();
+  if (w == 0) {
+    if (lane < 4)
+      __hip_atomic_store(&part[4 * blockIdx.x + lane],
+                         (red[4 * lane] + red[4 * lane + 2]) + (red[4 * lane + 1] + red[4 * lane + 3]),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0)
+      last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  if (w < 8) {
+    const double v =
+        tid < 4 * (int)gridDim.x ? __hip_atomic_load(&part[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+    const double r = wave_sum(v);
+    if (lane == 0) red[w] = r;
+  }
+  __syncthreads();
+  if (w == 0) {
+    const double r = wave_sum(lane < 8 ? red[lane] : 0.0);
+    if (lane == 0) {
+      *out = r;
+      *done = 0;   // for the next call, which the stream orders after this one
+    }
+  }
 }
 
-static double* g_dot_scratch = nullptr;
-int dev_dot(const double* x, const double* y, size_t n, double* d_out) {
-  if (!g_dot_scratch) {
-    g_dot_scratch = dalloc<double>(kDotGrid);
-    TTG_REQUIRE(g_dot_scratch, "dot scratch allocation failed");
+// x . y into *out once the stream is done
+static int dev_dot(const double* x, const double* y, size_t n, double* out) {
+  static double* scratch = nullptr;   // partial sums and the counter
+  static double* host = nullptr;
+  if (!scratch) {
+    scratch = dalloc<double>(kDotParts + 1);
+    TTG_REQUIRE(scratch, "dot scratch allocation failed");
+    fill_f64(scratch, kDotParts + 1, 0.0);
   }
-  hipLaunchKernelGGL(k_dot_partial, dim3(kDotGrid), dim3(256), 0, stream(), x, y, n, g_dot_scratch);
-  hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(512), 0, stream(), g_dot_scratch, kDotGrid, d_out);
+  if (!host) TTG_HIP(hipHostMalloc((void**)&host, sizeof(double)));
+  const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>((n + 1023) / 1024, kDotGrid));
+  hipLaunchKernelGGL(k_dot, dim3(g), dim3(1024), 0, stream(), x, y, n, scratch, (unsigned*)(scratch + kDotParts), host);
+  TTG_HIP(hipGetLastError());
+  TTG_HIP(hipStreamSynchronize(stream()));
+  *out = *host;
   return 0;
 }
 
@@ -491,35 +539,18 @@ int ttg_tensor_set_random(ttg_tensor t, uint64_t seed) {
 }
 
 // ---------------------------------------------------------------- vector ops
-static double* g_scalar = nullptr;
-static double* g_scalar_host = nullptr;
-
-static int read_scalar(double* out) {
-  if (!g_scalar_host) TTG_HIP(hipHostMalloc((void**)&g_scalar_host, sizeof(double)));
-  TTG_HIP(hipMemcpyAsync(g_scalar_host, g_scalar, sizeof(double), hipMemcpyDeviceToHost, stream()));
-  TTG_HIP(hipStreamSynchronize(stream()));
-  *out = *g_scalar_host;
-  return 0;
-}
-
 int ttg_dot(ttg_tensor x, ttg_tensor y, double* out) {
   PhaseTimer _phase("ttg_dot");
   TTG_REQUIRE(x && y, "null tensor");
   TTG_REQUIRE(same_structure(x, y), "dot: tensors have different block lists");
-  if (!g_scalar) g_scalar = dalloc<double>(1);
-  TTG_REQUIRE(g_scalar, "scalar allocation failed");
-  TTG_TRY(dev_dot(x->d_data, y->d_data, x->m->total, g_scalar));
-  return read_scalar(out);
+  return dev_dot(x->d_data, y->d_data, x->m->total, out);
 }
 
 int ttg_nrm2(ttg_tensor x, double* out) {
   PhaseTimer _phase("ttg_nrm2");
   TTG_REQUIRE(x, "null tensor");
-  if (!g_scalar) g_scalar = dalloc<double>(1);
-  TTG_REQUIRE(g_scalar, "scalar allocation failed");
-  TTG_TRY(dev_dot(x->d_data, x->d_data, x->m->total, g_scalar));
   double s;
-  TTG_TRY(read_scalar(&s));
+  TTG_TRY(dev_dot(x->d_data, x->d_data, x->m->total, &s));
   *out = std::sqrt(s);
   return 0;
 }

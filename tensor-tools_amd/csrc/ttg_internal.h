@@ -229,7 +229,4 @@ int meta_dag(const TMeta& o, MetaPtr* out);
 bool same_meta(const MetaPtr& a, const MetaPtr& b);
 bool same_structure(ttg_tensor a, ttg_tensor b);
 int block_scan_sum(const int64_t* in, int64_t* out_excl, int n);
-
-// device reductions shared by the vector ops
-int dev_dot(const double* x, const double* y, size_t n, double* d_out);
 }  // namespace ttg

@@ -172,7 +172,7 @@ void* tth_big_heff(void* b, void* x) {
     return bq->op();
   )
 }
-// device time per product (ms) over n graph replays, x widened to the
+// device time per product (ms) over n products, x widened to the
 // operator's block list first; ms3: the three stage kernels timed apart
 int tth_big_time(void* b, void* x, int n, double* ms, double* ms3) {
   TTH_GUARD(-1,

@@ -199,7 +199,7 @@ class PBig:
         return _check(_lib().tth_big_heff(self.h, x.h), "heff")
 
     def time(self, x: PTensor, n: int):
-        """(ms per product over n HIP-graph replays, ms of each stage kernel)"""
+        """(ms per product over n products, ms of each stage kernel)"""
         ms = _d(0)
         ms3 = np.zeros(3)
         _ok(_lib().tth_big_time(self.h, x.h, n, C.byref(ms), ms3), "time")

@@ -268,7 +268,7 @@ def contract(A: DTensor, B: DTensor, pairs, prec=FP64) -> DTensor:
 
 
 class Heff:
-    """y = ((L*x)*W12)*R, three planned stages replayed from a HIP graph."""
+    """y = ((L*x)*W12)*R, three planned stages."""
 
     def __init__(self, L: DTensor, W12: DTensor, R: DTensor, x_like: DTensor, pairs3, prec=FP64):
         enc = []
