@@ -240,7 +240,7 @@ int ttg_embed(ttg_tensor src, ttg_tensor dst) {
   int* err = sc.get<int>(1);
   TTG_TRY(sc.ok("embed"));
   int herr = 0;
-  TTG_HIP(hipMemsetAsync(err, 0, sizeof(int), s));
+  TTG_TRY(h2d(err, &herr, sizeof(int)));
   fill_f64(dst->d_data, dst->m->total, 0.0);
   if (nd) {
     hipLaunchKernelGGL(k_tuple_keys, dim3((nd + 255) / 256), dim3(256), 0, s, dst->m->view(), keys, ids);

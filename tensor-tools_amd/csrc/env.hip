@@ -101,7 +101,7 @@ int ttg_env_update(ttg_tensor psi, ttg_tensor env, ttg_tensor W, int direction, 
   TTG_TRY(ensure_init());
   const EnvPairs e = env_pairs(direction);
   MetaPtr psid;
-  TTG_TRY(meta_dag(*psi->m, &psid));
+  TTG_TRY(meta_dag(psi->m, &psid));
   TTG_TRY(check_pairs(*psid, *env->m, e.n[0], e.pa[0], e.pb[0], 0));
   std::unique_ptr<ttg_plan_s> p[3];
   {

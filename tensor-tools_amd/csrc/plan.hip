@@ -857,9 +857,10 @@ int plan_clone(const ttg_plan_s& src, int prec, ttg_plan* out) {
   p->d_tuples = dalloc<int>(6 * nt);
   TTG_REQUIRE(p->d_tasks && p->d_cblk && p->d_tuples, (std::string("plan: ") + ttg_last_error()).c_str());
   hipStream_t s = stream();
-  TTG_HIP(hipMemcpyAsync(p->d_tasks, src.d_tasks, sizeof(GemmTask) * nt, hipMemcpyDeviceToDevice, s));
-  TTG_HIP(hipMemcpyAsync(p->d_cblk, src.d_cblk, sizeof(CBlock) * nb, hipMemcpyDeviceToDevice, s));
-  TTG_HIP(hipMemcpyAsync(p->d_tuples, src.d_tuples, sizeof(int) * 6 * nt, hipMemcpyDeviceToDevice, s));
+  const DevPiece cp[3] = {{p->d_tasks, src.d_tasks, sizeof(GemmTask) * nt},
+                          {p->d_cblk, src.d_cblk, sizeof(CBlock) * nb},
+                          {p->d_tuples, src.d_tuples, sizeof(int) * 6 * nt}};
+  TTG_TRY(dev_copy(cp, 3));
   if (tk_of(prec) != tk_of(src.prec) && p->nblocksC > 0)
     hipLaunchKernelGGL(k_plan_ktiles, dim3((p->nblocksC + 255) / 256), dim3(256), 0, s, p->nblocksC,
                        p->d_cblk, p->d_tasks, tk_of(prec));

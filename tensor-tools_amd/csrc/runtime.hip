@@ -137,7 +137,65 @@ int side_join() {
   return 0;
 }
 
-// ---------------------------------------------------------------- staging
+// ---------------------------------------------------------------- copies
+// Copies between buffers of the device and pinned host memory: one launch for
+// up to kCopyPieces of them, 16 bytes a lane (the library's buffers are aligned to
+// that; single bytes at the end and for any other address).  A
+// planning call or an SVD makes a dozen copies of a few hundred bytes, and a
+// hipMemcpyAsync is a launch too (2.9 us of the GPU, as one of these is) that
+// costs the host more: the Davidson call at m=1024 took 2281 us with 73 of them and
+// takes 1808 us with 15 launches of k_copy, a 20-site sweep at m=48 107 and 98 ms
+// (4270 and 2407).
+namespace {
+constexpr int kCopyPieces = 16;
+struct CopyArgs {
+  char* dst[kCopyPieces];
+  const char* src[kCopyPieces];
+  size_t bytes[kCopyPieces];
+};
+
+__global__ void __launch_bounds__(256) k_copy(CopyArgs a) {
+  const int p = blockIdx.y;
+  char* __restrict__ d = a.dst[p];
+  const char* __restrict__ s = a.src[p];
+  const size_t n = a.bytes[p];
+  const size_t i0 = blockIdx.x * (size_t)256 + threadIdx.x, step = gridDim.x * (size_t)256;
+  const unsigned low = (unsigned)((size_t)d | (size_t)s);
+  size_t done = 0;
+  if ((low & 15) == 0) {
+    for (size_t i = i0; i < n / 16; i += step) ((uint4*)d)[i] = ((const uint4*)s)[i];
+    done = n & ~size_t(15);
+  }
+  for (size_t i = done + i0; i < n; i += step) d[i] = s[i];
+}
+
+// the pieces collected for one launch
+struct CopyList {
+  CopyArgs a;
+  int n = 0;
+};
+
+int copy_launch(CopyList& l) {
+  if (!l.n) return 0;
+  size_t most = 0;
+  for (int i = 0; i < l.n; i++) most = std::max(most, l.a.bytes[i]);
+  // four 16-byte elements a thread
+  const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>((most + 16383) / 16384, 4096));
+  hipLaunchKernelGGL(k_copy, dim3(g, l.n), dim3(256), 0, g_rt.stream, l.a);
+  l.n = 0;
+  TTG_HIP(hipGetLastError());
+  return 0;
+}
+
+int copy_add(CopyList& l, void* dst, const void* src, size_t bytes) {
+  if (!bytes) return 0;
+  if (l.n == kCopyPieces) TTG_TRY(copy_launch(l));
+  l.a.dst[l.n] = (char*)dst;
+  l.a.src[l.n] = (const char*)src;
+  l.a.bytes[l.n++] = bytes;
+  return 0;
+}
+
 // Small host-to-device copies go through a pinned ring: the bytes are copied
 // into the ring and the device copy is queued from there, so the call returns
 // at once and the caller's buffer may go out of scope (a copy queued from
@@ -145,8 +203,9 @@ int side_join() {
 // queued on the library stream; a copy that would wrap the ring first waits
 // for that stream, which has then finished every earlier copy out of the
 // ring.  Copies above a quarter of the ring are queued directly.
-namespace {
 constexpr size_t kRingBytes = size_t(8) << 20;
+// above this a copy to or from the host is left to the runtime
+constexpr size_t kCopyKernelMax = size_t(256) << 10;
 struct Ring {
   char* p = nullptr;
   size_t off = 0;
@@ -155,27 +214,44 @@ struct Readback {
   char* p = nullptr;
   size_t cap = 0;
 } g_rb;
-}  // namespace
+// uploads staged in the ring that an UploadBatch has not launched yet
+CopyList g_pending;
+int g_batches = 0;
 
-int h2d(void* dst, const void* src, size_t bytes) {
-  if (!bytes) return 0;
-  TTG_TRY(ensure_init());
-  hipStream_t s = g_rt.stream;
-  if (bytes > kRingBytes / 4) {
-    TTG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-    TTG_HIP(hipStreamSynchronize(s));   // the caller's buffer may be released on return
+// room for `bytes` in the ring; its place in *off
+int ring_room(size_t bytes, size_t* off) {
+  if (!g_ring.p) TTG_HIP(hipHostMalloc((void**)&g_ring.p, kRingBytes));
+  *off = (g_ring.off + 255) & ~size_t(255);
+  if (*off + bytes > kRingBytes) {
+    TTG_TRY(copy_launch(g_pending));
+    TTG_HIP(hipStreamSynchronize(g_rt.stream));
+    *off = 0;
+  }
+  g_ring.off = *off + bytes;
+  return 0;
+}
+
+int ring_copy(void* dst, size_t off, size_t bytes) {
+  if (bytes > kCopyKernelMax) {
+    TTG_HIP(hipMemcpyAsync(dst, g_ring.p + off, bytes, hipMemcpyHostToDevice, g_rt.stream));
     return 0;
   }
-  if (!g_ring.p) TTG_HIP(hipHostMalloc((void**)&g_ring.p, kRingBytes));
-  size_t off = (g_ring.off + 255) & ~size_t(255);
-  if (off + bytes > kRingBytes) {
-    TTG_HIP(hipStreamSynchronize(s));
-    off = 0;
-  }
-  memcpy(g_ring.p + off, src, bytes);
-  TTG_HIP(hipMemcpyAsync(dst, g_ring.p + off, bytes, hipMemcpyHostToDevice, s));
-  g_ring.off = off + bytes;
-  return 0;
+  TTG_TRY(copy_add(g_pending, dst, g_ring.p + off, bytes));
+  return g_batches ? 0 : copy_launch(g_pending);
+}
+}  // namespace
+
+UploadBatch::UploadBatch() { g_batches++; }
+UploadBatch::~UploadBatch() { (void)flush(); }
+int UploadBatch::flush() {
+  if (!open_) return 0;
+  open_ = false;
+  return --g_batches ? 0 : copy_launch(g_pending);
+}
+
+int h2d(void* dst, const void* src, size_t bytes) {
+  const H2DPiece p{src, 0, bytes};
+  return h2d_pieces(dst, &p, 1);
 }
 
 int h2d_pieces(void* dst, const H2DPiece* pieces, int n) {
@@ -185,20 +261,23 @@ int h2d_pieces(void* dst, const H2DPiece* pieces, int n) {
   TTG_TRY(ensure_init());
   hipStream_t s = g_rt.stream;
   if (total > kRingBytes / 4) {   // large: one direct copy per piece
-    for (int i = 0; i < n; i++) TTG_TRY(h2d((char*)dst + pieces[i].off, pieces[i].src, pieces[i].bytes));
+    for (int i = 0; i < n; i++)
+      if (pieces[i].bytes)
+        TTG_HIP(hipMemcpyAsync((char*)dst + pieces[i].off, pieces[i].src, pieces[i].bytes, hipMemcpyHostToDevice, s));
+    TTG_HIP(hipStreamSynchronize(s));   // the caller's buffers may be released on return
     return 0;
   }
-  if (!g_ring.p) TTG_HIP(hipHostMalloc((void**)&g_ring.p, kRingBytes));
-  size_t off = (g_ring.off + 255) & ~size_t(255);
-  if (off + total > kRingBytes) {
-    TTG_HIP(hipStreamSynchronize(s));
-    off = 0;
-  }
+  size_t off;
+  TTG_TRY(ring_room(total, &off));
   for (int i = 0; i < n; i++)
     if (pieces[i].bytes) memcpy(g_ring.p + off + pieces[i].off, pieces[i].src, pieces[i].bytes);
-  TTG_HIP(hipMemcpyAsync(dst, g_ring.p + off, total, hipMemcpyHostToDevice, s));
-  g_ring.off = off + total;
-  return 0;
+  return ring_copy(dst, off, total);
+}
+
+int dev_copy(const DevPiece* pieces, int n) {
+  CopyList l;
+  for (int i = 0; i < n; i++) TTG_TRY(copy_add(l, pieces[i].dst, pieces[i].src, pieces[i].bytes));
+  return copy_launch(l);
 }
 
 int d2h_wait(const D2HPiece* pieces, int n) {
@@ -214,12 +293,16 @@ int d2h_wait(const D2HPiece* pieces, int n) {
     TTG_HIP(hipHostMalloc((void**)&g_rb.p, cap));
     g_rb.cap = cap;
   }
+  CopyList l;
   size_t off = 0;
   for (int i = 0; i < n; i++) {
-    if (pieces[i].bytes)
+    if (pieces[i].bytes > kCopyKernelMax)
       TTG_HIP(hipMemcpyAsync(g_rb.p + off, pieces[i].src, pieces[i].bytes, hipMemcpyDeviceToHost, s));
+    else
+      TTG_TRY(copy_add(l, g_rb.p + off, pieces[i].src, pieces[i].bytes));
     off += (pieces[i].bytes + 255) & ~size_t(255);
   }
+  TTG_TRY(copy_launch(l));
   TTG_HIP(hipStreamSynchronize(s));
   off = 0;
   for (int i = 0; i < n; i++) {

@@ -652,11 +652,15 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
   int* rot = sc.get<int>(pitems.size());
   int* anyd = sc.get<int>(1);
   TTG_TRY(sc.ok("svd: block Jacobi"));
-  std::vector<int> hact(ns, 1);
-  TTG_TRY(h2d_vec(d_sec, sec));
-  TTG_TRY(h2d_vec(d_pit, pitems));
-  TTG_TRY(h2d_vec(d_tit, titems));
-  TTG_TRY(h2d_vec(act, hact));
+  {
+    UploadBatch up;
+    TTG_TRY(h2d_vec(d_sec, sec));
+    TTG_TRY(h2d_vec(d_pit, pitems));
+    TTG_TRY(h2d_vec(d_tit, titems));
+    TTG_TRY(h2d_vec(act, std::vector<int>(ns, 1)));
+    TTG_TRY(h2d_vec(flag, std::vector<int>(ns, 0)));
+    TTG_TRY(up.flush());
+  }
   // largest diagonal per sector and the convergence floor, on the device
   if (floor_rel > 0)
     hipLaunchKernelGGL(k_bjac_floor, dim3(ns), dim3(256), 0, s, d_sec, ns, d_goff, G, floor_rel);
@@ -666,7 +670,6 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
   // which the previous call of the same kind (LR-reduced or plain Gram
   // matrices) converged, less two: a sweep after convergence finds every
   // sector inactive and its launches return at once.
-  TTG_HIP(hipMemsetAsync(flag, 0, sizeof(int) * ns, s));
   static int prev_sweeps[2] = {0, 0};
   int& prev = prev_sweeps[floor_rel > 0 ? 1 : 0];
   const int first_check = std::max(0, prev - 2);
@@ -1282,9 +1285,11 @@ static int run_host_gemm(HostGemm& hg, const double* A, const double* B, double*
   p.d_cblk = dalloc<CBlock>(hg.cblk.size());
   TTG_REQUIRE(p.d_tasks && p.d_cblk, (std::string("svd: ") + ttg_last_error()).c_str());
   hipStream_t s = stream();
+  UploadBatch up;
   TTG_TRY(h2d_vec(p.d_tasks, hg.tasks));
   TTG_TRY(h2d_vec(p.d_cblk, hg.cblk));
   TTG_TRY(build_tiles(p, hg.cblk));
+  TTG_TRY(up.flush());
   TTG_TRY(gemm_launch(p, A, B, C, true, s));
   return 0;   // p's destructor returns the device arrays to the pool (stream-ordered reuse)
 }
@@ -1544,12 +1549,12 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   int* ssec = sc.get<int>(soff[nQ]);
   int* order = sc.get<int>(soff[nQ]);
   double* ssorted = sc.get<double>(soff[nQ]);
-  int* newdim = sc.get<int>(nQ);
   double* tout = sc.get<double>(2);
   TTG_TRY(sc.ok("svd"));
   Pack pk;
   const size_t o_moff = pk.add(moff), o_goff = pk.add(goff), o_eoff = pk.add(eoff),
-               o_soff = pk.add(soff), o_selo = pk.add(selo), o_nq = pk.add(nq), o_kq = pk.add(kq);
+               o_soff = pk.add(soff), o_selo = pk.add(selo), o_nq = pk.add(nq), o_kq = pk.add(kq),
+               o_nd = pk.add(std::vector<int>(nQ, 0)), o_bad = pk.add(std::vector<int>(1, 0));
   TTG_TRY(pk.upload(sc, "svd"));
   int64_t* d_moff = pk.at<int64_t>(o_moff);
   int64_t* d_goff = pk.at<int64_t>(o_goff);
@@ -1558,6 +1563,8 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   int64_t* d_selo = pk.at<int64_t>(o_selo);
   int* d_nq = pk.at<int>(o_nq);
   int* d_kq = pk.at<int>(o_kq);
+  int* newdim = pk.at<int>(o_nd);   // zero
+  int* bad = pk.at<int>(o_bad);     // zero
   // ---- 2. gather
   fill_f64(mat, moff[nQ], 0.0);
   hipLaunchKernelGGL(k_svd_gather, dim3(std::min(nb, 4096)), dim3(256), 0, s, m.view(), nleft,
@@ -1579,10 +1586,7 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   // a sector whose Gram matrix overflowed (entries of A above ~1e154) or that
   // holds a NaN has no meaningful eigenpairs: fail before the eigensolver
   {
-    int* bad = sc.get<int>(1);
-    TTG_TRY(sc.ok("svd"));
     int hbad = 0;
-    TTG_TRY(h2d(bad, &hbad, sizeof(int)));
     hipLaunchKernelGGL(k_svd_finite, dim3(nQ), dim3(256), 0, s, nQ, d_nq, d_goff, G, bad);
     const D2HPiece pc{&hbad, bad, sizeof(int)};
     TTG_TRY(d2h_wait(&pc, 1));
@@ -1632,7 +1636,6 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
     hipLaunchKernelGGL(k_svd_gather_sel, dim3(nQ, std::min(kmax, 64)), dim3(256), 0, s, d_nq, d_kq, d_goff,
                        Vev, d_soff, selidx, d_selo, Esel);
   }
-  TTG_HIP(hipMemsetAsync(newdim, 0, sizeof(int) * nQ, s));
   {
     const int T = (int)soff[nQ];
     if (T > 0)
@@ -1666,6 +1669,7 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   for (int j = nleft; j < m.rank; j++) rsrc.push_back({&m, j});
   MetaPtr mid;
   int arrOut = 1, arrIn = 0;
+  UploadBatch up;   // the tables of the results, in one launch
   TTG_TRY(meta_shell(1, &arrOut, &nm, mq.data(), md.data(), &mid));
   MetaPtr midIn;
   TTG_TRY(meta_shell(1, &arrIn, &nm, mq.data(), md.data(), &midIn));
@@ -1705,6 +1709,17 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   Pack pko;
   const size_t o_mid = pko.add(midnum), o_ub0 = pko.add(ublk0), o_vb0 = pko.add(vblk0), o_sout = pko.add(sout);
   TTG_TRY(pko.upload(sc, "svd"));
+  std::vector<int64_t> umo(nQ + 1, 0), wmo(nQ + 1, 0);
+  for (int q = 0; q < nQ; q++) {
+    umo[q + 1] = umo[q] + rows[q] * nd[q];
+    wmo[q + 1] = wmo[q] + (int64_t)nd[q] * cols[q];
+  }
+  Pack pkm;
+  const size_t o_umo = pkm.add(umo), o_wmo = pkm.add(wmo);
+  TTG_TRY(pkm.upload(sc, "svd"));
+  int64_t* d_umo = pkm.at<int64_t>(o_umo);
+  int64_t* d_wmo = pkm.at<int64_t>(o_wmo);
+  TTG_TRY(up.flush());
   int* d_mid = pko.at<int>(o_mid);
   int* d_ub0 = pko.at<int>(o_ub0);
   int* d_vb0 = pko.at<int>(o_vb0);
@@ -1721,19 +1736,9 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   hipLaunchKernelGGL(k_svd_svals, dim3(nQ), dim3(64), 0, s, nQ, newdim, d_soff, svals, d_sout, Sv->d_data);
   // absorbed factor: MoveFromLeft  W = E^T A (k x cols), U = E (rows x k)
   //                  MoveFromRight U = A E (rows x k),   W = E^T (k x cols)
-  std::vector<int64_t> umo(nQ + 1, 0), wmo(nQ + 1, 0);
-  for (int q = 0; q < nQ; q++) {
-    umo[q + 1] = umo[q] + rows[q] * nd[q];
-    wmo[q + 1] = wmo[q] + (int64_t)nd[q] * cols[q];
-  }
   double* Umat = sc.get<double>(umo[nQ]);
   double* Wmat = sc.get<double>(wmo[nQ]);
   TTG_TRY(sc.ok("svd"));
-  Pack pkm;
-  const size_t o_umo = pkm.add(umo), o_wmo = pkm.add(wmo);
-  TTG_TRY(pkm.upload(sc, "svd"));
-  int64_t* d_umo = pkm.at<int64_t>(o_umo);
-  int64_t* d_wmo = pkm.at<int64_t>(o_wmo);
   {
     HostGemm hg;
     for (int q = 0; q < nQ; q++) {

@@ -9,9 +9,11 @@ namespace ttg {
 
 // ---------------------------------------------------------------- meta
 TMeta::~TMeta() {
-  dfree(d_idx);
-  dfree(d_qi);
-  dfree(d_off);
+  if (!base) {
+    dfree(d_idx);
+    dfree(d_qi);
+    dfree(d_off);
+  }
   dfree(d_lut);
 }
 
@@ -145,19 +147,23 @@ bool same_structure(ttg_tensor a, ttg_tensor b) { return same_meta(a->m, b->m); 
 bool same_meta(const MetaPtr& a, const MetaPtr& b) {
   if (a == b) return true;
   if (!a || !b) return false;
-  const TMeta &x = *a, &y = *b;
+  TMeta &x = *a, &y = *b;
   if (x.nblocks != y.nblocks || x.total != y.total || !x.same_indices(y)) return false;
   // compare block lists on the host (small)
-  std::vector<int> qa((size_t)x.nblocks * x.rank), qb(qa.size());
-  if (!qa.empty()) {
-    const D2HPiece pc[2] = {{qa.data(), x.d_qi, qa.size() * sizeof(int)},
-                            {qb.data(), y.d_qi, qb.size() * sizeof(int)}};
-    if (d2h_wait(pc, 2) != 0) {
-      set_error("block list comparison: device copy failed");
-      return false;
+  const size_t n = (size_t)x.nblocks * x.rank;
+  D2HPiece pc[2];
+  int np = 0;
+  for (TMeta* m : {&x, &y})
+    if (m->h_qi.size() != n) {
+      m->h_qi.resize(n);
+      pc[np++] = {m->h_qi.data(), m->d_qi, n * sizeof(int)};
     }
+  if (np && d2h_wait(pc, np) != 0) {
+    for (int i = 0; i < np; i++) (pc[i].dst == x.h_qi.data() ? x : y).h_qi.clear();
+    set_error("block list comparison: device copy failed");
+    return false;
   }
-  return qa == qb;
+  return x.h_qi == y.h_qi;
 }
 
 // ---------------------------------------------------------------- kernels
@@ -302,24 +308,24 @@ void fill_f64(double* d, size_t n, double v) {
 }
 
 // the same sectors and block list with every arrow flipped (qtensor::dag,
-// qtensor.cpp:1575-1581): a new structure object, the blocks copied on the
-// device
-int meta_dag(const TMeta& o, MetaPtr* out) {
+// qtensor.cpp:1575-1581): a new structure object on the same device tables,
+// which nothing writes once a structure is complete
+int meta_dag(const MetaPtr& o, MetaPtr* out) {
   auto m = std::make_shared<TMeta>();
-  m->rank = o.rank;
-  m->h_idx = o.h_idx;
-  for (int j = 0; j <= MAXR; j++) m->idx_off[j] = o.idx_off[j];
-  for (int j = 0; j < o.rank; j++) {
-    m->arrow[j] = 1 - o.arrow[j];
-    m->nsec[j] = o.nsec[j];
+  m->rank = o->rank;
+  m->nblocks = o->nblocks;
+  m->total = o->total;
+  m->h_idx = o->h_idx;
+  m->h_qi = o->h_qi;
+  for (int j = 0; j <= MAXR; j++) m->idx_off[j] = o->idx_off[j];
+  for (int j = 0; j < o->rank; j++) {
+    m->arrow[j] = 1 - o->arrow[j];
+    m->nsec[j] = o->nsec[j];
   }
-  TTG_TRY(upload_idx(*m));
-  TTG_TRY(meta_alloc_blocks(*m, o.nblocks, o.total));
-  if (o.nblocks)
-    TTG_HIP(hipMemcpyAsync(m->d_qi, o.d_qi, sizeof(int) * (size_t)o.nblocks * o.rank,
-                           hipMemcpyDeviceToDevice, stream()));
-  TTG_HIP(hipMemcpyAsync(m->d_off, o.d_off, sizeof(int64_t) * ((size_t)o.nblocks + 1),
-                         hipMemcpyDeviceToDevice, stream()));
+  m->d_idx = o->d_idx;
+  m->d_qi = o->d_qi;
+  m->d_off = o->d_off;
+  m->base = o->base ? o->base : o;
   *out = m;
   return 0;
 }
@@ -341,8 +347,9 @@ int tensor_f32(ttg_tensor t, const float** out) {
 // ---------------------------------------------------------------- initBlock
 // One workgroup walks the sector combinations in chunks of 1024 (index 0
 // fastest), flags zero-flux tuples and compacts them with a block scan.
-// phase 0 counts (nblocks, total) into hdr; phase 1 writes qi and offsets.
-__global__ void __launch_bounds__(1024) k_init_blocks(MetaView m, int64_t ncomb, int phase,
+// Writes (nblocks, total) to hdr, in pinned host memory, and, if there are
+// arrays for them, qi and offsets.
+__global__ void __launch_bounds__(1024) k_init_blocks(MetaView m, int64_t ncomb,
                                                       int* __restrict__ qi_out,
                                                       int64_t* __restrict__ off_out,
                                                       int64_t* __restrict__ hdr) {
@@ -373,7 +380,7 @@ __global__ void __launch_bounds__(1024) k_init_blocks(MetaView m, int64_t ncomb,
     int64_t tot_n, tot_s;
     int64_t pn = block_excl_scan<1024>((int64_t)legal, scan_lds, &tot_n);
     int64_t ps = block_excl_scan<1024>(size, scan_lds + 32, &tot_s);
-    if (phase == 1 && legal) {
+    if (qi_out && legal) {
       int64_t b = carry_n + pn;
       for (int j = 0; j < m.rank; j++) qi_out[b * m.rank + j] = pos[j];
       off_out[b] = carry_s + ps;
@@ -384,7 +391,7 @@ __global__ void __launch_bounds__(1024) k_init_blocks(MetaView m, int64_t ncomb,
   if (threadIdx.x == 0) {
     hdr[0] = carry_n;
     hdr[1] = carry_s;
-    if (phase == 1) off_out[carry_n] = carry_s;
+    if (qi_out) off_out[carry_n] = carry_s;
   }
 }
 
@@ -398,6 +405,7 @@ int ttg_tensor_create(int rank, const int* arrows, const int* nsec, const int* q
                       const int* qdim, int nblocks, const int* block_qi, ttg_tensor* out) {
   PhaseTimer _phase("ttg_tensor_create");
   MetaPtr m;
+  UploadBatch up;
   TTG_TRY(meta_shell(rank, arrows, nsec, qn, qdim, &m));
   TTG_REQUIRE(nblocks >= 0, "nblocks < 0");
   std::vector<int64_t> off(nblocks + 1, 0);
@@ -413,6 +421,7 @@ int ttg_tensor_create(int rank, const int* arrows, const int* nsec, const int* q
   TTG_TRY(meta_alloc_blocks(*m, nblocks, (size_t)off[nblocks]));
   if (nblocks) TTG_TRY(h2d(m->d_qi, block_qi, sizeof(int) * (size_t)nblocks * rank));
   TTG_TRY(h2d_vec(m->d_off, off));
+  TTG_TRY(up.flush());
   TTG_TRY(tensor_from_meta(m, true, out));
   return 0;
 }
@@ -427,20 +436,24 @@ int ttg_tensor_init_blocks(int rank, const int* arrows, const int* nsec, const i
     ncomb *= nsec[j];
     TTG_REQUIRE(ncomb < ((int64_t)1 << 40), "initBlock: too many sector combinations");
   }
-  Scratch sc;
-  int64_t* hdr = sc.get<int64_t>(2);
-  TTG_TRY(sc.ok("initBlock"));
-  int64_t h[2];
-  hipLaunchKernelGGL(k_init_blocks, dim3(1), dim3(1024), 0, stream(), m->view(), ncomb, 0,
-                     (int*)nullptr, (int64_t*)nullptr, hdr);
-  {
-    const D2HPiece pc{h, hdr, sizeof(h)};
-    TTG_TRY(d2h_wait(&pc, 1));
+  // up to kInitOnce combinations the tables take that many entries and one
+  // launch fills them; above that a first launch counts
+  constexpr int64_t kInitOnce = 4096;
+  static int64_t* hdr = nullptr;
+  if (!hdr) TTG_HIP(hipHostMalloc((void**)&hdr, 2 * sizeof(int64_t)));
+  const bool once = ncomb <= kInitOnce;
+  if (once) TTG_TRY(meta_alloc_blocks(*m, (int)ncomb, 0));
+  hipLaunchKernelGGL(k_init_blocks, dim3(1), dim3(1024), 0, stream(), m->view(), ncomb, m->d_qi, m->d_off, hdr);
+  TTG_HIP(hipGetLastError());
+  TTG_HIP(hipStreamSynchronize(stream()));
+  TTG_REQUIRE(hdr[0] < (1 << 30), "initBlock: too many blocks");
+  if (once) {
+    m->nblocks = (int)hdr[0];
+    m->total = (size_t)hdr[1];
+  } else {
+    TTG_TRY(meta_alloc_blocks(*m, (int)hdr[0], (size_t)hdr[1]));
+    hipLaunchKernelGGL(k_init_blocks, dim3(1), dim3(1024), 0, stream(), m->view(), ncomb, m->d_qi, m->d_off, hdr);
   }
-  TTG_REQUIRE(h[0] < (1 << 30), "initBlock: too many blocks");
-  TTG_TRY(meta_alloc_blocks(*m, (int)h[0], (size_t)h[1]));
-  hipLaunchKernelGGL(k_init_blocks, dim3(1), dim3(1024), 0, stream(), m->view(), ncomb, 1,
-                     m->d_qi, m->d_off, hdr);
   return tensor_from_meta(m, true, out);
 }
 
@@ -497,7 +510,7 @@ int ttg_tensor_dag(ttg_tensor t) {
   PhaseTimer _phase("ttg_tensor_dag");
   TTG_REQUIRE(t, "null tensor");
   MetaPtr m;
-  TTG_TRY(meta_dag(*t->m, &m));
+  TTG_TRY(meta_dag(t->m, &m));
   t->m = m;
   return 0;
 }
@@ -512,10 +525,8 @@ int ttg_tensor_copy(ttg_tensor src, ttg_tensor* out) {
   PhaseTimer _phase("ttg_tensor_copy");
   TTG_REQUIRE(src, "null tensor");
   TTG_TRY(tensor_from_meta(src->m, false, out));
-  if (src->m->total)
-    TTG_HIP(hipMemcpyAsync((*out)->d_data, src->d_data, src->m->total * sizeof(double),
-                           hipMemcpyDeviceToDevice, stream()));
-  return 0;
+  const DevPiece pc{(*out)->d_data, src->d_data, src->m->total * sizeof(double)};
+  return dev_copy(&pc, 1);
 }
 
 int ttg_tensor_free(ttg_tensor t) {

@@ -89,6 +89,27 @@ struct H2DPiece {
   size_t bytes;
 };
 int h2d_pieces(void* dst, const H2DPiece* pieces, int n);
+// While one of these lives, uploads (h2d and its forms) are staged but not
+// launched; flush(), or the end of the object, launches them together.  No
+// kernel that reads an upload may be launched before.
+class UploadBatch {
+ public:
+  UploadBatch();
+  ~UploadBatch();
+  UploadBatch(const UploadBatch&) = delete;
+  UploadBatch& operator=(const UploadBatch&) = delete;
+  int flush();
+
+ private:
+  bool open_ = true;
+};
+// copies between device buffers on the library stream, several in one launch
+struct DevPiece {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+int dev_copy(const DevPiece* pieces, int n);
 // device-to-host copies of several ranges into pinned staging, one wait for
 // the library stream, then into the destinations
 struct D2HPiece {
@@ -190,6 +211,8 @@ struct TMeta {
   // lazily built: sector-combination -> block id table (for embedding)
   int* d_lut = nullptr;
   int64_t lut_size = 0;
+  std::vector<int> h_qi;           // host copy of the block list, read when it is first compared
+  std::shared_ptr<TMeta> base;     // the structure that owns d_idx, d_qi and d_off, if not this one
   ~TMeta();
   MetaView view() const;
   int q0(int j, int s) const { return h_idx[3 * (idx_off[j] + s)]; }
@@ -223,7 +246,7 @@ int tensor_from_meta(const MetaPtr& m, bool zero, ttg_tensor* out);
 inline void mark_written(ttg_tensor t) { t->version++; }
 int tensor_f32(ttg_tensor t, const float** out);
 // flipped-arrow copy of a block structure (qtensor::dag)
-int meta_dag(const TMeta& o, MetaPtr* out);
+int meta_dag(const MetaPtr& o, MetaPtr* out);
 // same index sectors and block list (hence the same packed offsets); equal
 // pointers short-cut, otherwise the block lists are compared on the host
 bool same_meta(const MetaPtr& a, const MetaPtr& b);

@@ -57,3 +57,43 @@ def test_product_over_its_input(prec):
     want = y.data()
     h.apply(dx, dx)
     assert np.array_equal(dx.data(), want)
+
+
+# list lengths at the ends of 16-byte elements, and above the size that one
+# copy launch takes (256 KiB)
+@pytest.mark.parametrize("nb", [1, 2, 3, 5, 7, 1023, 1025, 32768, 40001])
+def test_block_lists(nb):
+    n = max(2, int(np.ceil(np.sqrt(nb))))
+    i = make_index(INWARD, "i", LINK, 0, [((q, 0), 1) for q in range(n)])
+    j = make_index(OUTWARD, "j", LINK, 0, [((q, 0), 1 + q % 3) for q in range(n)])
+    qi = np.array([(b // n, b % n) for b in range(nb)], dtype=np.int32)
+    x = random_tensor([i, j], np.random.default_rng(nb), block_qi=qi)
+    a, b = T.DTensor.from_flat(x), T.DTensor.from_flat(x)
+    assert np.array_equal(np.asarray(a.meta()[0]).reshape(-1, 2), qi)
+    assert a.dot(b) == b.dot(a)          # compares the lists
+    c = a.copy()
+    T.check(T.lib().ttg_tensor_dag(a.h))
+    T.check(T.lib().ttg_tensor_dag(a.h))
+    assert a.dot(c) == c.dot(c)          # the same structure again
+    assert np.array_equal(c.data(), x.data)
+    other = qi.copy()
+    if nb > 1 and nb < n * n:            # as many blocks, one at another place
+        other[-1] = (n - 1, n - 1)
+        if tuple(other[-1]) != tuple(qi[-1]) and (n - 1) % 3 == qi[-1][1] % 3:
+            d = T.DTensor.from_flat(random_tensor([i, j], np.random.default_rng(1), block_qi=other))
+            with pytest.raises(RuntimeError):
+                a.dot(d)
+    del b, c
+
+
+def test_dag_outlives_its_source():
+    """a flipped structure shares the tables of the one it came from"""
+    rng = np.random.default_rng(0)
+    i = make_index(INWARD, "i", LINK, 0, [((q, 0), 3) for q in range(40)])
+    j = make_index(OUTWARD, "j", LINK, 0, [((q, 0), 2) for q in range(40)])
+    x = random_tensor([i, j], rng)
+    a = T.DTensor.from_flat(x)
+    T.check(T.lib().ttg_tensor_dag(a.h))   # the only holder of the first structure is now the second
+    others = [T.DTensor.from_flat(random_tensor([i, j], rng)) for _ in range(50)]
+    assert np.array_equal(np.asarray(a.meta()[0]).reshape(-1, 2), x.block_qi)
+    del others
