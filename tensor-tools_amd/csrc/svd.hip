@@ -206,17 +206,121 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // values below 1e-7 of the largest, under the Gram matrix's own resolution of
 // ~sqrt(eps)), and the rounding noise in the null space of a rank-deficient
 // sector's Gram matrix never passes the relative test alone.
+//
+// Sectors of more than 16 rows go through a pivoted Cholesky factorisation
+// P^T G P = R^T R first (as the large ones, 4c): the iteration then runs on
+// G' = R R^T, r x r, which is nearly diagonal and holds no null space, and
+// V = R^T W Lambda^(-1/2), which one Gram-Schmidt step makes orthonormal to rounding
+// (2e-15 where the rotations alone gave 2e-14).  The matrix stays in the registers of the
+// 8 waves (8 rows each), every wave keeps the remaining diagonal and finds the pivot for
+// itself, and one row a step passes through LDS.  On the sectors of an m = 100 state (up to 60
+// rows, rank-deficient) k_jacobi took 445 us and takes 89, at m = 333 531 and 258.  The route is taken
+// when the r columns are all that the selection can use: r >= kq, the values
+// kept before truncation, or a cutoff above kLrCutoff, the weight (of the
+// whole tensor's) that 64 rows below kPcTol of the largest can hold.
 constexpr double kJacFloor = 1e-14;   // convergence floor relative to the largest diagonal
+constexpr double kPcTol = 1e-15;      // a remaining diagonal below this of the largest ends the factorisation
+constexpr double kLrCutoff = kJW * kPcTol * 1.5;
 
+// LDS of k_jacobi
+struct JacLds {
+  double s[kJS];                 // the matrix, later W^T
+  double qts[2 * 4 * kJQt];
+  double r[kJS];                 // rows of R
+  double row[2][kJW];            // pivot row of a step, in turn; later the eigenvalues
+  double dmax;
+  int sig;
+};
+
+// Pivoted Cholesky of G0 (n x n): rows of R to L.r (zero beyond row r and column
+// n); returns r.  Ties go to the lower index.
+__device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, int wave, int lane) {
+  double x[8];   // G(8 wave + s, lane)
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int i = 8 * wave + s;
+    x[s] = i < n && lane < n ? 0.5 * (G0[i + (int64_t)n * lane] + G0[lane + (int64_t)n * i]) : 0.0;
+  }
+  double d = lane < n ? G0[lane * (int64_t)(n + 1)] : 0.0;
+  bool open = lane < n;
+  for (int e = threadIdx.x; e < kJS; e += kJThreads) L.r[e] = 0.0;
+  double stop = 0.0;
+  int k = 0;
+  for (; k < n; k++) {
+    const double v = open ? d : -1.0;
+    double m = v;
+    m = fmax(m, lane_xor<1>(m));
+    m = fmax(m, lane_xor<2>(m));
+    m = fmax(m, lane_xor<4>(m));
+    m = fmax(m, lane_xor<8>(m));
+    m = fmax(m, lane_xor<16>(m));
+    m = fmax(m, lane_xor<32>(m));
+    if (k == 0) stop = kPcTol * m;
+    if (!(m > stop)) break;   // the same in every wave
+    const int p = __builtin_ctzll(__ballot(v == m));
+    double* row = L.row[k & 1];
+    if (wave == p >> 3)
+#pragma unroll
+      for (int s = 0; s < 8; s++)
+        if ((p & 7) == s) row[lane] = x[s];
+    const double inv = 1.0 / sqrt(m);
+    __syncthreads();
+    const double rv = open ? (lane == p ? m : row[lane]) * inv : 0.0;
+    open = open && lane != p;
+    if (wave == 0) L.r[k * kJP + lane] = rv;
+    d = fma(-rv, rv, d);
+    typedef int i2 __attribute__((ext_vector_type(2)));
+    const i2 w = __builtin_bit_cast(i2, rv);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+      i2 u;
+      u[0] = __builtin_amdgcn_readlane(w[0], 8 * wave + s);
+      u[1] = __builtin_amdgcn_readlane(w[1], 8 * wave + s);
+      x[s] = fma(-__builtin_bit_cast(double, u), rv, x[s]);
+    }
+  }
+  __syncthreads();
+  return k;
+}
+
+// G' = R R^T into L.s (16 NPR square)
 template <int NPR>
-__device__ __forceinline__ void jacobi_sector(double* S, double* Qts, int* sig, double* red, int n, const double* G0,
-                                              double* Vg, double* ev, int max_sweeps, double floor_rel) {
+__device__ __forceinline__ void jac_gram(JacLds& L, int n, int wave, int lane) {
+  const int j = lane & 15, g = lane >> 4;
+  for (int t = wave; t < NPR * (NPR + 1) / 2; t += 8) {
+    int b = 0;
+    while ((b + 1) * (b + 2) / 2 <= t) b++;
+    const int a = t - b * (b + 1) / 2;   // a <= b
+    jac_v4d r = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 0; k < n; k += 4)
+      r = __builtin_amdgcn_mfma_f64_16x16x4f64(L.r[(16 * a + j) * kJP + k + g], L.r[(16 * b + j) * kJP + k + g], r, 0,
+                                               0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int i = 16 * a + g + 4 * s, c = 16 * b + j;
+      L.s[i * kJP + c] = r[s];
+      L.s[c * kJP + i] = r[s];
+    }
+  }
+}
+
+// Eigenpairs of the matrix G0 (n x n, r = 0) or of G' (r x r, from L.r) and from
+// them those of G0.
+template <int NPR>
+__device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, const double* G0, double* Vg, double* ev,
+                                              int max_sweeps, double floor_rel, int wave, int lane) {
   constexpr int W = 16 * NPR;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x;
+  double* S = L.s;
+  if (r == 0) {
 #pragma unroll 8
-  for (int e = tid; e < W * W; e += kJThreads) {
-    const int i = e % W, j = e / W;
-    S[j * kJP + i] = (i < n && j < n) ? 0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]) : 0.0;
+    for (int e = tid; e < W * W; e += kJThreads) {
+      const int i = e % W, j = e / W;
+      S[j * kJP + i] = (i < n && j < n) ? 0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]) : 0.0;
+    }
+  } else {
+    jac_gram<NPR>(L, n, wave, lane);
+    floor_rel = 0.0;   // the relative test alone
   }
   double vt[2 * NPR][2];
   jac_identity<NPR>(vt, wave, lane);
@@ -224,51 +328,138 @@ __device__ __forceinline__ void jacobi_sector(double* S, double* Qts, int* sig, 
   if (wave == 0) {   // largest diagonal element: the scale of the convergence floor
     double m = lane < W ? fabs(S[lane * kJP + lane]) : 0.0;
     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-    if (lane == 0) *red = m;
+    if (lane == 0) L.dmax = m;
   }
   int par = 0;
   for (int sweep = 0; sweep < max_sweeps; sweep++) {
-    if (tid == 0) *sig = 0;
+    if (tid == 0) L.sig = 0;
     __syncthreads();
-    jac_sweep<NPR>(S, Qts, vt, wave, lane, par, floor_rel * *red, sig);
+    jac_sweep<NPR>(S, L.qts, vt, wave, lane, par, floor_rel * L.dmax, &L.sig);
     __syncthreads();
     // every thread reads the flag before thread 0 may clear it for the next
     // sweep: the barrier between the read and the reset keeps the decision
     // uniform over the workgroup
-    const int rotated = *sig;
+    const int rotated = L.sig;
     __syncthreads();
     if (!rotated) break;
   }
-  for (int i = tid; i < n; i += kJThreads) ev[i] = S[i * kJP + i];
-  if (wave >= 4) {   // V(i, c) = V^T(c, i): consecutive lanes down a column of V
-    const int i = 16 * (wave - 4) + (lane & 15);
+  if (r == 0) {
+    for (int i = tid; i < n; i += kJThreads) ev[i] = S[i * kJP + i];
+    if (wave >= 4) {   // V(i, c) = V^T(c, i): consecutive lanes down a column of V
+      const int i = 16 * (wave - 4) + (lane & 15);
+#pragma unroll
+      for (int b = 0; b < 2 * NPR; b++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int c = 8 * b + (lane >> 4) + 4 * h;
+          if (i < n && c < n) Vg[i + (int64_t)n * c] = vt[b][h];
+        }
+    }
+    return;
+  }
+  // V = R^T W Lambda^(-1/2); columns c >= r are zero, with eigenvalue zero
+  double* lam = L.row[0];
+  if (tid < kJW) {
+    lam[tid] = tid < r ? S[tid * kJP + tid] : 0.0;
+    if (tid < n) ev[tid] = lam[tid];
+  }
+  __syncthreads();
+  if (wave >= 4 && wave < 4 + NPR) {
 #pragma unroll
     for (int b = 0; b < 2 * NPR; b++)
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int c = 8 * b + (lane >> 4) + 4 * h;
-        if (i < n && c < n) Vg[i + (int64_t)n * c] = vt[b][h];
-      }
+      for (int h = 0; h < 2; h++) S[(8 * b + (lane >> 4) + 4 * h) * kJP + 16 * (wave - 4) + (lane & 15)] = vt[b][h];
   }
+  __syncthreads();
+  // tiles (a, b) of V^T: rows c, columns i; X = V^T (r rows) afterwards in L.r
+  const int j = lane & 15, g = lane >> 4, nt = (n + 15) / 16;
+  constexpr int kMine = (NPR * 4 + 7) / 8;   // tiles a wave can have
+  jac_v4d v[kMine];
+#pragma unroll
+  for (int u = 0; u < kMine; u++) {
+    const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
+    v[u] = {0.0, 0.0, 0.0, 0.0};
+    if (t < NPR * nt) {
+#pragma unroll
+      for (int k = 0; k < W; k += 4)
+        v[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * a + j) * kJP + k + g], L.r[(k + g) * kJP + 16 * b + j], v[u],
+                                                    0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const double l = lam[16 * a + g + 4 * s];
+        v[u][s] *= l > 0.0 ? 1.0 / sqrt(l) : 0.0;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kMine; u++) {
+    const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
+    if (t < NPR * nt)
+#pragma unroll
+      for (int s = 0; s < 4; s++) L.r[(16 * a + g + 4 * s) * kJP + 16 * b + j] = v[u][s];
+  }
+  __syncthreads();
+  // X is orthonormal to the rounding of R^T W, eps sqrt(lambda_1 / lambda_c): one
+  // Gram-Schmidt step in the order of the eigenvalues takes that to eps,
+  // X <- C X, C(c, a) = -(X X^T)(c, a) for lambda_a > lambda_c, (3 - |x_c|^2) / 2 at c
+  for (int t = wave; t < NPR * (NPR + 1) / 2; t += 8) {
+    int b = 0;
+    while ((b + 1) * (b + 2) / 2 <= t) b++;
+    const int a = t - b * (b + 1) / 2;
+    jac_v4d m = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 0; k < n; k += 4)
+      m = __builtin_amdgcn_mfma_f64_16x16x4f64(L.r[(16 * a + j) * kJP + k + g], L.r[(16 * b + j) * kJP + k + g], m, 0, 0,
+                                               0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int i = 16 * a + g + 4 * s, c = 16 * b + j;
+      const double li = lam[i], lc = lam[c];
+      const bool first = li > lc || (li == lc && i < c);   // x_i is corrected before x_c
+      S[c * kJP + i] = i == c ? 1.5 - 0.5 * m[s] : first ? -m[s] : 0.0;
+      if (i != c) S[i * kJP + c] = first ? 0.0 : -m[s];
+    }
+  }
+  __syncthreads();
+  for (int t = wave; t < NPR * nt; t += 8) {
+    const int a = t % NPR, b = t / NPR;
+    jac_v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < W; k += 4)
+      x = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * a + j) * kJP + k + g], L.r[(k + g) * kJP + 16 * b + j], x, 0, 0,
+                                               0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int c = 16 * a + g + 4 * s, i = 16 * b + j;
+      if (i < n && c < n) Vg[i + (int64_t)n * c] = x[s];
+    }
+  }
+  for (int e = tid; e < n * (n - W); e += kJThreads) Vg[(int64_t)n * W + e] = 0.0;
 }
 
+// kq: the eigenpairs a sector can use (null: every one, no factorisation);
+// drop: fewer will do, the others are below the cutoff
 __global__ void __launch_bounds__(kJThreads)
-k_jacobi(const int* __restrict__ nq, const int64_t* __restrict__ goff, const double* __restrict__ Gin,
-         double* __restrict__ Vout, double* __restrict__ evals, const int64_t* __restrict__ eoff, int max_sweeps,
-         int nmax_here, double floor_rel) {
-  __shared__ __attribute__((aligned(16))) double lds[kJLds];
-  __shared__ double red;
-  __shared__ int sig;
+k_jacobi(const int* __restrict__ nq, const int* __restrict__ kq, int drop, const int64_t* __restrict__ goff,
+         const double* __restrict__ Gin, double* __restrict__ Vout, double* __restrict__ evals,
+         const int64_t* __restrict__ eoff, int max_sweeps, int nmax_here, double floor_rel) {
+  __shared__ __attribute__((aligned(16))) JacLds L;
   const int q = blockIdx.x;
   const int n = nq[q];
   if (n == 0 || n > nmax_here) return;   // larger sectors: block Jacobi
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double* G0 = Gin + goff[q];      // full n x n column-major
   double* Vg = Vout + goff[q];           // eigenvectors, the same layout
   double* ev = evals + eoff[q];
-  double* Qts = lds + kJS;
-  if (n <= 16) jacobi_sector<1>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
-  else if (n <= 32) jacobi_sector<2>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
-  else jacobi_sector<4>(lds, Qts, &sig, &red, n, G0, Vg, ev, max_sweeps, floor_rel);
+  int r = 0;
+  if (kq && n > 16) {
+    r = jac_cholesky(L, n, G0, wave, lane);
+    if (!drop && r < kq[q]) r = 0;
+  }
+  const int w = r ? r : n;
+  if (w <= 16) jacobi_sector<1>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else if (w <= 32) jacobi_sector<2>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else jacobi_sector<4>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
 }
 
 // 4b. Sectors larger than kJacBlockMin: two-sided block Jacobi.  The padded
@@ -716,7 +907,6 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
 //                  from the trailing matrix minus the panel's earlier rows
 //                  (left-looking inside the panel, rows held in LDS)
 //   k_pchol_update trailing matrix G <- G - R_panel^T R_panel (rank nb)
-constexpr double kPcTol = 1e-15;
 constexpr int kPcThreads = 1024;
 struct PcSector {
   int n, q;
@@ -1429,7 +1619,7 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
   }
   // eigenpairs of G' (relative convergence test only)
   if (any_small) {
-    hipLaunchKernelGGL(k_jacobi, dim3(ns), dim3(kJThreads), 0, s, d_r2, d_goff2, G2, W2, ev2, d_eoff2, 40,
+    hipLaunchKernelGGL(k_jacobi, dim3(ns), dim3(kJThreads), 0, s, d_r2, (const int*)nullptr, 0, d_goff2, G2, W2, ev2, d_eoff2, 40,
                        kJacBlockMin, 0.0);
     TTG_HIP(hipGetLastError());
   }
@@ -1609,7 +1799,7 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
       TTG_TRY(side_fork(&js));
       forked = true;
     }
-    hipLaunchKernelGGL(k_jacobi, dim3(nQ), dim3(kJThreads), 0, js, d_nq, d_goff, G, Vev, ev, d_eoff, 40,
+    hipLaunchKernelGGL(k_jacobi, dim3(nQ), dim3(kJThreads), 0, js, d_nq, d_kq, (int)(cutoff > kLrCutoff), d_goff, G, Vev, ev, d_eoff, 40,
                        kJacBlockMin, kJacFloor);
     TTG_HIP(hipGetLastError());
   }
