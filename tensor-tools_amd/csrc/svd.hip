@@ -21,6 +21,7 @@
 //   6. the absorbed factor as a second grouped GEMM (U^T A or A V), then the
 //      slicing of U, V and S into blocks.
 #include <algorithm>
+#include <type_traits>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -216,11 +217,14 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // itself, and one row a step passes through LDS.  On the sectors of an m = 100 state (up to 60
 // rows, rank-deficient) k_jacobi took 445 us and takes 89, at m = 333 531 and 258.  The route is taken
 // when the r columns are all that the selection can use: r >= kq, the values
-// kept before truncation, or a cutoff above kLrCutoff, the weight (of the
-// whole tensor's) that 64 rows below kPcTol of the largest can hold.
+// kept before truncation, with no pivot among them below kLrCond of the
+// largest diagonal (the factors of a worse conditioned sector lose up to ten times
+// more than those of the plain iteration), or a cutoff above kLrCutoff, the
+// weight (of the whole tensor's) that 64 rows below kPcTol of the largest can hold.
 constexpr double kJacFloor = 1e-14;   // convergence floor relative to the largest diagonal
 constexpr double kPcTol = 1e-15;      // a remaining diagonal below this of the largest ends the factorisation
 constexpr double kLrCutoff = kJW * kPcTol * 1.5;
+constexpr double kLrCond = 1e-8;
 
 // LDS of k_jacobi
 struct JacLds {
@@ -232,20 +236,16 @@ struct JacLds {
   int sig;
 };
 
-// Pivoted Cholesky of G0 (n x n): rows of R to L.r (zero beyond row r and column
-// n); returns r.  Ties go to the lower index.
-__device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, int wave, int lane) {
-  double x[8];   // G(8 wave + s, lane)
-#pragma unroll
-  for (int s = 0; s < 8; s++) {
-    const int i = 8 * wave + s;
-    x[s] = i < n && lane < n ? 0.5 * (G0[i + (int64_t)n * lane] + G0[lane + (int64_t)n * i]) : 0.0;
-  }
-  double d = lane < n ? G0[lane * (int64_t)(n + 1)] : 0.0;
-  bool open = lane < n;
-  for (int e = threadIdx.x; e < kJS; e += kJThreads) L.r[e] = 0.0;
-  double stop = 0.0;
+// Pivoted Cholesky of a matrix of up to 64 rows in the registers of 8 waves: x[s] is
+// element (8 wave + s, lane), d the remaining diagonal of index `lane`, kept by every
+// wave, `open` an index not yet taken.  Row k of R goes to r[k kJP + ..], the index of
+// step k to lane k's `order`; ends after n steps or when stop(k, pivot) says so, and
+// returns the steps.  Ties go to the lower index.  `row`: two rows of LDS.
+template <class Stop>
+__device__ __forceinline__ int cholesky64(double (&x)[8], double d, bool open, int n, double* r, double (*row)[kJW],
+                                          int wave, int lane, int& order, Stop stop) {
   int k = 0;
+  order = 0;
   for (; k < n; k++) {
     const double v = open ? d : -1.0;
     double m = v;
@@ -255,19 +255,19 @@ __device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, 
     m = fmax(m, lane_xor<8>(m));
     m = fmax(m, lane_xor<16>(m));
     m = fmax(m, lane_xor<32>(m));
-    if (k == 0) stop = kPcTol * m;
-    if (!(m > stop)) break;   // the same in every wave
+    if (stop(k, m)) break;   // the same in every wave
     const int p = __builtin_ctzll(__ballot(v == m));
-    double* row = L.row[k & 1];
+    double* rk = row[k & 1];
     if (wave == p >> 3)
 #pragma unroll
       for (int s = 0; s < 8; s++)
-        if ((p & 7) == s) row[lane] = x[s];
-    const double inv = 1.0 / sqrt(m);
+        if ((p & 7) == s) rk[lane] = x[s];
+    const double inv = jac_rsqrt(m);
     __syncthreads();
-    const double rv = open ? (lane == p ? m : row[lane]) * inv : 0.0;
+    const double rv = open ? (lane == p ? m : rk[lane]) * inv : 0.0;
     open = open && lane != p;
-    if (wave == 0) L.r[k * kJP + lane] = rv;
+    if (lane == k) order = p;
+    if (wave == 0) r[k * kJP + lane] = rv;
     d = fma(-rv, rv, d);
     typedef int i2 __attribute__((ext_vector_type(2)));
     const i2 w = __builtin_bit_cast(i2, rv);
@@ -281,6 +281,34 @@ __device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, 
   }
   __syncthreads();
   return k;
+}
+
+// Pivoted Cholesky of G0 (n x n): rows of R to L.r (zero beyond row r and column
+// n); returns r, and in `good` the rows with pivots above kLrCond of the largest
+// diagonal.
+__device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, int wave, int lane, int& good) {
+  double x[8];
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int i = 8 * wave + s;
+    x[s] = i < n && lane < n ? 0.5 * (G0[i + (int64_t)n * lane] + G0[lane + (int64_t)n * i]) : 0.0;
+  }
+  for (int e = threadIdx.x; e < kJS; e += kJThreads) L.r[e] = 0.0;
+  __syncthreads();
+  double tol = 0.0, fair = 0.0;
+  int order, g = 0;
+  const int r = cholesky64(x, lane < n ? G0[lane * (int64_t)(n + 1)] : 0.0, lane < n, n, L.r, L.row, wave, lane, order,
+                           [&](int k, double m) {
+                             if (k == 0) {
+                               tol = kPcTol * m;
+                               fair = kLrCond * m;
+                             }
+                             if (!(m > tol)) return true;
+                             g += m > fair;   // (the pivots descend)
+                             return false;
+                           });
+  good = g;
+  return r;
 }
 
 // G' = R R^T into L.s (16 NPR square)
@@ -453,8 +481,9 @@ k_jacobi(const int* __restrict__ nq, const int* __restrict__ kq, int drop, const
   double* ev = evals + eoff[q];
   int r = 0;
   if (kq && n > 16) {
-    r = jac_cholesky(L, n, G0, wave, lane);
-    if (!drop && r < kq[q]) r = 0;
+    int good;
+    r = jac_cholesky(L, n, G0, wave, lane, good);
+    if (!drop && good < kq[q]) r = 0;
   }
   const int w = r ? r : n;
   if (w <= 16) jacobi_sector<1>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
@@ -886,43 +915,56 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
   return 0;   // the scratch goes back to the pool in stream order
 }
 
-// 4c. LR preconditioning of the large sectors (cutoff > 0).  A sector's
-// Gram matrix of a DMRG state is numerically rank-deficient (a few hundred
-// of its rows carry weight), and the Jacobi iteration on G spends most of
+// 4c. LR preconditioning of the large sectors.  A sector's Gram matrix of
+// a DMRG state is numerically rank-deficient (a few hundred of its rows
+// carry weight), and that of a site to be canonicalised when it has more rows on
+// the isometric side than on the other; the Jacobi iteration on G spends most of
 // its sweeps decoupling that null space from the rest.  A pivoted Cholesky
 // factorisation P^T G P = R^T R stops at the numerical rank r (largest
 // remaining diagonal below 1e-15 of the largest diagonal) and gives
 // G' = R R^T (r x r, the same nonzero eigenvalues, no null space).  Jacobi
 // on G' with the relative convergence test alone (no absolute floor: G' is
 // positive definite) converges in about a third of the sweeps, at size r,
-// and G's eigenvectors follow as V = R^T W Lambda^(-1/2), orthonormal to the
-// relative accuracy of W.  The n - r null-space columns are left zero with
-// eigenvalue 0: a zero singular value is never kept when cutoff > 0
-// (qtensor_op.cpp:1294-1300).
+// and G's eigenvectors follow as X = R^T W Lambda^(-1/2), orthonormal to the
+// relative accuracy of W and to eps sqrt(lambda_1 / lambda_c); one Gram-Schmidt
+// step in the order of the eigenvalues makes that 2e-15 (1e-12 before).  The
+// n - r null-space columns are left zero with eigenvalue 0: a zero singular value
+// is never kept when cutoff > 0 (qtensor_op.cpp:1294-1300).  Without a cutoff
+// the rule is that of the small sectors (4): the r columns cover the kq
+// values asked for and no pivot among them is below kLrCond of the largest
+// diagonal; otherwise the sector's Gram matrix is formed again and solved by block Jacobi.
+// (A site of m = 701: 11 sweeps of 5 rounds on G, 7 of 3 on G', 2600 to 1870 us.)
 // R is stored by original column index (row k of R at k n + j), so neither
 // G' nor V needs the permutation.
-//   k_pchol_init   d = diag(G), no column pivoted yet, dmax per sector
-//   k_pchol_panel  one workgroup per sector: nb pivot steps (largest
-//                  remaining diagonal, ties to the lower index), each row of R
-//                  from the trailing matrix minus the panel's earlier rows
-//                  (left-looking inside the panel, rows held in LDS)
-//   k_pchol_update trailing matrix G <- G - R_panel^T R_panel (rank nb)
-constexpr int kPcThreads = 1024;
+//   k_pchol_init   d = diag(G), dmax per sector
+//   k_pchol_panel  the next up to 64 pivots, from a 64 x 64 principal submatrix
+//   k_pchol_update their rows of R, and G <- G - R_panel^T R_panel
+constexpr int kPcThreads = 512;
+constexpr int kPcNbMax = 64;   // candidates of a panel: a wave's lanes
 struct PcSector {
   int n, q;
+  int kq;         // eigenpairs the selection can use
+  int pad;
   int64_t goff;   // G (trailing matrix, overwritten) and R, n x n each
-  int64_t doff;   // diagonal / pivot flags, n each
+  int64_t doff;   // remaining diagonal, pivots in order, step of each column (-1: none), n each
+};
+struct PcState {
+  double dmax;    // largest diagonal of G
+  double least;   // smallest of the first kq pivots
+  int rank;       // -1: not finished
+  int k0, k1;     // rows of R that the last panel wrote
+  int panels, pad;
 };
 
 __global__ void __launch_bounds__(kPcThreads) k_pchol_init(const PcSector* ps, const double* G, double* d,
-                                                           int* piv, int* rank, double* dmax) {
+                                                           int* pos, PcState* st) {
   __shared__ double red[kPcThreads / 64];
   const PcSector P = ps[blockIdx.x];
   double mx = 0.0;
   for (int j = threadIdx.x; j < P.n; j += blockDim.x) {
     const double v = G[P.goff + j + (int64_t)P.n * j];
     d[P.doff + j] = v;
-    piv[P.doff + j] = 0;
+    pos[P.doff + j] = -1;
     mx = fmax(mx, v);
   }
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
@@ -931,157 +973,287 @@ __global__ void __launch_bounds__(kPcThreads) k_pchol_init(const PcSector* ps, c
   if (threadIdx.x == 0) {
     double m = 0.0;
     for (int w = 0; w < (int)(blockDim.x >> 6); w++) m = fmax(m, red[w]);
-    dmax[blockIdx.x] = m;
-    rank[blockIdx.x] = -1;
+    st[blockIdx.x] = PcState{m, m, -1, 0, 0, 0, 0};
   }
 }
 
-// dynamic LDS: nb panel rows (nb x n), d (n), pivot flags (n ints)
-__global__ void __launch_bounds__(kPcThreads) k_pchol_panel(const PcSector* ps, int k0, int nb,
-                                                            const double* A, double* R, double* dg,
-                                                            int* pivg, int* rank, const double* dmax) {
-  extern __shared__ __attribute__((aligned(16))) double pc_lds[];
-  __shared__ double rv[kPcThreads / 64];
-  __shared__ int ri[kPcThreads / 64];
-  __shared__ int s_p, s_stop;
-  __shared__ double s_rkk;
+// A panel takes its pivots from the (up to) 64 largest remaining diagonals at
+// its start: k_pchol_panel, one workgroup a sector, factorises that 64 x 64
+// principal submatrix in registers (cholesky64), and k_pchol_update forms the
+// panel's rows of R by forward substitution, column by column, where it needs
+// them, and takes R_panel^T R_panel from the trailing matrix.  The panel ends early
+// when its best candidate is below kPcLoose of the largest diagonal that is
+// not a candidate (which only decrease): a pivot is never less than that part
+// of the largest remaining one, and a panel has one pivot at least (1/32 took 11 panels
+// where this takes 16, but an element of R may be the square root of that above
+// its pivot: the smallest kept values' vectors were up to 2.4 times less accurate, and
+// are as accurate as with the largest pivot in every step here).  A step of the
+// panel is a chain of latencies, about 0.3 us; with whole rows of R formed in every
+// step, by one workgroup, it was 2.5 us, whether the pivot's column came from
+// memory or from LDS.  Sectors of up to 388 rows (m = 1500, rank 248): 16 panels of 20.1 us
+// and 16 updates of 14.1, before 9 of 69.3 and 9 of 12.2.
+constexpr int kPcMaxN = 8181;          // largest sector (the remaining diagonal is held in LDS)
+constexpr double kPcLoose = 0.125;
+// state of one panel for the update: column k of the substitution at L[64 k ..]
+// (elements t > k, and 1 / the diagonal at k)
+constexpr int kPcL = kPcNbMax * kPcNbMax;
+
+__global__ void __launch_bounds__(kJThreads) k_pchol_panel(const PcSector* ps, const double* A, const double* dg,
+                                                           int* piv, int* pos, double* Lg, PcState* st) {
+  extern __shared__ __attribute__((aligned(16))) double pc_lds[];   // d (n): -1 for pivots taken
+  __shared__ double s_r[kJS], s_row[2][kJW], s_dc[kPcNbMax], s_max[8];
+  __shared__ int s_cand[kPcNbMax], s_cnt[2][8];
   const PcSector P = ps[blockIdx.x];
-  const int n = P.n, tid = threadIdx.x;
-  if (k0 >= n || rank[blockIdx.x] >= 0) return;   // finished sector
-  double* Rp = pc_lds;                 // panel row s at s * n
-  double* d = pc_lds + (int64_t)nb * n;
-  int* piv = (int*)(d + n);
-  for (int j = tid; j < n; j += blockDim.x) {
-    d[j] = dg[P.doff + j];
-    piv[j] = pivg[P.doff + j];
+  PcState& T = st[blockIdx.x];
+  const int n = P.n, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int k0 = T.k1;
+  const bool finished = T.rank >= 0;
+  __syncthreads();
+  if (finished) {                      // nothing for the update either
+    if (tid == 0) T.k0 = k0;
+    return;
+  }
+  double* d = pc_lds;
+  double top = -1.0;
+  for (int j = tid; j < n; j += kJThreads) {
+    const double v = pos[P.doff + j] >= 0 ? -1.0 : dg[P.doff + j];
+    d[j] = v;
+    top = fmax(top, v);
+  }
+  for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o));
+  if (lane == 0) s_max[wave] = top;
+  for (int e = tid; e < kJS; e += kJThreads) s_r[e] = 0.0;
+  if (tid < kPcNbMax) s_dc[tid] = -1.0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; w++) top = fmax(top, s_max[w]);
+  const double tol = kPcTol * T.dmax;
+  // Candidates: those above the smallest step of a scale of quarter octaves that at
+  // most 64 open columns reach, found by bisection between the threshold and the
+  // largest diagonal; then some of the next step until there are 64.
+  int turn = 0;
+  auto total = [&](int mine) {         // the sum of a wave-uniform count over the waves
+    if (lane == 0) s_cnt[turn][wave] = mine;
+    __syncthreads();
+    int c = 0;
+#pragma unroll
+    for (int w = 0; w < 8; w++) c += s_cnt[turn][w];
+    turn ^= 1;
+    return c;
+  };
+  auto key = [](double v) { return v > 0.0 ? (int)(__builtin_bit_cast(uint64_t, v) >> 50) : -1; };
+  auto reach = [&](int k) {
+    int c = 0;
+    for (int j0 = 64 * wave; j0 < n; j0 += kJThreads) c += __popcll(__ballot(j0 + lane < n && key(d[j0 + lane]) >= k));
+    return total(c);
+  };
+  int lo = max(key(tol), 0), hi = key(top) + 1;   // reach(hi) <= 64; reach(lo) > 64, unless every column above the threshold is taken
+  if (reach(lo) <= kPcNbMax) hi = lo;
+  else
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (reach(mid) <= kPcNbMax) hi = mid;
+      else lo = mid;
+    }
+  const bool rest = hi > lo;           // open columns above the threshold that are no candidates
+  for (int pass = 0, base = 0; pass < (rest ? 2 : 1); pass++) {
+    int mine = 0;
+    for (int j0 = 64 * wave; j0 < n; j0 += kJThreads) {
+      const int k = j0 + lane < n ? key(d[j0 + lane]) : -1;
+      mine += __popcll(__ballot(pass == 0 ? k >= hi : k == lo));
+    }
+    const int* cnt = s_cnt[turn];
+    const int all = total(mine);
+    int at = base;
+    for (int w = 0; w < wave; w++) at += cnt[w];
+    for (int j0 = 64 * wave; j0 < n; j0 += kJThreads) {
+      const int j = j0 + lane;
+      const double v = j < n ? d[j] : -1.0;
+      const int k = key(v);
+      const bool in = pass == 0 ? k >= hi : k == lo;
+      const uint64_t m = __ballot(in);
+      const int c = at + __popcll(m & ((1ull << lane) - 1ull));
+      if (in && c < kPcNbMax) {
+        s_cand[c] = j;
+        s_dc[c] = v;
+      }
+      at += __popcll(m);
+    }
+    base += all;
   }
   __syncthreads();
-  const double tol = kPcTol * dmax[blockIdx.x];
-  const int kend = min(k0 + nb, n);
-  int k = k0;
-  for (; k < kend; k++) {
-    double bv = -1.0;
-    int bi = n;
-    for (int j = tid; j < n; j += blockDim.x)
-      if (!piv[j] && (d[j] > bv || (d[j] == bv && j < bi))) { bv = d[j]; bi = j; }
-    for (int o = 32; o > 0; o >>= 1) {
-      const double ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
-    if ((tid & 63) == 0) { rv[tid >> 6] = bv; ri[tid >> 6] = bi; }
-    __syncthreads();
-    if (tid < 64) {   // the waves' candidates, reduced by wave 0 (same order rule)
-      constexpr int kW = kPcThreads / 64;
-      double v = tid < kW ? rv[tid] : -1.0;
-      int i = tid < kW ? ri[tid] : n;
-      for (int o = kW / 2; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(v, o);
-        const int oi = __shfl_xor(i, o);
-        if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
-      }
-      if (tid == 0) {
-        s_stop = !(v > tol) || i >= n;
-        s_p = i;
-        s_rkk = s_stop ? 0.0 : sqrt(v);
-        if (!s_stop) piv[i] = 1;
-      }
-    }
-    __syncthreads();
-    if (s_stop) break;
-    const int p = s_p, ks = k - k0;
-    const double rkk = s_rkk;
-    const double irkk = 1.0 / rkk;
-    for (int j = tid; j < n; j += blockDim.x) {
-      double v;
-      if (j == p) {
-        v = rkk;
-      } else if (piv[j]) {
-        v = 0.0;
-      } else {
-        v = A[P.goff + j + (int64_t)n * p];   // trailing matrix, column p (symmetric)
-#pragma unroll 8
-        for (int t = 0; t < ks; t++) v -= Rp[t * n + p] * Rp[t * n + j];
-        v *= irkk;
-        d[j] -= v * v;
-      }
-      Rp[ks * n + j] = v;
-      R[P.goff + (int64_t)k * n + j] = v;
-    }
-    __syncthreads();
+  // the largest open diagonal that is not a candidate is below the next step of the scale
+  const double next = rest ? __builtin_bit_cast(double, (uint64_t)hi << 50) : 0.0;
+  const double dc = s_dc[lane];
+  const bool real = dc > 0.0;
+  const int cand = real ? s_cand[lane] : 0, nc = __popcll(__ballot(real));
+  double x[8];
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int i = 8 * wave + s;
+    x[s] = i < nc && real ? A[P.goff + (int64_t)n * s_cand[i] + cand] : 0.0;
   }
-  for (int j = tid; j < n; j += blockDim.x) {
-    dg[P.doff + j] = d[j];
-    pivg[P.doff + j] = piv[j];
+  double least = T.least;
+  bool small = nc == 0;
+  int order;
+  const int ks = cholesky64(x, dc, real, nc, s_r, s_row, wave, lane, order, [&](int k, double m) {
+    small = !(m > tol);
+    if (small || m < kPcLoose * next) return true;
+    if (k0 + k < P.kq) least = fmin(least, m);
+    return false;
+  });
+  double* L = Lg + (int64_t)kPcL * blockIdx.x;
+#pragma unroll
+  for (int s = 0; s < 8; s++) {
+    const int k = 8 * wave + s, t = lane;
+    const double v = s_r[k * kJP + order];   // R(k, pivot of step t)
+    L[kPcNbMax * k + t] = k >= ks || t >= ks || t < k ? 0.0 : t == k ? 1.0 / v : v;
   }
-  if (tid == 0 && k < kend) rank[blockIdx.x] = k;   // stopped inside this panel
+  const int col = __shfl(cand, order);
+  if (wave == 0 && lane < ks) {
+    piv[P.doff + k0 + lane] = col;
+    pos[P.doff + col] = k0 + lane;
+  }
+  if (tid == 0) {
+    T.least = least;
+    T.k0 = k0;
+    T.k1 = k0 + ks;
+    T.panels++;
+    // nothing left, or nothing above the threshold among the candidates and the rest (with no
+    // pivot taken the rest is at most a step of the scale above the candidates)
+    if (k0 + ks >= n || (small && (ks == 0 || !(next > tol)))) T.rank = k0 + ks;
+  }
 }
 
-// G[i, j] -= sum_{k in panel rows} R[k, i] R[k, j], 64 x 64 tiles, 256 threads
-// (launched with 256).  The panel rows' two 64-column pieces are staged in LDS
-// with one batch of loads (a loop over k with a global load per step would
-// wait one memory latency per k); the sums run over k in ascending order.
-constexpr int kPcNbMax = 32;
-__global__ void __launch_bounds__(256) k_pchol_update(const PcSector* ps, int k0, int nb, const int* rank,
-                                                      double* A, const double* R) {
-  __shared__ double Ri[kPcNbMax][64];
-  __shared__ double Rj[kPcNbMax][64];
+// Rows of R of a panel for 64 columns: forward substitution, a thread per column
+// (y in registers, the coefficients from LDS), and G[i, j] -= sum_k R[k, i] R[k, j], 64 x 64
+// tiles on the FP64 matrix cores.  The workgroups on the diagonal write R and the
+// remaining diagonal.  Rows of a column are zero after the step that takes it.
+constexpr int kPcP = 66;   // LDS pitch of a row of R: 64 columns
+__device__ __forceinline__ void pc_rows(const double* __restrict__ Acol, int64_t n, const int* __restrict__ piv,
+                                        const double* L, int ks, double (&y)[kPcNbMax]) {
+  // steps and rows in groups of 8; groups beyond ks are skipped, and steps beyond it in
+  // the last group have zero coefficients
+#pragma unroll
+  for (int tb = 0; tb < kPcNbMax; tb += 8) {
+    if (tb < ks) {
+#pragma unroll
+      for (int t = tb; t < tb + 8; t++) y[t] = Acol[n * piv[min(t, ks - 1)]];
+    }
+  }
+#pragma unroll
+  for (int kb = 0; kb < kPcNbMax; kb += 8) {
+    if (kb < ks) {
+#pragma unroll
+      for (int tb = kb; tb < kPcNbMax; tb += 8) {
+        if (tb < ks) {
+#pragma unroll
+          for (int k = kb; k < kb + 8; k++) {
+            if (tb == kb) y[k] *= L[kPcNbMax * k + k];
+#pragma unroll
+            for (int t = tb == kb ? k + 1 : tb; t < tb + 8; t++) y[t] = fma(-L[kPcNbMax * k + t], y[k], y[t]);
+          }
+        }
+      }
+    }
+  }
+}
+__global__ void __launch_bounds__(256) k_pchol_update(const PcSector* ps, const PcState* st, const int* piv,
+                                                      const int* pos, const double* __restrict__ Lg, double* A,
+                                                      double* R, double* dg) {
+  // the coefficients and, when every row is formed, the rows (two workgroups a CU)
+  __shared__ __attribute__((aligned(16))) double lds[2 * kPcNbMax * kPcP];
   const PcSector P = ps[blockIdx.y];
-  const int n = P.n;
-  const int nt = (n + 63) / 64;
-  if ((int)blockIdx.x >= nt * nt || k0 >= n) return;
-  const int rk = rank[blockIdx.y];
-  const int k1 = rk >= 0 ? min(rk, min(k0 + nb, n)) : min(k0 + nb, n);
-  if (k1 <= k0) return;   // uniform over the workgroup
-  const int nk = k1 - k0;   // <= nb <= kPcNbMax (the host caps nb)
-  const int i0 = (blockIdx.x % nt) * 64, j0 = (blockIdx.x / nt) * 64;
+  const int n = P.n, nt = (n + 63) / 64;
+  const int bi = blockIdx.x % nt, bj = blockIdx.x / nt;
+  const int k0 = st[blockIdx.y].k0, ks = st[blockIdx.y].k1 - k0;
+  const bool finished = st[blockIdx.y].rank >= 0;
+  if (bj >= nt || ks == 0 || (finished && bi != bj)) return;   // (a finished sector needs no trailing matrix)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   {
-    constexpr int kPer = kPcNbMax * 64 / 256;   // entries per thread (256 threads)
-    double vi[kPer], vj[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-      const int e = threadIdx.x + 256 * u, kk = e >> 6, c = e & 63;
-      const double* rk_ = R + P.goff + (int64_t)(k0 + kk) * n;
-      vi[u] = (kk < nk && i0 + c < n) ? rk_[i0 + c] : 0.0;
-      vj[u] = (kk < nk && j0 + c < n) ? rk_[j0 + c] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < kPer; u++) {
-      const int e = threadIdx.x + 256 * u, kk = e >> 6, c = e & 63;
-      Ri[kk][c] = vi[u];
-      Rj[kk][c] = vj[u];
-    }
+    const double* src = Lg + (int64_t)kPcL * blockIdx.y;
+    const int rows = (ks + 7) & ~7;
+    for (int e = threadIdx.x; e < kPcNbMax * rows; e += 256) lds[e] = src[e];
   }
   __syncthreads();
-  const int il = threadIdx.x & 63, jl = (threadIdx.x >> 6) * 16;
-  const int i = i0 + il, jb = j0 + jl;
-  if (i >= n) return;
-  double acc[16];
+  const bool mine = wave < (bi == bj ? 1 : 2);
+  double y[kPcNbMax];
+  const int cc = min(64 * (wave ? bj : bi) + lane, n - 1);
+  if (mine) pc_rows(A + P.goff + cc, n, piv + P.doff + k0, lds, ks, y);
+  __syncthreads();
+  if (mine) {
+    const int taken = pos[P.doff + cc], last = taken >= 0 ? taken - k0 : kPcNbMax;
+    double* Y = lds + wave * kPcNbMax * kPcP + lane;
 #pragma unroll
-  for (int u = 0; u < 16; u++) acc[u] = 0.0;
-  for (int kk = 0; kk < nk; kk++) {
-    const double ri_ = Ri[kk][il];
+    for (int t = 0; t < kPcNbMax; t++)
+      if (t < ((ks + 3) & ~3)) Y[t * kPcP] = t <= last ? y[t] : 0.0;
+  }
+  __syncthreads();
+  const double* Yi = lds;
+  const double* Yj = lds + (bi == bj ? 0 : kPcNbMax * kPcP);
+  if (bi == bj)
+    for (int t = wave; t < ks; t += 4)
+      if (64 * bi + lane < n) R[P.goff + (int64_t)(k0 + t) * n + 64 * bi + lane] = Yi[t * kPcP + lane];
+  if (finished) return;
+  // wave w: rows 16 w .. 16 w + 15 of the tile, its four 16-column pieces; D[l/16 + 4 r][l%16]
+  const int j = lane & 15, g = lane >> 4;
+  jac_v4d acc[4] = {};
+  for (int k = 0; k < ks; k += 4) {    // (rows of Y beyond ks are zero)
+    const double a = Yj[(k + g) * kPcP + 16 * wave + j];
 #pragma unroll
-    for (int u = 0; u < 16; u++) acc[u] += ri_ * Rj[kk][jl + u];
+    for (int u = 0; u < 4; u++)
+      acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, Yi[(k + g) * kPcP + 16 * u + j], acc[u], 0, 0, 0);
+  }
+  // columns that are pivots stay as they are: other workgroups read them here, and
+  // nothing reads them later
+  bool open[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int col = 64 * bj + 16 * wave + g + 4 * r;
+    open[r] = col < n && pos[P.doff + col] < 0;
   }
 #pragma unroll
-  for (int u = 0; u < 16; u++)
-    if (jb + u < n) A[P.goff + i + (int64_t)n * (jb + u)] -= acc[u];
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = 64 * bi + 16 * u + j, col = 64 * bj + 16 * wave + g + 4 * r;
+      if (row < n && open[r]) {
+        double* e = A + P.goff + row + (int64_t)n * col;
+        const double v = *e - acc[u][r];
+        *e = v;
+        if (row == col) dg[P.doff + row] = v;
+      }
+    }
 }
 
-// V columns c < r: (R^T W)_c / sqrt(lambda_c), eigenvalue lambda_c; columns
-// c >= r: zero, eigenvalue 0
-__global__ void k_lr_finish(const PcSector* ps, const int* rk, const int64_t* eoff2, const double* ev2,
-                            const int64_t* eoff, double* Vev, double* ev) {
+// X (in G's place): columns c < r of R^T W scaled by 1 / sqrt(lambda_c), eigenvalue lambda_c;
+// columns c >= r of V: zero, eigenvalue 0
+__global__ void k_lr_scale(const PcSector* ps, const int* rk, const int64_t* eoff2, const double* ev2,
+                           const int64_t* eoff, double* X, double* Vev, double* ev) {
   const PcSector P = ps[blockIdx.y];
   const int n = P.n, r = rk[blockIdx.y];
   const int c = blockIdx.x;
   if (c >= n) return;
   const double lam = c < r ? ev2[eoff2[blockIdx.y] + c] : 0.0;
-  const double sc = (c < r && lam > 0.0) ? 1.0 / sqrt(lam) : 0.0;
-  double* col = Vev + P.goff + (int64_t)n * c;
+  const double sc = lam > 0.0 ? 1.0 / sqrt(lam) : 0.0;
+  double* col = (c < r ? X : Vev) + P.goff + (int64_t)n * c;
   for (int i = threadIdx.x; i < n; i += blockDim.x) col[i] = c < r ? col[i] * sc : 0.0;
   if (threadIdx.x == 0) ev[eoff[P.q] + c] = lam;
+}
+
+// The Gram-Schmidt coefficients of X from M = X^T X (r x r): column c of V is X C_c,
+// C(a, c) = -M(a, c) for lambda_a > lambda_c, (3 - M(c, c)) / 2 at c
+__global__ void __launch_bounds__(256) k_lr_order(const int* rk, const int64_t* goff2, const int64_t* eoff2,
+                                                  const double* ev2, const double* M, double* C) {
+  const int r = rk[blockIdx.y], c = blockIdx.x;
+  if (c >= r) return;
+  const double* lam = ev2 + eoff2[blockIdx.y];
+  const int64_t o = goff2[blockIdx.y] + (int64_t)r * c;
+  const double lc = lam[c];
+  for (int a = threadIdx.x; a < r; a += 256) {
+    const double la = lam[a], m = M[o + a];
+    C[o + a] = a == c ? 1.5 - 0.5 * m : (la > lc || (la == lc && a < c)) ? -m : 0.0;
+  }
 }
 
 // 5a. per sector: eigen order (descending), top-k singular values in the
@@ -1522,8 +1694,10 @@ class Pack {
   char* d_ = nullptr;
 };
 
-// eigenpairs of the large sectors `big` through the LR step (see 4c)
-static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, const std::vector<int64_t>& goff,
+// eigenpairs of the large sectors `big` through the LR step (see 4c); without
+// `drop`, the sectors that the step cannot serve go to `plain`
+static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, const std::vector<int>& kq, bool drop,
+                    std::vector<int>& plain, const std::vector<int64_t>& goff,
                     const std::vector<int64_t>& eoff, const int64_t* d_eoff, int64_t gtotal, double* G,
                     double* Vev, double* ev, hipStream_t s) {
   PhaseTimer _phase("lr_eigen");
@@ -1533,62 +1707,57 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
   int64_t dtot = 0;
   for (int li = 0; li < ns; li++) {
     const int q = big[li];
-    ps[li] = PcSector{nq[q], q, goff[q], dtot};
+    ps[li] = PcSector{nq[q], q, kq[q], 0, goff[q], dtot};
     dtot += nq[q];
     nmax = std::max(nmax, nq[q]);
   }
-  // panel rows: nb rows of n doubles, d and the flags in the 160 KiB of LDS
-  const int nb = std::max(1, std::min(kPcNbMax, (int)(163840 / (8 * (int64_t)nmax)) - 2));
-  const size_t lds = sizeof(double) * ((size_t)nb * nmax + nmax) + sizeof(int) * nmax;
-  TTG_REQUIRE(lds <= 163840, "svd: sector too large for the pivoted Cholesky panel");
+  TTG_REQUIRE(nmax <= kPcMaxN, "svd: sector too large for the pivoted Cholesky panel");
+  const size_t lds = sizeof(double) * nmax;
   Scratch sc;
   PcSector* d_ps = sc.get<PcSector>(ns);
   double* R = sc.get<double>(gtotal);
   double* dg = sc.get<double>(dtot);
-  int* pg = sc.get<int>(dtot);
-  int* rank = sc.get<int>(ns);
-  double* dmax = sc.get<double>(ns);
+  int* piv = sc.get<int>(dtot);
+  int* pos = sc.get<int>(dtot);
+  double* Lg = sc.get<double>((size_t)kPcL * ns);
+  PcState* d_st = sc.get<PcState>(ns);
   TTG_TRY(sc.ok("svd: LR step"));
   TTG_TRY(h2d_vec(d_ps, ps));
-  hipLaunchKernelGGL(k_pchol_init, dim3(ns), dim3(kPcThreads), 0, s, d_ps, G, dg, pg, rank, dmax);
+  hipLaunchKernelGGL(k_pchol_init, dim3(ns), dim3(kPcThreads), 0, s, d_ps, G, dg, pos, d_st);
   TTG_HIP(hipFuncSetAttribute((const void*)k_pchol_panel, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds));
   const int nt = (nmax + 63) / 64;
   // Panels are launched up to one more than the previous call needed, then
-  // the ranks are read back; only if a sector is still running are the rest
-  // launched (a finished sector's launches exit at once, but each launch
-  // still costs a few microseconds).  The panels run in the same order
-  // either way.
+  // the ranks are read back, and while a sector is running some more follow
+  // (a finished sector's launches exit at once, but each launch still costs
+  // a few microseconds).
   static int prev_panels = 0;
-  const int all_panels = (nmax + nb - 1) / nb;
-  int target = prev_panels > 0 ? std::min(all_panels, prev_panels + 1) : all_panels;
-  std::vector<int> rk(ns);
-  int k0 = 0;
-  for (;;) {
-    for (; k0 < target * nb && k0 < nmax; k0 += nb) {
-      hipLaunchKernelGGL(k_pchol_panel, dim3(ns), dim3(kPcThreads), lds, s, d_ps, k0, nb, G, R, dg, pg, rank,
-                         dmax);
-      hipLaunchKernelGGL(k_pchol_update, dim3(nt * nt, ns), dim3(256), 0, s, d_ps, k0, nb, rank, G, R);
+  int more = prev_panels > 0 ? prev_panels + 1 : (nmax + kPcNbMax - 1) / kPcNbMax;
+  std::vector<PcState> pst(ns);
+  for (int done = 0; done <= nmax; done += more, more = 4) {   // every panel takes a pivot or ends its sector
+    for (int i = 0; i < more; i++) {
+      hipLaunchKernelGGL(k_pchol_panel, dim3(ns), dim3(kJThreads), lds, s, d_ps, G, dg, piv, pos, Lg, d_st);
+      hipLaunchKernelGGL(k_pchol_update, dim3(nt * nt, ns), dim3(256), 0, s, d_ps, d_st, piv, pos, Lg, G, R, dg);
     }
-    const D2HPiece pc{rk.data(), rank, sizeof(int) * ns};
+    const D2HPiece pc{pst.data(), d_st, sizeof(PcState) * ns};
     TTG_TRY(d2h_wait(&pc, 1));
-    bool running = false;   // a sector with neither a rank nor all its columns done
-    for (int li = 0; li < ns; li++) running |= rk[li] < 0 && k0 < ps[li].n;
-    if (!running || k0 >= nmax) break;
-    target = all_panels;
+    bool running = false;
+    for (const PcState& t : pst) running |= t.rank < 0;
+    if (!running) break;
   }
-  {
-    int need = 0;   // panels this call needed: up to each sector's stopping panel
-    for (int li = 0; li < ns; li++)
-      need = std::max(need, rk[li] < 0 ? (ps[li].n + nb - 1) / nb : rk[li] / nb + 1);
-    prev_panels = std::min(need, all_panels);
-  }
+  prev_panels = 0;
+  for (const PcState& t : pst) prev_panels = std::max(prev_panels, t.panels);
   std::vector<int> r2(ns);
   std::vector<int64_t> goff2(ns + 1, 0), eoff2(ns + 1, 0);
   bool any_small = false;
   std::vector<int> big2;
   for (int li = 0; li < ns; li++) {
-    const int r = rk[li] < 0 ? ps[li].n : rk[li];
+    TTG_REQUIRE(pst[li].rank >= 0, "svd: the pivoted Cholesky factorisation did not end");
+    int r = pst[li].rank;
+    if (!drop && (r < ps[li].kq || pst[li].least < kLrCond * pst[li].dmax)) {
+      plain.push_back(big[li]);
+      r = 0;
+    }
     r2[li] = r;
     goff2[li + 1] = goff2[li] + (int64_t)r * r;
     eoff2[li + 1] = eoff2[li] + r;
@@ -1624,21 +1793,27 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
     TTG_HIP(hipGetLastError());
   }
   if (!big2.empty()) TTG_TRY(block_jacobi(big2, r2, d_goff2, d_eoff2, G2, W2, ev2, s, 40, 0.0));
-  // V = R^T W Lambda^(-1/2): A(j, k) = R[k n + j], B(k, c) = W[k + r c]
-  {
-    HostGemm hv;
-    for (int li = 0; li < ns; li++) {
-      const int n = ps[li].n, r = r2[li];
-      if (r == 0) continue;
-      hv.tasks.push_back(gtask(ps[li].goff, goff2[li], n, 1, r, n, 1, r, r, r));
-      const int t = (int)hv.tasks.size() - 1;
-      hv.cblk.push_back(CBlock{ps[li].goff, n, r, t, t + 1});
-    }
-    TTG_TRY(run_host_gemm(hv, R, W2, Vev));
+  // X = R^T W Lambda^(-1/2), in G's place: A(j, k) = R[k n + j], B(k, c) = W[k + r c];
+  // M = X^T X, in G2's: A(c, i) = X[i + n c], B(i, a) = X[i + n a];
+  // V = X C: A(i, a) = X[i + n a], B(a, c) = C[a + r c]
+  HostGemm hx, hm, hv;
+  for (int li = 0; li < ns; li++) {
+    const int n = ps[li].n, r = r2[li];
+    if (r == 0) continue;
+    const int t = (int)hx.tasks.size();
+    hx.tasks.push_back(gtask(ps[li].goff, goff2[li], n, 1, r, n, 1, r, r, r));
+    hx.cblk.push_back(CBlock{ps[li].goff, n, r, t, t + 1});
+    hm.tasks.push_back(gtask(ps[li].goff, ps[li].goff, r, n, n, 1, 1, r, n, n));
+    hm.cblk.push_back(CBlock{goff2[li], r, r, t, t + 1});
+    hv.tasks.push_back(gtask(ps[li].goff, goff2[li], n, 1, r, n, 1, r, r, r));
+    hv.cblk.push_back(CBlock{ps[li].goff, n, r, t, t + 1});
   }
-  hipLaunchKernelGGL(k_lr_finish, dim3(nmax, ns), dim3(256), 0, s, d_ps, d_r2, d_eoff2, ev2, d_eoff, Vev, ev);
+  TTG_TRY(run_host_gemm(hx, R, W2, G));
+  hipLaunchKernelGGL(k_lr_scale, dim3(nmax, ns), dim3(256), 0, s, d_ps, d_r2, d_eoff2, ev2, d_eoff, G, Vev, ev);
+  TTG_TRY(run_host_gemm(hm, G, G, G2));
+  hipLaunchKernelGGL(k_lr_order, dim3(nmax, ns), dim3(256), 0, s, d_r2, d_goff2, d_eoff2, ev2, G2, W2);
   TTG_HIP(hipGetLastError());
-  return 0;
+  return run_host_gemm(hv, G, W2, Vev);
 }
 
 }  // namespace ttg
@@ -1760,18 +1935,23 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   hipLaunchKernelGGL(k_svd_gather, dim3(std::min(nb, 4096)), dim3(256), 0, s, m.view(), nleft,
                      A->d_data, t, nuL, nuR, nQ, d_moff, mat);
   // ---- 3. Gram on MFMA
-  {
+  auto gram = [&](const std::vector<int>& of) {
     HostGemm hg;
-    for (int q = 0; q < nQ; q++) {
-      const int n = nq[q];
+    for (int q : of) {
+      const int n = nq[q], t = (int)hg.tasks.size();
       const int64_t r = rows[q], c = cols[q];
       if (fromLeft)   // G = A A^T : A(m=i, k=j) = mat[i + r j]; B(k=j, n=i') = mat[i' + r j]
         hg.tasks.push_back(gtask(moff[q], moff[q], (int)r, 1, (int)c, r, r, (int)r, 1, (int)c));
       else            // G = A^T A : A(m=j, k=i) = mat[i + r j]; B(k=i, n=j') = mat[i + r j']
         hg.tasks.push_back(gtask(moff[q], moff[q], (int)c, r, (int)r, 1, 1, (int)c, r, (int)r));
-      hg.cblk.push_back(CBlock{goff[q], n, n, q, q + 1});
+      hg.cblk.push_back(CBlock{goff[q], n, n, t, t + 1});
     }
-    TTG_TRY(run_host_gemm(hg, mat, mat, G));
+    return run_host_gemm(hg, mat, mat, G);
+  };
+  {
+    std::vector<int> every(nQ);
+    std::iota(every.begin(), every.end(), 0);
+    TTG_TRY(gram(every));
   }
   // a sector whose Gram matrix overflowed (entries of A above ~1e154) or that
   // holds a NaN has no meaningful eigenpairs: fail before the eigensolver
@@ -1803,12 +1983,22 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
                        kJacBlockMin, kJacFloor);
     TTG_HIP(hipGetLastError());
   }
-  // large sectors: the LR step when the truncation drops zero singular
-  // values (cutoff > 0), else block Jacobi on G
+  // large sectors: the LR step, and without a cutoff (every value is kept) block
+  // Jacobi on G, formed again, for those it cannot serve
   int brc = 0;
-  if (!big.empty())
-    brc = cutoff > 0 ? lr_eigen(big, nq, goff, eoff, d_eoff, goff[nQ], G, Vev, ev, s)
-                     : block_jacobi(big, nq, d_goff, d_eoff, G, Vev, ev, s, 40, kJacFloor);
+  std::vector<int> plain, lr;
+  for (int q : big) (cutoff > 0 || nq[q] <= kPcMaxN ? lr : plain).push_back(q);
+  if (!lr.empty()) {
+    brc = lr_eigen(lr, nq, kq, cutoff > 0, plain, goff, eoff, d_eoff, goff[nQ], G, Vev, ev, s);
+    if (brc && !(cutoff > 0)) {   // (no room for its arrays, say)
+      plain = big;
+      brc = 0;
+    }
+  }
+  if (!brc && !plain.empty()) {
+    brc = gram(plain);
+    if (!brc) brc = block_jacobi(plain, nq, d_goff, d_eoff, G, Vev, ev, s, 40, kJacFloor);
+  }
   if (forked) {
     // join before anything else, the error path included: the scratch the
     // side stream reads goes back to the pool when this call returns

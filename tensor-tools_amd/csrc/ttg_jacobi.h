@@ -70,6 +70,20 @@ __device__ __forceinline__ void jac_rotation(double app, double aqq, double apq,
   s = td * c;
 }
 
+// x^(-1/2) for x > 0 of any size: the hardware estimate (better than 2^-20) of
+// the value scaled by a power of four, and two Newton steps
+__device__ __forceinline__ double jac_rsqrt(double x) {
+  const int ex = __builtin_amdgcn_frexp_exp(x) & ~1;
+  const double m = __builtin_amdgcn_ldexp(x, -ex);
+  double y = __builtin_amdgcn_rsq(m);
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const double e = fma(-m * y, y, 1.0);
+    y = fma(0.5 * y, e, y);
+  }
+  return __builtin_amdgcn_ldexp(y, -(ex >> 1));
+}
+
 constexpr double kJacRel = 1e-12;   // an off-diagonal below this of sqrt(a_pp a_qq) is converged
 
 __device__ __forceinline__ bool jac_significant(double app, double aqq, double apq, double floor_abs) {

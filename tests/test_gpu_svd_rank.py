@@ -86,3 +86,29 @@ def test_kept_values_within_the_rank():
     assert np.abs(s - want).max() < 1e-12
     for u, _, _ in out.values():
         assert np.linalg.norm(u.T @ u - np.eye(u.shape[1]), 2) < 1e-13
+
+
+LARGE = [(65, 65, 30), (65, 65, 65), (100, 40, 40), (128, 128, 64), (130, 200, 127), (200, 300, 200), (300, 300, 150),
+         (300, 150, 90), (70, 70, 1), (80, 80, 0)]
+
+
+@pytest.mark.parametrize("direction", [T.MOVE_FROM_LEFT, T.MOVE_FROM_RIGHT])
+@pytest.mark.parametrize("cutoff", [0.0, 1e-10])
+def test_large_sectors(direction, cutoff):
+    check(LARGE, direction, cutoff)
+
+
+@pytest.mark.parametrize("cutoff", [0.0, 1e-10])
+def test_equal_diagonals(cutoff):
+    """more equal remaining diagonals than a panel has candidates"""
+    n = 150
+    i = make_index(INWARD, "i", LINK, 0, [((0, 0), n)])
+    j = make_index(OUTWARD, "j", LINK, 0, [((0, 0), n)])
+    A = T.DTensor.from_flat(FlatTensor([i, j], np.array([[0, 0]], np.int32), 3.0 * np.eye(n).reshape(-1)))
+    h = [C.c_void_p() for _ in range(3)]
+    T.check(T.lib().ttg_svd(A.h, 1, T.MOVE_FROM_LEFT, cutoff, 0, C.byref(h[0]), C.byref(h[1]), C.byref(h[2]),
+                            C.byref(C.c_double(0)), C.byref(C.c_int64(0))))
+    u, s, v = (T.DTensor(x, []).data() for x in h)
+    u, v = u.reshape(n, n, order="F"), v.reshape(n, n, order="F")
+    assert np.abs(s - 3.0).max() < 1e-12
+    assert np.abs(u @ v - 3.0 * np.eye(n)).max() < 1e-12
