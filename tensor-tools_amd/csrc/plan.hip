@@ -25,58 +25,145 @@ __device__ inline uint32_t qcode(int q0, int q1) {
   return ((uint32_t)(q0 + 32768) << 16) | (uint32_t)(q1 + 32768);
 }
 
+// One operand of a contraction as the planning kernels read it, made on the host:
+// kernel arguments lie in host memory, and a list of positions that is walked in
+// them is a chain of slow loads.
+struct OperandSpec {
+  const int *idx, *qi;
+  const int64_t* off;
+  int nblocks, rank, nf, np;
+  unsigned free;               // bit j: index j is not contracted
+  int start[MAXR];             // of index j's sectors in idx
+  unsigned wf[MAXR], wm[MAXR]; // place values of index j in the free and in the contracted tuple
+  int sign[MAXR];              // of index j's QN in q: +1, -1, or 0 (contracted)
+  int pair[MAXR];              // index of pair p
+};
+
 // Sorted keys and groups of one plan (device scratch, nmax entries each).
 // q is a function of the left tuple, so the blocks of A with one left tuple are
-// a run of sSA, in ascending mid order: the candidates of every result block
-// with that left tuple, in the reference's mid order.
+// a run of SA, in ascending mid order: the candidates of every result block
+// with that left tuple, in the reference's mid order.  What a result block
+// needs of a block, a tuple or a q group is one record: its address depends on the
+// record before, and every such step is a load that misses to memory (about
+// 0.9 us).
+struct PlanRec {          // a block of A or B
+  uint64_t key;           // (left, mid) or (mid, right)
+  int64_t off;            // of its data
+  int id, ext;            // ext: product of the free extents
+  unsigned e0, s0, s1;    // the free indices folded into one mixed-radix index (Fold)
+  int n, pad[2];
+  unsigned dk[MAXR], sk[MAXR];   // extent and stride of the index of pair p
+};
+struct PlanL {            // a left tuple: first entry of SA, blocks, blocks of all earlier ones
+  int sa0, cnt, lpre, pad;
+};
+struct PlanR {            // a right tuple, one block of B that has it, and its extent
+  unsigned right;
+  int rep;
+  int64_t N;
+};
+struct PlanQ {            // a q group
+  int64_t base, cand;     // first result block, first candidate
+  int l0, nL, r0;         // first left tuple, left tuples, first right tuple
+  int lpre, wid;          // L[l0].lpre, candidates per right tuple
+  int pad[3];
+};
 struct PlanSets {
   uint64_t *kUL, *kSA, *kUR, *kSB;   // keys by block (the path of many blocks)
   uint64_t *sUL, *sSA, *sUR, *sSB;   // sorted: (q, left), (left, mid), (q, right), (mid, right)
   int *svSA, *svUR, *svSB;           // block ids in those orders
-  uint64_t *uL, *uR;                 // unique (q, left), (q, right)
-  int *lsa0, *lcnt, *lpre;           // per left tuple: first entry of sSA, blocks, blocks of all earlier ones (nuL + 1)
-  int *rrep;                         // per right tuple: one block of B that has it
-  int *qL0, *qL1, *qR0, *qR1;        // per q: ranges of uL and uR
-  int64_t *qbase, *qcand;            // per q: first result block, first candidate (nQ + 1)
+  uint64_t *uL, *uR;                 // unique (q, left), (q, right) (the path of many blocks)
+  int* qL0;                          // first left tuple of every q (the path of many blocks)
+  PlanRec *SA, *SB;                  // blocks in the orders of sSA and sSB
+  PlanL* L;                          // (one more: the total in lpre)
+  PlanR* R;
+  PlanQ* Q;
 };
 
-__device__ inline void plan_key_a(const MetaView& A, const PairSpec& ps, int i, uint64_t& ul, uint64_t& sa) {
-  const int* qi = A.qi + (size_t)i * A.rank;
+// fold (extent, stride) components in order: extent-1 ones are dropped,
+// contiguous runs merged; n counts the components, the first two are kept.
+// 32 bits: an operand block of 2^28 elements or more is refused (opmax).
+struct Fold {
+  int n = 0;
+  unsigned e0 = 1, ce = 0, cs = 0, s0 = 0, s1 = 0;   // ce: extent of the open component (0: none)
+  __device__ __forceinline__ void close() {
+    const bool open = ce != 0;
+    e0 = open && n == 0 ? ce : e0;
+    s0 = open && n == 0 ? cs : s0;
+    s1 = open && n == 1 ? cs : s1;
+    n += open;
+    ce = 0;
+  }
+  __device__ __forceinline__ void add(unsigned ext, unsigned st) {
+    if (ext == 1) return;
+    if (ce != 0 && st == ce * cs) { ce *= ext; return; }
+    close();
+    ce = ext;
+    cs = st;
+  }
+};
+
+// keys of block i: (q, free tuple), the free and the contracted tuple; with REC its
+// record as well, but for the key
+template <bool REC>
+__device__ __forceinline__ void plan_block(const OperandSpec& M, int i, uint64_t& uq, unsigned& fr, unsigned& mid,
+                                           PlanRec& r, int64_t& ext) {
+  int s[MAXR], e0[MAXR], e1[MAXR];
+  unsigned d[MAXR];
+  if (REC) r.off = M.off[i];
+#pragma unroll
+  for (int j = 0; j < MAXR; j++) s[j] = j < M.rank ? M.qi[(size_t)i * M.rank + j] : 0;
+#pragma unroll
+  for (int j = 0; j < MAXR; j++) {
+    const int* e = M.idx + (j < M.rank ? 3 * (M.start[j] + s[j]) : 0);
+    e0[j] = e1[j] = 0;
+    d[j] = 1;
+    if (j < M.rank) {
+      e0[j] = e[0];
+      e1[j] = e[1];
+      d[j] = e[2];
+    }
+  }
   int q0 = 0, q1 = 0;
-  uint64_t left = 0, mid = 0;
-  for (int j = 0; j < ps.nfa; j++) {
-    int p = ps.fa[j], s = qi[p];
-    const int* e = A.idx + 3 * (A.idx_off[p] + s);
-    int sg = A.arrow[p] == 0 ? 1 : -1;          // Inward +, Outward - (:617-621)
-    q0 += sg * e[0];
-    q1 += sg * e[1];
-    left = left * A.nsec[p] + s;
+  fr = mid = 0;
+  ext = 1;
+#pragma unroll
+  for (int j = 0; j < MAXR; j++) {
+    q0 += M.sign[j] * e0[j];
+    q1 += M.sign[j] * e1[j];
+    fr += M.wf[j] * (unsigned)s[j];
+    mid += M.wm[j] * (unsigned)s[j];
+    ext *= (M.free >> j) & 1 ? d[j] : 1u;
   }
-  for (int t = 0; t < ps.np; t++) {
-    int p = ps.pa[t];
-    mid = mid * A.nsec[p] + qi[p];
+  uq = ((uint64_t)qcode(q0, q1) << 32) | fr;
+  if (REC) {
+    Fold f;
+    unsigned st[MAXR], acc = 1;   // strides of the stored (unpermuted) block
+#pragma unroll
+    for (int j = 0; j < MAXR; j++) {
+      st[j] = acc;
+      if ((M.free >> j) & 1) f.add(d[j], acc);
+      acc *= d[j];
+    }
+    f.close();
+    r.id = i;
+    r.ext = (int)min(ext, (int64_t)0x7fffffff);   // (a block of 2^28 elements is refused, opmax)
+    r.e0 = f.e0;
+    r.s0 = f.s0;
+    r.s1 = f.s1;
+    r.n = f.n;
+#pragma unroll
+    for (int p = 0; p < MAXR; p++) {
+      r.dk[p] = 1;
+      r.sk[p] = 0;
+      if (p < M.np)
+#pragma unroll
+        for (int j = 0; j < MAXR; j++) {
+          r.dk[p] = j == M.pair[p] ? d[j] : r.dk[p];
+          r.sk[p] = j == M.pair[p] ? st[j] : r.sk[p];
+        }
+    }
   }
-  ul = ((uint64_t)qcode(q0, q1) << 32) | left;
-  sa = (left << 32) | mid;
-}
-__device__ inline void plan_key_b(const MetaView& B, const PairSpec& ps, int i, uint64_t& ur, uint64_t& sb) {
-  const int* qi = B.qi + (size_t)i * B.rank;
-  int q0 = 0, q1 = 0;
-  uint64_t right = 0, mid = 0;
-  for (int j = 0; j < ps.nfb; j++) {
-    int p = ps.fb[j], s = qi[p];
-    const int* e = B.idx + 3 * (B.idx_off[p] + s);
-    int sg = B.arrow[p] == 0 ? -1 : 1;          // Inward -, Outward + (:629-633)
-    q0 += sg * e[0];
-    q1 += sg * e[1];
-    right = right * B.nsec[p] + s;
-  }
-  for (int t = 0; t < ps.np; t++) {
-    int p = ps.pb[t];
-    mid = mid * B.nsec[p] + qi[p];
-  }
-  ur = ((uint64_t)qcode(q0, q1) << 32) | right;
-  sb = (mid << 32) | right;
 }
 
 // ---- groups of the sorted keys (one workgroup) ---------------------------
@@ -120,157 +207,217 @@ __device__ inline int64_t block_prefix(int64_t v, int64_t* lds, int64_t* total) 
   return base + x - v;
 }
 
-// Unique left and right tuples, q groups, and the first result block and first
-// candidate of every group.  The sorted keys are read from, and the unique
-// ones written to, LDS or global memory (cuL may be sUL, cuR may be sUR); the
-// other results go to w's global arrays and the header to both headers.
-__device__ __forceinline__ void plan_groups(const uint64_t* sUL, const uint64_t* sSA, const uint64_t* sUR, const int* svUR,
-                                            uint64_t* cuL, uint64_t* cuR, int nA, int nB, const PlanSets& w,
-                                            int* lds_i, int64_t* lds_l, PlanHdr* hdr, PlanHdr* host) {
-  const int nt = blockDim.x, tid = threadIdx.x;
-  int nuL = 0, nuR = 0, nQ = 0;
-  int64_t blocks_before = 0;   // blocks of A before the chunk
-  for (int base = 0; base < nA; base += nt) {
-    const int i = base + tid;
-    const uint64_t key = i < nA ? sUL[i] : 0;
-    const bool f = i < nA && (i == 0 || key != sUL[i - 1]);
-    int tot;
-    const int pos = nuL + block_rank(f, lds_i, &tot);
-    int cnt = 0, a0 = 0;
-    if (f) {
-      const uint64_t left = key & 0xffffffffull;
-      a0 = lower_bound_u64(sSA, nA, left << 32);
-      cnt = lower_bound_u64(sSA, nA, (left + 1) << 32) - a0;
-    }
-    int64_t all;
-    const int64_t pre = block_prefix(cnt, lds_l, &all);
-    if (f) {
-      cuL[pos] = key;
-      w.lsa0[pos] = a0;
-      w.lcnt[pos] = cnt;
-      w.lpre[pos] = (int)(blocks_before + pre);
-    }
-    nuL += tot;
-    blocks_before += all;
-  }
-  for (int base = 0; base < nB; base += nt) {
-    const int i = base + tid;
-    const uint64_t key = i < nB ? sUR[i] : 0;
-    const bool f = i < nB && (i == 0 || key != sUR[i - 1]);
-    int tot;
-    const int pos = nuR + block_rank(f, lds_i, &tot);   // (its barriers: every read of the chunk comes before a write)
-    if (f) {
-      cuR[pos] = key;
-      w.uR[pos] = key;
-      w.rrep[pos] = svUR[i];
-    }
-    nuR += tot;
-  }
-  if (tid == 0) w.lpre[nuL] = (int)blocks_before;
-  __syncthreads();
-  // q groups of the left tuples (ascending q; A's mid-QN set, :622-623)
-  for (int base = 0; base < nuL; base += nt) {
-    const int i = base + tid;
-    const bool f = i < nuL && (i == 0 || (cuL[i] >> 32) != (cuL[i - 1] >> 32));
-    int tot;
-    const int pos = nQ + block_rank(f, lds_i, &tot);
-    if (f) w.qL0[pos] = i;
-    nQ += tot;
+// ---- up to kPlanSmall blocks per operand: keys, sorts and groups in one
+// workgroup's LDS, a thread per block.  The four key arrays are sorted in runs of 64, a
+// run a wave in its registers (a key's place is the number of keys below it), and
+// the runs merged by binary searches in the other runs.  The q groups follow from
+// three prefix sums, of values packed into one word.  At 168 blocks the sort took
+// 50000 cycles as bitonic networks in LDS and takes 12000, the groups 13000 and 9000; what
+// bounds the rest is the keys' two dependent loads (6000 to 9000): 24 us before, 16 now,
+// 12.8 at 10 blocks.
+constexpr int kPlanSmall = 1024;
+struct PlanLds {
+  uint64_t K[4][kPlanSmall];         // (q, left), (left, mid), (q, right), (mid, right); ~0 beyond the blocks
+  uint64_t S[4][kPlanSmall];         // runs; later the unique keys
+  unsigned short V[kPlanSmall], W[4][kPlanSmall];      // block ids of (q, right); of S
+  unsigned short place[2][kPlanSmall];                 // of every block in SA and SB
+  int64_t N[kPlanSmall];             // free extent of B's blocks
+  int lpre[kPlanSmall + 1], qL0[kPlanSmall];
+  uint64_t sums[kPlanThreads / 64];
+};
+
+// exclusive prefix sum of packed fields over the workgroup, and the total
+__device__ __forceinline__ uint64_t plan_scan64(uint64_t v, uint64_t* sums, uint64_t* total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  uint64_t x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint64_t y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
   }
   __syncthreads();
-  int64_t nblk = 0, ncand = 0;
-  for (int base = 0; base < nQ; base += nt) {
-    const int t = base + tid;
-    int64_t cnt = 0, cand = 0;
-    if (t < nQ) {
-      const int l0 = w.qL0[t], l1 = t + 1 < nQ ? w.qL0[t + 1] : nuL;
-      const uint64_t qc = cuL[l0] >> 32;
-      const int r0 = lower_bound_u64(cuR, nuR, qc << 32), r1 = lower_bound_u64(cuR, nuR, (qc + 1) << 32);
-      w.qL1[t] = l1;
-      w.qR0[t] = r0;
-      w.qR1[t] = r1;
-      cnt = (int64_t)(l1 - l0) * (r1 - r0);
-      cand = (int64_t)(w.lpre[l1] - w.lpre[l0]) * (r1 - r0);
-    }
-    int64_t tot, tot2;
-    const int64_t pb = block_prefix(cnt, lds_l, &tot), pc = block_prefix(cand, lds_l, &tot2);
-    if (t < nQ) {
-      w.qbase[t] = nblk + pb;
-      w.qcand[t] = ncand + pc;
-    }
-    nblk += tot;
-    ncand += tot2;
+  if (lane == 63) sums[w] = x;
+  __syncthreads();
+  uint64_t base = 0, tot = 0;
+#pragma unroll
+  for (int k = 0; k < kPlanThreads / 64; k++) {
+    const uint64_t c = k < nw ? sums[k] : 0;
+    base += k < w ? c : 0;
+    tot += c;
   }
-  if (tid == 0) {
-    w.qbase[nQ] = nblk;
-    w.qcand[nQ] = ncand;
-    hdr->nQ = host->nQ = nQ;
-    hdr->nblocksC = host->nblocksC = nblk;
-    hdr->ncand = host->ncand = ncand;
-  }
+  *total = tot;
+  return base + x - v;
 }
 
-// ---- up to kPlanSmall blocks per operand: keys, sorts and groups in one
-// workgroup's LDS (one launch and 12 us where the three kernels below take
-// 23 us and two launch gaps at a few hundred blocks).  The four key arrays
-// are sorted together by bitonic networks of P entries, P the power of two
-// above both block counts.
-constexpr int kPlanSmall = 1024;
-__global__ void __launch_bounds__(kPlanThreads) k_plan_small(MetaView A, MetaView B, PairSpec ps, int P, PlanSets w,
-                                                             PlanHdr* hdr, PlanHdr* host) {
-  __shared__ uint64_t K[4][kPlanSmall];   // (q, left), (left, mid), (q, right), (mid, right)
-  __shared__ int V[3][kPlanSmall];        // block ids of the last three
-  __shared__ int lds_i[kPlanThreads / 64];
-  __shared__ int64_t lds_l[kPlanThreads / 64];
-  const int tid = threadIdx.x, nA = A.nblocks, nB = B.nblocks;
-  for (int i = tid; i < P; i += blockDim.x) {
-    uint64_t ul = ~0ull, sa = ~0ull, ur = ~0ull, sb = ~0ull;   // above every key: a tuple's half is below 2^32 - 1
-    if (i < nA) plan_key_a(A, ps, i, ul, sa);
-    if (i < nB) plan_key_b(B, ps, i, ur, sb);
-    K[0][i] = ul;
-    K[1][i] = sa;
-    K[2][i] = ur;
-    K[3][i] = sb;
-    V[0][i] = V[1][i] = V[2][i] = i;
+// keys below a (and below b) of an ascending array of P entries, P a power of two
+__device__ __forceinline__ void plan_count2(const uint64_t* k, int P, uint64_t a, uint64_t b, int& ca, int& cb) {
+  ca = cb = 0;
+  for (int s = P >> 1; s > 0; s >>= 1) {
+    const uint64_t x = k[ca + s - 1], y = k[cb + s - 1];
+    ca += x < a ? s : 0;
+    cb += y < b ? s : 0;
   }
-  const int half = P >> 1, hs = 31 - __builtin_clz(half | 1);   // half = 1 << hs (P >= 2)
-  for (int k = 2; k <= P; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      __syncthreads();
-      for (int c = tid; c < 4 * half; c += blockDim.x) {
-        const int a = c >> hs, e = c & (half - 1);
-        const int i = 2 * e - (e & (j - 1)), l = i + j;
-        const uint64_t x = K[a][i], y = K[a][l];
-        // equal keys keep block order (a repeated block is found at its first id)
-        const bool after = x > y || (x == y && a > 0 && V[a - 1][i] > V[a - 1][l]);
-        if (after == ((i & k) == 0)) {
-          K[a][i] = y;
-          K[a][l] = x;
-          if (a > 0) {
-            const int t = V[a - 1][i];
-            V[a - 1][i] = V[a - 1][l];
-            V[a - 1][l] = t;
-          }
-        }
+  const uint64_t x = k[ca], y = k[cb];
+  ca += x < a;
+  cb += y < b;
+}
+
+__global__ void __launch_bounds__(kPlanThreads) k_plan_small(OperandSpec A, OperandSpec B, PlanSets w, PlanHdr* hdr,
+                                                             PlanHdr* host) {
+  __shared__ PlanLds L;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+  const int nA = A.nblocks, nB = B.nblocks;
+  const int runs = (max(max(nA, nB), 1) + 63) >> 6;   // of 64 keys
+  int P = 64;
+  while (P < 64 * runs) P *= 2;
+  PlanRec ra{}, rb{};                 // of blocks tid of A and B
+  {
+    uint64_t k[4] = {~0ull, ~0ull, ~0ull, ~0ull};     // above every key: a tuple's half is below 2^32 - 1
+    unsigned f, m;
+    int64_t ext;
+    if (tid < nA) {
+      plan_block<true>(A, tid, k[0], f, m, ra, ext);
+      k[1] = ra.key = (uint64_t)f << 32 | m;          // (left, mid)
+    }
+    if (tid < nB) {
+      plan_block<true>(B, tid, k[2], f, m, rb, ext);
+      k[3] = rb.key = (uint64_t)m << 32 | f;          // (mid, right)
+      L.N[tid] = ext;
+    }
+    for (int i = tid; i < P; i += blockDim.x)
+#pragma unroll
+      for (int a = 0; a < 4; a++) L.K[a][i] = i == tid ? k[a] : ~0ull;
+  }
+  __syncthreads();
+  for (int t = wave; t < 4 * runs; t += nw) {
+    const int a = t & 3, i = (t >> 2) * 64 + lane;
+    const uint64_t key = L.K[a][i];
+    const unsigned lo = (unsigned)key, hi = (unsigned)(key >> 32);
+    // keys of the run below this one; equal keys keep block order, and so does the
+    // padding, behind all n keys
+    const int n = min(64, max(0, (a < 2 ? nA : nB) - (t >> 2) * 64));
+    int c = 0;
+    for (int e0 = 0; e0 < n; e0 += 8) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int e = e0 + u;
+        const uint64_t o = (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)hi, e) << 32 |
+                           (unsigned)__builtin_amdgcn_readlane((int)lo, e);
+        c += (o < key) | ((o == key) & (e < lane));
       }
     }
+    if (lane >= n) c = lane;
+    L.S[a][(t >> 2) * 64 + c] = key;
+    L.W[a][(t >> 2) * 64 + c] = (unsigned short)i;
+  }
   __syncthreads();
-  for (int i = tid; i < nA; i += blockDim.x) {
-    w.sSA[i] = K[1][i];
-    w.svSA[i] = V[0][i];
+  for (int t = wave; t < 4 * runs; t += nw) {
+    const int a = t & 3, run = t >> 2;
+    const uint64_t key = L.S[a][64 * run + lane];
+    int c = lane;
+    for (int o = 0; o < runs; o++) {
+      if (o == run) continue;
+      // keys of run o before this one: below it, or equal in an earlier run
+      const uint64_t lim = o < run ? key + 1 : key;   // (~0, padding: it goes last in any order, handled below)
+      const uint64_t* r = &L.S[a][64 * o];
+      int n = 0;
+#pragma unroll
+      for (int s = 32; s > 0; s >>= 1) n += r[n + s - 1] < lim ? s : 0;
+      n += r[n] < lim;
+      c += n;
+    }
+    if (key != ~0ull) {
+      L.K[a][c] = key;
+      const unsigned short id = L.W[a][64 * run + lane];
+      if (a == 2) L.V[c] = id;
+      else if (a) L.place[a >> 1][id] = (unsigned short)c;
+    }
   }
-  for (int i = tid; i < nB; i += blockDim.x) {
-    w.sSB[i] = K[3][i];
-    w.svSB[i] = V[2][i];
+  for (int i = tid; i < P; i += blockDim.x) {         // (places of no key)
+    if (i >= nA) L.K[0][i] = L.K[1][i] = ~0ull;
+    if (i >= nB) L.K[2][i] = L.K[3][i] = ~0ull;
   }
-  plan_groups(K[0], K[1], K[2], V[1], K[0], K[2], nA, nB, w, lds_i, lds_l, hdr, host);
+  __syncthreads();
+  if (tid < nA) w.SA[L.place[0][tid]] = ra;
+  if (tid < nB) {
+    w.SB[L.place[1][tid]] = rb;
+    w.sSB[L.place[1][tid]] = rb.key;
+  }
+  // unique left and right tuples, and the blocks of A of every left one
+  const uint64_t kl = tid < nA ? L.K[0][tid] : ~0ull, kr = tid < nB ? L.K[2][tid] : ~0ull;
+  const bool fl = tid < nA && (tid == 0 || kl != L.K[0][tid - 1]);
+  const bool fr = tid < nB && (tid == 0 || kr != L.K[2][tid - 1]);
+  int a0 = 0, a1 = 0;
+  if (fl) plan_count2(L.K[1], P, (kl & 0xffffffffull) << 32, ((kl & 0xffffffffull) + 1) << 32, a0, a1);
+  uint64_t tot;
+  const uint64_t pre = plan_scan64((uint64_t)fl | (uint64_t)fr << 16 | (uint64_t)(a1 - a0) << 32, L.sums, &tot);
+  const int nuL = (int)(tot & 0xffff), nuR = (int)(tot >> 16 & 0xffff), all = (int)(tot >> 32);
+  uint64_t *cuL = L.S[0], *cuR = L.S[2];
+  if (fl) {
+    const int l = (int)(pre & 0xffff), lp = (int)(pre >> 32);
+    cuL[l] = kl;
+    L.lpre[l] = lp;
+    w.L[l] = PlanL{a0, a1 - a0, lp, 0};
+  }
+  if (fr) {
+    const int r = (int)(pre >> 16 & 0xffff), rep = L.V[tid];
+    cuR[r] = kr;
+    w.R[r] = PlanR{(unsigned)kr, rep, L.N[rep]};
+  }
+  if (tid == 0) L.lpre[nuL] = all;
+  if (tid >= nuR && tid < P) cuR[tid] = ~0ull;   // (the workgroup has P threads at least)
+  __syncthreads();
+  // q groups of the left tuples (ascending q; A's mid-QN set, :622-623)
+  const bool fq = tid < nuL && (tid == 0 || (cuL[tid] >> 32) != (cuL[tid - 1] >> 32));
+  const int qi = (int)plan_scan64(fq, L.sums, &tot), nQ = (int)tot;
+  if (fq) L.qL0[qi] = tid;
+  __syncthreads();
+  PlanQ q{};
+  uint64_t mine = 0;
+  if (tid < nQ) {
+    q.l0 = L.qL0[tid];
+    const int l1 = tid + 1 < nQ ? L.qL0[tid + 1] : nuL;
+    const uint64_t qc = cuL[q.l0] >> 32;
+    q.nL = l1 - q.l0;
+    int r1;
+    plan_count2(cuR, P, qc << 32, qc == 0xffffffffull ? ~0ull : (qc + 1) << 32, q.r0, r1);
+    const int nR = r1 - q.r0;
+    q.lpre = L.lpre[q.l0];
+    q.wid = L.lpre[l1] - q.lpre;
+    mine = (uint64_t)(q.nL * nR) | (uint64_t)(q.wid * nR) << 32;   // both at most nA * nB <= 2^20
+  }
+  const uint64_t at = plan_scan64(mine, L.sums, &tot);
+  if (tid < nQ) {
+    q.base = (int64_t)(at & 0xffffffffull);
+    q.cand = (int64_t)(at >> 32);
+    w.Q[tid] = q;
+  }
+  if (tid == 0) {
+    hdr->nQ = nQ;
+    hdr->nblocksC = (int64_t)(tot & 0xffffffffull);
+    hdr->ncand = (int64_t)(tot >> 32);
+    hdr->done = 0;
+    if (host) {
+      host->nblocksC = hdr->nblocksC;
+      host->ncand = hdr->ncand;
+    }
+  }
 }
 
 // ---- more blocks: keys, stable rank sort (grid.y selects the array), groups
-__global__ void k_plan_keys(MetaView A, MetaView B, PairSpec ps, PlanSets w) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < A.nblocks) plan_key_a(A, ps, i, w.kUL[i], w.kSA[i]);
-  if (i < B.nblocks) plan_key_b(B, ps, i, w.kUR[i], w.kSB[i]);
+__global__ void k_plan_keys(OperandSpec A, OperandSpec B, PlanSets w) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  PlanRec none;
+  unsigned f, m;
+  int64_t ext;
+  if (i < A.nblocks) {
+    plan_block<false>(A, i, w.kUL[i], f, m, none, ext);
+    w.kSA[i] = (uint64_t)f << 32 | m;
+  }
+  if (i < B.nblocks) {
+    plan_block<false>(B, i, w.kUR[i], f, m, none, ext);
+    w.kSB[i] = (uint64_t)m << 32 | f;
+  }
 }
 
 struct SortJob {
@@ -304,10 +451,117 @@ __global__ void __launch_bounds__(256) k_rank_sort(SortJobs jobs) {
   }
 }
 
-__global__ void __launch_bounds__(kPlanThreads) k_plan_groups(int nA, int nB, PlanSets w, PlanHdr* hdr, PlanHdr* host) {
+// Unique left and right tuples, q groups, and the first result block and first
+// candidate of every group, by one workgroup (the path of many blocks).
+__global__ void __launch_bounds__(kPlanThreads) k_plan_groups(OperandSpec B, int nA, int nB, PlanSets w,
+                                                              PlanHdr* hdr, PlanHdr* host) {
   __shared__ int lds_i[kPlanThreads / 64];
   __shared__ int64_t lds_l[kPlanThreads / 64];
-  plan_groups(w.sUL, w.sSA, w.sUR, w.svUR, w.uL, w.uR, nA, nB, w, lds_i, lds_l, hdr, host);
+  const uint64_t *sUL = w.sUL, *sSA = w.sSA, *sUR = w.sUR;
+  uint64_t *cuL = w.uL, *cuR = w.uR;
+  const int nt = blockDim.x, tid = threadIdx.x;
+  int nuL = 0, nuR = 0, nQ = 0;
+  int64_t blocks_before = 0;   // blocks of A before the chunk
+  for (int base = 0; base < nA; base += nt) {
+    const int i = base + tid;
+    const uint64_t key = i < nA ? sUL[i] : 0;
+    const bool f = i < nA && (i == 0 || key != sUL[i - 1]);
+    int tot;
+    const int pos = nuL + block_rank(f, lds_i, &tot);
+    int cnt = 0, a0 = 0;
+    if (f) {
+      const uint64_t left = key & 0xffffffffull;
+      a0 = lower_bound_u64(sSA, nA, left << 32);
+      cnt = lower_bound_u64(sSA, nA, (left + 1) << 32) - a0;
+    }
+    int64_t all;
+    const int64_t pre = block_prefix(cnt, lds_l, &all);
+    if (f) {
+      cuL[pos] = key;
+      w.L[pos] = PlanL{a0, cnt, (int)(blocks_before + pre), 0};
+    }
+    nuL += tot;
+    blocks_before += all;
+  }
+  for (int base = 0; base < nB; base += nt) {
+    const int i = base + tid;
+    const uint64_t key = i < nB ? sUR[i] : 0;
+    const bool f = i < nB && (i == 0 || key != sUR[i - 1]);
+    int tot;
+    const int pos = nuR + block_rank(f, lds_i, &tot);   // (its barriers: every read of the chunk comes before a write)
+    if (f) {
+      cuR[pos] = key;
+      const int rep = w.svUR[i];
+      uint64_t uq;
+      unsigned f, m;
+      PlanRec none;
+      int64_t N;
+      plan_block<false>(B, rep, uq, f, m, none, N);
+      w.R[pos] = PlanR{(unsigned)key, rep, N};
+    }
+    nuR += tot;
+  }
+  if (tid == 0) w.L[nuL].lpre = (int)blocks_before;
+  __syncthreads();
+  // q groups of the left tuples (ascending q; A's mid-QN set, :622-623)
+  for (int base = 0; base < nuL; base += nt) {
+    const int i = base + tid;
+    const bool f = i < nuL && (i == 0 || (cuL[i] >> 32) != (cuL[i - 1] >> 32));
+    int tot;
+    const int pos = nQ + block_rank(f, lds_i, &tot);
+    if (f) w.qL0[pos] = i;
+    nQ += tot;
+  }
+  __syncthreads();
+  int64_t nblk = 0, ncand = 0;
+  for (int base = 0; base < nQ; base += nt) {
+    const int t = base + tid;
+    int64_t cnt = 0, cand = 0;
+    PlanQ q{};
+    if (t < nQ) {
+      q.l0 = w.qL0[t];
+      const int l1 = t + 1 < nQ ? w.qL0[t + 1] : nuL;
+      const uint64_t qc = cuL[q.l0] >> 32;
+      q.nL = l1 - q.l0;
+      q.r0 = lower_bound_u64(cuR, nuR, qc << 32);
+      const int nR = lower_bound_u64(cuR, nuR, (qc + 1) << 32) - q.r0;
+      q.lpre = w.L[q.l0].lpre;
+      q.wid = w.L[l1].lpre - q.lpre;
+      cnt = (int64_t)q.nL * nR;
+      cand = (int64_t)q.wid * nR;
+    }
+    int64_t tot, tot2;
+    const int64_t pb = block_prefix(cnt, lds_l, &tot), pc = block_prefix(cand, lds_l, &tot2);
+    if (t < nQ) {
+      q.base = nblk + pb;
+      q.cand = ncand + pc;
+      w.Q[t] = q;
+    }
+    nblk += tot;
+    ncand += tot2;
+  }
+  if (tid == 0) {
+    hdr->nQ = nQ;
+    hdr->nblocksC = host->nblocksC = nblk;
+    hdr->ncand = host->ncand = ncand;
+    hdr->done = 0;
+  }
+}
+
+// the records of the sorted blocks
+__global__ void __launch_bounds__(256) k_plan_recs(OperandSpec A, OperandSpec B, PlanSets w) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  auto rec = [&](const OperandSpec& M, int id, uint64_t key) {
+    PlanRec r{};
+    uint64_t uq;
+    unsigned f, m;
+    int64_t ext;
+    plan_block<true>(M, id, uq, f, m, r, ext);
+    r.key = key;
+    return r;
+  };
+  if (i < A.nblocks) w.SA[i] = rec(A, w.svSA[i], w.sSA[i]);
+  if (i < B.nblocks) w.SB[i] = rec(B, w.svSB[i], w.sSB[i]);
 }
 
 // ---- per result block: tuple, dims, task enumeration ---------------------
@@ -321,28 +575,6 @@ struct BlkStat {
   int votes[4];        // tasks with unit stride: A m, A k, B k, B n
 };
 
-// fold (extent, stride) components in order: extent-1 ones are dropped,
-// contiguous runs merged; n counts the components, the first two are kept.
-// 32 bits: an operand block of 2^28 elements or more is refused (opmax).
-struct Fold {
-  int n = 0;
-  unsigned e0 = 1, ce = 0, cs = 0, s0 = 0, s1 = 0;   // ce: extent of the open component (0: none)
-  __device__ __forceinline__ void close() {
-    const bool open = ce != 0;
-    e0 = open && n == 0 ? ce : e0;
-    s0 = open && n == 0 ? cs : s0;
-    s1 = open && n == 1 ? cs : s1;
-    n += open;
-    ce = 0;
-  }
-  __device__ __forceinline__ void add(unsigned ext, unsigned st) {
-    if (ext == 1) return;
-    if (ce != 0 && st == ce * cs) { ce *= ext; return; }
-    close();
-    ce = ext;
-    cs = st;
-  }
-};
 // the same for K, whose components have a stride in each operand
 struct FoldK {
   int n = 0;
@@ -366,238 +598,81 @@ struct FoldK {
     cb = sb;
   }
 };
-// extent and stride of index p (uniform, runtime) of a block of extents d:
-// products of selects, so the array stays in registers
-__device__ __forceinline__ unsigned ext_of(const unsigned (&d)[MAXR], int p) {
-  unsigned r = 1;
-#pragma unroll
-  for (int j = 0; j < MAXR; j++) r *= j == p ? d[j] : 1u;
-  return r;
+// v combined over the lanes of a wave
+template <class T, class Op>
+__device__ __forceinline__ T wave_all(T v, Op op) {
+  v = op(v, lane_xor<1>(v));
+  v = op(v, lane_xor<2>(v));
+  v = op(v, lane_xor<4>(v));
+  v = op(v, lane_xor<8>(v));
+  v = op(v, lane_xor<16>(v));
+  return op(v, lane_xor<32>(v));
 }
-__device__ __forceinline__ unsigned stride_of(const unsigned (&d)[MAXR], int p) {
-  unsigned r = 1;
-#pragma unroll
-  for (int j = 0; j < MAXR - 1; j++) r *= j < p ? d[j] : 1u;
-  return r;
+template <class T>
+__device__ __forceinline__ T wave_sum(T v) {
+  return wave_all(v, [](T a, T b) { return a + b; });
 }
-
-__device__ inline int64_t wave_sum_i64(int64_t v) {
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-  return v;
-}
-__device__ inline int wave_sum_i32(int v) {
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-  return v;
-}
-__device__ inline double wave_sum_f64(double v) {
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-  return v;
-}
-__device__ inline int64_t wave_max_i64(int64_t v) {
-  for (int d = 32; d >= 1; d >>= 1) {
-    const int64_t o = __shfl_xor(v, d);
-    v = o > v ? o : v;
-  }
-  return v;
+template <class T>
+__device__ __forceinline__ T wave_max(T v) {
+  return wave_all(v, [](T a, T b) { return a > b ? a : b; });
 }
 
-// One wave per result block (q -> right -> left).  Its candidates are A's
-// blocks with its left tuple, in ascending mid order (qtensor.cpp:696-722); the
-// lanes take 64 at a time and look up the B block (mid, right).  The tasks of
-// the block are written one after another from its first candidate slot, each
-// at the prefix sum of the matches before it, so the tasks, their k-tile
-// offsets and the counts come out of one pass.  The B keys are staged in LDS
-// when they fit (stage_b): the lookups are a chain of dependent loads.
-constexpr int kPlanStageB = 4096;
-__global__ void __launch_bounds__(256) k_plan_blocks(MetaView A, MetaView B, PairSpec ps, PlanSets w, int stage_b,
-                                                     const PlanHdr* hdr, BlkStat* stat, int* c_qi, GemmTask* tasks,
-                                                     int* tuples, int TK) {
-  extern __shared__ uint64_t lds_sb[];
-  const int nB = B.nblocks;
-  if (stage_b) {
-    for (int i = threadIdx.x; i < nB; i += 256) lds_sb[i] = w.sSB[i];
-    __syncthreads();
-  }
-  const int lane = threadIdx.x & 63;
-  const int b = (int)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
-  const int nQ = (int)hdr->nQ;
-  if (b >= hdr->nblocksC) return;   // the whole wave
-  // q group containing b: the last t with qbase[t] <= b
-  int t = -1;
-  for (int i = 0; i < nQ; i += 64)
-    t += __popcll(__ballot(i + lane < nQ && w.qbase[i + lane] <= b));
-  const int local = (int)(b - w.qbase[t]);
-  const int l0 = w.qL0[t], nL = w.qL1[t] - l0;
-  const int ri = local / nL, l = l0 + local % nL, r = w.qR0[t] + ri;
-  const int sa0 = w.lsa0[l], cnt = w.lcnt[l];
-  const int64_t t0 = w.qcand[t] + (int64_t)ri * (w.lpre[l0 + nL] - w.lpre[l0]) + (w.lpre[l] - w.lpre[l0]);
-  const uint32_t right = (uint32_t)w.uR[r];
-  const int rep = w.rrep[r];
-  unsigned freeA = 0, freeB = 0;   // uniform
-  for (int j = 0; j < ps.nfa; j++) freeA |= 1u << ps.fa[j];
-  for (int j = 0; j < ps.nfb; j++) freeB |= 1u << ps.fb[j];
-  const int rankC = ps.nfa + ps.nfb;
-  int64_t N = 1;
-  {
-    int k = ps.nfa;
+// What the scan and the tile choice need of the result blocks, one workgroup: packed
+// offsets and the block table, on the device and in pinned host memory (hcb, when
+// the table is read back that way), the result's index table, and the totals.  Writes
+// to host memory come last: a barrier would wait for them.
+struct ScanLds {
+  int64_t sums[kPlanThreads / 64];
+  PlanHdr H;
+  int M[kPlanThreads], N[kPlanThreads], kt[kPlanThreads];   // of the first chunk of blocks
+};
+struct ScanOut {
+  int64_t* c_off;
+  int* c_idx;
+  CBlock *cblk, *hcb;
+  PlanHdr* host;
+  const int* seg[MAXR];   // the result's index table: pieces of the operands' ones
+  int len[MAXR];          // (ints)
+};
+__device__ __forceinline__ void plan_scan(ScanLds& L, const BlkStat* stat, int TK, const ScanOut& out, int64_t nQ, int n,
+                                          int64_t ncand) {
+  PlanHdr& H = L.H;
+  {   // the index table, its loads before its stores
+    int v[MAXR], *to = out.c_idx;
 #pragma unroll
-    for (int j = 0; j < MAXR; j++)
-      if ((freeB >> j) & 1) {
-        const int s = B.qi[(size_t)rep * B.rank + j];
-        N *= B.idx[3 * (B.idx_off[j] + s) + 2];
-        if (lane == 0) c_qi[(size_t)b * rankC + k] = s;
-        k++;
-      }
-  }
-  int64_t M = 1;
-  int nt = 0, kt = 0;   // tasks and k-tiles of the block so far (uniform)
-  double fl = 0.0;
-  int votes[4] = {0, 0, 0, 0}, ktmax = 0, bad = 0;
-  int64_t opmax = 0;
-  for (int c0 = 0; c0 < cnt; c0 += 64) {
-    const int ca = c0 + lane;
-    bool valid = false;
-    GemmTask g{};
-    int64_t K = 1;
-    int ktl = 0, ablk = 0, bblk = 0;
-    if (ca < cnt) {
-      ablk = w.svSA[sa0 + ca];
-      const uint64_t akey = w.sSA[sa0 + ca];
-      const bool again = ca > 0 && w.sSA[sa0 + ca - 1] == akey;   // a repeated block counts once
-      const uint64_t key = (akey << 32) | right;                  // (mid, right)
-      unsigned dA[MAXR];
-      int qA[MAXR];
+    for (int j = 0; j < MAXR; j++) v[j] = (int)threadIdx.x < out.len[j] ? out.seg[j][threadIdx.x] : 0;
 #pragma unroll
-      for (int j = 0; j < MAXR; j++) qA[j] = j < A.rank ? A.qi[(size_t)ablk * A.rank + j] : 0;
-#pragma unroll
-      for (int j = 0; j < MAXR; j++) dA[j] = j < A.rank ? A.idx[3 * (A.idx_off[j] + qA[j]) + 2] : 1;
-      M = 1;
-#pragma unroll
-      for (int j = 0; j < MAXR; j++) M *= (freeA >> j) & 1 ? dA[j] : 1;
-      if (ca == 0) {
-        int k = 0;
-#pragma unroll
-        for (int j = 0; j < MAXR; j++)
-          if ((freeA >> j) & 1) c_qi[(size_t)b * rankC + k++] = qA[j];
-      }
-      const uint64_t* sb = stage_b ? lds_sb : w.sSB;
-      const int ib = lower_bound_u64(sb, nB, key);
-      if (!again && ib < nB && sb[ib] == key) {
-        valid = true;
-        bblk = w.svSB[ib];
-        unsigned dB[MAXR];
-#pragma unroll
-        for (int j = 0; j < MAXR; j++)
-          dB[j] = j < B.rank ? B.idx[3 * (B.idx_off[j] + B.qi[(size_t)bblk * B.rank + j]) + 2] : 1;
-        g.a_off = A.off[ablk];
-        g.b_off = B.off[bblk];
-        Fold fm, fn;
-        unsigned sA = 1, sB = 1;   // strides of the stored (unpermuted) blocks
-#pragma unroll
-        for (int j = 0; j < MAXR; j++) {
-          if ((freeA >> j) & 1) fm.add(dA[j], sA);
-          if ((freeB >> j) & 1) fn.add(dB[j], sB);
-          sA *= dA[j];
-          sB *= dB[j];
-        }
-        fm.close();
-        fn.close();
-        g.em0 = fm.e0; g.sam0 = fm.s0; g.sam1 = fm.s1;
-        g.en0 = fn.e0; g.sbn0 = fn.s0; g.sbn1 = fn.s1;
-        // the contraction order forwards, and reversed: taken when it folds
-        // better, or when it puts the longer component first (the GEMM walks k
-        // in chunks of the first component, so a short first component wastes
-        // chunk slots)
-        FoldK fk, fr;
-        for (int p = 0; p < ps.np; p++) {
-          const int z = ps.np - 1 - p;
-          const unsigned ext = ext_of(dB, ps.pb[p]);
-          K *= ext;
-          fk.add(ext, stride_of(dA, ps.pa[p]), stride_of(dB, ps.pb[p]));
-          fr.add(ext_of(dB, ps.pb[z]), stride_of(dA, ps.pa[z]), stride_of(dB, ps.pb[z]));
-        }
-        fk.close();
-        fr.close();
-        const bool rev = (fk.n > 2 && fr.n <= 2) || (fk.n == 2 && fr.n == 2 && fr.e0 > fk.e0);
-        g.ek0 = rev ? fr.e0 : fk.e0;
-        g.sak0 = rev ? fr.a0 : fk.a0;
-        g.sak1 = rev ? fr.a1 : fk.a1;
-        g.sbk0 = rev ? fr.b0 : fk.b0;
-        g.sbk1 = rev ? fr.b1 : fk.b1;
-        g.K = (int)K;
-        g.nk1 = (int)(K / g.ek0);
-        if (fm.n > 2 || fn.n > 2 || (rev ? fr.n : fk.n) > 2) bad = 1;
-        ktl = g.nk1 * ((g.ek0 + TK - 1) / TK);   // K walk in TK-wide chunks of the first k component (gemm.hip)
-        votes[0] += g.sam0 == 1 || M == 1;
-        votes[1] += g.sak0 == 1 || K == 1;
-        votes[2] += g.sbk0 == 1 || K == 1;
-        votes[3] += g.sbn0 == 1 || N == 1;
-        ktmax = max(ktmax, (int)K);
-        const int64_t oa = M * K, ob = K * N;
-        opmax = oa > opmax ? oa : opmax;
-        opmax = ob > opmax ? ob : opmax;
-        fl += 2.0 * (double)M * (double)N * (double)K;
-      }
+    for (int j = 0; j < MAXR; j++) {
+      if ((int)threadIdx.x < out.len[j]) to[threadIdx.x] = v[j];
+      for (int e = threadIdx.x + blockDim.x; e < out.len[j]; e += blockDim.x) to[e] = out.seg[j][e];
+      to += out.len[j];
     }
-    // position and k-tile offset: exclusive prefix sums over the lanes
-    const uint64_t vm = __ballot(valid);
-    const int pos = __popcll(vm & ((1ull << lane) - 1ull));
-    int incl = ktl;
-    for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(incl, d);
-      if (lane >= d) incl += y;
-    }
-    if (valid) {
-      g.kt0 = kt + incl - ktl;
-      tasks[t0 + nt + pos] = g;
-      int* tu = tuples + 6 * (t0 + nt + pos);
-      tu[0] = b; tu[1] = ablk; tu[2] = bblk; tu[3] = (int)M; tu[4] = (int)N; tu[5] = (int)K;
-    }
-    nt += __popcll(vm);
-    kt += __shfl(incl, 63);
   }
-  fl = wave_sum_f64(fl);
-  for (int v = 0; v < 4; v++) votes[v] = wave_sum_i32(votes[v]);
-  for (int d = 32; d >= 1; d >>= 1) {
-    ktmax = max(ktmax, __shfl_xor(ktmax, d));
-    bad = max(bad, __shfl_xor(bad, d));
-  }
-  opmax = wave_max_i64(opmax);
-  if (lane == 0)   // lane 0 holds the block's first candidate, so its M
-    stat[b] = BlkStat{t0, opmax, fl, (int)M, (int)N, nt, kt, ktmax, bad, {votes[0], votes[1], votes[2], votes[3]}};
-}
-
-// ---- scan over the result blocks (one workgroup) --------------------------
-// Packed offsets and the block table, on the device and in pinned host memory
-// (hcb, when the table is read back that way), the result's index table, and
-// the totals.  The per-shape totals of the tile choice are a wave's each.
-__global__ void __launch_bounds__(kPlanThreads) k_plan_scan(MetaView A, MetaView B, PairSpec ps, const BlkStat* stat,
-                                                            int TK, int64_t* c_off, int* c_idx, CBlock* cblk,
-                                                            CBlock* hcb, PlanHdr* hdr, PlanHdr* host) {
-  __shared__ int64_t lds[kPlanThreads / 64];
-  __shared__ PlanHdr H;
-  const int n = (int)hdr->nblocksC, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
   for (int k = tid; k < (int)(sizeof(PlanHdr) / 8); k += blockDim.x) ((int64_t*)&H)[k] = 0;
   __syncthreads();
   if (tid == 0) {
-    H.nQ = hdr->nQ;
+    H.nQ = nQ;
     H.nblocksC = n;
-    H.ncand = hdr->ncand;
+    H.ncand = ncand;
   }
   int64_t total = 0, nt = 0, opmax = 0;
-  int vote[4] = {0, 0, 0, 0}, nkt = 0, nmax = 0, ktmax = 0, bad = 0;
+  int64_t vote[4] = {0, 0, 0, 0};
+  int nkt = 0, nmax = 0, ktmax = 0, bad = 0;
   double fl = 0.0;
+  CBlock first{};   // of the first chunk, for the host (all of it up to a block a thread)
   for (int base = 0; base < n; base += blockDim.x) {
     const int i = base + tid;
     BlkStat s{};
     if (i < n) s = stat[i];
     int64_t tot;
-    const int64_t off = total + block_prefix((int64_t)s.M * s.N, lds, &tot);
+    const int64_t off = total + block_prefix((int64_t)s.M * s.N, L.sums, &tot);
     if (i < n) {
       const CBlock cb{off, s.M, s.N, (int)s.t0, (int)(s.t0 + s.nt), s.nkt, 0};
-      c_off[i] = off;
-      cblk[i] = cb;
-      if (hcb) hcb[i] = cb;
+      out.c_off[i] = off;
+      out.cblk[i] = cb;
+      if (base == 0) first = cb;
+      else if (out.hcb) out.hcb[i] = cb;
       nt += s.nt;
       fl += s.flops;
       nkt = max(nkt, s.nkt);
@@ -607,20 +682,24 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_scan(MetaView A, MetaView
       bad |= s.bad;
       for (int v = 0; v < 4; v++) vote[v] += s.votes[v];
     }
+    if (base == 0) {
+      L.M[tid] = s.M;
+      L.N[tid] = s.N;
+      L.kt[tid] = s.nkt;
+    }
     total += tot;
   }
-  // the workgroup's totals: a wave's by shuffles, the waves' by LDS atomics
+  __syncthreads();
+  // the workgroup's totals: a wave's by lane exchanges, the waves' by LDS atomics
   // (integers and maxima; the FLOP count is a sum of whole numbers)
-  nt = wave_sum_i64(nt);
-  fl = wave_sum_f64(fl);
-  opmax = wave_max_i64(opmax);
-  for (int v = 0; v < 4; v++) vote[v] = wave_sum_i32(vote[v]);
-  for (int d = 32; d >= 1; d >>= 1) {
-    nkt = max(nkt, __shfl_xor(nkt, d));
-    nmax = max(nmax, __shfl_xor(nmax, d));
-    ktmax = max(ktmax, __shfl_xor(ktmax, d));
-    bad |= __shfl_xor(bad, d);
-  }
+  nt = wave_sum(nt);
+  fl = wave_sum(fl);
+  opmax = wave_max(opmax);
+  for (int v = 0; v < 4; v++) vote[v] = wave_sum(vote[v]);
+  nkt = wave_max(nkt);
+  nmax = wave_max(nmax);
+  ktmax = wave_max(ktmax);
+  bad = wave_max(bad);
   typedef unsigned long long u64;
   if (lane == 0) {
     atomicAdd((u64*)&H.ntasks, (u64)nt);
@@ -637,34 +716,210 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_scan(MetaView A, MetaView
     const int TM = cfg_tm(c), TN = cfg_tn(c);
     int64_t tiles = 0;
     double padded = 0.0;
-    for (int i = lane; i < n; i += 64) {
-      const int tm = (stat[i].M + TM - 1) / TM, tn = (stat[i].N + TN - 1) / TN;
+    auto add = [&](int M, int N, int kt) {
+      const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
       tiles += (int64_t)tm * tn;
-      padded += (double)(tm * TM) * (double)(tn * TN) * ((double)stat[i].nkt * TK);
-    }
-    tiles = wave_sum_i64(tiles);
-    padded = wave_sum_f64(padded);
+      padded += (double)(tm * TM) * (double)(tn * TN) * ((double)kt * TK);
+    };
+    for (int i = lane; i < min(n, (int)blockDim.x); i += 64) add(L.M[i], L.N[i], L.kt[i]);
+    for (int i = blockDim.x + lane; i < n; i += 64) add(stat[i].M, stat[i].N, stat[i].nkt);
+    tiles = wave_sum(tiles);
+    padded = wave_sum(padded);
     if (lane == 0) {
       H.tiles[c] = tiles;
       H.padded[c] = padded;
     }
   }
-  // the result's sectors: A's free indices, then B's
-  {
-    int o = 0;
-    for (int j = 0; j < ps.nfa + ps.nfb; j++) {
-      const MetaView& S = j < ps.nfa ? A : B;
-      const int p = j < ps.nfa ? ps.fa[j] : ps.fb[j - ps.nfa], len = 3 * S.nsec[p];
-      for (int e = tid; e < len; e += blockDim.x) c_idx[o + e] = S.idx[3 * S.idx_off[p] + e];
-      o += len;
-    }
-  }
   if (tid == 0) {
-    c_off[n] = total;
+    out.c_off[n] = total;
     H.totalC = total;
   }
   __syncthreads();
-  for (int k = tid; k < (int)(sizeof(PlanHdr) / 8); k += blockDim.x) ((int64_t*)host)[k] = ((const int64_t*)&H)[k];
+  for (int k = tid; k < (int)(sizeof(PlanHdr) / 8); k += blockDim.x) ((int64_t*)out.host)[k] = ((const int64_t*)&H)[k];
+  if (out.hcb && tid < n) out.hcb[tid] = first;
+}
+
+// One wave per result block (q -> right -> left), the workgroups striding over
+// them.  A block's candidates are A's blocks with its left tuple, in ascending mid
+// order (qtensor.cpp:696-722); the lanes take 64 at a time and look up the B block
+// (mid, right).  The tasks of the block are written one after another from its
+// first candidate slot, each at the prefix sum of the matches before it, so the
+// tasks, their k-tile offsets and the counts come out of one pass.  The B keys are
+// staged in LDS when they fit (stage_b): the lookups are a chain of dependent
+// loads.  What bounds it is that chain: four loads that miss (q group, tuple, blocks of A
+// and of B), 20000 cycles with the launch, the records written, 15000 for the scan.  The
+// workgroup that finishes last goes on with the scan, for `fuse` blocks or fewer (16.9 us at
+// 170 blocks for both; 15.8 and 9.1 as two kernels, and the gap between them); a
+// longer list goes to k_plan_scan's 1024 threads.
+constexpr int kPlanStageB = 4096;
+constexpr int kPlanGrid = 512;      // most workgroups of k_plan_blocks
+constexpr int64_t kPlanFuse = 2048;
+__global__ void __launch_bounds__(256) k_plan_blocks(OperandSpec A, OperandSpec B, PlanSets w, int stage_b,
+                                                     PlanHdr* hdr, BlkStat* stat, int* c_qi, GemmTask* tasks,
+                                                     int* tuples, int TK, int64_t fuse, ScanOut out) {
+  extern __shared__ uint64_t lds_sb[];
+  __shared__ ScanLds L;
+  __shared__ bool last;
+  const int nB = B.nblocks, lane = threadIdx.x & 63;
+  const int nQ = (int)hdr->nQ;
+  const int64_t nblk = hdr->nblocksC;
+  const int groups = (int)max((int64_t)1, min((nblk + 3) / 4, (int64_t)gridDim.x));   // workgroups with work
+  if ((int)blockIdx.x >= groups) return;
+  if (stage_b) {
+    for (int i = threadIdx.x; i < nB; i += 256) lds_sb[i] = w.sSB[i];
+    __syncthreads();
+  }
+  const int rankC = A.nf + B.nf, np = A.np;
+  // lane k: the result's index k as an index of A or B
+  int from = 0;
+  {
+    int k = 0;
+#pragma unroll
+    for (int j = 0; j < MAXR; j++)
+      if ((A.free >> j) & 1) from = lane == k++ ? j : from;
+#pragma unroll
+    for (int j = 0; j < MAXR; j++)
+      if ((B.free >> j) & 1) from = lane == k++ ? j : from;
+  }
+  const int wave0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  for (int64_t bb = wave0; bb < nblk; bb += 4 * (int64_t)groups) {
+    const int b = (int)bb;
+    // q group containing b: the last with base <= b
+    PlanQ q{};
+    for (int i = 0; i < nQ; i += 64) {
+      PlanQ mine{};
+      if (i + lane < nQ) mine = w.Q[i + lane];
+      const uint64_t m = __ballot(i + lane < nQ && mine.base <= b);
+      if (!m) break;
+      const int t = __popcll(m) - 1;
+      q.base = (int64_t)__builtin_amdgcn_readlane((int)mine.base, t);   // at most b
+      q.cand = (int64_t)(unsigned)__builtin_amdgcn_readlane((int)mine.cand, t) |
+               (int64_t)__builtin_amdgcn_readlane((int)(mine.cand >> 32), t) << 32;
+      q.l0 = __builtin_amdgcn_readlane(mine.l0, t);
+      q.nL = __builtin_amdgcn_readlane(mine.nL, t);
+      q.r0 = __builtin_amdgcn_readlane(mine.r0, t);
+      q.lpre = __builtin_amdgcn_readlane(mine.lpre, t);
+      q.wid = __builtin_amdgcn_readlane(mine.wid, t);
+      if (t < 63) break;
+    }
+    const int local = (int)(b - q.base), ri = local / q.nL;
+    const PlanL l = w.L[q.l0 + local % q.nL];
+    const PlanR r = w.R[q.r0 + ri];
+    const int64_t t0 = q.cand + (int64_t)ri * q.wid + (l.lpre - q.lpre);
+    const int sa0 = l.sa0, cnt = l.cnt;
+    const uint32_t right = r.right;
+    const int64_t N = r.N;
+    int64_t M = 1;
+    int ablk0 = 0;        // lane 0: the first candidate's block of A
+    int nt = 0, kt = 0;   // tasks and k-tiles of the block so far (uniform)
+    double fl = 0.0;
+    int votes[4] = {0, 0, 0, 0}, ktmax = 0, bad = 0;
+    int64_t opmax = 0;
+    for (int c0 = 0; c0 < cnt; c0 += 64) {
+      const int ca = c0 + lane;
+      bool valid = false;
+      GemmTask g{};
+      int64_t K = 1;
+      int ktl = 0, ablk = 0, bblk = 0;
+      if (ca < cnt) {
+        const PlanRec a = w.SA[sa0 + ca];
+        const uint64_t akey = a.key;
+        const bool again = ca > 0 && w.SA[sa0 + ca - 1].key == akey;   // a repeated block counts once
+        const uint64_t key = (akey << 32) | right;                     // (mid, right)
+        ablk = a.id;
+        if (c0 == 0) ablk0 = ablk;
+        M = a.ext;
+        const uint64_t* sb = stage_b ? lds_sb : w.sSB;
+        const int ib = lower_bound_u64(sb, nB, key);
+        if (!again && ib < nB && sb[ib] == key) {
+          valid = true;
+          const PlanRec o = w.SB[ib];
+          bblk = o.id;
+          g.a_off = a.off;
+          g.b_off = o.off;
+          g.em0 = a.e0; g.sam0 = a.s0; g.sam1 = a.s1;
+          g.en0 = o.e0; g.sbn0 = o.s0; g.sbn1 = o.s1;
+          // the contraction order forwards, and reversed: taken when it folds
+          // better, or when it puts the longer component first (the GEMM walks k
+          // in chunks of the first component, so a short first component wastes
+          // chunk slots)
+          FoldK fk, fr;
+#pragma unroll
+          for (int p = 0; p < MAXR; p++)
+            if (p < np) {
+              K *= o.dk[p];
+              fk.add(o.dk[p], a.sk[p], o.sk[p]);
+            }
+#pragma unroll
+          for (int p = MAXR - 1; p >= 0; p--)
+            if (p < np) fr.add(o.dk[p], a.sk[p], o.sk[p]);
+          fk.close();
+          fr.close();
+          const bool rev = (fk.n > 2 && fr.n <= 2) || (fk.n == 2 && fr.n == 2 && fr.e0 > fk.e0);
+          g.ek0 = rev ? fr.e0 : fk.e0;
+          g.sak0 = rev ? fr.a0 : fk.a0;
+          g.sak1 = rev ? fr.a1 : fk.a1;
+          g.sbk0 = rev ? fr.b0 : fk.b0;
+          g.sbk1 = rev ? fr.b1 : fk.b1;
+          g.K = (int)K;
+          g.nk1 = (int)(K / g.ek0);
+          if (a.n > 2 || o.n > 2 || (rev ? fr.n : fk.n) > 2) bad = 1;
+          ktl = g.nk1 * ((g.ek0 + TK - 1) / TK);   // K walk in TK-wide chunks of the first k component (gemm.hip)
+          votes[0] += g.sam0 == 1 || M == 1;
+          votes[1] += g.sak0 == 1 || K == 1;
+          votes[2] += g.sbk0 == 1 || K == 1;
+          votes[3] += g.sbn0 == 1 || N == 1;
+          ktmax = max(ktmax, (int)K);
+          const int64_t oa = M * K, ob = K * N;
+          opmax = oa > opmax ? oa : opmax;
+          opmax = ob > opmax ? ob : opmax;
+          fl += 2.0 * (double)M * (double)N * (double)K;
+        }
+      }
+      // position and k-tile offset: exclusive prefix sums over the lanes
+      const uint64_t vm = __ballot(valid);
+      const int pos = __popcll(vm & ((1ull << lane) - 1ull));
+      int incl = ktl;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(incl, d);
+        if (lane >= d) incl += y;
+      }
+      if (valid) {
+        g.kt0 = kt + incl - ktl;
+        tasks[t0 + nt + pos] = g;
+        int* tu = tuples + 6 * (t0 + nt + pos);
+        tu[0] = b; tu[1] = ablk; tu[2] = bblk; tu[3] = (int)M; tu[4] = (int)N; tu[5] = (int)K;
+      }
+      nt += __popcll(vm);
+      kt += __shfl(incl, 63);
+    }
+    // the block's tuple (loads that nothing waits for)
+    if (lane < rankC) {
+      const int ab = __builtin_amdgcn_readfirstlane(ablk0);
+      c_qi[(size_t)b * rankC + lane] =
+          lane < A.nf ? A.qi[(size_t)ab * A.rank + from] : B.qi[(size_t)r.rep * B.rank + from];
+    }
+    fl = wave_sum(fl);
+    for (int v = 0; v < 4; v++) votes[v] = wave_sum(votes[v]);
+    ktmax = wave_max(ktmax);
+    bad = wave_max(bad);
+    opmax = wave_max(opmax);
+    if (lane == 0)   // lane 0 holds the block's first candidate, so its M
+      stat[b] = BlkStat{t0, opmax, fl, (int)M, (int)N, nt, kt, ktmax, bad, {votes[0], votes[1], votes[2], votes[3]}};
+  }
+  if (nblk > fuse) return;   // k_plan_scan follows
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(&hdr->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)groups - 1;
+  __syncthreads();
+  if (last)
+    plan_scan(L, stat, TK, out, nQ, (int)nblk, hdr->ncand);
+}
+
+__global__ void __launch_bounds__(kPlanThreads) k_plan_scan(const BlkStat* stat, int TK, const PlanHdr* hdr,
+                                                            ScanOut out) {
+  __shared__ ScanLds L;
+  plan_scan(L, stat, TK, out, hdr->nQ, (int)hdr->nblocksC, hdr->ncand);
 }
 
 }  // namespace ttg
@@ -894,6 +1149,34 @@ static PlanHost* plan_host() {
   return h;
 }
 
+// A's QNs count Inward + and Outward - (qtensor.cpp:617-621), B's the other way
+// round (:629-633): `inward` is the sign of an Inward index
+static OperandSpec operand_spec(const TMeta& m, int nf, const int* f, int np, const int* pair, int inward) {
+  OperandSpec o{};
+  o.idx = m.d_idx;
+  o.qi = m.d_qi;
+  o.off = m.d_off;
+  o.nblocks = m.nblocks;
+  o.rank = m.rank;
+  o.nf = nf;
+  o.np = np;
+  for (int j = 0; j < m.rank; j++) o.start[j] = m.idx_off[j];
+  unsigned w = 1;
+  for (int k = nf - 1; k >= 0; k--) {   // the first index is the most significant
+    o.free |= 1u << f[k];
+    o.sign[f[k]] = m.arrow[f[k]] == 0 ? inward : -inward;
+    o.wf[f[k]] = w;
+    w *= (unsigned)m.nsec[f[k]];
+  }
+  w = 1;
+  for (int k = np - 1; k >= 0; k--) {
+    o.pair[k] = pair[k];
+    o.wm[pair[k]] = w;
+    w *= (unsigned)m.nsec[pair[k]];
+  }
+  return o;
+}
+
 int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const int* pb, int prec,
                int force_cfg, ttg_plan* out, bool defer_tiles) {
   PhaseTimer _phase("plan_build");
@@ -934,14 +1217,17 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
   PlanSets w{};
   const int nmax = std::max(1, std::max(nA, nB));
   const bool small = nmax <= kPlanSmall;
-  for (uint64_t** k : {&w.sUL, &w.sSA, &w.sUR, &w.sSB, &w.uL, &w.uR}) *k = sc.get<uint64_t>(nmax);
-  for (int** v : {&w.svSA, &w.svUR, &w.svSB, &w.lsa0, &w.lcnt, &w.rrep, &w.qL0, &w.qL1, &w.qR0, &w.qR1})
-    *v = sc.get<int>(nmax);
-  w.lpre = sc.get<int>(nmax + 1);
-  w.qbase = sc.get<int64_t>(nmax + 1);
-  w.qcand = sc.get<int64_t>(nmax + 1);
-  if (!small)
-    for (uint64_t** k : {&w.kUL, &w.kSA, &w.kUR, &w.kSB}) *k = sc.get<uint64_t>(nmax);
+  w.sSB = sc.get<uint64_t>(nmax);
+  w.SA = sc.get<PlanRec>(nmax);
+  w.SB = sc.get<PlanRec>(nmax);
+  w.L = sc.get<PlanL>(nmax + 1);
+  w.R = sc.get<PlanR>(nmax);
+  w.Q = sc.get<PlanQ>(nmax);
+  if (!small) {
+    for (uint64_t** k : {&w.kUL, &w.kSA, &w.kUR, &w.kSB, &w.sUL, &w.sSA, &w.sUR, &w.uL, &w.uR}) *k = sc.get<uint64_t>(nmax);
+    for (int** v : {&w.svSA, &w.svUR, &w.svSB, &w.qL0}) *v = sc.get<int>(nmax);
+  }
+  const OperandSpec va = operand_spec(*A, ps.nfa, ps.fa, np, ps.pa, 1), vb = operand_spec(*B, ps.nfb, ps.fb, np, ps.pb, -1);
   PlanHdr* d_hdr = sc.get<PlanHdr>(1);
   TTG_TRY(sc.ok("plan"));
   PlanHost* host = plan_host();
@@ -949,24 +1235,25 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
   // One host wait when every (A, B) block pair could be a result block or a
   // task without much memory: the arrays take that size.  Otherwise the counts
   // are read back first.
-  constexpr int64_t kPlanPairs = 4096;
+  constexpr int64_t kPlanPairs = 8192;
   const bool one_wait = (int64_t)nA * nB <= kPlanPairs;
   int64_t nbcap = std::max<int64_t>(1, (int64_t)nA * nB), ncap = nbcap;
 
   if (small) {
-    int P = 2;
-    while (P < nmax) P *= 2;
-    hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(std::min(kPlanThreads, std::max(256, P))), 0, s, A->view(), B->view(),
-                       ps, P, w, d_hdr, &host->groups);
+    // a thread per block, and a wave per run to sort
+    const int waves = std::min(kPlanThreads / 64, 4 * ((nmax + 63) / 64));
+    hipLaunchKernelGGL(k_plan_small, dim3(1), dim3(64 * waves), 0, s, va, vb, w, d_hdr,
+                       one_wait ? nullptr : &host->groups);
   } else {
-    hipLaunchKernelGGL(k_plan_keys, dim3((nmax + 255) / 256), dim3(256), 0, s, A->view(), B->view(), ps, w);
+    hipLaunchKernelGGL(k_plan_keys, dim3((nmax + 255) / 256), dim3(256), 0, s, va, vb, w);
     SortJobs jobs;
     jobs.j[0] = {w.kUL, w.sUL, nullptr, nA};
     jobs.j[1] = {w.kSA, w.sSA, w.svSA, nA};
     jobs.j[2] = {w.kUR, w.sUR, w.svUR, nB};
     jobs.j[3] = {w.kSB, w.sSB, w.svSB, nB};
     hipLaunchKernelGGL(k_rank_sort, dim3((nmax + 255) / 256, 4), dim3(256), 0, s, jobs);
-    hipLaunchKernelGGL(k_plan_groups, dim3(1), dim3(kPlanThreads), 0, s, nA, nB, w, d_hdr, &host->groups);
+    hipLaunchKernelGGL(k_plan_groups, dim3(1), dim3(kPlanThreads), 0, s, vb, nA, nB, w, d_hdr, &host->groups);
+    hipLaunchKernelGGL(k_plan_recs, dim3((nmax + 255) / 256), dim3(256), 0, s, va, vb, w);
   }
   if (!one_wait) {
     TTG_HIP(hipStreamSynchronize(s));
@@ -995,11 +1282,21 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
     return 1;
   }
   const int stage_b = nB <= kPlanStageB;
-  hipLaunchKernelGGL(k_plan_blocks, dim3((unsigned)((nbcap + 3) / 4)), dim3(256), stage_b ? sizeof(uint64_t) * nB : 0, s,
-                     A->view(), B->view(), ps, w, stage_b, d_hdr, stat, C->d_qi, p->d_tasks, p->d_tuples, tk_of(prec));
   const bool hcb_pinned = nbcap <= kPlanHostBlocks;
-  hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(nbcap <= 256 ? 256 : kPlanThreads), 0, s, A->view(), B->view(), ps, stat,
-                     tk_of(prec), C->d_off, C->d_idx, p->d_cblk, hcb_pinned ? host->cb : nullptr, d_hdr, &host->scan);
+  ScanOut so{C->d_off, C->d_idx, p->d_cblk, hcb_pinned ? host->cb : nullptr, &host->scan, {}, {}};
+  for (int j = 0; j < ps.nfa + ps.nfb; j++) {
+    const TMeta& m = j < ps.nfa ? *A : *B;
+    const int k = j < ps.nfa ? ps.fa[j] : ps.fb[j - ps.nfa];
+    so.seg[j] = m.d_idx + 3 * m.idx_off[k];
+    so.len[j] = 3 * m.nsec[k];
+  }
+  // the scan by the last workgroup, unless a table of this size wants more threads
+  const bool fused = nbcap <= kPlanFuse || one_wait;
+  hipLaunchKernelGGL(k_plan_blocks, dim3((unsigned)std::min<int64_t>((nbcap + 3) / 4, kPlanGrid)), dim3(256),
+                     stage_b ? sizeof(uint64_t) * nB : 0, s, va, vb, w, stage_b, d_hdr, stat, C->d_qi,
+                     p->d_tasks, p->d_tuples, tk_of(prec), fused ? nbcap : 0, so);
+  if (!fused)
+    hipLaunchKernelGGL(k_plan_scan, dim3(1), dim3(kPlanThreads), 0, s, stat, tk_of(prec), d_hdr, so);
   TTG_HIP(hipGetLastError());
   TTG_HIP(hipStreamSynchronize(s));
   const PlanHdr* h_hdr = &host->scan;

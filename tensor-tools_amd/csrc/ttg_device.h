@@ -6,6 +6,35 @@ namespace ttg {
 
 void fill_f64(double* d, size_t n, double v);
 
+// the value of lane l ^ X (X = 1, 2, 4, 8, 16, 32), on the vector ALU
+template <int X>
+__device__ __forceinline__ int lane_xor(int v) {
+  if constexpr (X == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);        // quad_perm 1,0,3,2
+  else if constexpr (X == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true);   // quad_perm 2,3,0,1
+  else if constexpr (X == 4)   // row_half_mirror (^ 7), quad_perm 3,2,1,0 (^ 3)
+    return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+  else if constexpr (X == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true);   // row_ror:8
+  else if constexpr (X == 16) {   // rows of 16: {0, 0, 2, 2} and {1, 1, 3, 3}
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (threadIdx.x & 16) ? r[0] : r[1];
+  } else {   // halves: {0, 0} and {1, 1}
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (threadIdx.x & 32) ? r[0] : r[1];
+  }
+}
+template <int X>
+__device__ __forceinline__ int64_t lane_xor(int64_t v) {
+  return (int64_t)(unsigned)lane_xor<X>((int)v) | (int64_t)lane_xor<X>((int)(v >> 32)) << 32;
+}
+template <int X>
+__device__ __forceinline__ double lane_xor(double v) {
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  i2 w = __builtin_bit_cast(i2, v);
+  w[0] = lane_xor<X>(w[0]);
+  w[1] = lane_xor<X>(w[1]);
+  return __builtin_bit_cast(double, w);
+}
+
 // Sum over a workgroup of NT threads (NT a multiple of 64).  lds >= NT/64.
 template <int NT>
 __device__ inline double block_sum(double v, double* lds) {

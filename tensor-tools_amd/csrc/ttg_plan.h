@@ -81,6 +81,7 @@ struct PlanHdr {
   int64_t opmax;                 // largest operand block (elements) of any task
   int64_t err;
   int64_t ncand;                 // (result block, A block) candidates: an upper bound of ntasks
+  unsigned done, pad;            // workgroups of the block pass that have finished
 };
 
 }  // namespace ttg
