@@ -610,13 +610,15 @@ __device__ __forceinline__ void skinny_rows(const Tile& tl, const CBlock& cb, co
 
 template <typename T, typename OutT>
 __global__ void __launch_bounds__(kThreads)
-k_skinny(const Tile* __restrict__ tiles, const CBlock* __restrict__ cblk,
+k_skinny(const Tile* __restrict__ tiles, int ntiles, int runs, const CBlock* __restrict__ cblk,
          const GemmTask* __restrict__ tasks, const T* __restrict__ A, const T* __restrict__ B,
          OutT* __restrict__ C) {
   static_assert(kSkinnyRows == kThreads, "one row per thread");
   __shared__ T Bs[kSkinnyK * kSkinnyN];
   __shared__ unsigned koff[kSkinnyK];
-  const Tile tl = tiles[blockIdx.x];
+  const int ti = runs ? xcd_item() : (int)blockIdx.x;
+  if (ti >= ntiles) return;   // the whole workgroup
+  const Tile tl = tiles[ti];
   const CBlock cb = cblk[tl.c];
   // the column count picks the accumulator width (uniform); blocks without
   // tasks are written as zeros by every form
@@ -628,8 +630,8 @@ k_skinny(const Tile* __restrict__ tiles, const CBlock* __restrict__ cblk,
 template <typename T, typename OutT>
 static void launch_skinny(const ttg_plan_s& p, const void* A, const void* B, void* C,
                           hipStream_t s) {
-  hipLaunchKernelGGL((k_skinny<T, OutT>), dim3(p.ntiles), dim3(kThreads), 0, s, p.d_tiles,
-                     p.d_cblk, p.d_tasks, (const T*)A, (const T*)B, (OutT*)C);
+  hipLaunchKernelGGL((k_skinny<T, OutT>), p.by_rows ? item_grid(p.ntiles) : dim3(p.ntiles), dim3(kThreads), 0, s,
+                     p.d_tiles, p.ntiles, p.by_rows, p.d_cblk, p.d_tasks, (const T*)A, (const T*)B, (OutT*)C);
 }
 
 // ------------------------------------------------------------------ split-K

@@ -138,37 +138,8 @@ int side_join() {
 }
 
 // ---------------------------------------------------------------- copies
-// Copies between buffers of the device and pinned host memory: one launch for
-// up to kCopyPieces of them, 16 bytes a lane (the library's buffers are aligned to
-// that; single bytes at the end and for any other address).  A
-// planning call or an SVD makes a dozen copies of a few hundred bytes, and a
-// hipMemcpyAsync is a launch too (2.9 us of the GPU, as one of these is) that
-// costs the host more: the Davidson call at m=1024 took 2281 us with 73 of them and
-// takes 1808 us with 15 launches of k_copy, a 20-site sweep at m=48 107 and 98 ms
-// (4270 and 2407).
+// Copies between buffers of the device and pinned host memory (k_copy, tensor.hip)
 namespace {
-constexpr int kCopyPieces = 16;
-struct CopyArgs {
-  char* dst[kCopyPieces];
-  const char* src[kCopyPieces];
-  size_t bytes[kCopyPieces];
-};
-
-__global__ void __launch_bounds__(256) k_copy(CopyArgs a) {
-  const int p = blockIdx.y;
-  char* __restrict__ d = a.dst[p];
-  const char* __restrict__ s = a.src[p];
-  const size_t n = a.bytes[p];
-  const size_t i0 = blockIdx.x * (size_t)256 + threadIdx.x, step = gridDim.x * (size_t)256;
-  const unsigned low = (unsigned)((size_t)d | (size_t)s);
-  size_t done = 0;
-  if ((low & 15) == 0) {
-    for (size_t i = i0; i < n / 16; i += step) ((uint4*)d)[i] = ((const uint4*)s)[i];
-    done = n & ~size_t(15);
-  }
-  for (size_t i = done + i0; i < n; i += step) d[i] = s[i];
-}
-
 // the pieces collected for one launch
 struct CopyList {
   CopyArgs a;
@@ -181,10 +152,9 @@ int copy_launch(CopyList& l) {
   for (int i = 0; i < l.n; i++) most = std::max(most, l.a.bytes[i]);
   // four 16-byte elements a thread
   const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>((most + 16383) / 16384, 4096));
-  hipLaunchKernelGGL(k_copy, dim3(g, l.n), dim3(256), 0, g_rt.stream, l.a);
+  const int n = l.n;
   l.n = 0;
-  TTG_HIP(hipGetLastError());
-  return 0;
+  return copy_pieces(l.a, g, n);
 }
 
 int copy_add(CopyList& l, void* dst, const void* src, size_t bytes) {

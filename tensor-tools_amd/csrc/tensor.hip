@@ -307,6 +307,37 @@ void fill_f64(double* d, size_t n, double v) {
   hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, stream(), d, n, v);
 }
 
+// Copies between buffers of the device and pinned host memory: one launch for
+// up to kCopyPieces of them, 16 bytes a lane (the library's buffers are aligned to
+// that; single bytes at the end and for any other address).  A
+// planning call or an SVD makes a dozen copies of a few hundred bytes, and a
+// hipMemcpyAsync is a launch too (2.9 us of the GPU, as one of these is) that
+// costs the host more: the Davidson call at m=1024 took 2281 us with 73 of them and
+// takes 1808 us with 15 launches of k_copy, a 20-site sweep at m=48 107 and 98 ms
+// (4270 and 2407).
+// (It stands here, beside kernels that every program launches: a source file's kernels
+// are loaded at the first launch of one of them, some milliseconds.)
+__global__ void __launch_bounds__(256) k_copy(CopyArgs a) {
+  const int p = blockIdx.y;
+  char* __restrict__ d = a.dst[p];
+  const char* __restrict__ s = a.src[p];
+  const size_t n = a.bytes[p];
+  const size_t i0 = blockIdx.x * (size_t)256 + threadIdx.x, step = gridDim.x * (size_t)256;
+  const unsigned low = (unsigned)((size_t)d | (size_t)s);
+  size_t done = 0;
+  if ((low & 15) == 0) {
+    for (size_t i = i0; i < n / 16; i += step) ((uint4*)d)[i] = ((const uint4*)s)[i];
+    done = n & ~size_t(15);
+  }
+  for (size_t i = done + i0; i < n; i += step) d[i] = s[i];
+}
+
+int copy_pieces(const CopyArgs& a, unsigned g, int n) {
+  hipLaunchKernelGGL(k_copy, dim3(g, n), dim3(256), 0, stream(), a);
+  TTG_HIP(hipGetLastError());
+  return 0;
+}
+
 // the same sectors and block list with every arrow flipped (qtensor::dag,
 // qtensor.cpp:1575-1581): a new structure object on the same device tables,
 // which nothing writes once a structure is complete

@@ -103,6 +103,14 @@ class UploadBatch {
  private:
   bool open_ = true;
 };
+// one launch of k_copy: n pieces, g workgroups each
+constexpr int kCopyPieces = 16;
+struct CopyArgs {
+  char* dst[kCopyPieces];
+  const char* src[kCopyPieces];
+  size_t bytes[kCopyPieces];
+};
+int copy_pieces(const CopyArgs& a, unsigned g, int n);
 // copies between device buffers on the library stream, several in one launch
 struct DevPiece {
   void* dst;

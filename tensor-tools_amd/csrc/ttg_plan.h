@@ -26,7 +26,8 @@ struct CBlock {
   int64_t c_off;
   int M, N;
   int t0, t1;
-  int nkt, pad;
+  int nkt;
+  int left;   // number of the block's left tuple: blocks that share one share rows and blocks of A
 };
 
 // One workgroup work item: rows [m0, m0+TM) x cols [n0, n0+TN) of block c
@@ -97,6 +98,7 @@ struct ttg_plan_s {
   int cfg = ttg::TILE_64x64;
   int ntiles = 0;
   bool a_mcontig = true, b_kcontig = true;
+  bool by_rows = false;   // the vector kernel's items stand by rows (build_tiles)
   // split-BF16 operand format: packed_in, the MFMA stage reads both operands
   // as pre-split words (bf16 hi << 16 | bf16 lo, see split_word); split_out,
   // the vector-ALU stage writes its result as such words

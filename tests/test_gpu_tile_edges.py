@@ -49,3 +49,31 @@ def test_edges(make, prec, cfg, monkeypatch):
 def test_more_shapes(make, prec, cfg, monkeypatch):
     A, B = make(np.random.default_rng(11))
     run(A, B, prec, cfg, monkeypatch)
+
+
+def test_rows_of_a_large_operand():
+    """The vector kernel's items of an operand above 256 MB stand by rows, not by result
+    block: every result block against a sum over its tasks."""
+    rng = np.random.default_rng(2)
+    i = make_index(INWARD, "i", LINK, 0, sec([0, 2], [4000, 3700]))
+    j = make_index(INWARD, "j", LINK, 0, sec([0, 2], [1511, 1489]))
+    k = make_index(OUTWARD, "k", LINK, 0, sec([0, 2, 4], [2, 1, 2]))
+    s = make_index(INWARD, "s", LINK, 0, sec([0, 2], [1, 2]))
+    n = make_index(OUTWARD, "n", LINK, 0, sec([0, 2, 4, 6], [2, 3, 1, 2]))
+    A, B = random_tensor([i, j, k], rng), random_tensor([k.dag(), s, n], rng)
+    assert A.data.nbytes > 256 << 20
+    dA, dB = T.DTensor.from_flat(A), T.DTensor.from_flat(B)
+    plan = T.Plan(dA, dB, [(2, 0)])
+    C = plan.new_output()
+    plan.execute(dA, dB, C)
+    got, (_, co) = C.data(), C.meta()
+    ao, bo = A.block_offsets(), B.block_offsets()
+    tasks = plan.tasks()
+    assert len({t[0] for t in tasks}) == len(co) - 1
+    for c in range(len(co) - 1):
+        want = 0.0
+        for _, a, b, M, N, K in tasks[tasks[:, 0] == c]:
+            want = want + A.data[ao[a]:ao[a + 1]].reshape(M, K, order="F") @ \
+                B.data[bo[b]:bo[b + 1]].reshape(K, N, order="F")
+        # two products of five terms' sizes at most
+        assert np.abs(got[co[c]:co[c + 1]].reshape(want.shape, order="F") - want).max() < 1e-13
