@@ -16,7 +16,9 @@
 // of 63 rounds of 32 rotations, but 49 of the 63 rounds touch one wave's
 // 16 x 16 tile (no workgroup barrier), and the rest of the matrix moves
 // through LDS 7 times per sweep instead of 63.  What bounds it is the chain of
-// a round: read the 2 x 2 block, the rotation, one cross-lane copy, write.
+// a round: the rotation, one cross-lane copy, the exchange of the 2 x 2 blocks.  A
+// 64 x 64 subproblem of the block Jacobi, with its load and eigenvalue order, took
+// 61.2 us as 63 rounds through LDS and takes 29.3.
 //
 // Lane layout of v_mfma_f64_16x16x4 (lane l: A[l%16][l/16], B[l/16][l%16],
 // result register r: D[l/16 + 4r][l%16]): a tile T held as T[l/16 + 4s][l%16]
