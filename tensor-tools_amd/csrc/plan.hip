@@ -910,6 +910,9 @@ __global__ void __launch_bounds__(256) k_plan_blocks(OperandSpec A, OperandSpec 
                         q.l0 + local % q.nL, 0};
   }
   if (nblk > fuse) return;   // k_plan_scan follows
+  // Every wave waits for its own stores: a barrier orders them within the
+  // workgroup only, and what thread 0 waits for before the counter are its own wave's
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
   __syncthreads();
   if (threadIdx.x == 0)
     last = __hip_atomic_fetch_add(&hdr->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)groups - 1;
