@@ -599,16 +599,6 @@ struct FoldK {
     cb = sb;
   }
 };
-// v combined over the lanes of a wave
-template <class T, class Op>
-__device__ __forceinline__ T wave_all(T v, Op op) {
-  v = op(v, lane_xor<1>(v));
-  v = op(v, lane_xor<2>(v));
-  v = op(v, lane_xor<4>(v));
-  v = op(v, lane_xor<8>(v));
-  v = op(v, lane_xor<16>(v));
-  return op(v, lane_xor<32>(v));
-}
 template <class T>
 __device__ __forceinline__ T wave_sum(T v) {
   return wave_all(v, [](T a, T b) { return a + b; });

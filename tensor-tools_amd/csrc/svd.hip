@@ -285,19 +285,21 @@ __device__ __forceinline__ int cholesky64(double (&x)[8], double d, bool open, i
 
 // Pivoted Cholesky of G0 (n x n): rows of R to L.r (zero beyond row r and column
 // n); returns r, and in `good` the rows with pivots above kLrCond of the largest
-// diagonal.
-__device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, int wave, int lane, int& good) {
+// diagonal.  dg: the diagonal, scaled by 2^-ex as the matrix is on its way in.
+__device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, double dg, int ex, int wave, int lane,
+                                            int& good) {
   double x[8];
 #pragma unroll
   for (int s = 0; s < 8; s++) {
     const int i = 8 * wave + s;
-    x[s] = i < n && lane < n ? 0.5 * (G0[i + (int64_t)n * lane] + G0[lane + (int64_t)n * i]) : 0.0;
+    x[s] = i < n && lane < n ? __builtin_amdgcn_ldexp(0.5 * (G0[i + (int64_t)n * lane] + G0[lane + (int64_t)n * i]), -ex)
+                             : 0.0;
   }
   for (int e = threadIdx.x; e < kJS; e += kJThreads) L.r[e] = 0.0;
   __syncthreads();
   double tol = 0.0, fair = 0.0;
   int order, g = 0;
-  const int r = cholesky64(x, lane < n ? G0[lane * (int64_t)(n + 1)] : 0.0, lane < n, n, L.r, L.row, wave, lane, order,
+  const int r = cholesky64(x, dg, lane < n, n, L.r, L.row, wave, lane, order,
                            [&](int k, double m) {
                              if (k == 0) {
                                tol = kPcTol * m;
@@ -333,9 +335,9 @@ __device__ __forceinline__ void jac_gram(JacLds& L, int n, int wave, int lane) {
 }
 
 // Eigenpairs of the matrix G0 (n x n, r = 0) or of G' (r x r, from L.r) and from
-// them those of G0.
+// them those of G0, both scaled by 2^-ex.
 template <int NPR>
-__device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, const double* G0, double* Vg, double* ev,
+__device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, const double* G0, double* Vg, double* ev,
                                               int max_sweeps, double floor_rel, int wave, int lane) {
   constexpr int W = 16 * NPR;
   const int tid = threadIdx.x;
@@ -344,7 +346,8 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, const dou
 #pragma unroll 8
     for (int e = tid; e < W * W; e += kJThreads) {
       const int i = e % W, j = e / W;
-      S[j * kJP + i] = (i < n && j < n) ? 0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]) : 0.0;
+      S[j * kJP + i] =
+          (i < n && j < n) ? __builtin_amdgcn_ldexp(0.5 * (G0[i + (int64_t)n * j] + G0[j + (int64_t)n * i]), -ex) : 0.0;
     }
   } else {
     jac_gram<NPR>(L, n, wave, lane);
@@ -372,7 +375,7 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, const dou
     if (!rotated) break;
   }
   if (r == 0) {
-    for (int i = tid; i < n; i += kJThreads) ev[i] = S[i * kJP + i];
+    for (int i = tid; i < n; i += kJThreads) ev[i] = __builtin_amdgcn_ldexp(S[i * kJP + i], ex);
     if (wave >= 4) {   // V(i, c) = V^T(c, i): consecutive lanes down a column of V
       const int i = 16 * (wave - 4) + (lane & 15);
 #pragma unroll
@@ -389,7 +392,7 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, const dou
   double* lam = L.row[0];
   if (tid < kJW) {
     lam[tid] = tid < r ? S[tid * kJP + tid] : 0.0;
-    if (tid < n) ev[tid] = lam[tid];
+    if (tid < n) ev[tid] = __builtin_amdgcn_ldexp(lam[tid], ex);
   }
   __syncthreads();
   if (wave >= 4 && wave < 4 + NPR) {
@@ -479,16 +482,19 @@ k_jacobi(const int* __restrict__ nq, const int* __restrict__ kq, int drop, const
   const double* G0 = Gin + goff[q];      // full n x n column-major
   double* Vg = Vout + goff[q];           // eigenvectors, the same layout
   double* ev = evals + eoff[q];
+  const double dg = lane < n ? G0[lane * (int64_t)(n + 1)] : 0.0;
+  // (even: R's scale is a power of two as well)
+  const int ex = __builtin_amdgcn_frexp_exp(wave_all(fabs(dg), [](double a, double b) { return fmax(a, b); })) & ~1;
   int r = 0;
   if (kq && n > 16) {
     int good;
-    r = jac_cholesky(L, n, G0, wave, lane, good);
+    r = jac_cholesky(L, n, G0, __builtin_amdgcn_ldexp(dg, -ex), ex, wave, lane, good);
     if (!drop && good < kq[q]) r = 0;
   }
   const int w = r ? r : n;
-  if (w <= 16) jacobi_sector<1>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
-  else if (w <= 32) jacobi_sector<2>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
-  else jacobi_sector<4>(L, n, r, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  if (w <= 16) jacobi_sector<1>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else if (w <= 32) jacobi_sector<2>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else jacobi_sector<4>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
 }
 
 // 4b. Sectors larger than kJacBlockMin: two-sided block Jacobi.  The padded
@@ -515,9 +521,9 @@ typedef double bj_v4d __attribute__((ext_vector_type(4)));
 struct BJSector {
   int n, N, nbk, q;                    // size, padded size, blocks, sector id
   int64_t gp, qp;                      // offsets of padded G / V and of the pair Q's
-  double dmax;                         // largest diagonal of the Gram matrix
   double floor;                        // off-diagonal size below which nothing rotates
-  int pb, pad;                         // index of the sector's first pair in the pair list
+  int pb;                              // index of the sector's first pair in the pair list
+  int ex;                              // G is held scaled by 2^-ex (its largest diagonal below 1)
 };
 
 // circle method over m = 2 npair indices: pair k of round r (a < b)
@@ -530,38 +536,34 @@ __device__ inline void circle_pair(int m, int r, int k, int& a, int& b) {
 // subproblem entry t (0..63) of pair k of round r is global index
 // (t < kBJ ? a : b) * kBJ + t % kBJ, (a, b) = circle_pair(nbk, r, k)
 
-// sec[li].dmax = max_i |G_ii| of the sector, sec[li].floor = floor_rel * dmax
-__global__ void __launch_bounds__(256) k_bjac_floor(BJSector* sec, int nsec, const int64_t* goff, const double* G,
-                                                    double floor_rel) {
+// Gp: the padded matrix scaled by a power of two (ex), Vp: identity; and
+// sec[li].floor = floor_rel max_i |G_ii|, scaled
+__global__ void __launch_bounds__(256) k_bjac_init(BJSector* sec, int nsec, const int64_t* goff, const double* G,
+                                                   double* Gp, double* Vp, double floor_rel) {
   __shared__ double red[4];
-  const int li = blockIdx.x;
+  const int li = blockIdx.y;
   if (li >= nsec) return;
-  const int q = sec[li].q, n = sec[li].n;
-  const double* g = G + goff[q];
+  const int n = sec[li].n, N = sec[li].N;
+  const int64_t gp = sec[li].gp;
+  const double* g = G + goff[sec[li].q];
   double mx = 0.0;
   for (int i = threadIdx.x; i < n; i += blockDim.x) mx = fmax(mx, fabs(g[i + (int64_t)n * i]));
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const double m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
-    sec[li].dmax = m;
-    sec[li].floor = floor_rel * m;
+  mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  const int ex = __builtin_amdgcn_frexp_exp(mx);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sec[li].floor = floor_rel * __builtin_amdgcn_ldexp(mx, -ex);
+    sec[li].ex = ex;
   }
-}
-
-__global__ void k_bjac_init(const BJSector* sec, int nsec, const int64_t* goff, const double* G,
-                            double* Gp, double* Vp) {
-  const int li = blockIdx.y;
-  if (li >= nsec) return;
-  const BJSector S = sec[li];
-  const double* g = G + goff[S.q];
-  const int64_t NN = (int64_t)S.N * S.N;
+  const int64_t NN = (int64_t)N * N;
   for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < NN;
        e += (int64_t)gridDim.x * blockDim.x) {
-    const int i = (int)(e % S.N), j = (int)(e / S.N);
-    Gp[S.gp + e] = (i < S.n && j < S.n) ? 0.5 * (g[i + (int64_t)S.n * j] + g[j + (int64_t)S.n * i]) : 0.0;
-    Vp[S.gp + e] = i == j ? 1.0 : 0.0;
+    const int i = (int)(e % N), j = (int)(e / N);
+    Gp[gp + e] = (i < n && j < n) ? __builtin_amdgcn_ldexp(0.5 * (g[i + (int64_t)n * j] + g[j + (int64_t)n * i]), -ex)
+                                  : 0.0;
+    Vp[gp + e] = i == j ? 1.0 : 0.0;
   }
 }
 
@@ -831,7 +833,7 @@ __global__ void k_bjac_finish(const BJSector* sec, int nsec, const int64_t* goff
        e += (int64_t)gridDim.x * blockDim.x) {
     const int i = (int)(e % S.n), j = (int)(e / S.n);
     Vout[goff[S.q] + e] = Vp[S.gp + i + (int64_t)S.N * j];
-    if (i == j) evals[eoff[S.q] + i] = Gp[S.gp + i + (int64_t)S.N * i];
+    if (i == j) evals[eoff[S.q] + i] = __builtin_amdgcn_ldexp(Gp[S.gp + i + (int64_t)S.N * i], S.ex);
   }
 }
 
@@ -850,7 +852,7 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
     const int q = big[li], n = nq[q];
     const int N = (n + kSub - 1) / kSub * kSub;
     const int nbk = N / kBJ, npair = nbk / 2;
-    sec[li] = BJSector{n, N, nbk, q, gp, qp, 0.0, 0.0, (int)pitems.size(), 0};
+    sec[li] = BJSector{n, N, nbk, q, gp, qp, 0.0, (int)pitems.size(), 0};
     gp += (int64_t)N * N;
     qp += (int64_t)npair * kSub * kSub;
     maxr = std::max(maxr, nbk - 1);
@@ -881,10 +883,7 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
     TTG_TRY(h2d_vec(flag, std::vector<int>(ns, 0)));
     TTG_TRY(up.flush());
   }
-  // largest diagonal per sector and the convergence floor, on the device
-  if (floor_rel > 0)
-    hipLaunchKernelGGL(k_bjac_floor, dim3(ns), dim3(256), 0, s, d_sec, ns, d_goff, G, floor_rel);
-  hipLaunchKernelGGL(k_bjac_init, dim3(64, ns), dim3(256), 0, s, d_sec, ns, d_goff, G, Gp, Vp);
+  hipLaunchKernelGGL(k_bjac_init, dim3(64, ns), dim3(256), 0, s, d_sec, ns, d_goff, G, Gp, Vp, floor_rel);
   // Outer sweeps.  The active flags move on the device (k_bjac_sweep_end),
   // so the host reads the "any sector active" word only from the sweep at
   // which the previous call of the same kind (LR-reduced or plain Gram

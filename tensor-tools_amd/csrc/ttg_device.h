@@ -35,6 +35,17 @@ __device__ __forceinline__ double lane_xor(double v) {
   return __builtin_bit_cast(double, w);
 }
 
+// v combined over the lanes of a wave
+template <class T, class Op>
+__device__ __forceinline__ T wave_all(T v, Op op) {
+  v = op(v, lane_xor<1>(v));
+  v = op(v, lane_xor<2>(v));
+  v = op(v, lane_xor<4>(v));
+  v = op(v, lane_xor<8>(v));
+  v = op(v, lane_xor<16>(v));
+  return op(v, lane_xor<32>(v));
+}
+
 // Sum over a workgroup of NT threads (NT a multiple of 64).  lds >= NT/64.
 template <int NT>
 __device__ inline double block_sum(double v, double* lds) {

@@ -89,6 +89,9 @@ __device__ __forceinline__ double jac_rsqrt(double x) {
 
 constexpr double kJacRel = 1e-12;   // an off-diagonal below this of sqrt(a_pp a_qq) is converged
 
+// (compared squared: the callers scale a matrix by a power of two until its largest
+// diagonal is about 1.  A Gram matrix has the squares of a tensor's entries, and its own
+// squares leave the range of a double when those are below 1e-80 or above 1e77)
 __device__ __forceinline__ bool jac_significant(double app, double aqq, double apq, double floor_abs) {
   return apq * apq > (kJacRel * kJacRel) * fabs(app * aqq) && fabs(apq) > floor_abs;
 }
