@@ -211,19 +211,27 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // Sectors of more than 16 rows go through a pivoted Cholesky factorisation
 // P^T G P = R^T R first (as the large ones, 4c): the iteration then runs on
 // G' = R R^T, r x r, which is nearly diagonal and holds no null space, and
-// V = R^T W Lambda^(-1/2), which one Gram-Schmidt step makes orthonormal to rounding
+// V = R^T W Lambda^(-1/2), corrected to first order for the remainder that the
+// factorisation leaves out and made orthonormal to rounding by Gram-Schmidt steps
 // (2e-15 where the rotations alone gave 2e-14).  The matrix stays in the registers of the
 // 8 waves (8 rows each), every wave keeps the remaining diagonal and finds the pivot for
 // itself, and one row a step passes through LDS.  On the sectors of an m = 100 state (up to 60
-// rows, rank-deficient) k_jacobi took 445 us and takes 89, at m = 333 531 and 258.  The route is taken
-// when the r columns are all that the selection can use: r >= kq, the values
-// kept before truncation, with no pivot among them below kLrCond of the
-// largest diagonal (the factors of a worse conditioned sector lose up to ten times
-// more than those of the plain iteration), or a cutoff above kLrCutoff, the
-// weight (of the whole tensor's) that 64 rows below kPcTol of the largest can hold.
+// rows, rank-deficient) k_jacobi took 445 us and takes 94, at m = 333 531 and 249.
+// Why the correction: the remainder's diagonal is below kPcTol = 4.5 roundings of the
+// largest, and left out it moved the vectors near a cutoff of 1e-9 more than the rounding
+// of the Gram matrix does: the factors of states of m = 40 to 200 were off by 0.80e-12
+// (of the state's norm, geometric mean over 160 states) where the plain iteration's are by
+// 0.54e-12; with it they are by 0.29e-12, and k_jacobi takes 94 us at m = 100 instead of 89.
+// The route is taken when the r columns are all that the selection can use, and all above
+// kLrFix of the largest: r >= kq, the values kept before truncation, with no pivot among
+// them below kLrCond of the largest diagonal, or a cutoff above kLrCutoff.  (A cutoff c
+// keeps a value of weight w only if what follows weighs more than c in all, so the least
+// kept value is above c / 10 unless more than ten values share the tail; what the
+// factorisation leaves out weighs 64 kPcTol at most.)
 constexpr double kJacFloor = 1e-14;   // convergence floor relative to the largest diagonal
 constexpr double kPcTol = 1e-15;      // a remaining diagonal below this of the largest ends the factorisation
-constexpr double kLrCutoff = kJW * kPcTol * 1.5;
+constexpr double kLrFix = 1e-12;      // least eigenvalue (of the largest) whose vector is corrected for the remainder
+constexpr double kLrCutoff = 10 * kLrFix;
 constexpr double kLrCond = 1e-8;
 
 // LDS of k_jacobi
@@ -240,9 +248,10 @@ struct JacLds {
 // element (8 wave + s, lane), d the remaining diagonal of index `lane`, kept by every
 // wave, `open` an index not yet taken.  Row k of R goes to r[k kJP + ..], the index of
 // step k to lane k's `order`; ends after n steps or when stop(k, pivot) says so, and
-// returns the steps.  Ties go to the lower index.  `row`: two rows of LDS.
+// returns the steps; x is then what remains of the matrix at the open indices.  Ties go
+// to the lower index.  `row`: two rows of LDS.
 template <class Stop>
-__device__ __forceinline__ int cholesky64(double (&x)[8], double d, bool open, int n, double* r, double (*row)[kJW],
+__device__ __forceinline__ int cholesky64(double (&x)[8], double d, bool& open, int n, double* r, double (*row)[kJW],
                                           int wave, int lane, int& order, Stop stop) {
   int k = 0;
   order = 0;
@@ -284,11 +293,11 @@ __device__ __forceinline__ int cholesky64(double (&x)[8], double d, bool open, i
 }
 
 // Pivoted Cholesky of G0 (n x n): rows of R to L.r (zero beyond row r and column
-// n); returns r, and in `good` the rows with pivots above kLrCond of the largest
-// diagonal.  dg: the diagonal, scaled by 2^-ex as the matrix is on its way in.
+// n); returns r, in `good` the rows with pivots above kLrCond of the largest
+// diagonal, and in x rows 8 wave .. 8 wave + 7 of the remainder G0 - R^T R.  dg: the
+// diagonal, scaled by 2^-ex as the matrix is on its way in.
 __device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, double dg, int ex, int wave, int lane,
-                                            int& good) {
-  double x[8];
+                                            int& good, double (&x)[8]) {
 #pragma unroll
   for (int s = 0; s < 8; s++) {
     const int i = 8 * wave + s;
@@ -299,7 +308,8 @@ __device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, 
   __syncthreads();
   double tol = 0.0, fair = 0.0;
   int order, g = 0;
-  const int r = cholesky64(x, dg, lane < n, n, L.r, L.row, wave, lane, order,
+  bool open = lane < n;
+  const int r = cholesky64(x, dg, open, n, L.r, L.row, wave, lane, order,
                            [&](int k, double m) {
                              if (k == 0) {
                                tol = kPcTol * m;
@@ -310,6 +320,9 @@ __device__ __forceinline__ int jac_cholesky(JacLds& L, int n, const double* G0, 
                              return false;
                            });
   good = g;
+  const uint64_t left = __ballot(open);
+#pragma unroll
+  for (int s = 0; s < 8; s++) x[s] = open && (left >> (8 * wave + s) & 1) ? x[s] : 0.0;
   return r;
 }
 
@@ -335,10 +348,11 @@ __device__ __forceinline__ void jac_gram(JacLds& L, int n, int wave, int lane) {
 }
 
 // Eigenpairs of the matrix G0 (n x n, r = 0) or of G' (r x r, from L.r) and from
-// them those of G0, both scaled by 2^-ex.
+// them those of G0, both scaled by 2^-ex.  rem: the remainder's rows (jac_cholesky).
 template <int NPR>
-__device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, const double* G0, double* Vg, double* ev,
-                                              int max_sweeps, double floor_rel, int wave, int lane) {
+__device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, const double* G0, const double (&rem)[8],
+                                              double* Vg, double* ev, int max_sweeps, double floor_rel, int wave,
+                                              int lane) {
   constexpr int W = 16 * NPR;
   const int tid = threadIdx.x;
   double* S = L.s;
@@ -389,11 +403,8 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, c
     return;
   }
   // V = R^T W Lambda^(-1/2); columns c >= r are zero, with eigenvalue zero
-  double* lam = L.row[0];
-  if (tid < kJW) {
-    lam[tid] = tid < r ? S[tid * kJP + tid] : 0.0;
-    if (tid < n) ev[tid] = __builtin_amdgcn_ldexp(lam[tid], ex);
-  }
+  double *lam = L.row[0], *out = L.row[1];
+  if (tid < kJW) out[tid] = lam[tid] = tid < r ? S[tid * kJP + tid] : 0.0;
   __syncthreads();
   if (wave >= 4 && wave < 4 + NPR) {
 #pragma unroll
@@ -422,48 +433,93 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, c
       }
     }
   }
+  auto put = [&]() {   // X = v
+#pragma unroll
+    for (int u = 0; u < kMine; u++) {
+      const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
+      if (t < NPR * nt)
+#pragma unroll
+        for (int s = 0; s < 4; s++) L.r[(16 * a + g + 4 * s) * kJP + 16 * b + j] = v[u][s];
+    }
+  };
   __syncthreads();
+  put();
+  // The remainder E that the factorisation left out moves the vectors by E X / lambda
+  // to first order, and the eigenvalues by x_c^T E x_c: half of what it adds to |x_c|^2,
+  // times lambda_c.
+  const double least = kLrFix * L.dmax;
+  const bool fix = r < n;
+  if (fix) {
+#pragma unroll
+    for (int s = 0; s < 8; s++) S[(8 * wave + s) * kJP + lane] = rem[s];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMine; u++) {
+      const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
+      if (t >= NPR * nt) continue;
+      jac_v4d y = {0.0, 0.0, 0.0, 0.0};
+      for (int k = 0; k < n; k += 4)
+        y = __builtin_amdgcn_mfma_f64_16x16x4f64(L.r[(16 * a + j) * kJP + k + g], S[(k + g) * kJP + 16 * b + j], y, 0, 0,
+                                                 0);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const double l = lam[16 * a + g + 4 * s];
+        v[u][s] += l > least ? y[s] / l : 0.0;
+      }
+    }
+    __syncthreads();
+    put();
+  }
+  __syncthreads();
+  // X is orthonormal to the rounding of R^T W, eps sqrt(lambda_1 / lambda_c), and to E / lambda:
+  // a Gram-Schmidt step in the order of the eigenvalues squares that,
+  // X <- C X, C(c, a) = -(X X^T)(c, a) for lambda_a > lambda_c, (3 - |x_c|^2) / 2 at c
+  for (int round = fix ? 3 : 1; round > 0; round--) {
+    for (int t = wave; t < NPR * (NPR + 1) / 2; t += 8) {
+      int b = 0;
+      while ((b + 1) * (b + 2) / 2 <= t) b++;
+      const int a = t - b * (b + 1) / 2;
+      jac_v4d m = {0.0, 0.0, 0.0, 0.0};
+      for (int k = 0; k < n; k += 4)
+        m = __builtin_amdgcn_mfma_f64_16x16x4f64(L.r[(16 * a + j) * kJP + k + g], L.r[(16 * b + j) * kJP + k + g], m, 0,
+                                                 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int i = 16 * a + g + 4 * s, c = 16 * b + j;
+        const double li = lam[i], lc = lam[c];
+        const bool first = li > lc || (li == lc && i < c);   // x_i is corrected before x_c
+        S[c * kJP + i] = i == c ? 1.5 - 0.5 * m[s] : first ? -m[s] : 0.0;
+        if (i != c) S[i * kJP + c] = first ? 0.0 : -m[s];
+        else if (round == 3 && lc > least) out[c] = lc * (0.5 + 0.5 * m[s]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMine; u++) {
+      const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
+      v[u] = {0.0, 0.0, 0.0, 0.0};
+      if (t >= NPR * nt) continue;
+#pragma unroll
+      for (int k = 0; k < W; k += 4)
+        v[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * a + j) * kJP + k + g], L.r[(k + g) * kJP + 16 * b + j], v[u],
+                                                    0, 0, 0);
+    }
+    if (round > 1) {
+      __syncthreads();
+      put();
+      __syncthreads();
+    }
+  }
+  if (tid < n) ev[tid] = __builtin_amdgcn_ldexp(out[tid], ex);
 #pragma unroll
   for (int u = 0; u < kMine; u++) {
     const int t = wave + 8 * u, a = t % NPR, b = t / NPR;
     if (t < NPR * nt)
 #pragma unroll
-      for (int s = 0; s < 4; s++) L.r[(16 * a + g + 4 * s) * kJP + 16 * b + j] = v[u][s];
-  }
-  __syncthreads();
-  // X is orthonormal to the rounding of R^T W, eps sqrt(lambda_1 / lambda_c): one
-  // Gram-Schmidt step in the order of the eigenvalues takes that to eps,
-  // X <- C X, C(c, a) = -(X X^T)(c, a) for lambda_a > lambda_c, (3 - |x_c|^2) / 2 at c
-  for (int t = wave; t < NPR * (NPR + 1) / 2; t += 8) {
-    int b = 0;
-    while ((b + 1) * (b + 2) / 2 <= t) b++;
-    const int a = t - b * (b + 1) / 2;
-    jac_v4d m = {0.0, 0.0, 0.0, 0.0};
-    for (int k = 0; k < n; k += 4)
-      m = __builtin_amdgcn_mfma_f64_16x16x4f64(L.r[(16 * a + j) * kJP + k + g], L.r[(16 * b + j) * kJP + k + g], m, 0, 0,
-                                               0);
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const int i = 16 * a + g + 4 * s, c = 16 * b + j;
-      const double li = lam[i], lc = lam[c];
-      const bool first = li > lc || (li == lc && i < c);   // x_i is corrected before x_c
-      S[c * kJP + i] = i == c ? 1.5 - 0.5 * m[s] : first ? -m[s] : 0.0;
-      if (i != c) S[i * kJP + c] = first ? 0.0 : -m[s];
-    }
-  }
-  __syncthreads();
-  for (int t = wave; t < NPR * nt; t += 8) {
-    const int a = t % NPR, b = t / NPR;
-    jac_v4d x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < W; k += 4)
-      x = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * a + j) * kJP + k + g], L.r[(k + g) * kJP + 16 * b + j], x, 0, 0,
-                                               0);
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const int c = 16 * a + g + 4 * s, i = 16 * b + j;
-      if (i < n && c < n) Vg[i + (int64_t)n * c] = x[s];
-    }
+      for (int s = 0; s < 4; s++) {
+        const int c = 16 * a + g + 4 * s, i = 16 * b + j;
+        if (i < n && c < n) Vg[i + (int64_t)n * c] = v[u][s];
+      }
   }
   for (int e = tid; e < n * (n - W); e += kJThreads) Vg[(int64_t)n * W + e] = 0.0;
 }
@@ -486,15 +542,16 @@ k_jacobi(const int* __restrict__ nq, const int* __restrict__ kq, int drop, const
   // (even: R's scale is a power of two as well)
   const int ex = __builtin_amdgcn_frexp_exp(wave_all(fabs(dg), [](double a, double b) { return fmax(a, b); })) & ~1;
   int r = 0;
+  double rem[8] = {};
   if (kq && n > 16) {
     int good;
-    r = jac_cholesky(L, n, G0, __builtin_amdgcn_ldexp(dg, -ex), ex, wave, lane, good);
+    r = jac_cholesky(L, n, G0, __builtin_amdgcn_ldexp(dg, -ex), ex, wave, lane, good, rem);
     if (!drop && good < kq[q]) r = 0;
   }
   const int w = r ? r : n;
-  if (w <= 16) jacobi_sector<1>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
-  else if (w <= 32) jacobi_sector<2>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
-  else jacobi_sector<4>(L, n, r, ex, G0, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  if (w <= 16) jacobi_sector<1>(L, n, r, ex, G0, rem, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else if (w <= 32) jacobi_sector<2>(L, n, r, ex, G0, rem, Vg, ev, max_sweeps, floor_rel, wave, lane);
+  else jacobi_sector<4>(L, n, r, ex, G0, rem, Vg, ev, max_sweeps, floor_rel, wave, lane);
 }
 
 // 4b. Sectors larger than kJacBlockMin: two-sided block Jacobi.  The padded
@@ -1095,7 +1152,8 @@ __global__ void __launch_bounds__(kJThreads) k_pchol_panel(const PcSector* ps, c
   double least = T.least;
   bool small = nc == 0;
   int order;
-  const int ks = cholesky64(x, dc, real, nc, s_r, s_row, wave, lane, order, [&](int k, double m) {
+  bool open = real;
+  const int ks = cholesky64(x, dc, open, nc, s_r, s_row, wave, lane, order, [&](int k, double m) {
     small = !(m > tol);
     if (small || m < kPcLoose * next) return true;
     if (k0 + k < P.kq) least = fmin(least, m);
