@@ -986,9 +986,12 @@ static int block_jacobi(const std::vector<int>& big, const std::vector<int>& nq,
 // step in the order of the eigenvalues makes that 2e-15 (1e-12 before).  The
 // n - r null-space columns are left zero with eigenvalue 0: a zero singular value
 // is never kept when cutoff > 0 (qtensor_op.cpp:1294-1300).  Without a cutoff
-// the rule is that of the small sectors (4): the r columns cover the kq
-// values asked for and no pivot among them is below kLrCond of the largest
-// diagonal; otherwise the sector's Gram matrix is formed again and solved by block Jacobi.
+// the rule is: the r columns cover the kq values asked for, and no pivot among them
+// is below kLrCond of the largest diagonal, or kLrCondOpen when the factorisation
+// leaves indices out (r < n: nothing corrects for the remainder here); otherwise the sector's
+// Gram matrix is formed again and solved by block Jacobi.  The smallest singular values of
+// 130 x 65 and 600 x 300 sectors were off by 6e-15 and 8e-14 of the largest (block Jacobi:
+// 4e-14, 2e-13) with pivots from 2e-4, by 6e-14 and 3e-13 from 3e-6, and by 2e-12 from 1e-7.
 // (A site of m = 701: 11 sweeps of 5 rounds on G, 7 of 3 on G', 2600 to 1870 us.)
 // R is stored by original column index (row k of R at k n + j), so neither
 // G' nor V needs the permutation.
@@ -1050,6 +1053,7 @@ __global__ void __launch_bounds__(kPcThreads) k_pchol_init(const PcSector* ps, c
 // and 16 updates of 14.1, before 9 of 69.3 and 9 of 12.2.
 constexpr int kPcMaxN = 8181;          // largest sector (the remaining diagonal is held in LDS)
 constexpr double kPcLoose = 0.125;
+constexpr double kLrCondOpen = 1e-4;
 // state of one panel for the update: column k of the substitution at L[64 k ..]
 // (elements t > k, and 1 / the diagonal at k)
 constexpr int kPcL = kPcNbMax * kPcNbMax;
@@ -1811,7 +1815,8 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
   for (int li = 0; li < ns; li++) {
     TTG_REQUIRE(pst[li].rank >= 0, "svd: the pivoted Cholesky factorisation did not end");
     int r = pst[li].rank;
-    if (!drop && (r < ps[li].kq || pst[li].least < kLrCond * pst[li].dmax)) {
+    const double cond = r < ps[li].n ? kLrCondOpen : kLrCond;
+    if (!drop && (r < ps[li].kq || pst[li].least < cond * pst[li].dmax)) {
       plain.push_back(big[li]);
       r = 0;
     }

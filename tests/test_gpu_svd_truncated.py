@@ -1,8 +1,8 @@
-"""Truncated SVD (ttg_svd) of small sectors whose singular values fall by many decades,
-so that the values at the cutoff are near the rounding of the Gram matrix: the kept
-part of a sector against numpy's SVD of the sector itself.
+"""Accuracy of the sector SVD (ttg_svd) where singular values fall by many decades, so that
+those at the cutoff, or the smallest, are near the rounding of the Gram matrix: factors
+and values against numpy's SVD of the sector itself.
 
-Tolerance.  The rounding dG of the Gram matrix mixes the kept singular vectors c with the
+Tolerance of the kept part.  The rounding dG of the Gram matrix mixes the kept singular vectors c with the
 left-out ones d by K = u_c^T dG u_d / (lambda_c - lambda_d) to first order, which moves the kept
 part by sqrt(sum K^2 (sigma_c^2 + sigma_d^2)).  That is computed here from the Gram matrix that
 numpy rounds (against 80-bit arithmetic).  The device's is rounded by as much, and an
@@ -65,3 +65,28 @@ def test_kept_part(direction, decades):
             ratios.append(off / rounding_effect(m.T, V.T, S, p))
         assert np.linalg.norm(iso.T @ iso - np.eye(p), 2) < 1e-13, (n, c, p)
     assert np.exp(np.mean(np.log(ratios))) < 2.0
+
+
+@pytest.mark.parametrize("n,c", [(40, 20), (64, 50), (130, 65), (300, 150), (300, 200)])
+@pytest.mark.parametrize("decades", [2, 3.5, 3.9])
+def test_values_of_sectors_with_a_null_space(n, c, decades):
+    """more rows than columns, no cutoff: the singular values down to the smallest, whose
+    squares are near 1e-8 of the largest.  The Gram matrix's rounding moves a value by
+    u_c^T dG u_c / (2 sigma_c), and an iteration of some eight sweeps that rounds it anew in each
+    by eight times that; the largest values by the n roundings of each sweep, halved by the root"""
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        u, v = (np.linalg.qr(rng.standard_normal((x, c)))[0] for x in (n, c))
+        m = (u * np.logspace(0, -decades, c)) @ v.T
+        i = make_index(INWARD, "i", LINK, 0, [((0, 0), n)])
+        j = make_index(OUTWARD, "j", LINK, 0, [((0, 0), c)])
+        A = T.DTensor.from_flat(FlatTensor([i, j], np.array([[0, 0]], np.int32), m.reshape(-1, order="F")))
+        h = [C.c_void_p() for _ in range(3)]
+        T.check(T.lib().ttg_svd(A.h, 1, T.MOVE_FROM_LEFT, 0.0, 0, C.byref(h[0]), C.byref(h[1]), C.byref(h[2]),
+                                C.byref(C.c_double(0)), C.byref(C.c_int64(0))))
+        _, s, _ = (T.DTensor(x, []).data() for x in h)
+        U, S, _ = np.linalg.svd(m, full_matrices=False)
+        x = m.astype(np.longdouble)
+        dg = (m @ m.T - x @ x.T).astype(float)
+        moved = np.abs(np.einsum("ic,ij,jc->c", U, dg, U) / (2 * S)).max()
+        assert np.abs(s - S).max() < 8 * moved + 8 * n * 2.0 ** -53 / 2, (seed, moved)
