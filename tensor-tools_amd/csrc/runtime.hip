@@ -34,6 +34,7 @@ struct Pool {
   size_t in_use = 0, peak = 0, cached = 0;
   size_t budget = SIZE_MAX;
   int64_t fail_at = 0;   // > 0: the fail_at-th request from now is refused (tests)
+  uint64_t refused = 0;  // requests refused so far
 } g_pool;
 
 // hand every cached buffer back to HIP (after the device is idle: a buffer
@@ -56,8 +57,11 @@ size_t size_class(size_t b) {
 }
 }  // namespace
 
+uint64_t pool_refusals() { return g_pool.refused; }
+
 void* dmalloc(size_t bytes) {
   if (g_pool.fail_at > 0 && --g_pool.fail_at == 0) {
+    g_pool.refused++;
     set_error("device allocation of " + std::to_string(bytes) + " bytes refused (injected failure)");
     return nullptr;
   }
@@ -72,6 +76,7 @@ void* dmalloc(size_t bytes) {
   } else {
     if (g_pool.in_use + g_pool.cached + sz > g_pool.budget) release_cache();
     if (g_pool.in_use + sz > g_pool.budget) {
+      g_pool.refused++;
       set_error("device allocation of " + std::to_string(sz) + " bytes refused: " +
                 std::to_string(g_pool.in_use >> 20) + " MiB live, budget " + std::to_string(g_pool.budget >> 20) +
                 " MiB (device memory less a reserve for the HIP runtime)");
@@ -85,6 +90,7 @@ void* dmalloc(size_t bytes) {
       release_cache();
       if (hipMalloc(&p, sz) != hipSuccess) {
         (void)hipGetLastError();
+        g_pool.refused++;
         set_error("device allocation of " + std::to_string(sz) + " bytes failed");
         return nullptr;
       }

@@ -2051,10 +2051,13 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   std::vector<int> plain, lr;
   for (int q : big) (cutoff > 0 || nq[q] <= kPcMaxN ? lr : plain).push_back(q);
   if (!lr.empty()) {
+    const std::string last = ttg_last_error();
+    const uint64_t refused = pool_refusals();
     brc = lr_eigen(lr, nq, kq, cutoff > 0, plain, goff, eoff, d_eoff, goff[nQ], G, Vev, ev, s);
-    if (brc && !(cutoff > 0)) {   // (no room for its arrays, say)
+    if (brc && !(cutoff > 0) && pool_refusals() != refused) {   // no room for its arrays
       plain = big;
       brc = 0;
+      set_error(last);
     }
   }
   if (!brc && !plain.empty()) {

@@ -134,6 +134,8 @@ int d2h_wait(const D2HPiece* pieces, int n);
 constexpr size_t kAllocTail = 16;
 void* dmalloc(size_t bytes);
 void dfree(void* p);
+// requests refused so far (a call that failed while the number rose failed for that)
+uint64_t pool_refusals();
 template <class T>
 T* dalloc(size_t n) { return (T*)dmalloc(n * sizeof(T) + (n == 0 ? 8 : 0)); }
 
