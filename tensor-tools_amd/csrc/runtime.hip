@@ -65,7 +65,7 @@ void* dmalloc(size_t bytes) {
     set_error("device allocation of " + std::to_string(bytes) + " bytes refused (injected failure)");
     return nullptr;
   }
-  size_t sz = size_class(bytes + kAllocTail);
+  size_t sz = size_class(bytes);
   auto it = g_pool.free_list.lower_bound(sz);
   void* p = nullptr;
   if (it != g_pool.free_list.end() && it->first <= sz + sz / 4) {
@@ -82,13 +82,15 @@ void* dmalloc(size_t bytes) {
                 " MiB (device memory less a reserve for the HIP runtime)");
       return nullptr;
     }
-    if (hipMalloc(&p, sz) != hipSuccess) {
+    // the tail lies behind the class: counted in it, a request that is a class itself (a
+    // power of two, say) would take the next one, up to 25% more
+    if (hipMalloc(&p, sz + kAllocTail) != hipSuccess) {
       // release cached buffers and retry once.  The failure is handled here,
       // so it is cleared from the runtime's last-error state: the next
       // launch check (hipGetLastError) would otherwise report it.
       (void)hipGetLastError();
       release_cache();
-      if (hipMalloc(&p, sz) != hipSuccess) {
+      if (hipMalloc(&p, sz + kAllocTail) != hipSuccess) {
         (void)hipGetLastError();
         g_pool.refused++;
         set_error("device allocation of " + std::to_string(sz) + " bytes failed");
