@@ -184,6 +184,9 @@ int copy_add(CopyList& l, void* dst, const void* src, size_t bytes) {
 constexpr size_t kRingBytes = size_t(8) << 20;
 // above this a copy to or from the host is left to the runtime
 constexpr size_t kCopyKernelMax = size_t(256) << 10;
+// and above this one on the device: 64 MB take 19.8 us either way, 128 MB 38 us by the
+// runtime and 42 by k_copy, 800 MB 305 and 349
+constexpr size_t kDevCopyMax = size_t(64) << 20;
 struct Ring {
   char* p = nullptr;
   size_t off = 0;
@@ -254,7 +257,13 @@ int h2d_pieces(void* dst, const H2DPiece* pieces, int n) {
 
 int dev_copy(const DevPiece* pieces, int n) {
   CopyList l;
-  for (int i = 0; i < n; i++) TTG_TRY(copy_add(l, pieces[i].dst, pieces[i].src, pieces[i].bytes));
+  for (int i = 0; i < n; i++) {
+    const DevPiece& p = pieces[i];
+    if (p.bytes > kDevCopyMax)
+      TTG_HIP(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToDevice, g_rt.stream));
+    else
+      TTG_TRY(copy_add(l, p.dst, p.src, p.bytes));
+  }
   return copy_launch(l);
 }
 
