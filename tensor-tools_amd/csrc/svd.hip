@@ -233,6 +233,7 @@ constexpr double kPcTol = 1e-15;      // a remaining diagonal below this of the 
 constexpr double kLrFix = 1e-12;      // least eigenvalue (of the largest) whose vector is corrected for the remainder
 constexpr double kLrCutoff = 10 * kLrFix;
 constexpr double kLrCond = 1e-8;
+constexpr int kSvdMaxN = 8192;        // largest sector
 
 // LDS of k_jacobi
 struct JacLds {
@@ -1051,7 +1052,8 @@ __global__ void __launch_bounds__(kPcThreads) k_pchol_init(const PcSector* ps, c
 // step, by one workgroup, it was 2.5 us, whether the pivot's column came from
 // memory or from LDS.  Sectors of up to 388 rows (m = 1500, rank 248): 16 panels of 20.1 us
 // and 16 updates of 14.1, before 9 of 69.3 and 9 of 12.2.
-constexpr int kPcMaxN = 8181;          // largest sector (the remaining diagonal is held in LDS)
+// the remaining diagonal is held in LDS, beside 39 KB of fixed size
+static_assert(sizeof(double) * kSvdMaxN + 40 * 1024 <= 160 * 1024, "the largest sector's diagonal fits");
 constexpr double kPcLoose = 0.125;
 constexpr double kLrCondOpen = 1e-4;
 // state of one panel for the update: column k of the substitution at L[64 k ..]
@@ -1772,7 +1774,6 @@ static int lr_eigen(const std::vector<int>& big, const std::vector<int>& nq, con
     dtot += nq[q];
     nmax = std::max(nmax, nq[q]);
   }
-  TTG_REQUIRE(nmax <= kPcMaxN, "svd: sector too large for the pivoted Cholesky panel");
   const size_t lds = sizeof(double) * nmax;
   Scratch sc;
   PcSector* d_ps = sc.get<PcSector>(ns);
@@ -1953,7 +1954,7 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   std::vector<int> nq(nQ), kq(nQ);
   for (int q = 0; q < nQ; q++) {
     const int64_t n = fromLeft ? rows[q] : cols[q];
-    TTG_REQUIRE(n <= 8192, "svd: sector larger than 8192");
+    TTG_REQUIRE(n <= kSvdMaxN, "svd: sector larger than 8192");
     nq[q] = (int)n;
     int kd = (int)std::min(rows[q], cols[q]);
     kq[q] = K > 0 ? (int)std::min<int64_t>(K, kd) : kd;   // rank-K SVD per sector
@@ -2048,12 +2049,11 @@ extern "C" int ttg_svd(ttg_tensor A, int nleft, int direction, double cutoff, in
   // large sectors: the LR step, and without a cutoff (every value is kept) block
   // Jacobi on G, formed again, for those it cannot serve
   int brc = 0;
-  std::vector<int> plain, lr;
-  for (int q : big) (cutoff > 0 || nq[q] <= kPcMaxN ? lr : plain).push_back(q);
-  if (!lr.empty()) {
+  std::vector<int> plain;
+  if (!big.empty()) {
     const std::string last = ttg_last_error();
     const uint64_t refused = pool_refusals();
-    brc = lr_eigen(lr, nq, kq, cutoff > 0, plain, goff, eoff, d_eoff, goff[nQ], G, Vev, ev, s);
+    brc = lr_eigen(big, nq, kq, cutoff > 0, plain, goff, eoff, d_eoff, goff[nQ], G, Vev, ev, s);
     if (brc && !(cutoff > 0) && pool_refusals() != refused) {   // no room for its arrays
       plain = big;
       brc = 0;
