@@ -740,8 +740,10 @@ __device__ __forceinline__ void plan_scan(ScanLds& L, const BlkStat* stat, int T
 // loads.  What bounds it is that chain: four loads that miss (q group, tuple, blocks of A
 // and of B), 20000 cycles with the launch, the records written, 15000 for the scan.  The
 // workgroup that finishes last goes on with the scan, for `fuse` blocks or fewer (16.9 us at
-// 170 blocks for both; 15.8 and 9.1 as two kernels, and the gap between them); a
-// longer list goes to k_plan_scan's 1024 threads.
+// 170 blocks for both; 15.8 and 9.1 as two kernels, and the gap between them): kPlanFuse
+// of them when the host has read the count, and whatever a plan of one wait comes
+// to (kPlanPairs), as the host does not know it.  A longer list goes to k_plan_scan's
+// 1024 threads.
 constexpr int kPlanStageB = 4096;
 constexpr int kPlanGrid = 512;      // most workgroups of k_plan_blocks
 constexpr int64_t kPlanFuse = 2048;
@@ -1307,7 +1309,8 @@ int plan_build(const MetaPtr& A, const MetaPtr& B, int np, const int* pa, const 
     so.seg[j] = m.d_idx + 3 * m.idx_off[k];
     so.len[j] = 3 * m.nsec[k];
   }
-  // the scan by the last workgroup, unless a table of this size wants more threads
+  // the scan by the last workgroup, unless a table of this size wants more threads (in a
+  // plan of one wait nbcap is only a bound, mostly far above the count)
   const bool fused = nbcap <= kPlanFuse || one_wait;
   hipLaunchKernelGGL(k_plan_blocks, dim3((unsigned)std::min<int64_t>((nbcap + 3) / 4, kPlanGrid)), dim3(256),
                      stage_b ? sizeof(uint64_t) * nB : 0, s, va, vb, w, stage_b, d_hdr, stat, C->d_qi,
