@@ -202,11 +202,11 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // LDS until a sweep holds no significant rotation: |a_pq| above 1e-12 of
 // sqrt(a_pp a_qq) (an off-diagonal d moves eigenvalues by ~d^2 / gap, so
 // the eigenvalues are exact to ~1e-24 relative) and above 1e-14 of the
-// largest diagonal.  Below that floor
-// a rotation moves no eigenvalue by more than 1e-14 of the largest (singular
-// values below 1e-7 of the largest, under the Gram matrix's own resolution of
-// ~sqrt(eps)), and the rounding noise in the null space of a rank-deficient
-// sector's Gram matrix never passes the relative test alone.
+// largest diagonal, and then for up to kJacExtra sweeps without that floor, until
+// one holds none by the relative test alone.  (The rounding noise in the null space of a
+// rank-deficient sector's Gram matrix never passes the relative test alone.  A
+// graded matrix, as a site's whose columns carry the singular values of its
+// neighbour, has small singular values that are no noise.)
 //
 // Sectors of more than 16 rows go through a pivoted Cholesky factorisation
 // P^T G P = R^T R first (as the large ones, 4c): the iteration then runs on
@@ -376,18 +376,24 @@ __device__ __forceinline__ void jacobi_sector(JacLds& L, int n, int r, int ex, c
     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
     if (lane == 0) L.dmax = m;
   }
-  int par = 0;
+  int par = 0, extra = 0;
+  double floor_abs = -1.0;
   for (int sweep = 0; sweep < max_sweeps; sweep++) {
     if (tid == 0) L.sig = 0;
     __syncthreads();
-    jac_sweep<NPR>(S, L.qts, vt, wave, lane, par, floor_rel * L.dmax, &L.sig);
+    if (sweep == 0) floor_abs = floor_rel * L.dmax;
+    jac_sweep<NPR>(S, L.qts, vt, wave, lane, par, floor_abs, &L.sig);
     __syncthreads();
     // every thread reads the flag before thread 0 may clear it for the next
     // sweep: the barrier between the read and the reset keeps the decision
     // uniform over the workgroup
     const int rotated = L.sig;
     __syncthreads();
-    if (!rotated) break;
+    if (extra ? !rotated || extra == kJacExtra : !rotated && floor_abs == 0.0) break;
+    if (extra || !rotated) {   // the floor's own end: without it from here
+      floor_abs = 0.0;
+      extra++;
+    }
   }
   if (r == 0) {
     for (int i = tid; i < n; i += kJThreads) ev[i] = __builtin_amdgcn_ldexp(S[i * kJP + i], ex);
@@ -567,8 +573,9 @@ k_jacobi(const int* __restrict__ nq, const int* __restrict__ kq, int drop, const
 // so a round moves G and V through memory once instead of once per scalar
 // rotation.  A sweep (nbk - 1 rounds) leaves a sector active while any
 // subproblem held an off-diagonal element above 1e-12 sqrt(g_ii g_jj) and
-// above the sector's floor, 1e-14 of the largest diagonal.  A subproblem
-// with nothing to rotate leaves Q_IJ = I and marks its pair unrotated; the
+// above the sector's floor, 1e-14 of the largest diagonal, and for up to kJacExtra
+// sweeps more while some are above the relative test.  A subproblem with
+// none leaves Q_IJ = I and marks its pair unrotated; the
 // tile products of a round skip the tiles whose pairs were both unrotated.
 constexpr int kJacBlockMin = kJW;
 constexpr int kBJ = 32;                // block width; subproblems are 2 kBJ
@@ -633,7 +640,7 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
              int* rotated, const double* Gp, double* Qp) {
   __shared__ __attribute__((aligned(16))) double lds[kJLds];
   __shared__ int perm[kSub], cnt[kSub];
-  __shared__ int sig;
+  __shared__ int sig, sweep_sig;   // (the sweep's own flag: sig is the test's before it)
   const int2 it = items[blockIdx.x];
   const int li = it.x, k = it.y;
   const BJSector S = sec[li];
@@ -669,18 +676,20 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
   }
   __syncthreads();
   {
-    // significance test of this subproblem (before rotating):
-    // |v| > 1e-12 sqrt(g_pp g_qq), compared squared; thread t's columns p are
-    // all t % 64 (so one diagonal load), its rows q = t / 64 + 8 i
+    // significance test of this subproblem (before rotating), bit 0: |v| > 1e-12
+    // sqrt(g_pp g_qq), compared squared, bit 1: above the floor as well; thread t's
+    // columns p are all t % 64 (so one diagonal load), its rows q = t / 64 + 8 i
     const int p = tid % kSub;
     const double gpp = M[p * kJP + p];
-    bool any = false;
+    bool any = false, big = false;
     for (int q = tid / kSub; q < kSub; q += kJThreads / kSub) {
       if (p == q) continue;
       const double v = M[q * kJP + p];
-      any |= v * v > (kJacRel * kJacRel) * fabs(gpp * M[q * kJP + q]) && fabs(v) > S.floor;
+      const bool here = v * v > (kJacRel * kJacRel) * fabs(gpp * M[q * kJP + q]);
+      any |= here;
+      big |= here & (fabs(v) > S.floor);
     }
-    if (any) sig = 1;
+    if (any) atomicOr(&sig, big ? 3 : 1);
   }
   __syncthreads();
   double* Qg = Qp + S.qp + (int64_t)k * kSub * kSub;   // column-major 64 x 64
@@ -690,13 +699,13 @@ k_bjac_solve(const BJSector* sec, const int2* items, int nitems, int r, const in
     return;
   }
   if (tid == 0) {
-    atomicOr(&flag[li], 1);
+    atomicOr(&flag[li], sig);
     rotated[blockIdx.x] = 1;
   }
   double vt[8][2];
   jac_identity<4>(vt, wave, lane);
   int par = 0;
-  jac_sweep<4>(M, Qts, vt, wave, lane, par, S.floor, &sig);
+  jac_sweep<4>(M, Qts, vt, wave, lane, par, S.floor, &sweep_sig);
   // Eigenpairs in descending order (the larger values to the pair's lower
   // block): a fixed order keeps values from swapping between blocks from
   // round to round, which otherwise holds the outer iteration at a linear rate.
@@ -862,7 +871,8 @@ __global__ void __launch_bounds__(256) k_bjac_apply(const BJSector* sec, const i
   }
 }
 
-// end of an outer sweep: a sector stays active while its sweep rotated
+// end of an outer sweep: a sector stays active (1) while its sweep rotated
+// anything above the floor, then (2, 3, ..) for kJacExtra sweeps while it rotates
 // anything; the flags start over for the next sweep; *any = some sector active
 __global__ void __launch_bounds__(256) k_bjac_sweep_end(int nsec, int* flag, int* act, int* any) {
   __shared__ int s_any;
@@ -870,10 +880,11 @@ __global__ void __launch_bounds__(256) k_bjac_sweep_end(int nsec, int* flag, int
   __syncthreads();
   int a = 0;
   for (int li = threadIdx.x; li < nsec; li += blockDim.x) {
-    const int f = flag[li];
-    act[li] = f;
+    const int f = flag[li], was = act[li];
+    const int now = !f || was == 0 ? 0 : was == 1 ? (f & 2 ? 1 : 2) : was < 1 + kJacExtra ? was + 1 : 0;
+    act[li] = now;
     flag[li] = 0;
-    a |= f;
+    a |= now;
   }
   if (a) atomicOr(&s_any, 1);
   __syncthreads();
