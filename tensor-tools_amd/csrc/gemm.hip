@@ -30,8 +30,8 @@
 // row l%16, and a column of C is stored by 16 consecutive lanes.
 //
 // What bounds the FP64 kernel (m=8192 and m=2048 H_eff operators): the FP64
-// matrix cores, busy for 55-70% of a launch, plus padding to 16 x 16 fragments
-// (6% and 25% more products).  Against the kernel this one replaced (8-byte
+// matrix cores, busy for 62-71% and 38-50% of a launch (counters, on the shapes that
+// operators take), padding to 16 x 16 fragments included (6% and 25% more products).  Against the kernel this one replaced (8-byte
 // loads and [row][k] LDS tiles for every operand, a persistent grid with one
 // run of items per workgroup, padding to the whole tile), stage times, FP64:
 // m=8192 2.56 -> 1.9 and 2.51 -> 1.8 ms (98 and 81 GFLOP), m=2048 70 -> 57 and
@@ -66,9 +66,10 @@ static dim3 item_grid(int nitems) {
 // k, copied from the operand's block to LDS.  A staging slot is 16 bytes: V
 // consecutive rows at one k (RC: rows contiguous in memory) or V consecutive k
 // of one row, and the LDS tile keeps that direction ([k][row] or [row][k]), so a
-// slot is stored as it was loaded and neither the stores nor the fragment reads
-// meet bank conflicts (with [row][k] for both, two thirds of the LDS cycles of a
-// row-contiguous operand were conflicts, and the LDS was 77% busy).
+// slot is stored as it was loaded.  Bank conflicts are 9-21% of the LDS cycles with a
+// k-contiguous B and none otherwise, with the LDS 17-35% busy at m=2048 (with [row][k]
+// for both operands, two thirds of the LDS cycles of a row-contiguous one were
+// conflicts, and the LDS was 77% busy).
 // 8-byte loads take the vector memory path as long as 16-byte ones (15 cycles
 // per wave instruction and CU, whatever the alignment and the segments: 33
 // against 67 bytes per cycle).  A 16-byte load needs dword alignment only; at

@@ -941,6 +941,9 @@ namespace ttg {
 //           element including the hi/lo split) plus fragment loads and loop,
 //   lat   = global-load latency (kLatency) shared by the occ workgroups a CU
 //           keeps resident (occupancy of the actual kernel instantiation).
+// (6 per FP64/FP32 element is what 8-byte loads took; with the kernel's 16-byte slots it
+// takes fewer, so the model sees the wide shapes a little dearer than they are.  The shapes
+// 96x64 and 64x96 are not in it: operators time them, tune_stage.)
 // A CU retires one workgroup k-tile per max(mfma, issue, lat / occ) cycles;
 // each work item adds its first load and its epilogue.  The launch takes
 // max(total work over the CUs, the longest item after split-K run at the

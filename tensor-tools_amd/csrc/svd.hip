@@ -216,12 +216,12 @@ __global__ void k_svd_gather(MetaView A, int nleft, const double* __restrict__ a
 // (2e-15 where the rotations alone gave 2e-14).  The matrix stays in the registers of the
 // 8 waves (8 rows each), every wave keeps the remaining diagonal and finds the pivot for
 // itself, and one row a step passes through LDS.  On the sectors of an m = 100 state (up to 60
-// rows, rank-deficient) k_jacobi took 445 us and takes 94, at m = 333 531 and 249.
+// rows, rank-deficient) k_jacobi took 445 us and takes 95, at m = 333 531 and 250.
 // Why the correction: the remainder's diagonal is below kPcTol = 4.5 roundings of the
 // largest, and left out it moved the vectors near a cutoff of 1e-9 more than the rounding
 // of the Gram matrix does: the factors of states of m = 40 to 200 were off by 0.80e-12
 // (of the state's norm, geometric mean over 160 states) where the plain iteration's are by
-// 0.54e-12; with it they are by 0.29e-12, and k_jacobi takes 94 us at m = 100 instead of 89.
+// 0.54e-12; with it they are by 0.29e-12, and k_jacobi takes 95 us at m = 100 instead of 89.
 // The route is taken when the r columns are all that the selection can use, and all above
 // kLrFix of the largest: r >= kq, the values kept before truncation, with no pivot among
 // them below kLrCond of the largest diagonal, or a cutoff above kLrCutoff.  (A cutoff c

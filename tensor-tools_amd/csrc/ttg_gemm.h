@@ -1,4 +1,5 @@
-// ttg_gemm.h -- device pieces shared by the grouped GEMM kernels.
+// ttg_gemm.h -- device pieces of the grouped GEMM kernels (gemm.hip): MFMA forms,
+// k walk, operand loads.
 #pragma once
 #include "ttg_internal.h"
 #include "ttg_plan.h"
